@@ -71,6 +71,26 @@ def test_q4g32_encode_bit_exact_and_round_trip(ops, u, oracle, N, K):
     assert np.all(np.abs(deq - Wf.astype(np.float64)) <= 0.5 * step * 1.01 + 1e-7)
 
 
+@pytest.mark.parametrize("N,K", [(1, 32), (3, 32), (129, 256), (7, 4128)])
+@pytest.mark.parametrize("top", [7.0, 1e-4, 7 * 2.0**-17, 65504.0])
+def test_q4g32_encode_halves_and_ragged_sizes(ops, u, oracle, N, K, top):
+    """Quotients that are halves exactly, and the fp16 numbers on either side of them: the codes stay exact."""
+    rng = np.random.default_rng(N * K)
+    Wf = np.zeros((N, K // 32, 32), dtype=np.float16)
+    Wf[..., 0] = np.float16(top)
+    scale = np.float16(max(float(np.float16(top)), 1e-4) / 7)
+    halves = (rng.integers(-7, 7, size=(N, K // 32, 31)) + 0.5) * np.float64(scale)
+    Wf[..., 1:] = np.clip(halves.astype(np.float16), -np.float16(top), np.float16(top))
+    pick = rng.integers(0, 3, size=Wf.shape)
+    near = np.where(pick == 1, np.nextafter(Wf, np.float16(0)), Wf)
+    Wf[..., 1:] = near[..., 1:]
+    Wf = Wf.reshape(N, K)
+    W, S = ops.q4g32_encode(u.dev(Wf))
+    W_ref, S_ref = oracle.q4g32_encode(Wf)
+    np.testing.assert_array_equal(u.host(W).view(np.uint32), W_ref)
+    np.testing.assert_array_equal(u.host(S).view(np.uint16), S_ref.view(np.uint16))
+
+
 @pytest.mark.parametrize("nbit,group_size", [(8, -1), (4, -1), (8, 64), (4, 64)])
 def test_encode_preprocess_gemm_chain_vs_unquantized(ops, u, oracle, nbit, group_size):
     """x @ w^T through the quantized path agrees with the unquantized fp16 product to the accuracy the
