@@ -2,6 +2,7 @@
 #ifndef RELAX_AMD_CSRC_INTB_COMMON_H_
 #define RELAX_AMD_CSRC_INTB_COMMON_H_
 
+#include "gemm_epilogue.h"
 #include "wq_device.h"
 #include "wq_host.h"
 
@@ -36,9 +37,15 @@ int intb_small_batch_dispatch(const uint16_t* A, const int8_t* B, const uint16_t
 struct IntbGemmEpilogue {
   IntbEpilogue e;
   int N;
+  // silu and gelu: bias and activation in a pass of their own (gemm_epilogue.h), relu with the store
+  __device__ bool activates() const { return e.activation >= 2; }
+  __device__ float column_bias(int n) const { return e.bias && !e.bias_stride ? (float)e.bias[n] : 0.0f; }
+  __device__ float activate(float v, float column_bias, int m, int n) const {
+    if (e.bias) v += e.bias_stride ? (float)e.bias[(int64_t)m * e.bias_stride + n] : column_bias;
+    return apply_activation(v, e.activation);
+  }
   __device__ half_t operator()(float v, int m, int n) const {
-    if (e.bias) v += (float)e.bias[e.bias_stride ? (int64_t)m * e.bias_stride + n : n];
-    v = apply_activation(v, e.activation);
+    v = activate(v, column_bias(n), m, n);
     if (e.residual) {
       const float r = (float)e.residual[(int64_t)m * N + n];
       if (e.binary_op == 1) v += r;
@@ -47,29 +54,24 @@ struct IntbGemmEpilogue {
     if (e.unary_op == 1) v = v > 0.0f ? v : 0.0f;
     return (half_t)v;
   }
-  // Row-wise form for 8 consecutive columns n .. n+7 (n % 8 == 0): same arithmetic, 16-byte accesses.
-  // (identity and relu only: eight inlined erf / exp evaluations next to 256 live accumulators
-  // make the compiler spill; silu and gelu keep the element-wise form)
-  __device__ bool wide_ok(int n_cols, const half_t* y) const {
-    return e.activation <= 1 && n_cols % 8 == 0 && e.bias_stride % 8 == 0 &&
-           ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(e.bias) |
-             reinterpret_cast<uintptr_t>(e.residual)) & 15u) == 0;
-  }
+  // what is left to do after the activation pass (or all of it, where there is none), for 8 consecutive columns n .. n+7
   __device__ half8_t apply8(const float (&v)[8], int m, int n) const {
     float f[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) f[i] = v[i];
-    if (e.bias) {
-      const half8_t b = *reinterpret_cast<const half8_t*>(e.bias + (e.bias_stride ? (int64_t)m * e.bias_stride + n : n));
+    if (!activates()) {
+      if (e.bias) {
+        const half8_t b = *reinterpret_cast<const half8_any_t*>(e.bias + (e.bias_stride ? (int64_t)m * e.bias_stride + n : n));
 #pragma unroll
-      for (int i = 0; i < 8; ++i) f[i] += (float)b[i];
-    }
-    if (e.activation == 1) {
+        for (int i = 0; i < 8; ++i) f[i] += (float)b[i];
+      }
+      if (e.activation == 1) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) f[i] = f[i] > 0.0f ? f[i] : 0.0f;
+        for (int i = 0; i < 8; ++i) f[i] = f[i] > 0.0f ? f[i] : 0.0f;
+      }
     }
     if (e.residual) {
-      const half8_t r = *reinterpret_cast<const half8_t*>(e.residual + (int64_t)m * N + n);
+      const half8_t r = *reinterpret_cast<const half8_any_t*>(e.residual + (int64_t)m * N + n);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         if (e.binary_op == 1) f[i] += (float)r[i];

@@ -216,16 +216,13 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
   }
   const IntbGemmEpilogue gep{ep, (int)n};
   // the fully LDS-staged kernel under the tile shape (11, 17 or 18) whose rounds of the machine come out
-  // shortest; fine-grained scales whose pairs are not 4-byte aligned: the register-staged kernel (1..4).
-  // silu / gelu run the element-wise epilogue, whose inlined exp / erf code does not fit next to the 256
-  // accumulator registers of the 256x256 tile (11): they choose between the other two
+  // shortest; fine-grained scales whose pairs are not 4-byte aligned: the register-staged kernel (1..4)
   const bool lds_ok = !group || (reinterpret_cast<uintptr_t>(scales) & 3u) == 0;
   int cfg = wq_gemm_cfg_override();
   if (!cfg && !lds_ok) cfg = choose_gemm_cfg(m, n, false);
   if (!cfg) {
     double best = 0;
     for (int c : {17, 18, 11}) {
-      if (c == 11 && activation >= WQ_ACT_SILU) continue;
       const double t = lds_cfg_cost(c, m, n, cu_count());
       if (!cfg || t < best) cfg = c, best = t;
     }

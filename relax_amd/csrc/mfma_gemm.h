@@ -176,27 +176,10 @@ void wq_mfma_gemm_kernel(typename Loader::Args bargs, const half_t* __restrict__
   // ---- epilogue ----
   // Row-wise through LDS (gemm_epilogue.h): the activation buffers are idle after the last
   // barrier of the loop, and each wavefront stages in a piece of its own.
-  if (epilogue.wide_ok(N, Y)) {
-    using ECfg = RowwiseEpilogueCfg<TM, TN>;
-    static_assert(WM * WN * ECfg::kBytesPerWave <= Cfg::kLdsBytes, "epilogue staging exceeds the activation buffers");
-    store_tile_rowwise<Epilogue, TM, TN>(acc, epilogue, Y, M, N, m0 + wm * TM * 32, n0 + wn * TN * 32,
-                                         lds + wave * ECfg::kBytesPerWave, lane);
-    return;
-  }
-  // element-wise: accumulator register r of lane (j, h) is element (row 8*(r/4) + 4*h + r%4, col j)
-#pragma unroll
-  for (int t = 0; t < TN; ++t) {
-    const int n = n0 + (wn * TN + t) * 32 + lj;
-    if (n >= N) continue;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-        if (m < M) Y[(int64_t)m * N + n] = epilogue(acc[i][t][r], m, n);
-      }
-    }
-  }
+  using ECfg = RowwiseEpilogueCfg<TM, TN>;
+  static_assert(WM * WN * ECfg::kBytesPerWave <= Cfg::kLdsBytes, "epilogue staging exceeds the activation buffers");
+  store_tile_rowwise<Epilogue, TM, TN>(acc, epilogue, Y, M, N, m0 + wm * TM * 32, n0 + wn * TN * 32,
+                                       lds + wave * ECfg::kBytesPerWave, lane);
 }
 
 template <class Loader, class Epilogue, int TM, int TN, int WM, int WN, int WPE>

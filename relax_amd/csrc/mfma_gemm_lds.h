@@ -315,27 +315,10 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
   // ---- epilogue ----
   // Row-wise through LDS (gemm_epilogue.h); the ring is idle now: every real read of it was
   // waited for before the last barrier, and each wavefront stages in a piece of its own.
-  if (epilogue.wide_ok(N, Y)) {
-    using ECfg = RowwiseEpilogueCfg<TME, TN>;
-    static_assert(4 * ECfg::kBytesPerWave <= Cfg::kLdsBytes, "epilogue staging exceeds the ring");
-    store_tile_rowwise<Epilogue, TME, TN>(acc, epilogue, Y, M, N, m0 + wm * TME * 32, n0 + wn * TN * 32,
-                                          lds + wave * ECfg::kBytesPerWave, lane);
-    return;
-  }
-  // element-wise: accumulator register r of lane (j, h) is element (row 8*(r/4) + 4*h + r%4, col j)
-#pragma unroll
-  for (int t = 0; t < TN; ++t) {
-    const int n = n0 + (wn * TN + t) * 32 + lj;
-    if (n >= N) continue;
-#pragma unroll
-    for (int i = 0; i < TME; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + (wm * TME + i) * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-        if (m < M) Y[(int64_t)m * N + n] = epilogue(acc[i][t][r], m, n);
-      }
-    }
-  }
+  using ECfg = RowwiseEpilogueCfg<TME, TN>;
+  static_assert(4 * ECfg::kBytesPerWave <= Cfg::kLdsBytes, "epilogue staging exceeds the ring");
+  store_tile_rowwise<Epilogue, TME, TN>(acc, epilogue, Y, M, N, m0 + wm * TME * 32, n0 + wn * TN * 32,
+                                        lds + wave * ECfg::kBytesPerWave, lane);
 }
 
 // Row slices (1, 2 or 4; 8 where the policy carries the extra copy of the tile body, `fine`) that the tiles of

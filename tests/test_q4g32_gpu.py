@@ -304,3 +304,27 @@ def test_kn_layout_conversion_bit_exact_and_linear(ops, u, oracle, N, K):
         x = rng.standard_normal((3, K)).astype(np.float16)
         got = u.host(ops.q4g32_linear(W, S, u.dev(x)))
         u.assert_close(got, oracle.q4g32_kn_linear(W_kn, S_kn, x), f"kn linear {N}x{K}")
+
+
+@pytest.mark.parametrize("cfg", [4, 11, 17, 18])
+@pytest.mark.parametrize("N", [129, 134, 263])
+def test_gemm_row_ends_in_part_of_eight_columns(ops, u, oracle, cfg, N):
+    """Rows of y that start at any half's address; nothing before or behind y is written."""
+    import torch
+    from relax_amd import _lib
+
+    M, K = 70, 128
+    x, W, S = oracle.make_q4g32_inputs(M, N, K, seed=N)
+    rng = np.random.default_rng(N)
+    bias, res = rng.standard_normal(N).astype(np.float16), rng.standard_normal((M, N)).astype(np.float16)
+    ybuf = torch.zeros(M * N + 16, dtype=torch.float16, device="cuda")
+    _lib.lib().wq_debug_set_gemm_config(cfg)
+    try:
+        ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x), bias=u.dev(bias), residual=u.dev(res),
+                         out=ybuf[8:8 + M * N].view(M, N), kernel="gemm")
+    finally:
+        _lib.lib().wq_debug_set_gemm_config(0)
+    got = u.host(ybuf)
+    u.assert_close(got[8:8 + M * N].reshape(M, N), oracle.q4g32_linear(W, S, x, bias=bias, residual=res, nthreads=8),
+                   f"cfg {cfg} N={N}")
+    assert not got[:8].any() and not got[8 + M * N:].any()
