@@ -26,7 +26,7 @@
 //
 // A weight policy provides
 //   kColBytes            packed bytes per column and K-step (32 or 64)
-//   kScaleBytes          bytes of scales per column and K-step staged in LDS (4 or 0)
+//   kScaleBytes          bytes of scales per column and K-step staged in LDS (0, 4, or 8 as two planes of 4)
 //   Args, Frag, Scale    kernel arguments; a lane's packed codes of one column for one step; what
 //                        pair() needs besides the codes (the scale in both halves of a register,
 //                        plus the zero point where the format has one)
@@ -35,6 +35,9 @@
 //   s_src(args, n, K)    global address (step 0) of the 4 scale bytes of column n       (kScaleBytes > 0)
 //   s_offset(args, ks)   byte offset of step ks from there                              (kScaleBytes > 0)
 //   read_scale(p, lh)    Scale from the 4 staged bytes of a column, for lane half lh    (kScaleBytes > 0)
+//   s_src2(args, n, K)   the same for the second plane                                  (kScaleBytes == 8)
+//   read_scale2(p, plane, n, lh)   Scale from the 4 staged bytes of column n at p and those at p + plane
+//                                                                                       (kScaleBytes == 8)
 //   const_scale(args, n) the Scale of column n                                          (kScaleBytes == 0)
 //   read(frag, bslot, n_local, lh)   LDS -> registers
 //   pair(frag, kk, j, scale)   dequantized weights (k = 8kk + 2j, 8kk + 2j + 1) of the lane's column,
@@ -46,6 +49,8 @@
 //   phase_begin(scale, kk)     called once per column sub-tile in front of the phase that unpacks the weights
 //                              of MFMA kk: fetches what pair_finish_at needs for them
 //   pair_finish_at(bits, scale, j)   pair_finish for pair j of that MFMA
+// and, only where K may end with half a step (K % 64 == 32):
+//   half_step(args, n, k0, K, lh, out[2])   the weights k0 + 16c + 8lh .. + 7 of column n, c = 0, 1
 #ifndef RELAX_AMD_CSRC_MFMA_GEMM_LDS_H_
 #define RELAX_AMD_CSRC_MFMA_GEMM_LDS_H_
 
@@ -78,7 +83,7 @@ struct LdsGemmCfg {
   static constexpr int kALoads = BM / 32;   // direct loads per wavefront per step (64 chunks each)
   static constexpr int kBLoads = BN * Policy::kColBytes / 4096;
   static_assert(BN % 128 == 0 && BN <= 256, "B tile: 128 or 256 columns");
-  static constexpr int kSLoads = Policy::kScaleBytes ? 1 : 0;
+  static constexpr int kSLoads = Policy::kScaleBytes / 4;
   static constexpr int kLoadsPerStage = kALoads + kBLoads + kSLoads;
 };
 
@@ -93,6 +98,11 @@ template <class P, class = void>
 struct ScalePerK : std::false_type {};
 template <class P>
 struct ScalePerK<P, std::void_t<decltype(&P::phase_begin)>> : std::true_type {};
+
+template <class P, class = void>
+struct HalfStep : std::false_type {};
+template <class P>
+struct HalfStep<P, std::void_t<decltype(&P::half_step)>> : std::true_type {};
 
 typedef const void __attribute__((address_space(1))) * wq_gptr_t;
 typedef void __attribute__((address_space(3))) * wq_lptr_t;
@@ -149,8 +159,10 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
     b_src[i] = Policy::b_src(wargs, n0, (wave * Cfg::kBLoads + i) * 64 + lane, N, K);
   // scales staged per step (format A): 64 columns per wavefront (with BN = 128 wavefronts 2
   // and 3 repeat the loads of wavefronts 0 and 1)
-  const char* s_src = nullptr;
-  if (Cfg::kSLoads) s_src = Policy::s_src(wargs, min(n0 + (wave * 64) % Cfg::BN + lane, N - 1), K);
+  const char* s_src[2] = {nullptr, nullptr};
+  const int s_col = min(n0 + (wave * 64) % Cfg::BN + lane, N - 1);
+  if (Cfg::kSLoads) s_src[0] = Policy::s_src(wargs, s_col, K);
+  if constexpr (Cfg::kSLoads == 2) s_src[1] = Policy::s_src2(wargs, s_col, K);
 
   // direct load number idx (0 .. L-1) of step ks
   auto issue_one = [&](int ks, int idx) {
@@ -163,8 +175,9 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
       __builtin_amdgcn_global_load_lds((wq_gptr_t)(b_src[i] + (int64_t)ks * Policy::kStepStride),
                                        (wq_lptr_t)(slot + Cfg::kBOff + (wave * Cfg::kBLoads + i) * 1024), 16, 0, 0);
     } else {
-      __builtin_amdgcn_global_load_lds((wq_gptr_t)(s_src + Policy::s_offset(wargs, ks)),
-                                       (wq_lptr_t)(slot + Cfg::kSOff + (wave * 64 % Cfg::BN) * 4), 4, 0, 0);
+      const int i = idx - kALoadsE - Cfg::kBLoads;
+      __builtin_amdgcn_global_load_lds((wq_gptr_t)(s_src[i] + Policy::s_offset(wargs, ks)),
+                                       (wq_lptr_t)(slot + Cfg::kSOff + i * (Cfg::BN * 4) + (wave * 64 % Cfg::BN) * 4), 4, 0, 0);
     }
   };
 
@@ -188,7 +201,8 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
     for (int t = 0; t < TN; ++t) {
       const int n = (wn * TN + t) * 32 + lj;
       Policy::read(bw[t], slot + Cfg::kBOff, n, lh);
-      if (Cfg::kSLoads) bs[t] = Policy::read_scale(slot + Cfg::kSOff + n * 4, lh);
+      if constexpr (Cfg::kSLoads == 2) bs[t] = Policy::read_scale2(slot + Cfg::kSOff + n * 4, Cfg::BN * 4, n, lh);
+      else if (Cfg::kSLoads) bs[t] = Policy::read_scale(slot + Cfg::kSOff + n * 4, lh);
     }
   };
   auto read_a = [&](const unsigned char* slot, int kk, half8_t (&dst)[TME]) {
@@ -309,6 +323,26 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
       for (int t = 0; t < TN; ++t)
         bop[nxt][t] = half8_t{dq[t][0].x, dq[t][0].y, dq[t][1].x, dq[t][1].y,
                               dq[t][2].x, dq[t][2].y, dq[t][3].x, dq[t][3].y};
+    }
+  }
+
+  // ---- the last 32 k of a K that is no multiple of 64: two MFMAs per sub-tile straight from global memory.
+  // Once per tile, so it is not worth a place in the pipeline; the operands split k between the lane halves
+  // like the MFMA does (both alike, so any split gives the same sum). ----
+  if constexpr (HalfStep<Policy>::value) {
+    const int k0 = ksteps << 6;
+    half8_t b[TN][2];
+#pragma unroll
+    for (int t = 0; t < TN; ++t) Policy::half_step(wargs, min(n0 + (wn * TN + t) * 32 + lj, N - 1), k0, K, lh, b[t]);
+#pragma unroll
+    for (int i = 0; i < TME; ++i) {
+      const half_t* const a = X + (int64_t)min(m0 + (wm * TME + i) * 32 + lj, M - 1) * K + k0 + 8 * lh;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const half8_t av = *reinterpret_cast<const half8_t*>(a + 16 * c);
+#pragma unroll
+        for (int t = 0; t < TN; ++t) acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, b[t][c], acc[i][t], 0, 0, 0);
+      }
     }
   }
 

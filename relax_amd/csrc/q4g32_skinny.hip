@@ -1,6 +1,7 @@
 // Format A (q4f16_1) small-batch entry: the shared small-batch kernel with the
 // group-32 int4 weight policy.
 #include "q4g32_common.h"
+#include "q4g32_dispatch.h"
 #include "skinny_gemm.h"
 
 namespace wq {
@@ -47,6 +48,45 @@ struct Q4G32SkinnyPolicy {
     }
   }
 };
+
+// The same for K % 64 == 32 and an even N: a row of S holds an odd number of scales, so which half of the
+// aligned pair a scale is depends on the row as well.  (An odd N would have the pair of its very last scale end
+// past S.)
+struct Q4G32OddGroupsSkinnyPolicy : Q4G32SkinnyPolicy {
+  static constexpr bool kCanScaleBlock = false;
+  static constexpr bool kMaskTail = true;
+  struct Lane : Q4G32SkinnyPolicy::Lane {
+    int odd;  // parity of the row
+  };
+  __device__ __forceinline__ static void init(Lane& l, const Args& a, int n, int K, int N) {
+    Q4G32SkinnyPolicy::init(l, a, n, K, N);
+    l.odd = n & 1;
+  }
+  __device__ __forceinline__ static const char* s_addr(const Lane& l, int k0) {
+    return l.s + (k0 >> 5) * 2 - (((k0 >> 5) + l.odd) & 1) * 2;
+  }
+  __device__ __forceinline__ static const char* s_pair_addr(const Lane& l, int k0) { return s_addr(l, k0); }
+  // the lane's group is 4 * step + kq
+  __device__ __forceinline__ static half_t pick_scale(const Lane& l, half2_t pair, int kq) {
+    return ((kq + l.odd) & 1) ? pair.y : pair.x;
+  }
+};
+
+int q4g32_half_step_rows(const uint32_t* W, const uint16_t* S, const uint16_t* x, const uint16_t* bias,
+                         const uint16_t* residual, uint16_t* y, int64_t M, int64_t N, int64_t K,
+                         hipStream_t stream) {
+  if (M == 0) return WQ_OK;
+  WQ_REQUIRE(M > 0 && M <= WQ_SMALL_BATCH_MAX_M && K > 0 && K % 64 == 32 && q4g32_half_step_rows_ok(x, N),
+             "wq_q4g32_linear: M=%lld, N=%lld, K=%lld", (long long)M, (long long)N, (long long)K);
+  WQ_REQUIRE(W && S && x && y, "wq_q4g32_linear: null pointer");
+  WQ_REQUIRE(aligned16(W) && (reinterpret_cast<uintptr_t>(S) & 3u) == 0,
+             "wq_q4g32_linear: W must be 16-byte aligned, S 4-byte aligned");
+  WQ_REQUIRE(N < (1ll << 30) && K < (1ll << 30), "wq_q4g32_linear: too large");
+  const Q4G32OddGroupsSkinnyPolicy::Args pargs{W, (const half_t*)S};
+  const Q4G32Epilogue epi{(const half_t*)bias, (const half_t*)residual, (int)N};
+  return launch_skinny_auto<Q4G32OddGroupsSkinnyPolicy, Q4G32Epilogue>("wq_q4g32_linear", pargs, x, y, epi, M, N,
+                                                                       K, stream);
+}
 
 }  // namespace wq
 

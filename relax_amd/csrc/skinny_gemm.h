@@ -30,6 +30,8 @@
 #ifndef RELAX_AMD_CSRC_SKINNY_GEMM_H_
 #define RELAX_AMD_CSRC_SKINNY_GEMM_H_
 
+#include <type_traits>
+
 #include "tuning.h"
 #include "wq_device.h"
 #include "wq_host.h"
@@ -61,8 +63,16 @@ typedef void __attribute__((address_space(3))) * wq_sk_lptr_t;
 //   sblock_addr(lane, g)       address of scale g of the lane's column (g % 8 == 0)       (kCanScaleBlock)
 //   scale_block_ok(args, K)    host: every 8 scales of a column are 16 aligned bytes      (kCanScaleBlock)
 //   pair_aligned(args)         host: whether those pairs are 4-byte aligned
+// and, where K may end inside the two halves of a 64-k piece,
+//   kMaskTail                  true: the activations that meet weights past K are zeroed as well (they are
+//                              other values of the row, and 0 * inf is not 0)
 constexpr int kScaleBlockMaxK = 11264;  // a column block's scales for all of K stay in LDS: K bytes
 inline int scale_block_stride(int K) { return ((K + 1023) >> 10) << 10; }
+
+template <class P, class = void>
+struct MaskTail : std::false_type {};
+template <class P>
+struct MaskTail<P, std::void_t<decltype(P::kMaskTail)>> : std::bool_constant<P::kMaskTail> {};
 
 template <typename Policy, int TH, int NW, int WAVES, bool SB = false>
 struct SkinnyCfg {
@@ -189,8 +199,8 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       for (int i = 0; i < TM; ++i) {
         // rows past the slab (M <= 8 uses half a tile) re-read a held row: never stored
         const int row = (16 * i + lj < Cfg::kRows) ? 16 * i + lj : 16 * i + (lj & 7);
-        const half8_t aop =
-            *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * kq + t) ^ (row & 15)) << 4));
+        half8_t aop = *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * kq + t) ^ (row & 15)) << 4));
+        if constexpr (MaskTail<Policy>::value) aop = k0 < K ? aop : half8_t{};
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, bop[t], acc[i], 0, 0, 0);
       }
     }

@@ -328,3 +328,40 @@ def test_gemm_row_ends_in_part_of_eight_columns(ops, u, oracle, cfg, N):
     u.assert_close(got[8:8 + M * N].reshape(M, N), oracle.q4g32_linear(W, S, x, bias=bias, residual=res, nthreads=8),
                    f"cfg {cfg} N={N}")
     assert not got[:8].any() and not got[8 + M * N:].any()
+
+
+# K % 64 == 32: a step of half the length at the end of a row, and rows of S with an odd number of scales.
+# (M, N, K): up to 64 rows the small-batch kernel (odd N: the GEMM), above it the GEMM; a K of one half step
+# alone, one step and a half, partial tiles of columns, the kernel with the activations in registers
+HALF_STEP = [(3, 64, 32), (2, 34, 8224), (5, 16384, 4128), (8, 70, 96), (17, 130, 160), (33, 258, 4128), (64, 4096, 1056),
+             (9, 71, 96), (100, 514, 2080), (65, 131, 32), (130, 129, 96), (300, 257, 4128), (257, 1000, 1056)]
+
+
+@pytest.mark.parametrize("cfg", [0, 11, 17, 18])
+@pytest.mark.parametrize("M,N,K", HALF_STEP)
+def test_k_with_half_a_step(ops, u, oracle, cfg, M, N, K):
+    from relax_amd import _lib
+
+    x, W, S = oracle.make_q4g32_inputs(M, N, K, seed=M + N + K)
+    rng = np.random.default_rng(K)
+    bias, res = rng.standard_normal(N).astype(np.float16), rng.standard_normal((M, N)).astype(np.float16)
+    _lib.lib().wq_debug_set_gemm_config(cfg)
+    try:
+        got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x), bias=u.dev(bias), residual=u.dev(res),
+                                      kernel="gemm" if cfg else "auto"))
+    finally:
+        _lib.lib().wq_debug_set_gemm_config(0)
+    u.assert_close(got, oracle.q4g32_linear(W, S, x, bias=bias, residual=res, nthreads=8), f"cfg {cfg} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("M,N", [(3, 64), (17, 130), (64, 256), (130, 131)])
+def test_infinite_activations_under_half_a_step(ops, u, oracle, M, N):
+    """Nothing of a row meets the (absent) weights past K: an infinity stays one."""
+    K = 160
+    x, W, S = oracle.make_q4g32_inputs(M, N, K, seed=3)
+    codes = np.random.default_rng(1).integers(8, 16, size=(N, K)).astype(np.uint8)  # no zero weight
+    W = oracle.q4_pack(codes)
+    x[1, 0], x[2, K - 1] = np.inf, -np.inf
+    got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x)))
+    assert np.all(got[1] == np.inf) and np.all(got[2] == -np.inf)
+    assert np.all(np.isfinite(got[3:])) and np.all(np.isfinite(got[0]))
