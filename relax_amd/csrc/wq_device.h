@@ -153,11 +153,34 @@ __device__ __forceinline__ void u4_word_minus8(uint32_t w, half2_t out[4]) {
   }
 }
 
+// 1 + erf(v / sqrt(2)) = erfc(-v / sqrt(2)), without a branch: with s = |v|, erfc(s / sqrt(2)) =
+// exp(-s^2 / 2) * erfcx(s / sqrt(2)), and log2 of the second factor is smooth: a polynomial of degree 10, fitted here
+// by weighted least squares on [0, 6.5], beyond which gelu is below half the smallest fp16 number.
+// The library's erff runs both of its branches for every wavefront: a gelu over the identity cost 10 us at M = 128 and
+// 23 us at M = 500 (int8, K = 8192, N = 28672), with this 0 and 17.  Against 64 bits over |v| <= 12 the gelu is off by
+// 3.8e-7 at most (with erff 4.5e-7) and 5.0e-8 root mean square (5.6e-8); in the lower tail, where 1 + erff cancels,
+// by 1e-5 of its value down to v = -5.5 (erff: 0.6).
+__device__ __forceinline__ float one_plus_erf(float v) {
+  const float s = fminf(fabsf(v), 6.5f);
+  float p = 2.076590099875375e-08f;
+  p = fmaf(p, s, -6.674745236523449e-07f);
+  p = fmaf(p, s, 9.097290785575751e-06f);
+  p = fmaf(p, s, -6.668477726634592e-05f);
+  p = fmaf(p, s, 0.00024993513943627477f);
+  p = fmaf(p, s, 5.384150063036941e-05f);
+  p = fmaf(p, s, -0.0070038847625255585f);
+  p = fmaf(p, s, 0.05247436836361885f);
+  p = fmaf(p, s, -0.2621358633041382f);
+  p = fmaf(p, s, 1.1511050462722778f);
+  const float tail = __builtin_amdgcn_exp2f(-fmaf(v * v, 0.72134752044448170368f, p * s));
+  return v < 0.0f ? tail : 2.0f - tail;
+}
+
 __device__ __forceinline__ float apply_activation(float v, int act) {
   switch (act) {
     case 1: return v > 0.0f ? v : 0.0f;
     case 2: return v / (1.0f + __expf(-v));
-    case 3: return 0.5f * v * (1.0f + erff(v * 0.70710678118654752440f));
+    case 3: return 0.5f * v * one_plus_erf(v);
     default: return v;
   }
 }

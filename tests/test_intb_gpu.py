@@ -322,3 +322,27 @@ def test_grouped_gemv_with_scales_at_any_alignment(ops, u, oracle, nbit):
     got_s = ops.fpA_intB_gemm(u.dev(x), P, shifted, weight_nbit=nbit, group_size=64)
     assert torch.equal(got_a, got_s)
     u.assert_close(u.host(got_a), ref, f"grouped gemv int{nbit}")
+
+
+@pytest.mark.parametrize("M", [1, 40, 300])
+def test_gelu_over_its_range(ops, u, M):
+    """x[m] = (v, 0, ...), w = 1: gelu(v) itself, against 64 bits.  Bound: the rounding to fp16 (2^-11 of the value,
+    2^-25 below the smallest normal number) and 2e-5 for the fp32 evaluation (1e-5 at v = -5.5)."""
+    import torch
+    from scipy.special import erfc
+
+    N = K = 64
+    v = np.concatenate([np.linspace(-8, 8, 64 * M - 5), [0.0, 100.0, -100.0, 60000.0, -60000.0]])
+    v = v.astype(np.float16)[:: 64][:M] if M > 1 else np.array([-3.25], np.float16)
+    if M > 4:
+        v[:4] = [60000.0, -60000.0, 0.0, -5.5]
+    x = np.zeros((M, K), np.float16)
+    x[:, 0] = v
+    q = torch.zeros((K, N), dtype=torch.int8, device="cuda")
+    q[0] = 1
+    B = ops.ft_preprocess_weight(q, 80, False)
+    got = u.host(ops.fpA_intB_gemm(u.dev(x), B, torch.ones(N, dtype=torch.float16, device="cuda"), weight_nbit=8,
+                                   activation="gelu", group_size=-1)).astype(np.float64)
+    v = v.astype(np.float64)[:, None]
+    ref = 0.5 * v * erfc(-v / np.sqrt(2))
+    assert np.all(np.abs(got - ref) <= np.abs(ref) * (2.0**-11 + 2e-5) + 2.0**-25)
