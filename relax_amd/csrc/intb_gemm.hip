@@ -156,6 +156,7 @@ static int intb_gemm_lds(int cfg, const char* who, const int8_t* B, const uint16
     case 12: return launch_gemm_lds<P, IntbGemmEpilogue, 4, 2, 1, 4, 2>(who, largs, A, C, gep, m, n, k, stream);
     case 17: return launch_gemm_lds<P, IntbGemmEpilogue, 4, 1, 1, 4, 2>(who, largs, A, C, gep, m, n, k, stream);
     case 18: return launch_gemm_lds<P, IntbGemmEpilogue, 8, 1, 1, 4, 1>(who, largs, A, C, gep, m, n, k, stream);
+    case 19: return launch_gemm_lds<P, IntbGemmEpilogue, 4, 1, 1, 4, 2, 2>(who, largs, A, C, gep, m, n, k, stream);
     default: return fail(WQ_EINVAL, "%s: unknown tile configuration %d", who, cfg);
   }
 }
@@ -204,8 +205,10 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
     // up to 128 rows of a small matrix: the tiled GEMM has too few tiles for 256 CUs, two passes of the
     // small-batch kernel (64 rows, then the rest) are faster: n <= 4096 (int8, k = 11008, m = 128: 70 -> 55 us;
     // k = 4096: 28.4 -> 26.9 us), and up to 96 rows of a long, moderately wide one (k = 13824, n = 5120, m = 96:
-    // 88 -> 75 us; k = n = 8192: 54 -> 50 us).  Wider matrices keep the GEMM (n = 11008, k = 4096: 31 against 36 us).
-    if (m <= 2 * WQ_SMALL_BATCH_MAX_M && small_ok && (n <= 4096 || (m <= 96 && n <= 8192 && k >= 8192))) {
+    // 88 -> 75 us; k = n = 8192: 54 -> 50 us).  Wider matrices keep the GEMM (n = 11008, k = 4096: 31 against 36 us),
+    // and more than 96 rows where the GEMM may halve K (n = 4096, k = 11008, m = 128: int8 56 -> 48 us, int4 58 -> 42).
+    if (m <= 2 * WQ_SMALL_BATCH_MAX_M && small_ok &&
+        ((n <= 4096 && (m <= 96 || k % 128 != 0)) || (m <= 96 && n <= 8192 && k >= 8192))) {
       const int64_t m0 = WQ_SMALL_BATCH_MAX_M;
       if (int rc = intb_small_batch_dispatch(A, B, scales, C, m0, n, k, group, nbit, ep, stream)) return rc;
       IntbEpilogue ep2 = ep;
@@ -215,11 +218,12 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
     }
   }
   const IntbGemmEpilogue gep{ep, (int)n};
-  // the fully LDS-staged kernel under the tile shape (11, 17 or 18) whose rounds of the machine come out
-  // shortest; fine-grained scales whose pairs are not 4-byte aligned: the register-staged kernel (1..4)
+  // the fully LDS-staged kernel: 19 where its tiles fit one round, else the tile shape (11, 17 or 18) whose rounds of
+  // the machine come out shortest; fine-grained scales whose pairs are not 4-byte aligned: the register-staged kernel (1..4)
   const bool lds_ok = !group || (reinterpret_cast<uintptr_t>(scales) & 3u) == 0;
   int cfg = wq_gemm_cfg_override();
   if (!cfg && !lds_ok) cfg = choose_gemm_cfg(m, n, false);
+  if (!cfg && lds_k_halves(m, n, k, cu_count())) cfg = 19;
   if (!cfg) {
     double best = 0;
     for (int c : {17, 18, 11}) {
@@ -227,6 +231,7 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
       if (!cfg || t < best) cfg = c, best = t;
     }
   }
+  if (cfg == 19 && k % 128 != 0) cfg = 17;
   if (cfg >= 11 && lds_ok) {
     if (group)
       return nbit == 8 ? intb_gemm_lds<8, true>(cfg, who, B, scales, A, C, gep, m, n, k, stream)
@@ -234,7 +239,7 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
     return nbit == 8 ? intb_gemm_lds<8, false>(cfg, who, B, scales, A, C, gep, m, n, k, stream)
                      : intb_gemm_lds<4, false>(cfg, who, B, scales, A, C, gep, m, n, k, stream);
   }
-  if (cfg >= 11) cfg = cfg == 17 ? 4 : cfg == 11 ? 1 : 2;
+  if (cfg >= 11) cfg = (cfg == 17 || cfg == 19) ? 4 : cfg == 11 ? 1 : 2;
   if (nbit == 8) {
     const IntbLoader<8>::Args bargs{(const uint4_t*)B, (const half_t*)scales, group};
     return launch_mfma_gemm_cfg<IntbLoader<8>, IntbGemmEpilogue>(cfg, who, bargs, A, C, gep, m, n, k, stream);

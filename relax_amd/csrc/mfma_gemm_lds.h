@@ -126,7 +126,12 @@ typedef void __attribute__((address_space(3))) * wq_lptr_t;
 // One barrier per K-step suffices (three slots shown): slot (ks+2)%3 = (ks-1)%3 is refilled by loads issued after
 // the barrier of step ks-1, and every wavefront has waited for its last LDS reads of that slot
 // (the phase-3 fragments of step ks-1) before that barrier.
-template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME>
+//
+// KW = 2: the workgroup has two sets of four wavefronts, each with a ring of its own; set 0 takes the first half of
+// the K-steps, set 1 the second half (K % 128 == 0: as many steps, so as many barriers, in both), and set 1 hands
+// its sums to set 0 through LDS.  For launches with no more tiles than CUs: a wavefront alone on its SIMD leaves the
+// matrix core idle whenever it waits, and a second workgroup for the CU does not exist.
+template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME, int KW = 1>
 __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs,
                                               const half_t* __restrict__ X, half_t* __restrict__ Y,
                                               const Epilogue& epilogue, int M, int N, int K, int m0,
@@ -139,10 +144,14 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
   static_assert(kALoadsE >= 1, "tile too small to split further");
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  static_assert(KW == 1 || KW == 2);
+  const int set = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) - 4 * set;
   const int wm = wave / WN, wn = wave % WN;
   const int lj = lane & 31, lh = lane >> 5;
-  const int ksteps = K >> 6;
+  const int ksteps = (K >> 6) / KW, ks0 = set * ksteps;  // this set's steps: ks0 .. ks0 + ksteps - 1
+  unsigned char* const lds_all = lds;
+  lds += set * Cfg::kLdsBytes;
 
   // ---- global sources of this lane's direct loads (rows past M / N are clamped:
   //      they only feed accumulators that are never stored) ----
@@ -164,19 +173,19 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
   if (Cfg::kSLoads) s_src[0] = Policy::s_src(wargs, s_col, K);
   if constexpr (Cfg::kSLoads == 2) s_src[1] = Policy::s_src2(wargs, s_col, K);
 
-  // direct load number idx (0 .. L-1) of step ks
+  // direct load number idx (0 .. L-1) of this set's step ks
   auto issue_one = [&](int ks, int idx) {
     unsigned char* slot = lds + (ks % Cfg::kStages) * Cfg::kStageBytes;
     if (idx < kALoadsE) {
-      __builtin_amdgcn_global_load_lds((wq_gptr_t)(a_src[idx] + (int64_t)ks * 128),
+      __builtin_amdgcn_global_load_lds((wq_gptr_t)(a_src[idx] + (int64_t)(ks0 + ks) * 128),
                                        (wq_lptr_t)(slot + Cfg::kAOff + (wave * kALoadsE + idx) * 1024), 16, 0, 0);
     } else if (idx < kALoadsE + Cfg::kBLoads) {
       const int i = idx - kALoadsE;
-      __builtin_amdgcn_global_load_lds((wq_gptr_t)(b_src[i] + (int64_t)ks * Policy::kStepStride),
+      __builtin_amdgcn_global_load_lds((wq_gptr_t)(b_src[i] + (int64_t)(ks0 + ks) * Policy::kStepStride),
                                        (wq_lptr_t)(slot + Cfg::kBOff + (wave * Cfg::kBLoads + i) * 1024), 16, 0, 0);
     } else {
       const int i = idx - kALoadsE - Cfg::kBLoads;
-      __builtin_amdgcn_global_load_lds((wq_gptr_t)(s_src[i] + Policy::s_offset(wargs, ks)),
+      __builtin_amdgcn_global_load_lds((wq_gptr_t)(s_src[i] + Policy::s_offset(wargs, ks0 + ks)),
                                        (wq_lptr_t)(slot + Cfg::kSOff + i * (Cfg::BN * 4) + (wave * 64 % Cfg::BN) * 4), 4, 0, 0);
     }
   };
@@ -346,13 +355,45 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
     }
   }
 
+  unsigned char* stage = lds;
+  if constexpr (KW == 2) {
+    // set 1's sums in register order, 16 bytes per lane; behind them set 0's staging
+    static_assert(!HalfStep<Policy>::value);
+    constexpr int kSumBytes = 4 * TME * TN * 4096;
+    static_assert(kSumBytes + 4 * RowwiseEpilogueCfg<TME, TN>::kBytesPerWave <= 2 * Cfg::kLdsBytes);
+    float4_t* const sums = reinterpret_cast<float4_t*>(lds_all) + wave * (TME * TN * 256) + lane;
+    __syncthreads();  // both rings are idle
+    if (set == 1) {
+#pragma unroll
+      for (int i = 0; i < TME; ++i)
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            sums[((i * TN + t) * 4 + q) * 64] = float4_t{acc[i][t][4 * q], acc[i][t][4 * q + 1], acc[i][t][4 * q + 2], acc[i][t][4 * q + 3]};
+    }
+    __syncthreads();
+    if (set == 1) return;
+#pragma unroll
+    for (int i = 0; i < TME; ++i)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float4_t o = sums[((i * TN + t) * 4 + q) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][t][4 * q + e] += o[e];
+        }
+    stage = lds_all + kSumBytes;
+  }
+
   // ---- epilogue ----
   // Row-wise through LDS (gemm_epilogue.h); the ring is idle now: every real read of it was
   // waited for before the last barrier, and each wavefront stages in a piece of its own.
   using ECfg = RowwiseEpilogueCfg<TME, TN>;
   static_assert(4 * ECfg::kBytesPerWave <= Cfg::kLdsBytes, "epilogue staging exceeds the ring");
   store_tile_rowwise<Epilogue, TME, TN>(acc, epilogue, Y, M, N, m0 + wm * TME * 32, n0 + wn * TN * 32,
-                                        lds + wave * ECfg::kBytesPerWave, lane);
+                                        stage + wave * ECfg::kBytesPerWave, lane);
 }
 
 // Row slices (1, 2 or 4; 8 where the policy carries the extra copy of the tile body, `fine`) that the tiles of
@@ -393,6 +434,29 @@ inline double lds_cfg_cost(int cfg, int64_t M, int64_t N, int cus) {
   return t;
 }
 
+// Configuration 19: 128 x 128 tiles with the K-steps of a tile split between two sets of wavefronts (KW = 2), for
+// launches that have no more such tiles than CUs.  Against the fastest of 17, 18 and 11: int8, K = 8192, N = 28672,
+// M = 128 93 -> 85 us; K = 4096, N = 11008, M = 200 41.5 -> 35.2 us, int4 38.7 -> 32.8 us; N = K = 1024, M = 128
+// 9.4 -> 7.9 us; over five such shapes, M = 70 .. 1024, 1 .. 28 % (one 3 % slower: int8, N = K = 8192, M = 128).
+inline bool lds_k_halves(int64_t M, int64_t N, int64_t K, int cus) {
+  return K % 128 == 0 && ((M + 127) / 128) * ((N + 127) / 128) <= cus;
+}
+
+// The same for 4-bit codes with a scale per group in front of the rule of choose_q4_lds_cfg, whose 256 x 128 tiles in
+// row slices are as fast where they fill the machine: four or eight slices on 7/8 of the CUs (N = 4096, K = 11008:
+// M = 256 69 against 73 us, M = 500 80 against 85), or tiles for 3/4 of them (N = 12288, K = 4096, M = 256 39.0
+// against 39.5; N = 5120, K = 13824, M = 640 122 against 124).  A last row of tiles with hardly a row in it costs
+// this form a whole tile too (N = 11008, K = 4096, M = 129: 38 against 39 us).  Elsewhere: N = 11008, K = 4096,
+// M = 128 33.5 -> 29.7, M = 200 38.6 -> 36.3 us; N = 5120, K = 13824, M = 300 113 -> 93 us.
+inline bool q4_lds_k_halves(int64_t M, int64_t N, int64_t K, int cus) {
+  const int64_t tiles_n = (N + 127) / 128, tiles = ((M + 127) / 128) * tiles_n;
+  if (K % 128 != 0 || tiles * 4 >= (int64_t)cus * 3 || (M - 1) % 128 < 15) return false;
+  const int64_t rest = ((M + 255) / 256) * tiles_n;  // fewer than 3/4 of the CUs, as well
+  const int split = lds_tail_split((int)rest, cus, cus, 8, 8, true);
+  const int64_t slices = tiles_n * ((M * split + 255) / 256);
+  return !(M > 128 && split >= 4 && slices * 8 >= (int64_t)cus * 7);
+}
+
 // Policy::kFineTail = true: the kernels of that policy also hold the tile body for slices of TM / 8 sub-tiles.
 template <class P, class = void>
 struct FineTail : std::false_type {};
@@ -403,8 +467,8 @@ struct FineTail<P, std::void_t<decltype(P::kFineTail)>> : std::bool_constant<P::
 // as fill complete rounds of the machine); the tiles of the last, partially filled
 // round are cut into `split` row slices of TM/split sub-tiles so that the round is
 // shorter instead of leaving most CUs idle while a few finish whole tiles.
-template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WAVES_PER_EU>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU, WAVES_PER_EU)))
+template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WAVES_PER_EU, int KW>
+__global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU, WAVES_PER_EU)))
 void gemm_lds_kernel(typename Policy::Args wargs, const half_t* __restrict__ X, half_t* __restrict__ Y,
                      Epilogue epilogue, int M, int N, int K, int tiles_m, int tiles_n, int n_full,
                      int split, int group_m) {
@@ -426,7 +490,7 @@ void gemm_lds_kernel(typename Policy::Args wargs, const half_t* __restrict__ X, 
     const int xcd = pid & 7, idx = pid >> 3;
     int tile_m, tile_n;
     tile_of(xcd * per + min(xcd, rem) + idx, tile_m, tile_n);
-    gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM>(wargs, X, Y, epilogue, M, N, K,
+    gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM, KW>(wargs, X, Y, epilogue, M, N, K,
                                                         tile_m * Cfg::BM, tile_n * Cfg::BN, lds);
     return;
   }
@@ -443,31 +507,31 @@ void gemm_lds_kernel(typename Policy::Args wargs, const half_t* __restrict__ X, 
   if (m0 >= M) return;  // a slice that lies entirely past the last row
   if (split == 2) {
     if constexpr (TM % 2 == 0)
-      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 2>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 2, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
   } else if (split == 4) {
     if constexpr (TM % 4 == 0)
-      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 4>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 4, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
   } else if (split == 8) {
     if constexpr (TM % 8 == 0 && FineTail<Policy>::value)
-      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 8>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 8, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
   } else {
-    gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+    gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
   }
 }
 
-template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE>
+template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int KW = 1>
 static int launch_gemm_lds(const char* who, const typename Policy::Args& wargs, const uint16_t* x,
                            uint16_t* y, const Epilogue& ep, int64_t M, int64_t N, int64_t K,
                            hipStream_t stream) {
   using Cfg = LdsGemmCfg<Policy, TM, TN, WM, WN, WPE>;
   const int tiles_m = (int)((M + Cfg::BM - 1) / Cfg::BM);
   const int tiles_n = (int)((N + Cfg::BN - 1) / Cfg::BN);
-  auto kern = gemm_lds_kernel<Policy, Epilogue, TM, TN, WM, WN, WPE>;
+  auto kern = gemm_lds_kernel<Policy, Epilogue, TM, TN, WM, WN, WPE, KW>;
   static DynamicLdsLimit limit;
-  WQ_HIP(limit.ensure(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes));
+  WQ_HIP(limit.ensure(reinterpret_cast<const void*>(kern), KW * Cfg::kLdsBytes));
   // Whole rounds of the machine run whole tiles; the tiles of the last, partial
   // round are cut into 2 or 4 row slices when that lets them all run at once.
-  const int per_cu = std::max(1, std::min(WPE, (160 * 1024) / Cfg::kLdsBytes));
+  const int per_cu = std::max(1, std::min(WPE / KW, (160 * 1024) / (KW * Cfg::kLdsBytes)));
   const int slots = cu_count() * per_cu;
   const int total = tiles_m * tiles_n;
   const int n_full = (total / slots) * slots;
@@ -481,7 +545,7 @@ static int launch_gemm_lds(const char* who, const typename Policy::Args& wargs, 
   while (group_m * 1.5 < want) group_m *= 2;
   group_m = std::max(1, std::min(group_m, tiles_m));
   if (n_full == 0) group_m = tiles_m;  // one partial round: M-fastest, workgroup i takes slice i
-  WQ_LAUNCH(who, kern, dim3((unsigned)(n_full + rest * split)), dim3(256), Cfg::kLdsBytes, stream, wargs,
+  WQ_LAUNCH(who, kern, dim3((unsigned)(n_full + rest * split)), dim3(256 * KW), KW * Cfg::kLdsBytes, stream, wargs,
             (const half_t*)x, (half_t*)y, ep, (int)M, (int)N, (int)K, tiles_m, tiles_n, n_full, split, group_m);
   return WQ_OK;
 }

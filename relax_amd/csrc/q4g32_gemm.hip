@@ -147,21 +147,24 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
   WQ_REQUIRE(W && S && x && y, "wq_q4g32_gemm: null pointer");
   WQ_REQUIRE(aligned16(W) && aligned16(x), "wq_q4g32_gemm: W and x must be 16-byte aligned");
   WQ_REQUIRE(M < (1ll << 30) && N < (1ll << 30) && K < (1ll << 30), "wq_q4g32_gemm: too large");
-  int cfg = tuning().gemm_cfg ? tuning().gemm_cfg : choose_q4_lds_cfg(M, N, cu_count());
+  int cfg = tuning().gemm_cfg                       ? tuning().gemm_cfg
+            : q4_lds_k_halves(M, N, K, cu_count()) ? 19
+                                                   : choose_q4_lds_cfg(M, N, cu_count());
   const Q4G32Loader::Args bargs{W, (const half_t*)S};
   const Q4G32LdsPolicy::Args largs{W, (const half_t*)S};
   const Q4G32Epilogue ep{(const half_t*)bias, (const half_t*)residual, (int)N};
-  // 11..18: the fully LDS-staged kernel (needs 4-byte aligned S); K % 64 == 32 has the three shapes that the
+  // 11..19: the fully LDS-staged kernel (needs 4-byte aligned S); K % 64 == 32 has the three shapes that the
   // choice above takes for most problems
   if (cfg >= 11 && K % 64 == 32 && ((uintptr_t)S & 3u) == 0) {
     switch (cfg) {
-      case 17: return launch_gemm_lds<Q4G32HalfStepPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 17: case 19: return launch_gemm_lds<Q4G32HalfStepPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 12: case 13:
       case 18: return launch_gemm_lds<Q4G32HalfStepPolicy, Q4G32Epilogue, 8, 1, 1, 4, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 11: case 14: return launch_gemm_lds<Q4G32HalfStepPolicy, Q4G32Epilogue, 8, 2, 1, 4, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       default: return fail(WQ_EINVAL, "wq_q4g32_gemm: unknown tile configuration %d", cfg);
     }
   }
+  if (cfg == 19 && K % 128 != 0) cfg = 17;
   if (cfg >= 11 && K % 64 == 0 && ((uintptr_t)S & 3u) == 0) {
     switch (cfg) {
       case 11: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 8, 2, 1, 4, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
@@ -170,10 +173,11 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
       case 14: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 4, 2, 2, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 17: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 18: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 8, 1, 1, 4, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 19: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       default: return fail(WQ_EINVAL, "wq_q4g32_gemm: unknown tile configuration %d", cfg);
     }
   }
-  if (cfg >= 11) cfg = cfg == 17 ? 4 : (cfg == 11 || cfg == 14) ? 1 : 2;  // 12, 13, 18 -> 128 x 256  // not eligible: register-staged kernel, same tile
+  if (cfg >= 11) cfg = (cfg == 17 || cfg == 19) ? 4 : (cfg == 11 || cfg == 14) ? 1 : 2;  // 12, 13, 18 -> 128 x 256  // not eligible: register-staged kernel, same tile
   return launch_mfma_gemm_cfg<Q4G32Loader, Q4G32Epilogue>(cfg, "wq_q4g32_gemm", bargs, x, y, ep, M,
                                                           N, K, stream);
 }

@@ -231,6 +231,27 @@ def test_gemm_tile_configurations(ops, u, oracle, nbit, cfg):
         _lib.lib().wq_debug_set_gemm_config(0)
 
 
+# K of one step per set of wavefronts, of fewer steps than the ring has slots, and of more
+@pytest.mark.parametrize("K", [128, 256, 384, 1152])
+@pytest.mark.parametrize("group_size", [-1, 64])
+@pytest.mark.parametrize("nbit", [8, 4])
+def test_k_halves_in_one_workgroup(ops, u, oracle, nbit, group_size, K):
+    """128 x 128 tiles whose K-steps two sets of wavefronts share: whole tiles and row slices of them."""
+    from relax_amd import _lib
+
+    _lib.lib().wq_debug_set_gemm_config(19)
+    try:
+        for split in (1, 0):
+            _lib.lib().wq_debug_set_gemm_tail_split(split)
+            for M, N in [(70, 64), (130, 320), (300, 192)]:
+                _run(ops, u, oracle, M, N, K, nbit, seed=M + K, group_size=group_size)
+                _run(ops, u, oracle, M, N, K, nbit, seed=M + K + 1, group_size=group_size, bias="row", activation="gelu",
+                     residual=True)
+    finally:
+        _lib.lib().wq_debug_set_gemm_tail_split(1)
+        _lib.lib().wq_debug_set_gemm_config(0)
+
+
 @pytest.mark.parametrize("M", [1, 16, 128, 256, 512])
 def test_int8_full_size_sampled(ops, u, oracle, M):
     """K=8192, N=28672 int8 per-channel.  The oracle checks a sample of output columns

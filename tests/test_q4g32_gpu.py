@@ -365,3 +365,23 @@ def test_infinite_activations_under_half_a_step(ops, u, oracle, M, N):
     got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x)))
     assert np.all(got[1] == np.inf) and np.all(got[2] == -np.inf)
     assert np.all(np.isfinite(got[3:])) and np.all(np.isfinite(got[0]))
+
+
+@pytest.mark.parametrize("K", [128, 256, 384, 1152])
+@pytest.mark.parametrize("M,N", [(70, 64), (130, 321), (300, 200)])
+def test_gemm_k_halves_in_one_workgroup(ops, u, oracle, M, N, K):
+    """128 x 128 tiles whose K-steps two sets of wavefronts share: whole tiles and row slices of them."""
+    from relax_amd import _lib
+
+    x, W, S = oracle.make_q4g32_inputs(M, N, K, seed=M + N + K)
+    res = np.random.default_rng(K).standard_normal((M, N)).astype(np.float16)
+    ref = oracle.q4g32_linear(W, S, x, residual=res, nthreads=8)
+    _lib.lib().wq_debug_set_gemm_config(19)
+    try:
+        for split in (1, 0):
+            _lib.lib().wq_debug_set_gemm_tail_split(split)
+            got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x), residual=u.dev(res), kernel="gemm"))
+            u.assert_close(got, ref, f"{M}x{N}x{K} split {split}")
+    finally:
+        _lib.lib().wq_debug_set_gemm_tail_split(1)
+        _lib.lib().wq_debug_set_gemm_config(0)
