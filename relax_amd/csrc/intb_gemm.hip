@@ -227,7 +227,7 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
   if (!cfg) {
     double best = 0;
     for (int c : {17, 18, 11}) {
-      const double t = lds_cfg_cost(c, m, n, cu_count());
+      const double t = lds_cfg_cost(c, m, n, k, activation >= WQ_ACT_SILU, cu_count());
       if (!cfg || t < best) cfg = c, best = t;
     }
   }

@@ -416,7 +416,13 @@ inline int lds_tail_split(int rest, int slots, int cus, int TM, int a_loads, boo
 // 256 x 128: 254; 256 x 256: 294); row slices of a cut tile run at 0.74 (halves) and 0.56 (quarters) of
 // them (a slice unpacks all columns of its tile whatever its height; fitted to launches that are one cut round:
 // N = 4096 .. 12288, M = 192 .. 1024, where 0.85 / 0.75 chose 256 x 256 tiles 10 .. 15 % too slow).  The model reproduces the measured times at M = 65 .. 2048 within 6 %.
-inline double lds_cfg_cost(int cfg, int64_t M, int64_t N, int cus) {
+//
+// An epilogue with an activation (exp, erf) adds time that does not depend on K: per round 4 us (17), 18 us (18),
+// 26 us (11) for whole tiles, less for slices.  Two workgroups per CU multiply through each other's epilogue, one
+// cannot.  Fitted to silu and gelu over seven (N, K), K = 1024 .. 12288, M = 128 .. 2048: the choice is 0.2 % slower
+// than the fastest on average and 6 % at most; without the term 10 % and 34 % (int8, N = 16384, K = 1024, M = 768:
+// 64.8 -> 52.9 us; N = 28672, K = 2048, M = 1536: 288 -> 242 us; N = 22016, K = 4096, M = 512: 137 -> 124 us).
+inline double lds_cfg_cost(int cfg, int64_t M, int64_t N, int64_t K, bool activates, int cus) {
   const int BM = cfg == 17 ? 128 : 256, BN = cfg == 11 ? 256 : 128, per_cu = cfg == 17 ? 2 : 1;
   const double rate_alone = cfg == 17 ? 193.0 : cfg == 18 ? 254.0 : 294.0;
   const double rate_full = cfg == 17 ? 243.0 : rate_alone;  // per CU, every slot taken
@@ -424,12 +430,14 @@ inline double lds_cfg_cost(int cfg, int64_t M, int64_t N, int cus) {
   const int slots = cus * per_cu;
   const int rest = (int)(tiles % slots);
   const double area = (double)BM * BN;
-  double t = (double)(tiles / slots) * per_cu * area / rate_full;
+  const double fixed = activates ? (cfg == 17 ? 4.0 : cfg == 18 ? 18.0 : 26.0) * 8192.0 / (double)K : 0.0;
+  double t = (double)(tiles / slots) * (per_cu * area / rate_full + fixed);
   if (rest) {
     const int split = lds_tail_split(rest, slots, cus, BM / 32, BM / 32);
     const bool alone = rest * split <= cus;
     const double slice = split == 4 ? 0.56 : split == 2 ? 0.74 : 1.0;
     t += area / split * (alone ? 1 : per_cu) / ((alone ? rate_alone : rate_full) * slice);
+    t += fixed / split * (alone && cfg == 17 ? 0.7 : 1.0);
   }
   return t;
 }
