@@ -5,8 +5,8 @@
 //     its output feeds wq_ft_preprocess_weight.
 //   format A (q4f16_1): the inverse of the decode in tests/python/dlight/test_gpu_gemv.py:198;
 //     the reference tree holds no encoder for it, the definition is stated below.
-// All arithmetic is float32 with IEEE division and round-half-away-from-zero, as the
-// llvm lowering of T.round does (src/target/llvm/intrin_rule_llvm.cc:84-86).
+// All arithmetic is float32, rounded as IEEE division and round-half-away-from-zero give it (the llvm lowering of
+// T.round, src/target/llvm/intrin_rule_llvm.cc:84-86).
 #include "wq_device.h"
 #include "wq_host.h"
 
