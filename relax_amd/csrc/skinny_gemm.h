@@ -318,12 +318,14 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
 
   // ---- the A operands of this wavefront's run of K (zero past M and past K) ----
   half8_t a[NSTEP][4];
-  int k0c[NSTEP];  // this lane's 32 weights of step s (any valid k when past K: they meet zeros)
+  int k0c[NSTEP];  // this lane's 32 weights of step s (any valid k when past K)
+  bool past[NSTEP];  // past K: the scale is zeroed too, the one fetched may be another row's and 0 * inf is not 0
 #pragma unroll
   for (int s = 0; s < NSTEP; ++s) {
     const int k0 = (wave * NSTEP + s) * 128 + 32 * kq;
     const bool held = lj < M && k0 < K;
-    k0c[s] = k0 < K ? k0 : 0;
+    past[s] = k0 >= K;
+    k0c[s] = past[s] ? 0 : k0;
     const half_t* src = held ? X + (int64_t)lj * K + k0 : X;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -381,8 +383,10 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
 #pragma unroll
       for (int p = 0; p < P; ++p) pieces[p] = *reinterpret_cast<const uint4_t*>(src + p * 1024 + lane * 16);
       const half2_t pair = *reinterpret_cast<const half2_t*>(src + P * 1024 + lane * 4);
+      typename Policy::Scale scale = Policy::pick_scale(pl0, pair, kq);
+      if (past[s]) scale = Policy::null_scale();
       half8_t bop[4];
-      Policy::dequant(pieces, Policy::pick_scale(pl0, pair, kq), bop);
+      Policy::dequant(pieces, scale, bop);
 #pragma unroll
       for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[s][t], bop[t], acc, 0, 0, 0);
       // the slot is free once its contents are in registers; it takes the step D ahead

@@ -367,6 +367,20 @@ def test_infinite_activations_under_half_a_step(ops, u, oracle, M, N):
     assert np.all(np.isfinite(got[3:])) and np.all(np.isfinite(got[0]))
 
 
+# the kernel with the activations in registers (N >= 16384), and the ring kernel; the last scale of row 200 shares
+# an aligned word with the first of row 201
+@pytest.mark.parametrize("M,N,K", [(5, 16384, 4128), (16, 16384, 8160), (9, 514, 4128), (40, 514, 4128)])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_non_finite_scale_stays_in_its_row(ops, u, oracle, M, N, K, value):
+    x, W, S = oracle.make_q4g32_inputs(M, N, K, seed=N)
+    want = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x)))
+    S[200, -1] = value
+    got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x)))
+    others = np.arange(N) != 200
+    np.testing.assert_array_equal(got[:, others], want[:, others])
+    assert np.all(np.isfinite(want)) and not np.any(np.isfinite(got[:, 200]))
+
+
 @pytest.mark.parametrize("K", [128, 256, 384, 1152])
 @pytest.mark.parametrize("M,N", [(70, 64), (130, 321), (300, 200)])
 def test_gemm_k_halves_in_one_workgroup(ops, u, oracle, M, N, K):
