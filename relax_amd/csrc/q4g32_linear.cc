@@ -13,8 +13,9 @@ extern "C" int wq_q4g32_linear(const uint32_t* W, const uint16_t* S, const uint1
   // for the next one that serves the call.
   const bool gemv_ok = K <= 32768;
   // K % 64 == 32 has a form of the small-batch kernel with its own scale addressing; before it, 3 .. 8 rows went
-  // through the streaming kernel in pairs and more through the GEMM (N = 11008, K = 4064: M = 4 16.5 -> 10.3 us,
-  // M = 8 30.6 -> 10.1, M = 19 65 -> 19, M = 64 66 -> 25)
+  // through the streaming kernel in pairs and more through the GEMM (N = 11008, K = 4064: M = 3 14.6 -> 10.7 us,
+  // M = 8 29.4 -> 10.7, M = 19 65 -> 19, M = 64 66 -> 25); like the kernel they left, up to 8 rows take the weights
+  // unrounded
   const bool half_step = K > 0 && K % 64 == 32 && wq::q4g32_half_step_rows_ok(x, N);
   const bool small_ok = (K % 64 == 0 || half_step) && (reinterpret_cast<uintptr_t>(S) & 3u) == 0;
   const auto small_batch = [&](const uint16_t* x_, const uint16_t* residual_, uint16_t* y_, int64_t M_) {

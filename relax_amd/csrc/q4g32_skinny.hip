@@ -72,6 +72,19 @@ struct Q4G32OddGroupsSkinnyPolicy : Q4G32SkinnyPolicy {
   }
 };
 
+// Up to 8 rows of such a K: (code - 7) * scale is not rounded to fp16, as in the streaming kernel that serves them
+// elsewhere (against 64 bits, K = 4064: 2.06e-4, most of it the rounding of y; with rounded weights 2.75e-4).
+// M = 8, streaming kernel / this / rounded weights: N = 11008, K = 4064 29.4 / 10.6 / 10.4 us, N = 4096, K = 11040
+// 45.3 / 11.8 / 11.1 us, N = 28672, K = 8160 112 / 44.2 / 43.1 us.
+struct Q4G32OddGroupsExactSkinnyPolicy : Q4G32OddGroupsSkinnyPolicy {
+  __device__ __forceinline__ static half8_t codes8(uint32_t word) {
+    const half2_t one = {(half_t)1.0f, (half_t)1.0f};
+    half2_t d[4];
+    q4_word_dequant_natural(word, one, d);
+    return half8_t{d[0].x, d[0].y, d[1].x, d[1].y, d[2].x, d[2].y, d[3].x, d[3].y};
+  }
+};
+
 int q4g32_half_step_rows(const uint32_t* W, const uint16_t* S, const uint16_t* x, const uint16_t* bias,
                          const uint16_t* residual, uint16_t* y, int64_t M, int64_t N, int64_t K,
                          hipStream_t stream) {
@@ -84,6 +97,9 @@ int q4g32_half_step_rows(const uint32_t* W, const uint16_t* S, const uint16_t* x
   WQ_REQUIRE(N < (1ll << 30) && K < (1ll << 30), "wq_q4g32_linear: too large");
   const Q4G32OddGroupsSkinnyPolicy::Args pargs{W, (const half_t*)S};
   const Q4G32Epilogue epi{(const half_t*)bias, (const half_t*)residual, (int)N};
+  if (M <= 8)
+    return launch_skinny_auto<Q4G32OddGroupsExactSkinnyPolicy, Q4G32Epilogue>("wq_q4g32_linear", pargs, x, y, epi, M,
+                                                                              N, K, stream);
   return launch_skinny_auto<Q4G32OddGroupsSkinnyPolicy, Q4G32Epilogue>("wq_q4g32_linear", pargs, x, y, epi, M, N,
                                                                        K, stream);
 }

@@ -66,6 +66,9 @@ typedef void __attribute__((address_space(3))) * wq_sk_lptr_t;
 // and, where K may end inside the two halves of a 64-k piece,
 //   kMaskTail                  true: the activations that meet weights past K are zeroed as well (they are
 //                              other values of the row, and 0 * inf is not 0)
+// and, for weights that are not rounded (up to 8 rows, kPieces == 1),
+//   codes8(word)               the codes of a word of codes as halves, exact (8 consecutive k); the products of a
+//                              group of 32 k are summed alone and scaled in fp32
 constexpr int kScaleBlockMaxK = 11264;  // a column block's scales for all of K stay in LDS: K bytes
 inline int scale_block_stride(int K) { return ((K + 1023) >> 10) << 10; }
 
@@ -73,6 +76,51 @@ template <class P, class = void>
 struct MaskTail : std::false_type {};
 template <class P>
 struct MaskTail<P, std::void_t<decltype(P::kMaskTail)>> : std::bool_constant<P::kMaskTail> {};
+
+template <class P, class = void>
+struct GroupSums : std::false_type {};
+template <class P>
+struct GroupSums<P, std::void_t<decltype(&P::codes8)>> : std::true_type {};
+
+// bits 0 .. n - 1 of `groups` groups, of which those up to K exist
+__device__ __forceinline__ uint32_t live_groups(int k0, int K, int groups) {
+  const int n = min(max((K - k0) >> 5, 0), groups);
+  return n >= 32 ? ~0u : (1u << n) - 1u;
+}
+
+// One step of 128 k with the scales outside the products (GroupSums).  MFMA g takes group g whole: a quarter kq of
+// the wavefront brings k 32g + 8kq .. + 7, so lane (j, kq) reads the word kq of the piece that lane (j, g) fetched
+// (4 bytes a lane, the 64 of them contiguous), and the scale that lane fetched.  a(g) is the A operand; groups past K,
+// whose bit first + g of `live` is clear, get a zero scale (a mask: a branch would keep the reads from being issued
+// together).
+template <class Policy, class AOp>
+__device__ __forceinline__ void mul_group_sums(float4_t& acc, const typename Policy::Lane& pl, const unsigned char* pieces,
+                                               const unsigned char* pairs, int lj, int kq, uint32_t live, int first, AOp a) {
+  static_assert(Policy::kPieces == 1 && Policy::kScaleDma);
+  const uint32_t* const w = reinterpret_cast<const uint32_t*>(pieces + lj * 16 + kq * 4);
+  const uint32_t* const p = reinterpret_cast<const uint32_t*>(pairs + lj * 4);
+  uint32_t word[4], pair[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    word[g] = w[g * 64];
+    pair[g] = p[g * 16] & (uint32_t)((int32_t)(live << (31 - first - g)) >> 31);
+  }
+  half8_t aop[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) aop[g] = a(g);
+  float s[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) s[g] = (float)Policy::pick_scale(pl, as_half2(pair[g]), g);
+  float4_t sum[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    sum[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop[g], Policy::codes8(word[g]), float4_t{}, 0, 0, 0);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = fmaf(s[g], sum[g][r], acc[r]);
+  }
+}
 
 template <typename Policy, int TH, int NW, int WAVES, bool SB = false>
 struct SkinnyCfg {
@@ -176,6 +224,17 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
 
   auto compute = [&](int it, int slot) {
     const int stage_off = slot * Cfg::kStageBytes;
+    const unsigned char* slab = lds + stage_off + kw * Cfg::kSlabBytes;
+    if constexpr (GroupSums<Policy>::value) {
+      static_assert(TM == 1);
+      const int k0 = 128 * (it * KW + kw);
+      const int row = lj < Cfg::kRows ? lj : lj & 7;
+      mul_group_sums<Policy>(acc[0], pl, w_area + stage_off, s_area + stage_off, lj, kq, live_groups(k0, K, 4), 0, [&](int g) {
+        const half8_t v = *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * g + kq) ^ (row & 15)) << 4));
+        return k0 + 32 * g < K ? v : half8_t{};
+      });
+      return;
+    }
     const int k0 = 128 * (it * KW + kw) + 32 * kq;
     uint4_t pieces[P];
 #pragma unroll
@@ -192,7 +251,6 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
     if (k0 >= K) s = Policy::null_scale();  // code * 0 = exact zero for the weights past K
     half8_t bop[4];
     Policy::dequant(pieces, s, bop);
-    const unsigned char* slab = lds + stage_off + kw * Cfg::kSlabBytes;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
 #pragma unroll
@@ -326,6 +384,16 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
     const bool held = lj < M && k0 < K;
     past[s] = k0 >= K;
     k0c[s] = past[s] ? 0 : k0;
+    if constexpr (GroupSums<Policy>::value) {  // operand t: k 8kq .. + 7 of group t
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int kt = (wave * NSTEP + s) * 128 + 32 * t;
+        const bool held_t = lj < M && kt < K;
+        const half8_t v = *reinterpret_cast<const half8_t*>(held_t ? X + (int64_t)lj * K + kt + 8 * kq : X);
+        a[s][t] = held_t ? v : half8_t{};
+      }
+      continue;
+    }
     const half_t* src = held ? X + (int64_t)lj * K + k0 : X;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -370,8 +438,12 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
 
   int slot = 0;  // of step 0 of the current tile
   int turn = 0;
+  uint32_t run_groups = 0;  // the 32-k groups of this wavefront's run that exist (GroupSums)
+  if constexpr (GroupSums<Policy>::value) run_groups = live_groups(wave * NSTEP * 128, K, 4 * NSTEP);
   for (int tile = blockIdx.x; tile < tiles; tile += grid) {
     set_tile(1, tile + (QA + 1) * grid);
+    if constexpr (GroupSums<Policy>::value) asm volatile("" : "+v"(run_groups));  // or a mask per group is kept: they spill
+    const uint32_t live = __builtin_amdgcn_readfirstlane(run_groups);
     float4_t acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int s = 0; s < NSTEP; ++s) {
@@ -379,16 +451,21 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
       int sl = slot + s;
       if (sl >= D) sl -= D;
       const unsigned char* src = ring + sl * Cfg::kStepBytes;
-      uint4_t pieces[P];
+      if constexpr (GroupSums<Policy>::value) {
+        mul_group_sums<Policy>(acc, pl0, src, src + P * 1024, lj, kq, live, 4 * s, [&](int g) { return a[s][g]; });
+        asm volatile("" : "+v"(acc));  // scaled in every step: left to the end of the tile the sums of all steps spill
+      } else {
+        uint4_t pieces[P];
 #pragma unroll
-      for (int p = 0; p < P; ++p) pieces[p] = *reinterpret_cast<const uint4_t*>(src + p * 1024 + lane * 16);
-      const half2_t pair = *reinterpret_cast<const half2_t*>(src + P * 1024 + lane * 4);
-      typename Policy::Scale scale = Policy::pick_scale(pl0, pair, kq);
-      if (past[s]) scale = Policy::null_scale();
-      half8_t bop[4];
-      Policy::dequant(pieces, scale, bop);
+        for (int p = 0; p < P; ++p) pieces[p] = *reinterpret_cast<const uint4_t*>(src + p * 1024 + lane * 16);
+        const half2_t pair = *reinterpret_cast<const half2_t*>(src + P * 1024 + lane * 4);
+        typename Policy::Scale scale = Policy::pick_scale(pl0, pair, kq);
+        if (past[s]) scale = Policy::null_scale();
+        half8_t bop[4];
+        Policy::dequant(pieces, scale, bop);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[s][t], bop[t], acc, 0, 0, 0);
+        for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[s][t], bop[t], acc, 0, 0, 0);
+      }
       // the slot is free once its contents are in registers; it takes the step D ahead
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       issue((s + D) / NSTEP - QA, (s + D) % NSTEP, sl);
@@ -548,6 +625,9 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
     if (nw == 2) WQ_SK_GO(1, 2, 8);
     WQ_SK_GO(1, 1, 8);
   }
+  if constexpr (GroupSums<Policy>::value) {
+    return fail(WQ_EINVAL, "%s: internal: more than 8 rows", who);
+  } else {
   if (M <= 16 && nw != 8) {
     if (nw == 4) WQ_SK_GO(2, 4, 8);
     if (nw == 2) WQ_SK_GO(2, 2, 8);
@@ -563,6 +643,7 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
   if (nw == 4) WQ_SK_GO(8, 4, 8);
   if (nw == 2) WQ_SK_GO(8, 2, 8);
   WQ_SK_GO(8, 1, 8);
+  }
 #undef WQ_SK_GO
 }
 

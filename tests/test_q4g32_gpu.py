@@ -367,6 +367,20 @@ def test_infinite_activations_under_half_a_step(ops, u, oracle, M, N):
     assert np.all(np.isfinite(got[3:])) and np.all(np.isfinite(got[0]))
 
 
+# the ring kernel (1 .. 2 column blocks side by side) and the one with the activations in registers
+@pytest.mark.parametrize("N,K", [(514, 4064), (8194, 1056), (16384, 4128), (16386, 8160), (514, 11040)])
+@pytest.mark.parametrize("M", [2, 3, 8])
+def test_weights_of_half_a_step_are_not_rounded(ops, u, oracle, M, N, K):
+    """Up to 8 rows (code - 7) * scale is not rounded to fp16.  Against 64 bits: the rounding of y to fp16 is 2.0e-4
+    (2^-11 / sqrt(3) of the binade, over the root mean square in it); with every weight rounded as well, 2.7e-4."""
+    x, W, S = oracle.make_q4g32_inputs(M, N, K, seed=K)
+    got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x))).astype(np.float64)
+    codes = (W[:, :, None] >> (4 * np.arange(8, dtype=np.uint32))) & 15
+    w = (codes.reshape(N, K // 32, 32).astype(np.float64) - 7) * S.astype(np.float64)[:, :, None]
+    ref = x.astype(np.float64) @ w.reshape(N, K).T
+    assert np.linalg.norm(got - ref) <= 2.35e-4 * np.linalg.norm(ref)
+
+
 # the kernel with the activations in registers (N >= 16384), and the ring kernel; the last scale of row 200 shares
 # an aligned word with the first of row 201
 @pytest.mark.parametrize("M,N,K", [(5, 16384, 4128), (16, 16384, 8160), (9, 514, 4128), (40, 514, 4128)])
