@@ -24,6 +24,9 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-fvisibility=hidden",
     "-Wall", "-Wno-unused-function",
+    # loops start on an instruction cache line: the main loop of the 256 x 256 GEMM tile, identical code, is 1 % faster there
+    # than in mid-line (q4f16_1, N = 22016, K = 4096, M = 8192: 1287 against 1302 us)
+    "-falign-loops=64",
     # keep the compiler from forming packed-fp32 VALU ops
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
