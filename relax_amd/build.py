@@ -24,12 +24,14 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-fvisibility=hidden",
     "-Wall", "-Wno-unused-function",
-    # loops start on an instruction cache line: the main loop of the 256 x 256 GEMM tile, identical code, is 1 % faster there
-    # than in mid-line (q4f16_1, N = 22016, K = 4096, M = 8192: 1287 against 1302 us)
-    "-falign-loops=64",
     # keep the compiler from forming packed-fp32 VALU ops
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+
+# Loops on instruction cache lines: the main loop of the 256 x 256 tile of the MFMA GEMM, the same code, is 1 % faster there
+# than in mid-line (q4f16_1, N = 22016, K = 4096, M = 8192: 1287 against 1302 us).  Not for the other sources: the loops of
+# the small-batch kernel are up to 2 % slower with it, as often as they are faster.
+SOURCE_FLAGS = {name: ["-falign-loops=64"] for name in ("q4g32_gemm.hip", "intb_gemm.hip")}
 
 
 def sources():
@@ -38,7 +40,7 @@ def sources():
 
 def _compile(src: str) -> str:
     obj = os.path.join(OBJDIR, os.path.basename(src) + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", src, "-o", obj]
+    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(os.path.basename(src), ()), "-c", src, "-o", obj]
     if src.endswith(".cc"):
         cmd.insert(1, "-x")
         cmd.insert(2, "hip")
