@@ -54,7 +54,6 @@ struct Q4G32SkinnyPolicy {
 // past S.)
 struct Q4G32OddGroupsSkinnyPolicy : Q4G32SkinnyPolicy {
   static constexpr bool kCanScaleBlock = false;
-  static constexpr bool kMaskTail = true;
   struct Lane : Q4G32SkinnyPolicy::Lane {
     int odd;  // parity of the row
   };

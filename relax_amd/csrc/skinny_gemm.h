@@ -63,19 +63,11 @@ typedef void __attribute__((address_space(3))) * wq_sk_lptr_t;
 //   sblock_addr(lane, g)       address of scale g of the lane's column (g % 8 == 0)       (kCanScaleBlock)
 //   scale_block_ok(args, K)    host: every 8 scales of a column are 16 aligned bytes      (kCanScaleBlock)
 //   pair_aligned(args)         host: whether those pairs are 4-byte aligned
-// and, where K may end inside the two halves of a 64-k piece,
-//   kMaskTail                  true: the activations that meet weights past K are zeroed as well (they are
-//                              other values of the row, and 0 * inf is not 0)
 // and, for weights that are not rounded (up to 8 rows, kPieces == 1),
 //   codes8(word)               the codes of a word of codes as halves, exact (8 consecutive k); the products of a
 //                              group of 32 k are summed alone and scaled in fp32
 constexpr int kScaleBlockMaxK = 11264;  // a column block's scales for all of K stay in LDS: K bytes
 inline int scale_block_stride(int K) { return ((K + 1023) >> 10) << 10; }
-
-template <class P, class = void>
-struct MaskTail : std::false_type {};
-template <class P>
-struct MaskTail<P, std::void_t<decltype(P::kMaskTail)>> : std::bool_constant<P::kMaskTail> {};
 
 template <class P, class = void>
 struct GroupSums : std::false_type {};
@@ -122,6 +114,12 @@ __device__ __forceinline__ void mul_group_sums(float4_t& acc, const typename Pol
   }
 }
 
+// What the slab holds past K, where the K-steps do not come out even among the wavefronts that share them: the
+// weights there are exact zeros, and zero times an infinite activation is not zero.  Zeros by address, because the loop
+// can take no more: a test or masks around the products cost up to 16 %, a last iteration of its own up to 11 %, this
+// 0.3 % on average over seven such (N, K) (4 % at most: AutoGPTQ, N = 4096, K = 11008, M = 48: 25.5 -> 26.6 us).
+static __device__ const uint4_t kZeroChunk = {0, 0, 0, 0};
+
 template <typename Policy, int TH, int NW, int WAVES, bool SB = false>
 struct SkinnyCfg {
   static constexpr int KW = WAVES / NW;
@@ -156,7 +154,7 @@ __device__ __forceinline__ void wait_newer_groups(int groups) {
   }
 }
 
-template <typename Policy, typename Epilogue, int TH, int NW, int WAVES, bool SB>
+template <typename Policy, typename Epilogue, int TH, int NW, int WAVES, bool SB, bool EVEN>
 __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
     typename Policy::Args pargs, const half_t* __restrict__ X, half_t* __restrict__ Y, Epilogue epi,
     int M, int N, int K, int stages) {
@@ -204,9 +202,17 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
 #pragma unroll
     for (int i = 0; i < Cfg::kXLoads; ++i) {
       const int kchunk = ks * 16 + x_chunk[i];     // 16-byte chunk index along the row
-      const int64_t off = (kchunk * 8 < K) ? (int64_t)kchunk * 16 : 0;
+      const char* src;
+      if constexpr (EVEN) {
+        // always inside the row; without the test the compiler puts the LDS reads of the loop one behind the other in
+        // some arrangements (q4f16_1, N = 22016, K = 4096, M = 64: 32.1 -> 36.6 us)
+        const int64_t off = (kchunk * 8 < K) ? (int64_t)kchunk * 16 : 0;
+        src = x_row[i] + off;
+      } else {
+        src = kchunk * 8 < K ? x_row[i] + (int64_t)kchunk * 16 : reinterpret_cast<const char*>(&kZeroChunk);
+      }
       __builtin_amdgcn_global_load_lds(
-          (wq_sk_gptr_t)(x_row[i] + off),
+          (wq_sk_gptr_t)src,
           (wq_sk_lptr_t)(lds + stage_off + kw * Cfg::kSlabBytes + (nw * Cfg::kXLoads + i) * 1024), 16, 0, 0);
     }
 #pragma unroll
@@ -230,8 +236,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       const int k0 = 128 * (it * KW + kw);
       const int row = lj < Cfg::kRows ? lj : lj & 7;
       mul_group_sums<Policy>(acc[0], pl, w_area + stage_off, s_area + stage_off, lj, kq, live_groups(k0, K, 4), 0, [&](int g) {
-        const half8_t v = *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * g + kq) ^ (row & 15)) << 4));
-        return k0 + 32 * g < K ? v : half8_t{};
+        return *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * g + kq) ^ (row & 15)) << 4));
       });
       return;
     }
@@ -257,8 +262,8 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       for (int i = 0; i < TM; ++i) {
         // rows past the slab (M <= 8 uses half a tile) re-read a held row: never stored
         const int row = (16 * i + lj < Cfg::kRows) ? 16 * i + lj : 16 * i + (lj & 7);
-        half8_t aop = *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * kq + t) ^ (row & 15)) << 4));
-        if constexpr (MaskTail<Policy>::value) aop = k0 < K ? aop : half8_t{};
+        const half8_t aop =
+            *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * kq + t) ^ (row & 15)) << 4));
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, bop[t], acc[i], 0, 0, 0);
       }
     }
@@ -538,21 +543,21 @@ inline SkinnyTuning skinny_tuning() {
   return SkinnyTuning{t.skinny_nw, t.skinny_stages, t.skinny_waves};
 }
 
-template <typename Policy, typename Epilogue, int TH, int NW, int WAVES, bool SB = false>
-static int launch_skinny(const char* who, const typename Policy::Args& pargs, const uint16_t* x, uint16_t* y,
-                         const Epilogue& epi, int64_t M, int64_t N, int64_t K, int want_stages,
-                         hipStream_t stream) {
+template <typename Policy, typename Epilogue, int TH, int NW, int WAVES, bool SB, bool EVEN>
+static int launch_skinny_form(const char* who, const typename Policy::Args& pargs, const uint16_t* x, uint16_t* y,
+                              const Epilogue& epi, int64_t M, int64_t N, int64_t K, int want_stages,
+                              hipStream_t stream) {
   // one fetch of all scales where the policy allows it and the block is small (two column
   // blocks at most: more would cost a workgroup per CU)
   if constexpr (!SB && Policy::kCanScaleBlock && NW <= 2) {
     if (K <= kScaleBlockMaxK && Policy::scale_block_ok(pargs, K) &&
         2 * SkinnyCfg<Policy, TH, NW, WAVES, true>::kStageBytes + NW * scale_block_stride((int)K) <=
             kSkinnyLdsBudget)
-      return launch_skinny<Policy, Epilogue, TH, NW, WAVES, true>(who, pargs, x, y, epi, M, N, K, want_stages,
-                                                                  stream);
+      return launch_skinny_form<Policy, Epilogue, TH, NW, WAVES, true, EVEN>(who, pargs, x, y, epi, M, N, K,
+                                                                             want_stages, stream);
   }
   using Cfg = SkinnyCfg<Policy, TH, NW, WAVES, SB>;
-  auto kern = skinny_gemm_kernel<Policy, Epilogue, TH, NW, WAVES, SB>;
+  auto kern = skinny_gemm_kernel<Policy, Epilogue, TH, NW, WAVES, SB, EVEN>;
   const int64_t blocks = (N + 16 * NW - 1) / (16 * NW);
   int stages = want_stages;
   if (stages > Cfg::kMaxAhead + 1) stages = Cfg::kMaxAhead + 1;
@@ -568,6 +573,20 @@ static int launch_skinny(const char* who, const typename Policy::Args& pargs, co
   WQ_LAUNCH(who, kern, dim3((unsigned)blocks), dim3(64 * WAVES), lds_bytes, stream, pargs,
             (const half_t*)x, (half_t*)y, epi, (int)M, (int)N, (int)K, stages);
   return WQ_OK;
+}
+
+// EVEN: K is whole steps for every wavefront (K % (128 * KW) == 0), so that nothing lies past it.
+template <typename Policy, typename Epilogue, int TH, int NW, int WAVES>
+static int launch_skinny(const char* who, const typename Policy::Args& pargs, const uint16_t* x, uint16_t* y,
+                         const Epilogue& epi, int64_t M, int64_t N, int64_t K, int want_stages,
+                         hipStream_t stream) {
+  if constexpr (!GroupSums<Policy>::value) {  // (those are for K % 64 == 32)
+    if (K % (128 * (WAVES / NW)) == 0)
+      return launch_skinny_form<Policy, Epilogue, TH, NW, WAVES, false, true>(who, pargs, x, y, epi, M, N, K,
+                                                                              want_stages, stream);
+  }
+  return launch_skinny_form<Policy, Epilogue, TH, NW, WAVES, false, false>(who, pargs, x, y, epi, M, N, K,
+                                                                           want_stages, stream);
 }
 
 // Picks the arrangement from the shape (timings of the Llama-7B layer shapes): few

@@ -167,6 +167,23 @@ def test_one_hot_rows_reproduce_the_dequantized_weight(ops, u, oracle, M):
         assert np.max(np.abs(got.astype(np.float64) - B[ks].astype(np.float64))) <= 2.0**-10 * np.max(np.abs(B))
 
 
+@pytest.mark.parametrize("M,K", [(3, 384), (16, 11008), (40, 384), (100, 11008)])
+def test_infinite_activations_where_the_steps_do_not_come_out_even(ops, u, M, K):
+    """The small-batch kernel multiplies the first activations of a row once, not again by the zero weights past K."""
+    import torch
+
+    N, gs = 64, 128
+    w = ops.gptq_prepare(torch.full((K // 8, N), 0x66666666, dtype=torch.int32, device="cuda"),
+                         torch.full((K // gs, N // 8), 0x11111111, dtype=torch.int32, device="cuda"),
+                         torch.full((K // gs, N), 0.01, dtype=torch.float16, device="cuda"),
+                         torch.arange(K, dtype=torch.int32, device="cuda") // gs)
+    x = np.random.default_rng(M).standard_normal((M, K)).astype(np.float16)
+    x[1, 0], x[2, 7] = np.inf, -np.inf
+    got = u.host(ops.gptq_linear(w, u.dev(x)))
+    assert np.all(got[1] == np.inf) and np.all(got[2] == -np.inf)
+    assert np.all(np.isfinite(got[3:])) and np.all(np.isfinite(got[0]))
+
+
 def test_linear_argument_errors(ops, u, oracle):
     from relax_amd import _lib
     from relax_amd._lib import WqError

@@ -345,6 +345,25 @@ def test_grouped_gemv_with_scales_at_any_alignment(ops, u, oracle, nbit):
     u.assert_close(u.host(got_a), ref, f"grouped gemv int{nbit}")
 
 
+@pytest.mark.parametrize("K", [192, 11008])
+@pytest.mark.parametrize("group_size", [-1, 64])
+@pytest.mark.parametrize("nbit", [8, 4])
+def test_infinite_activations_where_the_steps_do_not_come_out_even(ops, u, nbit, group_size, K):
+    """The small-batch kernel multiplies the first activations of a row once, not again by the zero weights past K."""
+    import torch
+
+    N = 128
+    q = torch.full((K, N if nbit == 8 else N // 2), 3 if nbit == 8 else 0x33, dtype=torch.int8, device="cuda")
+    B = ops.ft_preprocess_weight(q, 80, nbit == 4)
+    s = torch.full((N,) if group_size <= 0 else (K // 64, N), 0.01, dtype=torch.float16, device="cuda")
+    for M in (3, 16, 40, 64, 96):
+        x = np.random.default_rng(M).standard_normal((M, K)).astype(np.float16)
+        x[1, 0], x[2, 7] = np.inf, -np.inf
+        got = u.host(ops.fpA_intB_gemm(u.dev(x), B, s, weight_nbit=nbit, group_size=group_size))
+        assert np.all(got[1] == np.inf) and np.all(got[2] == -np.inf), M
+        assert np.all(np.isfinite(got[3:])) and np.all(np.isfinite(got[0])), M
+
+
 @pytest.mark.parametrize("M", [1, 40, 300])
 def test_gelu_over_its_range(ops, u, M):
     """x[m] = (v, 0, ...), w = 1: gelu(v) itself, against 64 bits.  Bound: the rounding to fp16 (2^-11 of the value,

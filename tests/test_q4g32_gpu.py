@@ -367,6 +367,19 @@ def test_infinite_activations_under_half_a_step(ops, u, oracle, M, N):
     assert np.all(np.isfinite(got[3:])) and np.all(np.isfinite(got[0]))
 
 
+# K-steps of 128 that leave some wavefronts of a workgroup with half a step, or with one step less than the others
+@pytest.mark.parametrize("K", [192, 4032, 11008])
+@pytest.mark.parametrize("M,N", [(3, 64), (16, 130), (40, 70), (64, 4096)])
+def test_infinite_activations_where_the_steps_do_not_come_out_even(ops, u, oracle, M, N, K):
+    """The first activations of a row are not multiplied a second time, by the zero weights past K."""
+    x, W, S = oracle.make_q4g32_inputs(M, N, K, seed=3)
+    codes = np.random.default_rng(1).integers(8, 16, size=(N, K)).astype(np.uint8)  # no zero weight
+    x[1, 0], x[2, 7] = np.inf, -np.inf
+    got = u.host(ops.q4g32_linear(u.dev(oracle.q4_pack(codes)), u.dev(S), u.dev(x)))
+    assert np.all(got[1] == np.inf) and np.all(got[2] == -np.inf)
+    assert np.all(np.isfinite(got[3:])) and np.all(np.isfinite(got[0]))
+
+
 # the ring kernel (1 .. 2 column blocks side by side) and the one with the activations in registers
 @pytest.mark.parametrize("N,K", [(514, 4064), (8194, 1056), (16384, 4128), (16386, 8160), (514, 11040)])
 @pytest.mark.parametrize("M", [2, 3, 8])
