@@ -206,9 +206,12 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
     // small-batch kernel (64 rows, then the rest) are faster: n <= 4096 (int8, k = 11008, m = 128: 70 -> 55 us;
     // k = 4096: 28.4 -> 26.9 us), and up to 96 rows of a long, moderately wide one (k = 13824, n = 5120, m = 96:
     // 88 -> 75 us; k = n = 8192: 54 -> 50 us).  Wider matrices keep the GEMM (n = 11008, k = 4096: 31 against 36 us),
-    // and more than 96 rows where the GEMM may halve K (n = 4096, k = 11008, m = 128: int8 56 -> 48 us, int4 58 -> 42).
+    // and more than 96 rows where the GEMM may halve K (n = 4096, k = 11008, m = 128: int8 56 -> 48 us, int4 58 -> 42),
+    // save int8 with a scale per 64, whose two passes are the faster form again above k = 8192 (n = 1024, m = 128,
+    // two passes / GEMM: k = 4096 24.6 / 22.7, k = 8192 41.2 / 40.8, k = 11008 52.7 / 54.1, k = 28672 119 / 134 us).
+    const bool halves = k % 128 == 0 && !(nbit == 8 && group && k > 8192);
     if (m <= 2 * WQ_SMALL_BATCH_MAX_M && small_ok &&
-        ((n <= 4096 && (m <= 96 || k % 128 != 0)) || (m <= 96 && n <= 8192 && k >= 8192))) {
+        ((n <= 4096 && (m <= 96 || !halves)) || (m <= 96 && n <= 8192 && k >= 8192))) {
       const int64_t m0 = WQ_SMALL_BATCH_MAX_M;
       if (int rc = intb_small_batch_dispatch(A, B, scales, C, m0, n, k, group, nbit, ep, stream)) return rc;
       IntbEpilogue ep2 = ep;

@@ -165,10 +165,11 @@ def test_one_and_two_rows_on_either_kernel(ops, u, oracle, nbit, group_size, row
 
 @pytest.mark.parametrize("nbit", [8, 4])
 def test_65_to_128_rows_in_two_small_batch_passes(ops, u, oracle, nbit):
-    """65 .. 128 rows of a small matrix run as two passes of the small-batch kernel (64 rows, then the rest), wider
-    ones as a tiled GEMM: both sides of the rule, with an epilogue that reads per-row operands."""
-    for M, N, K, g in [(65, 4096, 256, -1), (128, 1024, 1024, 64), (96, 5120, 8192, -1), (97, 5120, 8192, -1),
-                       (128, 4160, 512, 64)]:
+    """65 .. 96 rows of a small matrix, and up to 128 where a GEMM cannot halve K or (int8, a scale per 64, long K) gains
+    nothing by it, run as two passes of the small-batch kernel (64 rows, then the rest), others as a tiled GEMM: both
+    sides of the rule, with an epilogue that reads per-row operands."""
+    for M, N, K, g in [(65, 4096, 256, -1), (96, 1024, 1024, 64), (128, 1024, 1024, 64), (100, 512, 192, 64),
+                       (128, 1024, 8320, 64), (96, 5120, 8192, -1), (97, 5120, 8192, -1), (128, 4160, 512, 64)]:
         print(f"intb two passes nbit={nbit} M={M} N={N} K={K} g={g}", flush=True)
         _run(ops, u, oracle, M, N, K, nbit, seed=M + N, group_size=g, bias="full")
         _run(ops, u, oracle, M, N, K, nbit, seed=M + N + 1, group_size=g, bias="row", residual=True, binary_op="multiply")
