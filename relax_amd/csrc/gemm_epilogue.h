@@ -18,8 +18,9 @@
 //   float   activate(float acc, float column_bias, int m, int n)
 //                                  (the columns of such a format come in eights: its rows have no tail)
 // That pass is a rolled loop over LDS: inlined next to each of the 64 .. 256 accumulators of a lane it was
-// megabytes of code, and eight at a time spilled (int8, K = 8192, N = 28672, M = 500: gelu 342 -> 271 us, silu
-// 319 -> 266 us, of which 256 x 256 tiles, which now can take these calls, are most; identity 240 us).
+// megabytes of code, and eight at a time spilled.  With it 256 x 256 tiles can take these calls, which is most of the gain
+// (int8, K = 8192, N = 28672, M = 500, with the branch-free erf of wq_device.h: gelu 339 -> 249 us, silu 316 -> 251 us,
+// bias alone 234 us).
 #ifndef RELAX_AMD_CSRC_GEMM_EPILOGUE_H_
 #define RELAX_AMD_CSRC_GEMM_EPILOGUE_H_
 

@@ -218,9 +218,9 @@ static int launch_mfma_gemm_cfg(int cfg, const char* who, const typename Loader:
 
 // Tile shape from the problem shape, from timings at M = 96 .. 2048 of the Llama-7B shapes
 // (format A) and of K = 8192, N = 28672 (format B): what matters at mid M is the number of
-// tiles against 256 CUs.  Register-staged kernel (fine-grained format B, and format A when K is
-// not a multiple of 64): 64x128 up to M = 128, 128x128 up to 256, else 128x256.  Fully
-// LDS-staged kernel: 128x128 tiles, two workgroups per CU (17) up to M = 384, above that
+// tiles against 256 CUs.  Register-staged kernel (scales that are not 4-byte aligned): 64x128 up to
+// M = 128, 128x128 up to 256, else 128x256.  Fully LDS-staged kernel: 128x128 tiles, two workgroups per CU (17)
+// up to M = 384, above that
 // 256x256 with one wavefront per SIMD (11), except for narrow matrices at moderate M, where
 // 256x128 tiles (13) give the CUs twice as many tiles (N = 4096, K = 11008, M = 1024: 140 -> 131 us).
 inline int choose_gemm_cfg(int64_t M, int64_t N, bool lds_staged) {

@@ -11,7 +11,8 @@
 //       base + 16*l);
 //   B   BN columns x 32 or 64 B of packed codes, still packed, in the order the weight
 //       format's policy fetches them;
-//   S   (format A only) BN x 4 B: the two scales of the step.
+//   S   (formats with a scale per group) BN x 4 B: the two scales of the step, or the pair of a group; BN x 8 B where
+//       the two scales straddle aligned words (format A, K % 64 == 32).
 // A wavefront then reads, per K-step, TM*4 activation fragments, and per weight
 // sub-tile its 32 codes (16 or 32 bytes) plus one scale: MFMA lane (j, h) needs 8
 // K-values of column j per MFMA, so the weights are dequantized in registers by the
@@ -445,7 +446,9 @@ inline double lds_cfg_cost(int cfg, int64_t M, int64_t N, int64_t K, bool activa
 // Configuration 19: 128 x 128 tiles with the K-steps of a tile split between two sets of wavefronts (KW = 2), for
 // launches that have no more such tiles than CUs.  Against the fastest of 17, 18 and 11: int8, K = 8192, N = 28672,
 // M = 128 93 -> 85 us; K = 4096, N = 11008, M = 200 41.5 -> 35.2 us, int4 38.7 -> 32.8 us; N = K = 1024, M = 128
-// 9.4 -> 7.9 us; over five such shapes, M = 70 .. 1024, 1 .. 28 % (one 3 % slower: int8, N = K = 8192, M = 128).
+// 9.4 -> 7.9 us; over five such shapes, M = 70 .. 1024, 1 .. 28 %.  Slower at one of them only, int8, N = K = 8192,
+// M = 100 .. 128 (55.0 -> 55.8 us: rows of weights a power of two apart, read by a row slice on every CU); its neighbours
+// gain as elsewhere (N = 7936 53.2 -> 47.1, N = 8320 57.3 -> 42.8, K = 8320 53.8 -> 43.2 us), which leaves no rule to draw.
 inline bool lds_k_halves(int64_t M, int64_t N, int64_t K, int cus) {
   return K % 128 == 0 && ((M + 127) / 128) * ((N + 127) / 128) <= cus;
 }

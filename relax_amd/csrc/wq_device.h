@@ -156,8 +156,8 @@ __device__ __forceinline__ void u4_word_minus8(uint32_t w, half2_t out[4]) {
 // 1 + erf(v / sqrt(2)) = erfc(-v / sqrt(2)), without a branch: with s = |v|, erfc(s / sqrt(2)) =
 // exp(-s^2 / 2) * erfcx(s / sqrt(2)), and log2 of the second factor is smooth: a polynomial of degree 10, fitted here
 // by weighted least squares on [0, 6.5], beyond which gelu is below half the smallest fp16 number.
-// The library's erff runs both of its branches for every wavefront: a gelu over the identity cost 10 us at M = 128 and
-// 23 us at M = 500 (int8, K = 8192, N = 28672), with this 0 and 17.  Against 64 bits over |v| <= 12 the gelu is off by
+// The library's erff runs both of its branches for every wavefront; this costs what silu does (the figures are in
+// gemm_epilogue.h).  Against 64 bits over |v| <= 12 the gelu is off by
 // 3.8e-7 at most (with erff 4.5e-7) and 5.0e-8 root mean square (5.6e-8); in the lower tail, where 1 + erff cancels,
 // by 1e-5 of its value down to v = -5.5 (erff: 0.6).
 __device__ __forceinline__ float one_plus_erf(float v) {
