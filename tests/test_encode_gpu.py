@@ -82,13 +82,33 @@ def test_q4g32_encode_halves_and_ragged_sizes(ops, u, oracle, N, K, top):
     halves = (rng.integers(-7, 7, size=(N, K // 32, 31)) + 0.5) * np.float64(scale)
     Wf[..., 1:] = np.clip(halves.astype(np.float16), -np.float16(top), np.float16(top))
     pick = rng.integers(0, 3, size=Wf.shape)
-    near = np.where(pick == 1, np.nextafter(Wf, np.float16(0)), Wf)
-    Wf[..., 1:] = near[..., 1:]
+    with np.errstate(over="ignore"):  # above the largest fp16 number: clipped below
+        beyond = np.nextafter(Wf, np.copysign(np.float16(np.inf), Wf))
+    near = np.where(pick == 1, np.nextafter(Wf, np.float16(0)), np.where(pick == 2, beyond, Wf))
+    Wf[..., 1:] = np.clip(near[..., 1:], -np.float16(top), np.float16(top))
     Wf = Wf.reshape(N, K)
     W, S = ops.q4g32_encode(u.dev(Wf))
     W_ref, S_ref = oracle.q4g32_encode(Wf)
     np.testing.assert_array_equal(u.host(W).view(np.uint32), W_ref)
     np.testing.assert_array_equal(u.host(S).view(np.uint16), S_ref.view(np.uint16))
+
+
+def test_q4g32_encode_non_finite_values(ops, u):
+    """A NaN does not count for the maximum of its group and gets code 0; beside an infinity (an infinite scale) finite
+    values are 0, code 7, and the infinity itself (infinity over infinity) gets code 0.  Other groups are not touched."""
+    Wf = np.full((2, 128), 3.5, dtype=np.float16)
+    Wf[:, 1] = 7.0
+    Wf[0, 5], Wf[1, 40], Wf[1, 64:96] = np.nan, np.inf, np.nan
+    Wf[1, 41] = -np.inf
+    W, S = ops.q4g32_encode(u.dev(Wf))
+    codes = ((u.host(W).view(np.uint32)[:, :, None] >> (4 * np.arange(8, dtype=np.uint32))) & 15).reshape(2, 128)
+    want = np.full((2, 128), 14)
+    want[:, :32] = 11  # 3.5 with a scale of 1: a half, away from zero
+    want[:, 1] = 14
+    want[0, 5], want[1, 32:64], want[1, 40:42], want[1, 64:96] = 0, 7, 0, 0
+    np.testing.assert_array_equal(codes, want)
+    tiny, half = np.float16(np.float32(1e-4) / np.float32(7)), np.float16(0.5)
+    np.testing.assert_array_equal(u.host(S), np.array([[1, half, half, half], [1, np.inf, tiny, half]], np.float16))
 
 
 @pytest.mark.parametrize("nbit,group_size", [(8, -1), (4, -1), (8, 64), (4, 64)])

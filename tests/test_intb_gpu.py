@@ -212,7 +212,7 @@ def test_one_row_of_a_narrow_matrix(ops, u, oracle, nbit):
 @pytest.mark.parametrize("nbit", [8, 4])
 def test_gemm_tile_configurations(ops, u, oracle, nbit, cfg):
     """every tile shape of the register-staged (1-4) and the LDS-staged (11, 12, 17, 18) kernel, ragged M,
-    N smaller than a tile, with and without the row-wise epilogue (bias stride not a multiple of 8)."""
+    N smaller than a tile, a bias per row and one per element."""
     from relax_amd import _lib
 
     _lib.lib().wq_debug_set_gemm_config(cfg)
@@ -230,6 +230,53 @@ def test_gemm_tile_configurations(ops, u, oracle, nbit, cfg):
         _run(ops, u, oracle, 100, 128, 256, nbit, seed=cfg + 2, group_size=64, bias="row", activation="relu")
     finally:
         _lib.lib().wq_debug_set_gemm_config(0)
+
+
+@pytest.mark.parametrize("cfg", [4, 11, 17, 18, 19])
+@pytest.mark.parametrize("activation", ["identity", "relu", "silu", "gelu"])
+def test_gemm_epilogue_operands_at_any_address_and_stride(ops, u, oracle, cfg, activation):
+    """A bias per element with rows of N and of N + 3 halves, and bias, residual and output one half off a 16-byte
+    boundary; nothing before or behind the output is written."""
+    import torch
+    from relax_amd import _lib
+
+    M, N, K = 300, 192, 256
+    rng = np.random.default_rng(cfg)
+    x, A, s = oracle.make_intb_inputs(M, N, K, 8, seed=cfg)
+    P, dx, ds = ops.ft_preprocess_weight(u.dev(A), 80, False), u.dev(x), u.dev(s)
+    row, res = rng.standard_normal(N).astype(np.float16), rng.standard_normal((M, N)).astype(np.float16)
+
+    def off(a):  # the same values, two bytes off
+        buf = torch.zeros(a.size + 8, dtype=torch.float16, device="cuda")
+        buf[1:1 + a.size] = u.dev(a).reshape(-1)
+        return buf
+
+    L, act = _lib.lib(), ops.ACTIVATIONS[activation]
+    L.wq_debug_set_gemm_config(cfg)
+    try:
+        for stride in (N, N + 3):
+            full = rng.standard_normal((M, stride)).astype(np.float16)
+            b, y = off(full), torch.zeros(M * N + 16, dtype=torch.float16, device="cuda")
+            rc = L.wq_fpA_intB_gemm(dx.data_ptr(), P.data_ptr(), ds.data_ptr(), b[1:].data_ptr(), y[9:].data_ptr(), act, M, N,
+                                    K, -1, stride, 8, 0, 0, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0
+            ref = oracle.intb_linear(x, A, s, 8, bias=np.ascontiguousarray(full[:, :N]), bias_stride=N,
+                                     activation=activation, nthreads=8)
+            got = u.host(y)
+            u.assert_close(got[9:9 + M * N].reshape(M, N), ref, f"cfg {cfg} {activation} stride {stride}")
+            assert not got[:9].any() and not got[9 + M * N:].any()
+        b, r, y = off(row), off(res), torch.zeros(M * N + 16, dtype=torch.float16, device="cuda")
+        rc = L.wq_fpA_intB_gemm_residual(dx.data_ptr(), P.data_ptr(), ds.data_ptr(), b[1:].data_ptr(), r[1:].data_ptr(),
+                                         y[9:].data_ptr(), act, ops.BINARY_OPS["plus"], ops.UNARY_OPS["relu"], M, N, K, -1, 8,
+                                         0, 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        ref = oracle.intb_linear(x, A, s, 8, bias=row, residual=res, activation=activation, binary_op="plus",
+                                 unary_op="relu", nthreads=8)
+        got = u.host(y)
+        u.assert_close(got[9:9 + M * N].reshape(M, N), ref, f"cfg {cfg} {activation} residual")
+        assert not got[:9].any() and not got[9 + M * N:].any()
+    finally:
+        L.wq_debug_set_gemm_config(0)
 
 
 # K of one step per set of wavefronts, of fewer steps than the ring has slots, and of more

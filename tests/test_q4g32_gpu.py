@@ -267,8 +267,8 @@ def test_two_pass_small_batch_for_mid_m(ops, u, oracle):
 
 
 def test_gemm_row_wise_and_element_wise_epilogues_agree(ops, u, oracle):
-    """The GEMM stores 16 bytes per lane when N % 8 == 0 and y / residual are 16-byte aligned, single
-    elements otherwise: both paths, same numbers."""
+    """The GEMM stores eight columns per lane at any half's address: y and residual on a 16-byte boundary and two
+    bytes off one, same numbers."""
     import torch
 
     M, N, K = 300, 520, 1024
