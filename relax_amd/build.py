@@ -28,10 +28,7 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-# Loops on instruction cache lines: the main loop of the 256 x 256 tile of the MFMA GEMM, the same code, is 1 % faster there
-# than in mid-line (q4f16_1, N = 22016, K = 4096, M = 8192: 1287 against 1302 us).  Not for the other sources: the loops of
-# the small-batch kernel are up to 2 % slower with it, as often as they are faster.
-SOURCE_FLAGS = {name: ["-falign-loops=64"] for name in ("q4g32_gemm.hip", "intb_gemm.hip")}
+SOURCE_FLAGS = {"gemm_256.hip": ["-falign-loops=64"]}  # why: see that file
 
 
 def sources():

@@ -4,9 +4,9 @@
 // m <= 2 goes to the streaming GEMV (intb_gemv.hip), m <= 64 to the small-batch
 // kernel (intb_skinny.hip), larger m to the shared MFMA GEMM (mfma_gemm.h) with the
 // weight loaders below.
+#include "gemm_256.h"
 #include "intb_common.h"
 #include "mfma_gemm.h"
-#include "mfma_gemm_lds.h"
 
 int wq_gemm_cfg_override();
 
@@ -77,74 +77,6 @@ struct IntbLoader {
   }
 };
 
-
-// Weight policy of the fully LDS-staged kernel (mfma_gemm_lds.h) for the preprocessed layouts
-// with per-column scales.  A K-step (one 64-row tile) of I = 2 (int8) or 4 (int4) interleaved
-// columns is 128 contiguous bytes, so the B tile is fetched in whole 128-byte lines; the scale
-// of a column never changes and stays in a register.
-// GROUPED (scales fp16 [K/64, N], one per column and K-step): a lane stages the 4 bytes that hold
-// the scales of its column and the neighbouring one, and the reader takes its half.
-template <int NBIT, bool GROUPED = false>
-struct IntbLdsPolicy {
-  static constexpr int I = NBIT == 8 ? 2 : 4;
-  static constexpr int kColBytes = 128 / I;
-  static constexpr int kScaleBytes = GROUPED ? 4 : 0;
-  static constexpr int kStepStride = 128;
-  struct Args {
-    const uint4_t* B;
-    const half_t* scales;
-    int N;
-  };
-  struct Frag {
-    uint4_t w[NBIT == 8 ? 2 : 1];
-  };
-  __device__ __forceinline__ static const char* b_src(const Args& a, int n0, int q, int N, int K) {
-    const int group = min(n0 / I + (q >> 3), N / I - 1);  // columns past N re-read the last group
-    return reinterpret_cast<const char*>(a.B) + ((int64_t)group * (K >> 6)) * 128 + (q & 7) * 16;
-  }
-  using Scale = half2_t;  // the column's scale, twice
-  __device__ __forceinline__ static const char* s_src(const Args& a, int n, int) {
-    return reinterpret_cast<const char*>(a.scales + (n & ~1));  // the aligned pair of columns (N is even)
-  }
-  __device__ __forceinline__ static int64_t s_offset(const Args& a, int ks) { return (int64_t)ks * a.N * 2; }
-  // p = the 4 staged bytes of the lane's column; columns are staged 4 bytes apart from an 8-byte
-  // aligned base, so bit 2 of the address is the parity of the column
-  __device__ __forceinline__ static Scale read_scale(const unsigned char* p, int) {
-    const half2_t pair = *reinterpret_cast<const half2_t*>(p);
-    const half_t s = (reinterpret_cast<uintptr_t>(p) & 4) ? pair.y : pair.x;
-    return Scale{s, s};
-  }
-  __device__ __forceinline__ static Scale const_scale(const Args& a, int n) {
-    const half_t s = a.scales[n];
-    return Scale{s, s};
-  }
-  __device__ __forceinline__ static void read(Frag& f, const unsigned char* bslot, int n_local, int lh) {
-    if (NBIT == 8) {
-      const unsigned char* p = bslot + ((n_local >> 1) * 8 + (n_local & 1) * 4 + 2 * lh) * 16;
-      f.w[0] = *reinterpret_cast<const uint4_t*>(p);
-      f.w[NBIT == 8 ? 1 : 0] = *reinterpret_cast<const uint4_t*>(p + 16);
-    } else {
-      f.w[0] = *reinterpret_cast<const uint4_t*>(bslot + ((n_local >> 2) * 8 + (n_local & 3) * 2 + lh) * 16);
-    }
-  }
-  // int8: piece kk/2 holds 16 k; word j of it holds k = 2j, 2j+1 (bytes 0, 2) and 2j+8, 2j+9 (bytes 1, 3).
-  // int4: word j holds k = 2j + 8i, 2j + 8i + 1 in nibbles i, i + 4.
-  __device__ __forceinline__ static uint32_t pair_bits(const Frag& f, int kk, int j) {
-    if (NBIT == 8) {
-      const uint4_t& p = f.w[NBIT == 8 ? (kk >> 1) : 0];
-      const uint32_t word = j == 0 ? p.x : j == 1 ? p.y : j == 2 ? p.z : p.w;
-      return __builtin_amdgcn_perm(0x64646464u, word, (kk & 1) ? 0x04030401u : 0x04020400u);  // 1024 + u8
-    }
-    const uint32_t word = j == 0 ? f.w[0].x : j == 1 ? f.w[0].y : j == 2 ? f.w[0].z : f.w[0].w;
-    return and_or(word >> (4 * kk), 0x000F000Fu, 0x64006400u);                                // 1024 + u4
-  }
-  __device__ __forceinline__ static half2_t pair_finish(uint32_t bits, half2_t s2) {
-    const half_t o = (half_t)(NBIT == 8 ? 1152.0f : 1032.0f);  // 1024 + the bias of the stored codes
-    return (as_half2(bits) - half2_t{o, o}) * s2;
-  }
-  __device__ __forceinline__ static half2_t pair(const Frag& f, int kk, int j, half2_t s2) { return pair_finish(pair_bits(f, kk, j), s2); }
-};
-
 template <int NBIT, bool GROUPED>
 static int intb_gemm_lds(int cfg, const char* who, const int8_t* B, const uint16_t* scales, const uint16_t* A,
                          uint16_t* C, const IntbGemmEpilogue& gep, int64_t m, int64_t n, int64_t k,
@@ -152,7 +84,11 @@ static int intb_gemm_lds(int cfg, const char* who, const int8_t* B, const uint16
   using P = IntbLdsPolicy<NBIT, GROUPED>;
   const typename P::Args largs{(const uint4_t*)B, (const half_t*)scales, (int)n};
   switch (cfg) {
-    case 11: return launch_gemm_lds<P, IntbGemmEpilogue, 8, 2, 1, 4, 1>(who, largs, A, C, gep, m, n, k, stream);
+    case 11:
+      if constexpr (NBIT == 8 && !GROUPED)
+        return launch_gemm_lds<P, IntbGemmEpilogue, 8, 2, 1, 4, 1>(who, largs, A, C, gep, m, n, k, stream);
+      else
+        return intb_gemm_256<NBIT, GROUPED>(who, largs, A, C, gep, m, n, k, stream);
     case 12: return launch_gemm_lds<P, IntbGemmEpilogue, 4, 2, 1, 4, 2>(who, largs, A, C, gep, m, n, k, stream);
     case 17: return launch_gemm_lds<P, IntbGemmEpilogue, 4, 1, 1, 4, 2>(who, largs, A, C, gep, m, n, k, stream);
     case 18: return launch_gemm_lds<P, IntbGemmEpilogue, 8, 1, 1, 4, 1>(who, largs, A, C, gep, m, n, k, stream);

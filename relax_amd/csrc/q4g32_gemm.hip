@@ -3,8 +3,8 @@
 // loader for the q4f16_1 layout and the epilogue of the reference's prefill
 // PrimFunc (tests/python/dlight/test_gpu_matmul.py:378-401).
 #include "mfma_gemm.h"
+#include "gemm_256.h"
 #include "q4g32_common.h"
-#include "mfma_gemm_lds.h"
 
 namespace wq {
 
@@ -51,51 +51,7 @@ struct Q4G32Loader {
   }
 };
 
-
-// Weight policy of the fully LDS-staged kernel (mfma_gemm_lds.h) for format A: per K-step a
-// column is 32 bytes of codes (chunk (n, h) of the B tile = 16 bytes = one scale group) and two
-// scales (4 bytes, staged in LDS with the codes).
-struct Q4G32LdsPolicy {
-  static constexpr bool kFineTail = true;  // a last round of few tiles may be cut into eight row slices
-  static constexpr int kColBytes = 32;
-  static constexpr int kScaleBytes = 4;
-  static constexpr int kStepStride = 32;
-  struct Args {
-    const uint32_t* W;
-    const half_t* S;
-  };
-  struct Frag {
-    uint4_t w;
-  };
-  using Scale = half2_t;  // the group's scale, twice
-  __device__ __forceinline__ static const char* b_src(const Args& a, int n0, int q, int N, int K) {
-    const int n = q >> 1, h = q & 1;
-    return reinterpret_cast<const char*>(a.W + (int64_t)min(n0 + n, N - 1) * (K >> 3)) + h * 16;
-  }
-  __device__ __forceinline__ static const char* s_src(const Args& a, int n, int K) {
-    return reinterpret_cast<const char*>(a.S + (int64_t)n * (K >> 5));
-  }
-  __device__ __forceinline__ static int64_t s_offset(const Args&, int ks) { return (int64_t)ks * 4; }
-  __device__ __forceinline__ static Scale read_scale(const unsigned char* p, int lh) {
-    const half_t s = *reinterpret_cast<const half_t*>(p + lh * 2);
-    return Scale{s, s};
-  }
-  __device__ __forceinline__ static Scale const_scale(const Args&, int) { return Scale{(half_t)0.0f, (half_t)0.0f}; }
-  __device__ __forceinline__ static void read(Frag& f, const unsigned char* bslot, int n_local, int lh) {
-    f.w = *reinterpret_cast<const uint4_t*>(bslot + (n_local * 2 + lh) * 16);
-  }
-  __device__ __forceinline__ static uint32_t pair_bits(const Frag& f, int kk, int j) {
-    const uint32_t word = kk == 0 ? f.w.x : kk == 1 ? f.w.y : kk == 2 ? f.w.z : f.w.w;
-    return q4_pair_bits_natural(word, j);
-  }
-  __device__ __forceinline__ static half2_t pair_finish(uint32_t bits, half2_t s2) {
-    const half2_t off = {(half_t)1031.0f, (half_t)1031.0f};
-    return (as_half2(bits) - off) * s2;
-  }
-  __device__ __forceinline__ static half2_t pair(const Frag& f, int kk, int j, half2_t s2) { return pair_finish(pair_bits(f, kk, j), s2); }
-};
-
-// The same for K % 64 == 32.  A row of S then holds an odd number G of scales: in odd rows the pair of a K-step
+// Q4G32LdsPolicy for K % 64 == 32.  A row of S then holds an odd number G of scales: in odd rows the pair of a K-step
 // straddles two aligned words, so both are staged (in even rows the first one twice), and the last 32 k are half
 // a step.  Nothing past a row is read: the steps end one scale before its end, so the second word of an odd row
 // ends with that row's last scale, at the latest.
@@ -167,7 +123,7 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
   if (cfg == 19 && K % 128 != 0) cfg = 17;
   if (cfg >= 11 && K % 64 == 0 && ((uintptr_t)S & 3u) == 0) {
     switch (cfg) {
-      case 11: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 8, 2, 1, 4, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 11: return q4g32_gemm_256("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 12: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 2, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 13: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 2, 2, 2, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 14: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 4, 2, 2, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
