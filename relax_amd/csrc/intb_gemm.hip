@@ -144,7 +144,8 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
     // 88 -> 75 us; k = n = 8192: 54 -> 50 us).  Wider matrices keep the GEMM (n = 11008, k = 4096: 31 against 36 us),
     // and more than 96 rows where the GEMM may halve K (n = 4096, k = 11008, m = 128: int8 56 -> 48 us, int4 58 -> 42),
     // save int8 with a scale per 64, whose two passes are the faster form again above k = 8192 (n = 1024, m = 128,
-    // two passes / GEMM: k = 4096 24.6 / 22.7, k = 8192 41.2 / 40.8, k = 11008 52.7 / 54.1, k = 28672 119 / 134 us).
+    // two passes / GEMM: k = 4096 24.6 / 22.9, k = 8192 41.2 / 41.6, k = 11008 52.7 / 54.3, k = 28672 119 / 134 us;
+    // n = 4096, k = 8192 42.9 / 42.2).
     const bool halves = k % 128 == 0 && !(nbit == 8 && group && k > 8192);
     if (m <= 2 * WQ_SMALL_BATCH_MAX_M && small_ok &&
         ((n <= 4096 && (m <= 96 || !halves)) || (m <= 96 && n <= 8192 && k >= 8192))) {
