@@ -116,8 +116,7 @@ __device__ __forceinline__ void mul_group_sums(float4_t& acc, const typename Pol
 
 // What the slab holds past K, where the K-steps do not come out even among the wavefronts that share them: the
 // weights there are exact zeros, and zero times an infinite activation is not zero.  Zeros by address, because the loop
-// can take no more: a test or masks around the products cost up to 16 %, a last iteration of its own up to 11 %, this
-// 0.3 % on average over seven such (N, K) (4 % at most: AutoGPTQ, N = 4096, K = 11008, M = 48: 25.5 -> 26.6 us).
+// can take no more: a test or masks around the products cost up to 16 %, a last iteration of its own up to 11 %.
 static __device__ const uint4_t kZeroChunk = {0, 0, 0, 0};
 
 template <typename Policy, int TH, int NW, int WAVES, bool SB = false>
@@ -174,6 +173,10 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
   // ---- per-lane sources ----
   // slab load i of this wavefront: rows 4*li .. 4*li+3 of the slab, li = nw*kXLoads + i;
   // LDS position p of a row holds the 16-byte chunk p ^ (row & 15) (bank-conflict-free reads)
+  // kAhead: the arrangements where the choice of source below cost up to 4 % (AutoGPTQ, N = 4096, K = 11008, M = 48:
+  // 25.5 -> 26.6 us) request the operands of the next MFMAs before the last ones are multiplied and count addresses from the
+  // chunk of step 0, and are as fast as they were or faster (22.6 us); with eight wavefronts side by side that loses 5 %
+  constexpr bool kAhead = !EVEN && TH >= 4 && NW < 8;
   const char* x_row[Cfg::kXLoads];
   int x_chunk[Cfg::kXLoads];
 #pragma unroll
@@ -181,7 +184,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
     const int li = nw * Cfg::kXLoads + i;
     const int row = 4 * li + (lane >> 4);
     x_chunk[i] = (lane & 15) ^ (row & 15);
-    x_row[i] = reinterpret_cast<const char*>(X + (int64_t)min(row, M - 1) * K);
+    x_row[i] = reinterpret_cast<const char*>(X + (int64_t)min(row, M - 1) * K + (kAhead ? 8 * x_chunk[i] : 0));
   }
   typename Policy::Lane pl;
   Policy::init(pl, pargs, min(n0 + 16 * nw + lj, N - 1), K, N);  // clamped columns are never stored
@@ -208,6 +211,8 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
         // some arrangements (q4f16_1, N = 22016, K = 4096, M = 64: 32.1 -> 36.6 us)
         const int64_t off = (kchunk * 8 < K) ? (int64_t)kchunk * 16 : 0;
         src = x_row[i] + off;
+      } else if constexpr (kAhead) {
+        src = 8 * x_chunk[i] < K - 128 * ks ? x_row[i] + (int64_t)ks * 256 : reinterpret_cast<const char*>(&kZeroChunk);
       } else {
         src = kchunk * 8 < K ? x_row[i] + (int64_t)kchunk * 16 : reinterpret_cast<const char*>(&kZeroChunk);
       }
@@ -256,15 +261,33 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
     if (k0 >= K) s = Policy::null_scale();  // code * 0 = exact zero for the weights past K
     half8_t bop[4];
     Policy::dequant(pieces, s, bop);
+    // rows past the slab (M <= 8 uses half a tile) re-read a held row: never stored
+    auto a_operand = [&](int t, int i) {
+      const int row = (16 * i + lj < Cfg::kRows) ? 16 * i + lj : 16 * i + (lj & 7);
+      return *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * kq + t) ^ (row & 15)) << 4));
+    };
+    if constexpr (kAhead) {
+      half8_t aop[2][TM];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+      for (int i = 0; i < TM; ++i) aop[0][i] = a_operand(0, i);
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        // rows past the slab (M <= 8 uses half a tile) re-read a held row: never stored
-        const int row = (16 * i + lj < Cfg::kRows) ? 16 * i + lj : 16 * i + (lj & 7);
-        const half8_t aop =
-            *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * kq + t) ^ (row & 15)) << 4));
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, bop[t], acc[i], 0, 0, 0);
+      for (int t = 0; t < 4; ++t) {
+        if (t < 3) {
+#pragma unroll
+          for (int i = 0; i < TM; ++i) aop[(t + 1) & 1][i] = a_operand(t + 1, i);
+        }
+        __builtin_amdgcn_sched_barrier(0x6);  // only the unpacking may move past
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop[t & 1][i], bop[t], acc[i], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0x6);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_operand(t, i), bop[t], acc[i], 0, 0, 0);
       }
     }
   };
