@@ -24,7 +24,7 @@ struct Q4G32LdsPolicy {
   struct Frag {
     uint4_t w;
   };
-  using Scale = half2_t;  // the group's scale, twice
+  using Scale = half_t;  // the group's scale
   __device__ __forceinline__ static const char* b_src(const Args& a, int n0, int q, int N, int K) {
     const int n = q >> 1, h = q & 1;
     return reinterpret_cast<const char*>(a.W + (int64_t)min(n0 + n, N - 1) * (K >> 3)) + h * 16;
@@ -34,22 +34,19 @@ struct Q4G32LdsPolicy {
   }
   __device__ __forceinline__ static int64_t s_offset(const Args&, int ks) { return (int64_t)ks * 4; }
   __device__ __forceinline__ static Scale read_scale(const unsigned char* p, int lh) {
-    const half_t s = *reinterpret_cast<const half_t*>(p + lh * 2);
-    return Scale{s, s};
+    return *reinterpret_cast<const half_t*>(p + lh * 2);
   }
-  __device__ __forceinline__ static Scale const_scale(const Args&, int) { return Scale{(half_t)0.0f, (half_t)0.0f}; }
+  __device__ __forceinline__ static Scale const_scale(const Args&, int) { return (half_t)0.0f; }
   __device__ __forceinline__ static void read(Frag& f, const unsigned char* bslot, int n_local, int lh) {
     f.w = *reinterpret_cast<const uint4_t*>(bslot + (n_local * 2 + lh) * 16);
   }
   __device__ __forceinline__ static uint32_t pair_bits(const Frag& f, int kk, int j) {
     const uint32_t word = kk == 0 ? f.w.x : kk == 1 ? f.w.y : kk == 2 ? f.w.z : f.w.w;
-    return q4_pair_bits_natural(word, j);
-  }
-  __device__ __forceinline__ static half2_t pair_finish(uint32_t bits, half2_t s2) {
     const half2_t off = {(half_t)1031.0f, (half_t)1031.0f};
-    return (as_half2(bits) - off) * s2;
+    return as_u32(as_half2(q4_pair_bits_natural(word, j)) - off);
   }
-  __device__ __forceinline__ static half2_t pair(const Frag& f, int kk, int j, half2_t s2) { return pair_finish(pair_bits(f, kk, j), s2); }
+  __device__ __forceinline__ static half2_t pair_finish(uint32_t bits, Scale s) { return as_half2(bits) * half2_t{s, s}; }
+  __device__ __forceinline__ static half2_t pair(const Frag& f, int kk, int j, Scale s) { return pair_finish(pair_bits(f, kk, j), s); }
 };
 
 // Weight policy of the fully LDS-staged kernel (mfma_gemm_lds.h) for the preprocessed layouts
@@ -76,7 +73,7 @@ struct IntbLdsPolicy {
     const int group = min(n0 / I + (q >> 3), N / I - 1);  // columns past N re-read the last group
     return reinterpret_cast<const char*>(a.B) + ((int64_t)group * (K >> 6)) * 128 + (q & 7) * 16;
   }
-  using Scale = half2_t;  // the column's scale, twice
+  using Scale = half_t;  // the column's scale
   __device__ __forceinline__ static const char* s_src(const Args& a, int n, int) {
     return reinterpret_cast<const char*>(a.scales + (n & ~1));  // the aligned pair of columns (N is even)
   }
@@ -84,13 +81,10 @@ struct IntbLdsPolicy {
   // p = the 4 staged bytes of the lane's column; columns are staged 4 bytes apart from an 8-byte
   // aligned base, so bit 2 of the address is the parity of the column
   __device__ __forceinline__ static Scale read_scale(const unsigned char* p, int) {
-    const half2_t pair = *reinterpret_cast<const half2_t*>(p);
-    const half_t s = (reinterpret_cast<uintptr_t>(p) & 4) ? pair.y : pair.x;
-    return Scale{s, s};
+    return *reinterpret_cast<const half_t*>(p + ((reinterpret_cast<uintptr_t>(p) & 4) >> 1));
   }
   __device__ __forceinline__ static Scale const_scale(const Args& a, int n) {
-    const half_t s = a.scales[n];
-    return Scale{s, s};
+    return a.scales[n];
   }
   __device__ __forceinline__ static void read(Frag& f, const unsigned char* bslot, int n_local, int lh) {
     if (NBIT == 8) {
@@ -107,16 +101,14 @@ struct IntbLdsPolicy {
     if (NBIT == 8) {
       const uint4_t& p = f.w[NBIT == 8 ? (kk >> 1) : 0];
       const uint32_t word = j == 0 ? p.x : j == 1 ? p.y : j == 2 ? p.z : p.w;
-      return __builtin_amdgcn_perm(0x64646464u, word, (kk & 1) ? 0x04030401u : 0x04020400u);  // 1024 + u8
+      return minus(__builtin_amdgcn_perm(0x64646464u, word, (kk & 1) ? 0x04030401u : 0x04020400u), 1152.0f);  // 1024 + u8
     }
     const uint32_t word = j == 0 ? f.w[0].x : j == 1 ? f.w[0].y : j == 2 ? f.w[0].z : f.w[0].w;
-    return and_or(word >> (4 * kk), 0x000F000Fu, 0x64006400u);                                // 1024 + u4
+    return minus(and_or_b(word >> (4 * kk), 0x000F000Fu, 0x64006400u), 1032.0f);                                // 1024 + u4
   }
-  __device__ __forceinline__ static half2_t pair_finish(uint32_t bits, half2_t s2) {
-    const half_t o = (half_t)(NBIT == 8 ? 1152.0f : 1032.0f);  // 1024 + the bias of the stored codes
-    return (as_half2(bits) - half2_t{o, o}) * s2;
-  }
-  __device__ __forceinline__ static half2_t pair(const Frag& f, int kk, int j, half2_t s2) { return pair_finish(pair_bits(f, kk, j), s2); }
+  __device__ __forceinline__ static uint32_t minus(uint32_t bits, float o) { return as_u32(as_half2(bits) - half2_t{(half_t)o, (half_t)o}); }
+  __device__ __forceinline__ static half2_t pair_finish(uint32_t bits, Scale s) { return as_half2(bits) * half2_t{s, s}; }
+  __device__ __forceinline__ static half2_t pair(const Frag& f, int kk, int j, Scale s2) { return pair_finish(pair_bits(f, kk, j), s2); }
 };
 
 int q4g32_gemm_256(const char* who, const Q4G32LdsPolicy::Args& wargs, const uint16_t* x, uint16_t* y,

@@ -160,10 +160,11 @@ static int intb_gemm_common(const char* who, const uint16_t* A, const int8_t* B,
   const IntbGemmEpilogue gep{ep, (int)n};
   // the fully LDS-staged kernel: 19 where its tiles fit one round, else the tile shape (11, 17 or 18) whose rounds of
   // the machine come out shortest; fine-grained scales whose pairs are not 4-byte aligned: the register-staged kernel (1..4)
-  const bool lds_ok = !group || (reinterpret_cast<uintptr_t>(scales) & 3u) == 0;
+  // (and 32-bit offsets inside a tile, and down the rows of the scales)
+  const bool lds_ok = (!group || ((reinterpret_cast<uintptr_t>(scales) & 3u) == 0 && (k / 64) * n < (1ll << 30))) && k < kLdsGemmMaxK;
   int cfg = wq_gemm_cfg_override();
   if (!cfg && !lds_ok) cfg = choose_gemm_cfg(m, n, false);
-  if (!cfg && lds_k_halves(m, n, k, cu_count())) cfg = 19;
+  if (!cfg && lds_ok && lds_k_halves(m, n, k, cu_count())) cfg = 19;
   if (!cfg) {
     double best = 0;
     for (int c : {17, 18, 11}) {

@@ -1,9 +1,8 @@
 // Prefill GEMM, fully LDS-staged variant for the gfx950 matrix cores, both weight formats:
 //   y[m,n] = epilogue( sum_k x[m,k] * dequant(w)[n,k] )
 //
-// Every operand of a K-step (64 k) travels global -> LDS with the direct
-// global_load_lds_dwordx4 path: no staging registers, no VALU work, and the loads
-// of the next two or more steps are in flight while a step is multiplied (a ring of 3 slots, or of up to 6
+// Every operand of a K-step (64 k) travels global -> LDS with direct loads: no staging registers, no VALU work, and the
+// loads of the next two or more steps are in flight while a step is multiplied (a ring of 3 slots, or of up to 6
 // where one workgroup per CU leaves room in LDS; what pays is a 4-slot ring under 256 x 128 tiles).  Per slot:
 //   A   BM rows x 128 B of activations, 16-byte chunk c of row r at slot position
 //       c ^ ((r >> 1) & 7) (the swizzle is applied to the GLOBAL address each lane fetches,
@@ -105,8 +104,24 @@ struct HalfStep : std::false_type {};
 template <class P>
 struct HalfStep<P, std::void_t<decltype(&P::half_step)>> : std::true_type {};
 
+// Policy::kWide = true: 64-bit addresses, for a K whose byte offsets inside a tile do not fit 32 bits.
+template <class P, class = void>
+struct Wide : std::false_type {};
+template <class P>
+struct Wide<P, std::void_t<decltype(P::kWide)>> : std::bool_constant<P::kWide> {};
+// ... which they do below this one (256 rows of activations)
+constexpr int64_t kLdsGemmMaxK = 1 << 23;
+
 typedef const void __attribute__((address_space(1))) * wq_gptr_t;
 typedef void __attribute__((address_space(3))) * wq_lptr_t;
+// The direct loads are buffer loads and not global_load_lds: behind one of those, which may touch either memory, the
+// compiler waits for ALL outstanding LDS reads and loads wherever it waits for one.
+typedef __amdgpu_buffer_rsrc_t wq_rsrc_t;
+// Raw buffer descriptor from `base` on, which must be the same for the whole wavefront.  With `live` 0 instead of -1 nothing
+// lies inside it: a load brings zeros and touches no memory.
+__device__ __forceinline__ wq_rsrc_t wq_rsrc(const char* base, int live) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, live, 0x00027000);
+}
 
 // One output tile of TME*32*WM rows x BN columns starting at (m0, n0).  TME is the
 // number of 32-row sub-tiles per wavefront that are actually computed: TM for a full
@@ -124,6 +139,12 @@ typedef void __attribute__((address_space(3))) * wq_lptr_t;
 //               and s_barrier (everyone's have); then, between its MFMAs, the packed
 //               weights, the first activation fragments and the first weight pairs of
 //               step ks+1, so that step ks+1 starts multiplying at once.
+// The K loop is one basic block: the loads past the last step are issued too, against a descriptor that holds nothing, so
+// that the waits are constants.  Branches around them cost more than themselves, since the compiler moves the unpacking
+// across the end of a block, behind the barrier.  With buffer loads, the integers of a pair finished in its first slot and
+// no wait for the scale in front of phase 3: 540 -> 308 instructions per step, N = 22016, K = 4096, M = 8192 1292 -> 1207 us,
+// int4 N = 28672, K = 8192, M = 500 232 -> 219 us, N = 11008, K = 4096, M = 200 36.4 -> 35.4 us.
+//
 // One barrier per K-step suffices (three slots shown): slot (ks+2)%3 = (ks-1)%3 is refilled by loads issued after
 // the barrier of step ks-1, and every wavefront has waited for its last LDS reads of that slot
 // (the phase-3 fragments of step ks-1) before that barrier.
@@ -154,40 +175,55 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
   unsigned char* const lds_all = lds;
   lds += set * Cfg::kLdsBytes;
 
-  // ---- global sources of this lane's direct loads (rows past M / N are clamped:
-  //      they only feed accumulators that are never stored) ----
-  const char* a_src[kALoadsE];
+  // ---- global sources of this lane's direct loads: buffer descriptors at the tile's first row and column, byte offsets
+  //      from there (rows past M / N are clamped: they only feed accumulators that are never stored) ----
+  const char* const a_base = reinterpret_cast<const char*>(X + (int64_t)m0 * K);
+  using Off = std::conditional_t<Wide<Policy>::value, int64_t, uint32_t>;
+  Off a_off[kALoadsE];
 #pragma unroll
   for (int i = 0; i < kALoadsE; ++i) {
     const int s = (wave * kALoadsE + i) * 64 + lane;  // LDS chunk slot
     const int r = s >> 3, c = (s & 7) ^ WQ_SWZ(r);
-    a_src[i] = reinterpret_cast<const char*>(X + (int64_t)min(m0 + r, M - 1) * K) + c * 16;
+    a_off[i] = (Off)(min(m0 + r, M - 1) - m0) * (Off)(2 * (int64_t)K) + c * 16;
   }
-  const char* b_src[Cfg::kBLoads];
+  const char* const b_base = Policy::b_src(wargs, n0, 0, N, K);
+  Off b_off[Cfg::kBLoads];
 #pragma unroll
   for (int i = 0; i < Cfg::kBLoads; ++i)
-    b_src[i] = Policy::b_src(wargs, n0, (wave * Cfg::kBLoads + i) * 64 + lane, N, K);
+    b_off[i] = (Off)(Policy::b_src(wargs, n0, (wave * Cfg::kBLoads + i) * 64 + lane, N, K) - b_base);
   // scales staged per step (format A): 64 columns per wavefront (with BN = 128 wavefronts 2
   // and 3 repeat the loads of wavefronts 0 and 1)
-  const char* s_src[2] = {nullptr, nullptr};
+  const char* s_base = b_base;
+  Off s_off[2] = {0, 0};
   const int s_col = min(n0 + (wave * 64) % Cfg::BN + lane, N - 1);
-  if (Cfg::kSLoads) s_src[0] = Policy::s_src(wargs, s_col, K);
-  if constexpr (Cfg::kSLoads == 2) s_src[1] = Policy::s_src2(wargs, s_col, K);
+  if constexpr (Cfg::kSLoads > 0) {
+    s_base = Policy::s_src(wargs, n0, K);
+    s_off[0] = (Off)(Policy::s_src(wargs, s_col, K) - s_base);
+    if constexpr (Cfg::kSLoads == 2) s_off[1] = (Off)(Policy::s_src2(wargs, s_col, K) - s_base);
+  }
 
-  // direct load number idx (0 .. L-1) of this set's step ks
-  auto issue_one = [&](int ks, int idx) {
-    unsigned char* slot = lds + (ks % Cfg::kStages) * Cfg::kStageBytes;
-    if (idx < kALoadsE) {
-      __builtin_amdgcn_global_load_lds((wq_gptr_t)(a_src[idx] + (int64_t)(ks0 + ks) * 128),
-                                       (wq_lptr_t)(slot + Cfg::kAOff + (wave * kALoadsE + idx) * 1024), 16, 0, 0);
-    } else if (idx < kALoadsE + Cfg::kBLoads) {
-      const int i = idx - kALoadsE;
-      __builtin_amdgcn_global_load_lds((wq_gptr_t)(b_src[i] + (int64_t)(ks0 + ks) * Policy::kStepStride),
-                                       (wq_lptr_t)(slot + Cfg::kBOff + (wave * Cfg::kBLoads + i) * 1024), 16, 0, 0);
+  // direct load number idx (0 .. L-1) of this set's step ks into the slot at byte `slot` of the ring; past the last
+  // step nothing is read, so that the loop has neither a branch nor a second form of its waits
+  auto issue_one = [&](int ks, int slot, int idx) {
+    unsigned char* const to = lds + slot;
+    const int k = ks0 + ks;
+    const bool is_a = idx < kALoadsE, is_b = !is_a && idx < kALoadsE + Cfg::kBLoads;
+    const int i = is_a ? idx : is_b ? idx - kALoadsE : idx - kALoadsE - Cfg::kBLoads;
+    unsigned char* const dst = to + (is_a   ? Cfg::kAOff + (wave * kALoadsE + i) * 1024
+                                     : is_b ? Cfg::kBOff + (wave * Cfg::kBLoads + i) * 1024
+                                            : Cfg::kSOff + i * (Cfg::BN * 4) + (wave * 64 % Cfg::BN) * 4);
+    if constexpr (Wide<Policy>::value) {
+      const int kc = min(k, ks0 + ksteps - 1);
+      const char* const src = is_a   ? a_base + a_off[i] + (int64_t)kc * 128
+                              : is_b ? b_base + b_off[i] + (int64_t)kc * Policy::kStepStride
+                                     : s_base + s_off[i] + Policy::s_offset(wargs, kc);
+      if (is_a || is_b) __builtin_amdgcn_global_load_lds((wq_gptr_t)src, (wq_lptr_t)dst, 16, 0, 0);
+      else __builtin_amdgcn_global_load_lds((wq_gptr_t)src, (wq_lptr_t)dst, 4, 0, 0);
     } else {
-      const int i = idx - kALoadsE - Cfg::kBLoads;
-      __builtin_amdgcn_global_load_lds((wq_gptr_t)(s_src[i] + Policy::s_offset(wargs, ks0 + ks)),
-                                       (wq_lptr_t)(slot + Cfg::kSOff + i * (Cfg::BN * 4) + (wave * 64 % Cfg::BN) * 4), 4, 0, 0);
+      const int live = __builtin_amdgcn_readfirstlane(ks < ksteps ? -1 : 0);
+      if (is_a) __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(a_base, live), (wq_lptr_t)dst, 16, a_off[i], k * 128, 0, 0);
+      else if (is_b) __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(b_base, live), (wq_lptr_t)dst, 16, b_off[i], k * Policy::kStepStride, 0, 0);
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(s_base, live), (wq_lptr_t)dst, 4, s_off[i], (int)Policy::s_offset(wargs, k), 0, 0);
     }
   };
 
@@ -215,43 +251,27 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
       else if (Cfg::kSLoads) bs[t] = Policy::read_scale(slot + Cfg::kSOff + n * 4, lh);
     }
   };
-  auto read_a = [&](const unsigned char* slot, int kk, half8_t (&dst)[TME]) {
+  int a_lane[4];  // fragment kk of row lj of a sub-tile, from the slot on (WQ_SWZ is the same for all sub-tiles)
 #pragma unroll
-    for (int i = 0; i < TME; ++i) {
-      const int row = (wm * TME + i) * 32 + lj;
-      dst[i] = *reinterpret_cast<const half8_t*>(slot + Cfg::kAOff + row * 128 +
-                                                 (((4 * lh + kk) ^ WQ_SWZ(row)) << 4));
-    }
+  for (int kk = 0; kk < 4; ++kk)
+    a_lane[kk] = Cfg::kAOff + (wm * TME * 32 + lj) * 128 + (((4 * lh + kk) ^ WQ_SWZ(lj)) << 4);
+  auto read_a = [&](const unsigned char* slot, int kk, int i) {
+    return *reinterpret_cast<const half8_t*>(slot + a_lane[kk] + i * 4096);
   };
 
   // ---- prologue: steps 0 .. kStages - 2 in flight, operands of step 0 ready ----
   constexpr int AHEAD = Cfg::kStages - 1;  // steps of loads in flight while a step is multiplied
+  static_assert(AHEAD * L <= 63, "vmcnt holds 6 bits");
 #pragma unroll
   for (int st = 0; st < AHEAD; ++st) {
-    if (st < ksteps) {
 #pragma unroll
-      for (int idx = 0; idx < L; ++idx) issue_one(st, idx);
-    }
+    for (int idx = 0; idx < L; ++idx) issue_one(st, st * Cfg::kStageBytes, idx);
   }
-  // loads retire in order: step 0 has landed once at most the loads of the later steps are outstanding
-  static_assert(AHEAD * L <= 63, "vmcnt holds 6 bits");
-  const int first_later = min(AHEAD, ksteps) - 1;
-  if (first_later >= 5) {
-    WQ_WAITCNT_VM(5 * L);
-  } else if (first_later == 4) {
-    WQ_WAITCNT_VM(4 * L);
-  } else if (first_later == 3) {
-    WQ_WAITCNT_VM(3 * L);
-  } else if (first_later == 2) {
-    WQ_WAITCNT_VM(2 * L);
-  } else if (ksteps >= 2) {
-    WQ_WAITCNT_VM(L);
-  } else {
-    WQ_WAITCNT_VM(0);
-  }
+  WQ_WAITCNT_VM((AHEAD - 1) * L);  // loads retire in order: step 0 has landed
   __builtin_amdgcn_s_barrier();
   read_b(lds);
-  read_a(lds, 0, aop[0]);
+#pragma unroll
+  for (int i = 0; i < TME; ++i) aop[0][i] = read_a(lds, 0, i);
 #pragma unroll
   for (int t = 0; t < TN; ++t) {
     half2_t d[4];
@@ -261,39 +281,25 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
   }
 
   // Phase 3 prepares the next step unconditionally: in the last step it reads a slot that
-  // holds stale data and unpacks it for nobody.  (A run-time branch around those LDS reads
-  // would make the compiler wait for them before the first MFMA of the phase.)
+  // holds stale data and unpacks it for nobody.
+  int at = 0, last = AHEAD * Cfg::kStageBytes;  // slots of step ks and of ks - 1, which takes step ks + AHEAD
   for (int ks = 0; ks < ksteps; ++ks) {
-    const unsigned char* slot = lds + (ks % Cfg::kStages) * Cfg::kStageBytes;
-    const unsigned char* next_slot = lds + ((ks + 1) % Cfg::kStages) * Cfg::kStageBytes;
-    const bool ahead2 = ks + AHEAD < ksteps;  // there is a step to request in this one
-    const int later = min(AHEAD - 1, ksteps - 2 - ks);  // steps requested beyond ks + 1 when phase 3 waits
+    const int next = at == AHEAD * Cfg::kStageBytes ? 0 : at + Cfg::kStageBytes;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const int cur = kk & 1, nxt = cur ^ 1;
-      const unsigned char* const a_from = kk == 3 ? next_slot : slot;  // activation fragments of the next phase
+      const unsigned char* const a_from = lds + (kk == 3 ? next : at);  // activation fragments of the next phase
       const int a_kk = kk == 3 ? 0 : kk + 1;
       if (kk == 3) {
-        // loads of step ks+1 landed (those of ks+2 may be in flight), own LDS reads done
-        if (later >= 4) {
-          WQ_WAITCNT_VM_LGKM0(4 * L);
-        } else if (later == 3) {
-          WQ_WAITCNT_VM_LGKM0(3 * L);
-        } else if (later == 2) {
-          WQ_WAITCNT_VM_LGKM0(2 * L);
-        } else if (later == 1) {
-          WQ_WAITCNT_VM_LGKM0(L);
-        } else {
-          WQ_WAITCNT_VM_LGKM0(0);
-        }
+        // loads of step ks+1 landed (those of the later ones may be in flight), own LDS reads done
+        WQ_WAITCNT_VM_LGKM0((AHEAD - 1) * L);
         __builtin_amdgcn_s_barrier();
-        read_b(next_slot);
+        read_b(lds + next);
       }
       half2_t dq[TN][4];
       uint32_t pb[NPAIR];
-      // Slots of the unpacking: the bit patterns in the first half of the usable slots, the
-      // arithmetic in the second half; in phase 3 the packed weights were requested from LDS
-      // just above, so the first slots stay free.
+      // Slots of the unpacking: the exact integers in the first half of the usable slots, the products in the
+      // second half; in phase 3 the packed weights were requested from LDS just above, so the first slots stay free.
       const int first = kk < 3 ? 0 : NSLOT * 3 / 8, usable = NSLOT - first, half = usable / 2;
       if constexpr (ScalePerK<Policy>::value) {
 #pragma unroll
@@ -304,12 +310,10 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
       for (int sl = 0; sl < NSLOT; ++sl) {
         const int i = sl / TN, t = sl % TN;
         acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aop[cur][i], bop[cur][t], acc[i][t], 0, 0, 0);
-        // one activation fragment of the next phase per slot
-        if (sl < TME) {
-          const int row = (wm * TME + sl) * 32 + lj;
-          aop[nxt][sl] = *reinterpret_cast<const half8_t*>(a_from + Cfg::kAOff + row * 128 +
-                                                           (((4 * lh + a_kk) ^ WQ_SWZ(row)) << 4));
-        }
+        // the activation fragments of the next phase, evenly
+#pragma unroll
+        for (int r = 0; r < TME; ++r)
+          if (sl == r * TN + TN - 1) aop[nxt][r] = read_a(a_from, a_kk, r);
 #pragma unroll
         for (int p = 0; p < NPAIR; ++p) {
           const int tt = p >> 2, j = p & 3;
@@ -322,10 +326,10 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
         // direct loads of step ks+AHEAD, all in phase 0 (into the slot of step ks-1, free since the
         // barrier of its phase 3): timed on the GPU, one phase with loads and three without beat
         // the same loads spread over two phases (by 1-2 %) or over all four (by 15 %)
-        if (kk == 0 && ahead2) {
+        if (kk == 0) {
           const int l0 = sl * L / NSLOT, l1 = (sl + 1) * L / NSLOT;
 #pragma unroll
-          for (int idx = l0; idx < l1; ++idx) issue_one(ks + AHEAD, idx);
+          for (int idx = l0; idx < l1; ++idx) issue_one(ks + AHEAD, last, idx);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -334,6 +338,8 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
         bop[nxt][t] = half8_t{dq[t][0].x, dq[t][0].y, dq[t][1].x, dq[t][1].y,
                               dq[t][2].x, dq[t][2].y, dq[t][3].x, dq[t][3].y};
     }
+    last = at;
+    at = next;
   }
 
   // ---- the last 32 k of a K that is no multiple of 64: two MFMAs per sub-tile straight from global memory.
@@ -535,6 +541,7 @@ static int launch_gemm_lds(const char* who, const typename Policy::Args& wargs, 
                            uint16_t* y, const Epilogue& ep, int64_t M, int64_t N, int64_t K,
                            hipStream_t stream) {
   using Cfg = LdsGemmCfg<Policy, TM, TN, WM, WN, WPE>;
+  WQ_REQUIRE(Wide<Policy>::value || K < kLdsGemmMaxK, "%s: internal: K=%lld needs 64-bit addresses", who, (long long)K);
   const int tiles_m = (int)((M + Cfg::BM - 1) / Cfg::BM);
   const int tiles_n = (int)((N + Cfg::BN - 1) / Cfg::BN);
   auto kern = gemm_lds_kernel<Policy, Epilogue, TM, TN, WM, WN, WPE, KW>;

@@ -68,8 +68,7 @@ struct Q4G32HalfStepPolicy : Q4G32LdsPolicy {
   }
   // n_local has the parity of the column: tiles start at multiples of 128
   __device__ __forceinline__ static Scale read_scale2(const unsigned char* p, int plane, int n_local, int lh) {
-    const half_t s = *reinterpret_cast<const half_t*>(p + ((n_local & 1) ? (lh ? plane : 2) : 2 * lh));
-    return Scale{s, s};
+    return *reinterpret_cast<const half_t*>(p + ((n_local & 1) ? (lh ? plane : 2) : 2 * lh));
   }
   __device__ __forceinline__ static void half_step(const Args& a, int n, int k0, int K, int lh, half8_t out[2]) {
     const uint32_t* const w = a.W + (int64_t)n * (K >> 3) + (k0 >> 3) + lh;
@@ -79,7 +78,7 @@ struct Q4G32HalfStepPolicy : Q4G32LdsPolicy {
       const uint32_t word = w[2 * c];
       half2_t d[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) d[j] = pair_finish(q4_pair_bits_natural(word, j), Scale{s, s});
+      for (int j = 0; j < 4; ++j) d[j] = half2_t{s, s} * (as_half2(q4_pair_bits_natural(word, j)) - half2_t{(half_t)1031.0f, (half_t)1031.0f});
       out[c] = half8_t{d[0].x, d[0].y, d[1].x, d[1].y, d[2].x, d[2].y, d[3].x, d[3].y};
     }
   }
@@ -109,9 +108,10 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
   const Q4G32Loader::Args bargs{W, (const half_t*)S};
   const Q4G32LdsPolicy::Args largs{W, (const half_t*)S};
   const Q4G32Epilogue ep{(const half_t*)bias, (const half_t*)residual, (int)N};
-  // 11..19: the fully LDS-staged kernel (needs 4-byte aligned S); K % 64 == 32 has the three shapes that the
+  // 11..19: the fully LDS-staged kernel (needs 4-byte aligned S and 32-bit offsets inside a tile); K % 64 == 32 has the three shapes that the
   // choice above takes for most problems
-  if (cfg >= 11 && K % 64 == 32 && ((uintptr_t)S & 3u) == 0) {
+  const bool lds_ok = ((uintptr_t)S & 3u) == 0 && K < kLdsGemmMaxK;
+  if (cfg >= 11 && K % 64 == 32 && lds_ok) {
     switch (cfg) {
       case 17: case 19: return launch_gemm_lds<Q4G32HalfStepPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 12: case 13:
@@ -121,7 +121,7 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
     }
   }
   if (cfg == 19 && K % 128 != 0) cfg = 17;
-  if (cfg >= 11 && K % 64 == 0 && ((uintptr_t)S & 3u) == 0) {
+  if (cfg >= 11 && K % 64 == 0 && lds_ok) {
     switch (cfg) {
       case 11: return q4g32_gemm_256("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 12: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 2, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);

@@ -221,6 +221,10 @@ struct Q4N32LdsPolicy {
   }
 };
 
+struct Q4N32WidePolicy : Q4N32LdsPolicy {
+  static constexpr bool kWide = true;
+};
+
 }  // namespace wq
 
 extern "C" int wq_q4n32_prepare(const uint32_t* W, const uint16_t* S, uint32_t* W_nk, uint16_t* ST, int64_t K, int64_t N,
@@ -289,6 +293,8 @@ extern "C" int wq_q4n32_linear(const uint32_t* W_nk, const uint16_t* ST, const u
   }
   const Q4N32LdsPolicy::Args args{W_nk, (const half_t*)ST};
   const Q4G32Epilogue ep{(const half_t*)bias, (const half_t*)residual, (int)N};
+  if (K >= kLdsGemmMaxK)
+    return launch_gemm_lds<Q4N32WidePolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4n32_linear", {W_nk, (const half_t*)ST}, x, y, ep, M, N, K, stream);
   // the tile shapes of format A's GEMM (same code stream, same bytes per step)
   switch (tuning().gemm_cfg ? tuning().gemm_cfg : choose_q4_lds_cfg(M, N, cu_count())) {
     case 11: return launch_gemm_lds<Q4N32LdsPolicy, Q4G32Epilogue, 8, 2, 1, 4, 1>("wq_q4n32_linear", args, x, y, ep, M, N, K, stream);

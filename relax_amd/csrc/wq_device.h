@@ -32,6 +32,12 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t b
   return r;
 }
 
+// The same as an instruction the compiler knows (any three-input bit function; 0xEA = a & b | c): behind the inline
+// assembly it puts a wait state in front of the next packed fp16 instruction.  For kernels whose loads it also schedules.
+__device__ __forceinline__ uint32_t and_or_b(uint32_t a, uint32_t mask, uint32_t bits) {
+  return __builtin_amdgcn_bitop3_b32(a, mask, bits, 0xEA);
+}
+
 // ---------------------------------------------------------------------------
 // Format A: one uint32 holds 8 codes, code i in bits 4i..4i+3.
 // (w >> 4i) & 0x000F000F isolates code i in the low half-word and code i+4 in the
@@ -75,7 +81,7 @@ __device__ __forceinline__ void q4_word_dequant_natural(uint32_t w, half2_t s2, 
 __device__ __forceinline__ uint32_t q4_pair_bits_natural(uint32_t w, int j) {
   const uint32_t t = (w >> (8 * j)) & 0xFFu;
   const uint32_t u = (t << 12) | t;
-  return and_or(u, 0x000F000Fu, 0x64006400u);
+  return and_or_b(u, 0x000F000Fu, 0x64006400u);
 }
 // ... and (w_{2j}, w_{2j+1}) from it.
 __device__ __forceinline__ half2_t q4_pair_dequant_natural(uint32_t w, int j, half2_t s2) {

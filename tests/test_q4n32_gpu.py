@@ -130,3 +130,21 @@ def test_arguments(env):
     assert ops.q4n32_linear(W_nk, ST, torch.zeros((0, 64), dtype=torch.float16, device="cuda")).shape == (0, 64)
     y = ops.q4n32_linear(W_nk, ST, torch.ones((3, 64), dtype=torch.float16, device="cuda"))
     assert torch.count_nonzero(y) == 0  # zero scales
+
+
+def test_k_beyond_32_bit_offsets(env):
+    """From K = 2^23 on, the byte offsets of a 256-row tile do not fit 32 bits: the kernel form with 64-bit addresses.
+    One activation per row is not zero, so the product is a weight, bit for bit."""
+    ops, u, torch = env
+    M, N, K = 130, 32, (1 << 23) + 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    W_nk = torch.randint(-2**31, 2**31 - 1, (N, K // 8), dtype=torch.int32, device="cuda", generator=g)
+    ST = (torch.rand((1, K), device="cuda", generator=g) * 0.015 + 0.005).half()
+    x = torch.zeros((M, K), dtype=torch.float16, device="cuda")
+    ks = torch.cat([torch.tensor([0, 1, K // 2 - 1, K // 2, K - 65, K - 64, K - 1]),
+                    torch.randint(0, K, (M - 7,), generator=torch.Generator().manual_seed(6))]).cuda()
+    x[torch.arange(M, device="cuda"), ks] = 1.0
+    y = ops.q4n32_linear(W_nk, ST, x)
+    codes = (W_nk[:, ks // 8] >> (4 * (ks % 8)).int()[None, :]) & 15
+    want = ((codes.half() - 7) * ST[:, ks]).t()
+    assert torch.equal(y, want)
