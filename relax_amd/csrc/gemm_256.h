@@ -49,6 +49,17 @@ struct Q4G32LdsPolicy {
   __device__ __forceinline__ static half2_t pair(const Frag& f, int kk, int j, Scale s) { return pair_finish(pair_bits(f, kk, j), s); }
 };
 
+// The same with the weights in registers, from K = 256 on (the scales of four steps are fetched at a time).
+struct Q4G32RegPolicy : Q4G32LdsPolicy {
+  static constexpr bool kRegB = true, kFourScales = true;
+  __device__ __forceinline__ static const char* b_base(const Args& a, int n0, int K) {
+    return reinterpret_cast<const char*>(a.W + (int64_t)n0 * (K >> 3));
+  }
+  __device__ __forceinline__ static uint32_t b_lane(int n, int n0, int lh, int K) { return (uint32_t)(n - n0) * (uint32_t)(K >> 1) + lh * 16; }
+  __device__ __forceinline__ static const char* s_base(const Args& a, int n0, int K) { return s_src(a, n0, K); }
+  __device__ __forceinline__ static uint32_t s_lane(const Args&, int n, int n0, int K) { return (uint32_t)(n - n0) * (uint32_t)(K >> 4); }
+};
+
 // Weight policy of the fully LDS-staged kernel (mfma_gemm_lds.h) for the preprocessed layouts
 // with per-column scales.  A K-step (one 64-row tile) of I = 2 (int8) or 4 (int4) interleaved
 // columns is 128 contiguous bytes, so the B tile is fetched in whole 128-byte lines; the scale
@@ -111,7 +122,7 @@ struct IntbLdsPolicy {
   __device__ __forceinline__ static half2_t pair(const Frag& f, int kk, int j, Scale s2) { return pair_finish(pair_bits(f, kk, j), s2); }
 };
 
-int q4g32_gemm_256(const char* who, const Q4G32LdsPolicy::Args& wargs, const uint16_t* x, uint16_t* y,
+int q4g32_gemm_256(const char* who, const Q4G32RegPolicy::Args& wargs, const uint16_t* x, uint16_t* y,
                    const Q4G32Epilogue& ep, int64_t M, int64_t N, int64_t K, hipStream_t stream);
 
 template <int NBIT, bool GROUPED>  // defined for int4, and for int8 with a scale per 64

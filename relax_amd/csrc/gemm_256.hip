@@ -7,9 +7,9 @@
 
 namespace wq {
 
-int q4g32_gemm_256(const char* who, const Q4G32LdsPolicy::Args& wargs, const uint16_t* x, uint16_t* y,
+int q4g32_gemm_256(const char* who, const Q4G32RegPolicy::Args& wargs, const uint16_t* x, uint16_t* y,
                    const Q4G32Epilogue& ep, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
-  return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 8, 2, 1, 4, 1>(who, wargs, x, y, ep, M, N, K, stream);
+  return launch_gemm_lds<Q4G32RegPolicy, Q4G32Epilogue, 8, 2, 1, 4, 1>(who, wargs, x, y, ep, M, N, K, stream);
 }
 
 template <int NBIT, bool GROUPED>

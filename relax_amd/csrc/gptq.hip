@@ -304,6 +304,22 @@ struct GptqLdsPolicy {
   }
 };
 
+// The same with the weights in registers, where a group is an even number of K-steps: two steps share a pair.
+struct GptqRegPolicy : GptqLdsPolicy {
+  static constexpr bool kRegB = true, kFourScales = false;
+  __device__ __forceinline__ static const char* b_base(const Args& a, int n0, int K) {
+    return reinterpret_cast<const char*>(a.W + (int64_t)n0 * (K >> 3));
+  }
+  __device__ __forceinline__ static uint32_t b_lane(int n, int n0, int lh, int K) { return (uint32_t)(n - n0) * (uint32_t)(K >> 1) + lh * 16; }
+  __device__ __forceinline__ static const char* s_base(const Args& a, int n0, int K) { return s_src(a, n0, K); }
+  __device__ __forceinline__ static uint32_t s_lane(const Args& a, int n, int n0, int) { return (uint32_t)(n - n0) * (uint32_t)a.groups * 4; }
+  __device__ __forceinline__ static int s_step(const Args& a, int ks) { return (int)s_offset(a, ks); }
+  __device__ __forceinline__ static half2_t pair_finish(uint32_t bits, half2_t sz) {
+    const half_t o = sz.y + (half_t)1024.0f;
+    return (as_half2(bits) - half2_t{o, o}) * half2_t{sz.x, sz.x};
+  }
+};
+
 }  // namespace wq
 
 extern "C" int wq_gptq_dequantize(const uint32_t* qweight, const uint32_t* qzeros, const uint16_t* scales,
@@ -578,8 +594,17 @@ static int wq::gptq_linear_impl(const uint32_t* W_nk, const uint16_t* SZ, const 
   const int spg = (int)(gs / 64);
   const GptqLdsPolicy::Args largs{W_nk, (const half2_t*)SZ, (int)G, spg,
                                   spg > 1 ? (uint32_t)(((1ull << 32) + spg - 1) / spg) : 0u};
+  const int cfg = choose_q4_lds_cfg(M, N, cu_count());
+  if (spg % 2 == 0 && K >= 256) {
+    switch (cfg) {
+      case 17: return launch_gemm_lds<GptqRegPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);
+      case 18: return launch_gemm_lds<GptqRegPolicy, Q4G32Epilogue, 8, 1, 1, 4, 1>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);
+      case 13: return launch_gemm_lds<GptqRegPolicy, Q4G32Epilogue, 4, 2, 2, 2, 2>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);
+      default: return launch_gemm_lds<GptqRegPolicy, Q4G32Epilogue, 8, 2, 1, 4, 1>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);
+    }
+  }
   // tile shape as for q4f16_1 (N = K = 4096, M = 512 with 256 x 256 tiles: 47 us, with 256 x 128: 33 us)
-  switch (choose_q4_lds_cfg(M, N, cu_count())) {
+  switch (cfg) {
     case 17: return launch_gemm_lds<GptqLdsPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);
     case 18: return launch_gemm_lds<GptqLdsPolicy, Q4G32Epilogue, 8, 1, 1, 4, 1>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);
     case 13: return launch_gemm_lds<GptqLdsPolicy, Q4G32Epilogue, 4, 2, 2, 2, 2>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);

@@ -65,6 +65,12 @@
 
 namespace wq {
 
+// Policy::kRegB = true: weights and scales go from memory to registers (gemm_rb_tile).
+template <class P, class = void>
+struct RegB : std::false_type {};
+template <class P>
+struct RegB<P, std::void_t<decltype(P::kRegB)>> : std::bool_constant<P::kRegB> {};
+
 template <class Policy, int TM, int TN, int WM, int WN, int WPE>
 struct LdsGemmCfg {
   static_assert(WM * WN == 4, "four wavefronts per workgroup");
@@ -74,11 +80,11 @@ struct LdsGemmCfg {
   static constexpr int kAOff = 0;
   static constexpr int kBOff = BM * 128;
   static constexpr int kSOff = kBOff + BN * Policy::kColBytes;
-  static constexpr int kStageBytes = kSOff + BN * Policy::kScaleBytes;
+  static constexpr int kStageBytes = RegB<Policy>::value ? kBOff : kSOff + BN * Policy::kScaleBytes;
   // ring slots: loads of kStages - 1 steps are in flight while a step is multiplied; four where a
   // single workgroup per CU leaves room for them in the 160 KiB of LDS
   static constexpr int kFit = (158 * 1024) / kStageBytes;
-  static constexpr int kStages = WPE == 1 ? (kFit >= 6 ? 6 : kFit >= 4 ? kFit : 3) : 3;
+  static constexpr int kStages = RegB<Policy>::value ? 4 : WPE == 1 ? (kFit >= 6 ? 6 : kFit >= 4 ? kFit : 3) : 3;
   static constexpr int kLdsBytes = kStages * kStageBytes;
   static constexpr int kALoads = BM / 32;   // direct loads per wavefront per step (64 chunks each)
   static constexpr int kBLoads = BN * Policy::kColBytes / 4096;
@@ -121,6 +127,54 @@ typedef __amdgpu_buffer_rsrc_t wq_rsrc_t;
 // lies inside it: a load brings zeros and touches no memory.
 __device__ __forceinline__ wq_rsrc_t wq_rsrc(const char* base, int live) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, live, 0x00027000);
+}
+
+// What follows the K loop: the sums of the two sets of wavefronts (KW = 2), then the epilogue.
+template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME, int KW>
+__device__ __forceinline__ void finish_tile(float16_t (&acc)[TME][TN], half_t* __restrict__ Y, const Epilogue& epilogue,
+                                            int M, int N, int m0, int n0, unsigned char* lds_all, int set, int wave,
+                                            int lane) {
+  using Cfg = LdsGemmCfg<Policy, TM, TN, WM, WN, WPE>;
+  const int wm = wave / WN, wn = wave % WN;
+  unsigned char* stage = lds_all;
+  if constexpr (KW == 2) {
+    // set 1's sums in register order, 16 bytes per lane; behind them set 0's staging
+    static_assert(!HalfStep<Policy>::value);
+    constexpr int kSumBytes = 4 * TME * TN * 4096;
+    static_assert(kSumBytes + 4 * RowwiseEpilogueCfg<TME, TN>::kBytesPerWave <= 2 * Cfg::kLdsBytes);
+    float4_t* const sums = reinterpret_cast<float4_t*>(lds_all) + wave * (TME * TN * 256) + lane;
+    __syncthreads();  // both rings are idle
+    if (set == 1) {
+#pragma unroll
+      for (int i = 0; i < TME; ++i)
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            sums[((i * TN + t) * 4 + q) * 64] = float4_t{acc[i][t][4 * q], acc[i][t][4 * q + 1], acc[i][t][4 * q + 2], acc[i][t][4 * q + 3]};
+    }
+    __syncthreads();
+    if (set == 1) return;
+#pragma unroll
+    for (int i = 0; i < TME; ++i)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float4_t o = sums[((i * TN + t) * 4 + q) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][t][4 * q + e] += o[e];
+        }
+    stage = lds_all + kSumBytes;
+  }
+
+  // ---- epilogue ----
+  // Row-wise through LDS (gemm_epilogue.h); the ring is idle now: every real read of it was
+  // waited for before the last barrier, and each wavefront stages in a piece of its own.
+  using ECfg = RowwiseEpilogueCfg<TME, TN>;
+  static_assert(4 * ECfg::kBytesPerWave <= Cfg::kLdsBytes, "epilogue staging exceeds the ring");
+  store_tile_rowwise<Epilogue, TME, TN>(acc, epilogue, Y, M, N, m0 + wm * TME * 32, n0 + wn * TN * 32,
+                                        stage + wave * ECfg::kBytesPerWave, lane);
 }
 
 // One output tile of TME*32*WM rows x BN columns starting at (m0, n0).  TME is the
@@ -362,45 +416,240 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
     }
   }
 
-  unsigned char* stage = lds;
-  if constexpr (KW == 2) {
-    // set 1's sums in register order, 16 bytes per lane; behind them set 0's staging
-    static_assert(!HalfStep<Policy>::value);
-    constexpr int kSumBytes = 4 * TME * TN * 4096;
-    static_assert(kSumBytes + 4 * RowwiseEpilogueCfg<TME, TN>::kBytesPerWave <= 2 * Cfg::kLdsBytes);
-    float4_t* const sums = reinterpret_cast<float4_t*>(lds_all) + wave * (TME * TN * 256) + lane;
-    __syncthreads();  // both rings are idle
-    if (set == 1) {
+  finish_tile<Policy, Epilogue, TM, TN, WM, WN, WPE, TME, KW>(acc, Y, epilogue, M, N, m0, n0, lds_all, set, wave, lane);
+}
+
+// The same tile with the weights in registers.  With the wavefronts of a workgroup side by side (WM = 1) nobody shares a
+// wavefront's columns, so staging them in LDS buys nothing, and fetching them step by step is expensive: a format that
+// is contiguous along K gives a step 32 bytes of codes and 4 of scales per column, and every load touches a cache line
+// per column however little it takes of it (without the loads of the scales, 1 KB of the 41 KB of a step, N = 22016,
+// K = 4096, M = 8192 took 1120 instead of 1233 us, without those of the activations 1101).  So the codes of two steps
+// are requested together, one piece of a column behind the other, and the scales of four; the K loop is written out for four steps, which
+// makes the registers of a step and its slot in LDS fixed, and the ring of four slots holds activations only, a step
+// more ahead than with the weights in it.
+//
+// Order of the loads (all of a wavefront's loads retire in order, and the wait for the activations counts them): step ks
+// requests the activations of step ks + 3 in phase 0, the scales of the next four steps in phase 1 where ks % 4 == 0, and in
+// phase 3 of odd steps the weights of steps ks + 3 and ks + 4, whose registers it has just emptied.  The prologue issues its loads in the order that the steps before the first would have had.
+//
+// Such a policy provides besides pair_bits / pair_finish
+//   kStepStride            bytes between the steps of a column, of which a lane takes 16
+//   b_base(args, n0, K)    where the columns from n0 on begin, b_lane(n, n0, lh, K) the lane's first piece from there
+//   kFourScales            true: a scale per 32 k, contiguous along K, taken for four steps at a time;
+//                          false: a pair of halves that serves two steps
+//   b_base(args, n0, K)    where the columns from n0 on begin, b_lane(n, n0, lh, K) the lane's first piece from there
+//   s_base(args, n0, K), s_lane(args, n, n0, K)   the same for the scales
+//   s_step(args, ks)       bytes from there to the pair of step ks (not kFourScales)
+// Measured with the K loop below it, start of that change / before / now: N = 22016, K = 4096, M = 8192 1307 / 1219 / 1191 us;
+// N = 4096, K = 11008, M = 2048 194 / 187 / 178; N = 11008, K = 4096, M = 200 37.2 / 35.5 / 32.4; AutoGPTQ with a group of 128,
+// 128 x 128 tiles, 36.2 / - / 26.6 us.  fpA_intB stays with LDS: its 128-byte units are whole lines there, eight a load
+// (int8, N = 28672, K = 8192, M = 128: 84 us, in registers 88).
+template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME, int KW = 1>
+__device__ __forceinline__ void gemm_rb_tile(const typename Policy::Args& wargs, const half_t* __restrict__ X,
+                                             half_t* __restrict__ Y, const Epilogue& epilogue, int M, int N, int K, int m0,
+                                             int n0, unsigned char* lds_all) {
+  using Cfg = LdsGemmCfg<Policy, TM, TN, WM, WN, WPE>;
+  constexpr int kA = Cfg::kALoads * TME / TM;  // direct loads per wavefront and step
+  constexpr bool kFour = Policy::kFourScales;
+  constexpr int kB2 = kFour ? 2 * TN : 3 * TN;        // loads to registers per two steps
+  constexpr int NSLOT = TME * TN, NPAIR = TN * 4;
+  static_assert(kA >= 1 && Cfg::kStages == 4);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int set = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) - 4 * set;
+  const int wm = wave / WN, wn = wave % WN;
+  const int lj = lane & 31, lh = lane >> 5;
+  const int ksteps = (K >> 6) / KW, ks0 = set * ksteps;
+  unsigned char* const lds = lds_all + set * Cfg::kLdsBytes;
+
+  const char* const a_base = reinterpret_cast<const char*>(X + (int64_t)m0 * K);
+  uint32_t a_off[kA];
 #pragma unroll
-      for (int i = 0; i < TME; ++i)
+  for (int i = 0; i < kA; ++i) {
+    const int s = (wave * kA + i) * 64 + lane;
+    const int r = s >> 3, c = (s & 7) ^ WQ_SWZ(r);
+    a_off[i] = (uint32_t)(min(m0 + r, M - 1) - m0) * (uint32_t)(2 * K) + c * 16;
+  }
+  const char* const b_base = Policy::b_base(wargs, n0, K);
+  const char* const s_base = Policy::s_base(wargs, n0, K);
+  uint32_t b_off[TN], s_off[TN];
 #pragma unroll
-        for (int t = 0; t < TN; ++t)
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            sums[((i * TN + t) * 4 + q) * 64] = float4_t{acc[i][t][4 * q], acc[i][t][4 * q + 1], acc[i][t][4 * q + 2], acc[i][t][4 * q + 3]};
-    }
-    __syncthreads();
-    if (set == 1) return;
-#pragma unroll
-    for (int i = 0; i < TME; ++i)
-#pragma unroll
-      for (int t = 0; t < TN; ++t)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float4_t o = sums[((i * TN + t) * 4 + q) * 64];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[i][t][4 * q + e] += o[e];
-        }
-    stage = lds_all + kSumBytes;
+  for (int t = 0; t < TN; ++t) {
+    const int n = min(n0 + (wn * TN + t) * 32 + lj, N - 1);
+    b_off[t] = Policy::b_lane(n, n0, lh, K);
+    s_off[t] = Policy::s_lane(wargs, n, n0, K);
   }
 
-  // ---- epilogue ----
-  // Row-wise through LDS (gemm_epilogue.h); the ring is idle now: every real read of it was
-  // waited for before the last barrier, and each wavefront stages in a piece of its own.
-  using ECfg = RowwiseEpilogueCfg<TME, TN>;
-  static_assert(4 * ECfg::kBytesPerWave <= Cfg::kLdsBytes, "epilogue staging exceeds the ring");
-  store_tile_rowwise<Epilogue, TME, TN>(acc, epilogue, Y, M, N, m0 + wm * TME * 32, n0 + wn * TN * 32,
-                                        stage + wave * ECfg::kBytesPerWave, lane);
+  typename Policy::Frag bq[4][TN];  // the codes of four steps
+  uint4_t s_cur[TN], s_next[TN];    // scales of this set of four steps and of the next (kFour)
+  half2_t s_pair[2][TN];            // (not kFour)
+  // past the last step: descriptors that hold nothing
+  auto live = [&](int ks) { return __builtin_amdgcn_readfirstlane(ks < ksteps ? -1 : 0); };
+  auto issue_a = [&](int ks, int slot, int i) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(a_base, live(ks)), (wq_lptr_t)(lds + slot * Cfg::kStageBytes + (wave * kA + i) * 1024), 16,
+                                             a_off[i], (ks0 + ks) * 128, 0, 0);
+  };
+  auto load_b2 = [&](int ks, int slot, int idx) {  // what two steps need, idx 0 .. kB2 - 1
+    if (idx < 2 * TN) {
+      const int t = idx / 2, st = idx % 2;
+      bq[slot + st][t].w = __builtin_amdgcn_raw_buffer_load_b128(wq_rsrc(b_base, live(ks + st)), b_off[t], (ks0 + ks + st) * Policy::kStepStride, 0);
+    } else if constexpr (!kFour) {
+      const int t = idx - 2 * TN;
+      s_pair[slot >> 1][t] = as_half2(__builtin_amdgcn_raw_buffer_load_b32(wq_rsrc(s_base, live(ks)), s_off[t], Policy::s_step(wargs, ks0 + ks), 0));
+    }
+  };
+  // four steps' scales: the 8 from 2 ks on, or the last 8 of the row, moved down when they are taken over
+  auto s_start = [&](int ks) { return min(2 * (ks0 + ks), (K >> 5) - 8); };
+  auto load_s = [&](int ks, int t) {
+    s_next[t] = __builtin_amdgcn_raw_buffer_load_b128(wq_rsrc(s_base, live(ks)), s_off[t], 2 * s_start(ks), 0);
+  };
+  auto take_s = [&](int ks, int t) {
+    const int d = (2 * (ks0 + ks) - s_start(ks)) >> 1;
+    uint4_t v = s_next[t];
+    v = (d & 1) ? uint4_t{v.y, v.z, v.w, v.w} : v;
+    s_cur[t] = (d & 2) ? uint4_t{v.z, v.w, v.w, v.w} : v;
+  };
+  auto scale_of = [&](int u, int t) {
+    if constexpr (kFour) {
+      const uint32_t w = u == 0 ? s_cur[t].x : u == 1 ? s_cur[t].y : u == 2 ? s_cur[t].z : s_cur[t].w;
+      return as_half2(w >> (16 * lh)).x;
+    } else {
+      return s_pair[u >> 1][t];
+    }
+  };
+
+  float16_t acc[TME][TN];
+#pragma unroll
+  for (int i = 0; i < TME; ++i)
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][t][r] = 0.0f;
+  half8_t aop[2][TME], bop[2][TN];
+  std::conditional_t<kFour, half_t, half2_t> sc[TN];
+  // fragment kk of row lj of a sub-tile in slots 0 and 1, and in slots 2 and 3 (an LDS instruction reaches 64 KiB from its
+  // address register; left to itself the compiler keeps a register for everything beyond, and spills)
+  int a_lane[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      a_lane[h][kk] = set * Cfg::kLdsBytes + 2 * h * Cfg::kStageBytes + (wm * TME * 32 + lj) * 128 + (((4 * lh + kk) ^ WQ_SWZ(lj)) << 4);
+      asm volatile("" : "+v"(a_lane[h][kk]));
+    }
+  auto read_a = [&](int slot, int kk, int i) {
+    return *reinterpret_cast<const half8_t*>(lds_all + a_lane[slot >> 1][kk] + (slot & 1) * Cfg::kStageBytes + i * 4096);
+  };
+
+  // ---- prologue (the waits count on its order) ----
+  auto first_a = [&](int st) {
+#pragma unroll
+    for (int i = 0; i < kA; ++i) issue_a(st, st, i);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto first_b2 = [&](int st) {
+#pragma unroll
+    for (int i = 0; i < kB2; ++i) load_b2(st, st, i);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if constexpr (kFour) {
+#pragma unroll
+    for (int t = 0; t < TN; ++t) load_s(0, t);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  first_a(0);
+  first_b2(0);
+  first_a(1);
+  first_a(2);
+  first_b2(2);
+  WQ_WAITCNT_VM(2 * kA + 2 * kB2);  // step 0's activations have landed
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < TME; ++i) aop[0][i] = read_a(0, 0, i);
+#pragma unroll
+  for (int t = 0; t < TN; ++t) {
+    if constexpr (kFour) take_s(0, t);
+    sc[t] = scale_of(0, t);
+    half2_t d[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) d[j] = Policy::pair_finish(Policy::pair_bits(bq[0][t], 0, j), sc[t]);
+    bop[0][t] = half8_t{d[0].x, d[0].y, d[1].x, d[1].y, d[2].x, d[2].y, d[3].x, d[3].y};
+  }
+
+  auto step = [&](int ks, auto u_) {
+    constexpr int u = decltype(u_)::value, un = (u + 1) & 3;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const int cur = kk & 1, nxt = cur ^ 1;
+      if (kk == 3) {
+        // The activations of step ks + 1 have landed.  Requested after them: those of two steps, the weights of two
+        // steps, and the scales where a set of four was begun in this step or the two before.
+        WQ_WAITCNT_VM_LGKM0(2 * kA + kB2 + (kFour && u != 3 ? TN : 0));
+        __builtin_amdgcn_s_barrier();
+      }
+      half2_t dq[TN][4];
+      uint32_t pb[NPAIR];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int sl = 0; sl < NSLOT; ++sl) {
+        const int i = sl / TN, t = sl % TN;
+        acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aop[cur][i], bop[cur][t], acc[i][t], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < TME; ++r)  // the activation fragments of the next phase, evenly
+          if (sl == r * TN + TN - 1) aop[nxt][r] = kk == 3 ? read_a(un, 0, r) : read_a(u, kk + 1, r);
+        if (kk == 3 && sl == 0) {
+#pragma unroll
+          for (int tt = 0; tt < TN; ++tt) {
+            if constexpr (kFour) {
+              if (u == 3) take_s(ks + 1, tt);
+            }
+            sc[tt] = scale_of(un, tt);
+          }
+        }
+        // the exact integers in the first half of the slots, the products in the second
+#pragma unroll
+        for (int p = 0; p < NPAIR; ++p) {
+          const int tt = p >> 2, j = p & 3;
+          if (sl == p * (NSLOT / 2) / NPAIR) pb[p] = Policy::pair_bits(bq[kk == 3 ? un : u][tt], (kk + 1) & 3, j);
+          if (sl == NSLOT / 2 + p * (NSLOT - NSLOT / 2) / NPAIR) dq[tt][j] = Policy::pair_finish(pb[p], sc[tt]);
+        }
+        if (kk == 0) {
+#pragma unroll
+          for (int idx = sl * kA / NSLOT; idx < (sl + 1) * kA / NSLOT; ++idx) issue_a(ks + 3, (u + 3) & 3, idx);
+        }
+        if constexpr (kFour && u == 0) {
+          static_assert(NSLOT >= TN);
+          if (kk == 1 && sl < TN) load_s(ks + 4, sl);
+        }
+        if constexpr (u % 2 == 1) {
+          if (kk == 3) {
+#pragma unroll
+            for (int idx = sl * kB2 / NSLOT; idx < (sl + 1) * kB2 / NSLOT; ++idx) load_b2(ks + 3, (u + 3) & 3, idx);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int t = 0; t < TN; ++t) {
+        bop[nxt][t] = half8_t{dq[t][0].x, dq[t][0].y, dq[t][1].x, dq[t][1].y, dq[t][2].x, dq[t][2].y, dq[t][3].x, dq[t][3].y};
+        // (or the compiler moves the unpacking into the next step, behind the test for the end)
+        if (kk == 3) asm volatile("" : "+v"(bop[nxt][t]));
+      }
+    }
+  };
+  int ks = 0;
+  for (; ks + 4 <= ksteps; ks += 4) {  // (one way out: with a test behind every step the sums change registers at the end)
+    step(ks, std::integral_constant<int, 0>{});
+    step(ks + 1, std::integral_constant<int, 1>{});
+    step(ks + 2, std::integral_constant<int, 2>{});
+    step(ks + 3, std::integral_constant<int, 3>{});
+  }
+  if (ks < ksteps) step(ks, std::integral_constant<int, 0>{});
+  if (ks + 1 < ksteps) step(ks + 1, std::integral_constant<int, 1>{});
+  if (ks + 2 < ksteps) step(ks + 2, std::integral_constant<int, 2>{});
+  WQ_WAITCNT_VM(0);
+  __builtin_amdgcn_s_barrier();  // nothing is on its way to the ring, and nobody reads it
+  finish_tile<Policy, Epilogue, TM, TN, WM, WN, WPE, TME, KW>(acc, Y, epilogue, M, N, m0, n0, lds_all, set, wave, lane);
 }
 
 // Row slices (1, 2 or 4; 8 where the policy carries the extra copy of the tile body, `fine`) that the tiles of
@@ -484,6 +733,16 @@ struct FineTail<P, std::void_t<decltype(P::kFineTail)>> : std::bool_constant<P::
 // as fill complete rounds of the machine); the tiles of the last, partially filled
 // round are cut into `split` row slices of TM/split sub-tiles so that the round is
 // shorter instead of leaving most CUs idle while a few finish whole tiles.
+template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME, int KW>
+__device__ __forceinline__ void gemm_tile(const typename Policy::Args& wargs, const half_t* __restrict__ X,
+                                          half_t* __restrict__ Y, const Epilogue& epilogue, int M, int N, int K, int m0,
+                                          int n0, unsigned char* lds) {
+  if constexpr (RegB<Policy>::value)
+    gemm_rb_tile<Policy, Epilogue, TM, TN, WM, WN, WPE, TME, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+  else
+    gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WPE, TME, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+}
+
 template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WAVES_PER_EU, int KW>
 __global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU, WAVES_PER_EU)))
 void gemm_lds_kernel(typename Policy::Args wargs, const half_t* __restrict__ X, half_t* __restrict__ Y,
@@ -507,7 +766,7 @@ void gemm_lds_kernel(typename Policy::Args wargs, const half_t* __restrict__ X, 
     const int xcd = pid & 7, idx = pid >> 3;
     int tile_m, tile_n;
     tile_of(xcd * per + min(xcd, rem) + idx, tile_m, tile_n);
-    gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM, KW>(wargs, X, Y, epilogue, M, N, K,
+    gemm_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM, KW>(wargs, X, Y, epilogue, M, N, K,
                                                         tile_m * Cfg::BM, tile_n * Cfg::BN, lds);
     return;
   }
@@ -524,15 +783,15 @@ void gemm_lds_kernel(typename Policy::Args wargs, const half_t* __restrict__ X, 
   if (m0 >= M) return;  // a slice that lies entirely past the last row
   if (split == 2) {
     if constexpr (TM % 2 == 0)
-      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 2, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+      gemm_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 2, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
   } else if (split == 4) {
     if constexpr (TM % 4 == 0)
-      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 4, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+      gemm_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 4, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
   } else if (split == 8) {
     if constexpr (TM % 8 == 0 && FineTail<Policy>::value)
-      gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 8, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+      gemm_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM / 8, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
   } else {
-    gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
+    gemm_tile<Policy, Epilogue, TM, TN, WM, WN, WAVES_PER_EU, TM, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
   }
 }
 

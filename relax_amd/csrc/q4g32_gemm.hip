@@ -120,16 +120,19 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
       default: return fail(WQ_EINVAL, "wq_q4g32_gemm: unknown tile configuration %d", cfg);
     }
   }
-  if (cfg == 19 && K % 128 != 0) cfg = 17;
   if (cfg >= 11 && K % 64 == 0 && lds_ok) {
+    if (K < 256)  // fewer steps than the weights are requested ahead
+      return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+    if (cfg == 19 && K % 128 != 0) cfg = 17;
+    using P = Q4G32RegPolicy;
     switch (cfg) {
       case 11: return q4g32_gemm_256("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
-      case 12: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 2, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
-      case 13: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 2, 2, 2, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
-      case 14: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 4, 2, 2, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
-      case 17: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
-      case 18: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 8, 1, 1, 4, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
-      case 19: return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 12: return launch_gemm_lds<P, Q4G32Epilogue, 4, 2, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 13: return launch_gemm_lds<P, Q4G32Epilogue, 4, 2, 2, 2, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 14: return launch_gemm_lds<P, Q4G32Epilogue, 4, 4, 2, 2, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 17: return launch_gemm_lds<P, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 18: return launch_gemm_lds<P, Q4G32Epilogue, 8, 1, 1, 4, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
+      case 19: return launch_gemm_lds<P, Q4G32Epilogue, 4, 1, 1, 4, 2, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       default: return fail(WQ_EINVAL, "wq_q4g32_gemm: unknown tile configuration %d", cfg);
     }
   }

@@ -264,3 +264,14 @@ def test_prepare_padded_errors(ops, u, oracle):
     bad[3] = 4  # outside [0, G)
     with pytest.raises(WqError, match="outside"):
         ops.gptq_prepare_padded(u.dev(qw), u.dev(qz), u.dev(s), u.dev(bad))
+
+
+@pytest.mark.parametrize("M,N,K,gs", [(256, 264, 256, 128), (384, 264, 384, 128), (640, 4104, 640, 128), (1152, 264, 1152, 384),
+                                      (1024, 8200, 1024, 256), (320, 264, 320, 64)])
+def test_gemm_returns_the_weights_bit_exact(ops, u, oracle, M, N, K, gs):
+    """x = identity: the tiled GEMM with one pair of scale and zero point for every two K-steps (gs % 128 == 0), and
+    without."""
+    _, qw, qz, s, g_idx = oracle.make_gptq_inputs(1, N, K, gs, seed=K + gs, act_order=False)
+    w = ops.gptq_prepare(u.dev(qw), u.dev(qz), u.dev(s), u.dev(g_idx))
+    got = u.host(ops.gptq_linear(w, u.dev(np.eye(K, dtype=np.float16))))
+    np.testing.assert_array_equal(got, oracle.gptq_dequant(qw, qz, s, g_idx))

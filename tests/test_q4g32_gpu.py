@@ -426,3 +426,22 @@ def test_gemm_k_halves_in_one_workgroup(ops, u, oracle, M, N, K):
     finally:
         _lib.lib().wq_debug_set_gemm_tail_split(1)
         _lib.lib().wq_debug_set_gemm_config(0)
+
+
+@pytest.mark.parametrize("cfg", [11, 12, 13, 14, 17, 18, 19])
+@pytest.mark.parametrize("K", [192, 256, 320, 384, 448, 512, 704])
+def test_gemm_k_loop_ends_bit_exact(ops, u, oracle, cfg, K):
+    """x = identity returns the dequantized weights, bit for bit: every step, pair of steps and set of four scales, and
+    each remainder of the K loop that is written out for four steps (K = 192: the form for fewer)."""
+    from relax_amd import _lib
+
+    N = 300
+    _, W, S = oracle.make_q4g32_inputs(1, N, K, seed=K + cfg)
+    x = np.eye(K, dtype=np.float16)
+    want = oracle.q4g32_dequant(W, S).T
+    _lib.lib().wq_debug_set_gemm_config(cfg)
+    try:
+        got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x), kernel="gemm"))
+    finally:
+        _lib.lib().wq_debug_set_gemm_config(0)
+    np.testing.assert_array_equal(got, want)
