@@ -190,7 +190,8 @@ int wq_q4g32_gemv_list_status(wq_gemv_list_t* list, wq_stream_t stream);
 int wq_q4g32_gemv_list_poll(wq_gemv_list_t* list, int* host_word, wq_stream_t stream);
 void wq_q4g32_gemv_list_destroy(wq_gemv_list_t* list);
 /* How many linears of the list wait for an earlier one, and how many of those for the linear
- * directly in front of them (those cannot overlap with it; order lists to keep this number low). */
+ * directly in front of them, in the order given (a list of several rows is walked in that order, and those cannot
+ * overlap; a list of one row is walked in an order of its own, in which other linears lie between where there are any). */
 int wq_q4g32_gemv_list_info(const wq_gemv_list_t* list, int* dependencies, int* adjacent);
 /* Upper bound of one wait in ticks of the 100 MHz wall clock (default 2 s). */
 int wq_q4g32_gemv_list_set_spin_limit(wq_gemv_list_t* list, long long ticks);

@@ -82,7 +82,8 @@ __device__ __forceinline__ void lds_spin_until(const int* flag, int target) {
 }  // namespace wq
 
 struct wq_gemv_list {
-  std::vector<wq::GemvListDesc> descs;
+  std::vector<wq::GemvListDesc> descs;  // in the order they are walked
+  std::vector<int> given;               // which linear of the caller's list that is
   int n = 0;
   void* table = nullptr;  // device: descriptors
   int* sync = nullptr;    // device: counters

@@ -713,6 +713,59 @@ extern "C" wq_gemv_list_t* wq_gptq_gemv_list_create(const wq_gptq_gemv_desc* d, 
 #undef bad
 }
 
+namespace wq {
+// The order in which the kernel walks a list, as indices of the caller's.  A linear that reads what an earlier one wrote
+// can start some 13 us after that one has ended (its rows stored, counted, the count seen, the activations fetched past the
+// caches and rearranged), and whoever is walked in between hides that: the linears of a list have no other order among them,
+// since create refuses every overlap but this one.  So producers go first, a consumer follows once kNear bytes of codes
+// (about 20 us of the weight stream) lie behind its producer, and consumers and the others take turns, so that the waits of
+// the two x wavefronts do not queue up.  If nothing else can go, the consumer whose producer lies furthest back does.
+// Only the first kWindow linears not yet placed compete, so that what is staged together stays together.
+// Llama-2-7B-shaped layers in the order of the model (q, k and v; o; gate and up, which read o; down, which the next q, k
+// and v read), as given / 20 / 60 / 120 MB: 1 layer 34.4 / 32.2 / 29.1 / 29.2 us, 4 layers 151 / 135 / 98 / 81,
+// 16 layers 620 / 548 / 362 / 294; hidden size 1024, 32 layers: 859 / 163 / 163 / 163 (window 24: 168 / 170 / 171).
+// Lists of several rows are walked as given: their groups of workgroups run different linears side by side (4 layers,
+// M = 8: 108 us as given, 110 .. 136 in these orders).
+static std::vector<int> walk_order(const std::vector<GemvListDesc>& descs) {
+  constexpr int kWindow = 12;
+  constexpr double kNear = 120e6;
+  const int n = (int)descs.size();
+  std::vector<int> order;
+  std::vector<char> placed(n, 0);
+  std::vector<double> end(n, 0.0);  // of a placed linear: the bytes of codes up to and with it
+  double bytes = 0.0;
+  bool last_waits = true;
+  int first = 0;
+  while ((int)order.size() < n) {
+    while (placed[first]) ++first;
+    int free_consumer = -1, producer = -1, other = -1, furthest = -1;
+    for (int i = first, seen = 0; i < n && seen < kWindow; ++i) {
+      if (placed[i]) continue;
+      ++seen;
+      const int dep = (int)((descs[i].g_dep >> 16) & 0x7fffu) - 1;
+      if (dep < 0) {
+        if (other < 0) other = i;
+        if (producer < 0 && (descs[i].g_dep & kSignal)) producer = i;
+      } else if (placed[dep]) {
+        if (free_consumer < 0 && bytes - end[dep] >= kNear) free_consumer = i;
+        if (furthest < 0 || end[dep] < end[(int)((descs[furthest].g_dep >> 16) & 0x7fffu) - 1]) furthest = i;
+      }
+    }
+    if (producer >= 0) other = producer;
+    // (`first` itself waits for nothing that is not placed, so one of the candidates exists)
+    int next = furthest;
+    if (free_consumer >= 0 && (!last_waits || other < 0)) next = free_consumer;
+    else if (other >= 0) next = other;
+    last_waits = next != other;
+    placed[next] = 1;
+    bytes += 0.5 * descs[next].N * (double)((descs[next].g_dep & 0xffffu) << 5);
+    end[next] = bytes;
+    order.push_back(next);
+  }
+  return order;
+}
+}  // namespace wq
+
 static wq_gemv_list_t* wq::gemv_list_create(const char* who, const wq_q4g32_gemv_desc* d, const uint8_t* szl,
                                             const int32_t* const* perm, int n, int M, void* workspace,
                                             size_t workspace_bytes, hipStream_t stream) {
@@ -796,9 +849,24 @@ static wq_gemv_list_t* wq::gemv_list_create(const char* who, const wq_q4g32_gemv
       if (dep == i - 1) ++l->late;
     }
   }
+  l->given.resize(ne);
+  for (int i = 0; i < ne; ++i) l->given[i] = i;
   if (M > 1) {
     if (batch_list_plan(l.get()) != WQ_OK) return nullptr;
   } else {
+  l->given = walk_order(l->descs);
+  {
+    std::vector<int> at(ne);  // where a linear of the caller's list is walked
+    for (int i = 0; i < ne; ++i) at[l->given[i]] = i;
+    const std::vector<GemvListDesc> descs = l->descs;
+    const std::vector<wq_q4g32_gemv_desc> given = e;
+    for (int i = 0; i < ne; ++i) {
+      e[i] = given[l->given[i]];
+      GemvListDesc& g = l->descs[i] = descs[l->given[i]];
+      const int dep = (int)((g.g_dep >> 16) & 0x7fffu) - 1;
+      if (dep >= 0) g.g_dep = (g.g_dep & ~(0x7fffu << 16)) | (uint32_t)(at[dep] + 1) << 16;
+    }
+  }
   // launch shape: one workgroup of 16 wavefronts per CU.  Workgroup b owns the rows
   // n = local * workgroups + ((b - off) mod workgroups); `off` continues the round-robin where the
   // previous linear ended, so that the remainders of all linears spread over the workgroups.
@@ -944,7 +1012,7 @@ extern "C" int wq_q4g32_gemv_list_status(wq_gemv_list_t* l, wq_stream_t stream) 
   return fail(WQ_EDEVICE,
               "wq_q4g32_gemv_list: a wait for linear %d timed out (the grid was not resident at once?); "
               "results of that launch are undefined",
-              err - 1);
+              l->given[err - 1]);
 }
 
 extern "C" int wq_q4g32_gemv_list_poll(wq_gemv_list_t* l, int* host_word, wq_stream_t stream) {

@@ -212,6 +212,60 @@ def test_a_wait_that_runs_out_is_reported_and_every_wavefront_exits(env, oracle)
     u.assert_close(u.host(t1), oracle.q4g32_linear(b["W"], b["S"], r0[:, :4096], nthreads=8), "consumer after a reported time-out")
 
 
+@pytest.mark.parametrize("n,seed", [(2, 1), (5, 2), (13, 3), (40, 4), (90, 5)])
+def test_lists_are_walked_in_an_order_that_keeps_producers_in_front(env, oracle, n, seed):
+    """Random lists (odd heights, several consumers of one producer, chains, consumers directly behind their producer,
+    more linears than the walk looks ahead or the workgroup has buffers for): every linear equals the oracle on the
+    activations that it read."""
+    ops, u, torch = env
+    rng = np.random.default_rng(seed)
+    ys, ent, src, depth = [], [], [], []
+    for i in range(n):
+        K = int(rng.choice([32, 256, 1024, 2080]))
+        N = int(rng.choice([5, 33, 300, 1024, 2080]))
+        lin = _linear(oracle, u, torch, N, K, seed=100 * seed + i)
+        wide = [j for j in range(i) if ent[j][0]["W"].shape[0] >= K and depth[j] < 4]
+        if wide and rng.random() < 0.6:
+            j = int(rng.choice(wide[-3:]))
+            x = ys[j][:, :K]
+        else:
+            j, x = -1, u.dev((rng.standard_normal((1, K)) * 0.5).astype(np.float16))
+        ys.append(torch.zeros((1, N), dtype=torch.float16, device="cuda"))
+        ent.append((lin, x))
+        src.append(j)
+        depth.append(depth[j] + 1 if j >= 0 else 0)  # (fp16 holds the values of so many products)
+    gl = ops.Q4G32GemvList([(l["dW"], l["dS"], x, y) for (l, x), y in zip(ent, ys)])
+    assert gl.info() == (sum(j >= 0 for j in src), sum(j >= 0 and j == i - 1 for i, j in enumerate(src)))
+    print(f"gemv list: random list of {n}", flush=True)
+    for rep in range(2):
+        for y in ys:
+            y.zero_()
+        gl.run()
+        gl.status()
+        for i, ((l, x), y) in enumerate(zip(ent, ys)):
+            u.assert_close(u.host(y), oracle.q4g32_linear(l["W"], l["S"], u.host(x).copy()), f"linear {i} of {n}, rep {rep}")
+
+
+def test_a_wait_that_runs_out_names_the_linear_as_the_caller_counts(env, oracle):
+    """Linear 1 is walked first, since linear 2 reads it; the message still says 1."""
+    ops, u, torch = env
+    other, a, b = (_linear(oracle, u, torch, N, K, seed=s) for N, K, s in ((512, 4096, 41), (22016, 4096, 42), (512, 4096, 43)))
+    y = [torch.zeros((1, N), dtype=torch.float16, device="cuda") for N in (512, 22016, 512)]
+    gl = ops.Q4G32GemvList([(other["dW"], other["dS"], u.dev(other["x"]), y[0]), (a["dW"], a["dS"], u.dev(a["x"]), y[1]),
+                            (b["dW"], b["dS"], y[1][:, :4096], y[2])])
+    from relax_amd._lib import WqError
+
+    gl.set_spin_limit(0)
+    print("gemv list: spin limit 0, walked in another order", flush=True)
+    gl.run()
+    with pytest.raises(WqError, match="linear 1 timed out"):
+        gl.status()
+    gl.set_spin_limit(200_000_000)
+    gl.run()
+    gl.status()
+    u.assert_close(u.host(y[0]), oracle.q4g32_linear(other["W"], other["S"], other["x"], nthreads=8), "the other linear")
+
+
 def test_argument_errors(env, oracle):
     ops, u, torch = env
     from relax_amd._lib import WqError
