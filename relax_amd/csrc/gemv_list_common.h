@@ -56,6 +56,10 @@ static_assert(sizeof(GatherJob) == 32, "job layout");
 constexpr int kCounterStride = 16;   // ints between two counters (64 bytes: one cache line each)
 constexpr int kCountersPerLinear = 8;
 constexpr int kBufferFlags = 0x00020000;  // buffer resource word 3: 32-bit data format, no swizzle
+// Between two looks at a producer's counters, 64 cycles each.  Every workgroup looks, at memory, and the looks queue in front
+// of the signals they wait for: one linear behind the other, K = N = 1024, 7.8 us a linear at 4, 6.6 at 64; a Llama-2-7B
+// layer 30.0 -> 25.4 us.
+constexpr int kPollSleep = 64;
 constexpr int kDeviceScope = 16;          // cache policy bit sc1: the access is coherent over the whole device
 
 // error word: 1 + the linear a consumer waited for in vain, or kBatchInternalWait + a code: a hand-over

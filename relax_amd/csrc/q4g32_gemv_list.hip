@@ -407,7 +407,7 @@ __global__ __launch_bounds__(64 * (NC + XW + 1)) void q4g32_gemv_list_kernel(con
             __hip_atomic_store(sync + sync_error_index(nlin), dep + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           break;
         }
-        __builtin_amdgcn_s_sleep(4);
+        __builtin_amdgcn_s_sleep(kPollSleep);
       }
       // whatever this XCD's L2 still holds of an earlier content of x (the addresses are reused
       // from launch to launch) must not serve the loads that follow
