@@ -223,10 +223,14 @@ struct GptqSkinnyPolicy {
     l.inv = a.inv;
   }
   __device__ __forceinline__ static const char* w_addr(const Lane& l, int k0, int) { return l.w + (k0 >> 1); }
-  __device__ __forceinline__ static const char* s_addr(const Lane& l, int k0) {
+  static constexpr int kStepStride = 64;
+  __device__ __forceinline__ static const char* s_lane(const Lane& l) { return l.sz; }
+  __device__ __forceinline__ static uint32_t s_rel(const Lane& l, int k0) {
     const uint32_t g32 = (uint32_t)k0 >> 5;
-    return l.sz + (l.ratio == 1 ? g32 : __umulhi(g32, l.inv)) * 4;
+    return (l.ratio == 1 ? g32 : __umulhi(g32, l.inv)) * 4;
   }
+  static int64_t s_reach(const Args&, int64_t, int64_t K) { return 2 * K; }
+  __device__ __forceinline__ static const char* s_addr(const Lane& l, int k0) { return l.sz + s_rel(l, k0); }
   __device__ __forceinline__ static const char* s_pair_addr(const Lane& l, int k0) { return s_addr(l, k0); }
   static bool pair_aligned(const Args&) { return true; }
   __device__ __forceinline__ static Scale pick_scale(const Lane&, half2_t pair, int) { return pair; }

@@ -118,17 +118,6 @@ struct Wide<P, std::void_t<decltype(P::kWide)>> : std::bool_constant<P::kWide> {
 // ... which they do below this one (256 rows of activations)
 constexpr int64_t kLdsGemmMaxK = 1 << 23;
 
-typedef const void __attribute__((address_space(1))) * wq_gptr_t;
-typedef void __attribute__((address_space(3))) * wq_lptr_t;
-// The direct loads are buffer loads and not global_load_lds: behind one of those, which may touch either memory, the
-// compiler waits for ALL outstanding LDS reads and loads wherever it waits for one.
-typedef __amdgpu_buffer_rsrc_t wq_rsrc_t;
-// Raw buffer descriptor from `base` on, which must be the same for the whole wavefront.  With `live` 0 instead of -1 nothing
-// lies inside it: a load brings zeros and touches no memory.
-__device__ __forceinline__ wq_rsrc_t wq_rsrc(const char* base, int live) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, live, 0x00027000);
-}
-
 // What follows the K loop: the sums of the two sets of wavefronts (KW = 2), then the epilogue.
 template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME, int KW>
 __device__ __forceinline__ void finish_tile(float16_t (&acc)[TME][TN], half_t* __restrict__ Y, const Epilogue& epilogue,

@@ -27,7 +27,10 @@ struct Q4G32SkinnyPolicy {
   __device__ __forceinline__ static const char* w_addr(const Lane& l, int k0, int) { return l.w + (k0 >> 1); }
   __device__ __forceinline__ static const char* s_addr(const Lane& l, int k0) { return l.s + ((k0 >> 5) & ~1) * 2; }
   __device__ __forceinline__ static const char* s_pair_addr(const Lane& l, int k0) { return s_addr(l, k0); }
-  __device__ __forceinline__ static const char* sblock_addr(const Lane& l, int g) { return l.s + g * 2; }
+  static constexpr int kStepStride = 64;
+  __device__ __forceinline__ static const char* s_lane(const Lane& l) { return l.s; }
+  __device__ __forceinline__ static uint32_t s_rel(const Lane&, int k0) { return ((k0 >> 5) & ~1) * 2; }
+  static int64_t s_reach(const Args&, int64_t, int64_t K) { return K; }
   // rows of K/16 bytes: every 8 scales are 16 aligned bytes when K % 256 == 0 and S is aligned
   static bool scale_block_ok(const Args& a, int64_t K) {
     return K % 256 == 0 && (reinterpret_cast<uintptr_t>(a.S) & 15u) == 0;
@@ -54,6 +57,7 @@ struct Q4G32SkinnyPolicy {
 // past S.)
 struct Q4G32OddGroupsSkinnyPolicy : Q4G32SkinnyPolicy {
   static constexpr bool kCanScaleBlock = false;
+  static constexpr bool kOddStart = true;
   struct Lane : Q4G32SkinnyPolicy::Lane {
     int odd;  // parity of the row
   };
@@ -61,9 +65,8 @@ struct Q4G32OddGroupsSkinnyPolicy : Q4G32SkinnyPolicy {
     Q4G32SkinnyPolicy::init(l, a, n, K, N);
     l.odd = n & 1;
   }
-  __device__ __forceinline__ static const char* s_addr(const Lane& l, int k0) {
-    return l.s + (k0 >> 5) * 2 - (((k0 >> 5) + l.odd) & 1) * 2;
-  }
+  __device__ __forceinline__ static uint32_t s_rel(const Lane& l, int k0) { return ((k0 >> 5) - (((k0 >> 5) + l.odd) & 1)) * 2; }
+  __device__ __forceinline__ static const char* s_addr(const Lane& l, int k0) { return l.s + (int)s_rel(l, k0); }
   __device__ __forceinline__ static const char* s_pair_addr(const Lane& l, int k0) { return s_addr(l, k0); }
   // the lane's group is 4 * step + kq
   __device__ __forceinline__ static half_t pick_scale(const Lane& l, half2_t pair, int kq) {

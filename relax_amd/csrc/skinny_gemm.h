@@ -40,9 +40,6 @@ namespace wq {
 
 #define WQ_SK_WAITCNT_VM(n) __builtin_amdgcn_s_waitcnt(((n)&0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
-typedef const void __attribute__((address_space(1))) * wq_sk_gptr_t;
-typedef void __attribute__((address_space(3))) * wq_sk_lptr_t;
-
 // A Policy provides
 //   kPieces            16-byte pieces of codes per lane and step (32 k)
 //   kScaleDma          true: a scale per lane and step, fetched as the 4-byte pair that holds it
@@ -60,9 +57,12 @@ typedef void __attribute__((address_space(3))) * wq_sk_lptr_t;
 //                              along K, one per 32 k; where scale_block_ok(args, K) the ring kernel may
 //                              fetch all scales of a column block once, 16 bytes per lane, instead of a
 //                              pair per lane and step
-//   sblock_addr(lane, g)       address of scale g of the lane's column (g % 8 == 0)       (kCanScaleBlock)
+//                              (then scale g of the lane's column lies at s_lane(lane) + 2 g)
 //   scale_block_ok(args, K)    host: every 8 scales of a column are 16 aligned bytes      (kCanScaleBlock)
 //   pair_aligned(args)         host: whether those pairs are 4-byte aligned
+//   kStepStride                bytes between a lane's pieces of consecutive steps (128 k)
+//   s_lane(lane), s_rel(lane, k0)   s_addr(lane, k0) as a pointer and a 32-bit offset from it           (kScaleDma)
+//   s_reach(args, N, K)        host: no such offset inside 16 columns goes beyond this
 // and, for weights that are not rounded (up to 8 rows, kPieces == 1),
 //   codes8(word)               the codes of a word of codes as halves, exact (8 consecutive k); the products of a
 //                              group of 32 k are summed alone and scaled in fp32
@@ -73,6 +73,12 @@ template <class P, class = void>
 struct GroupSums : std::false_type {};
 template <class P>
 struct GroupSums<P, std::void_t<decltype(&P::codes8)>> : std::true_type {};
+
+// Policy::kOddStart = true: s_rel may be -2 (the pair begins in front of the column)
+template <class P, class = void>
+struct OddStart : std::false_type {};
+template <class P>
+struct OddStart<P, std::void_t<decltype(P::kOddStart)>> : std::bool_constant<P::kOddStart> {};
 
 // bits 0 .. n - 1 of `groups` groups, of which those up to K exist
 __device__ __forceinline__ uint32_t live_groups(int k0, int K, int groups) {
@@ -114,10 +120,23 @@ __device__ __forceinline__ void mul_group_sums(float4_t& acc, const typename Pol
   }
 }
 
-// What the slab holds past K, where the K-steps do not come out even among the wavefronts that share them: the
-// weights there are exact zeros, and zero times an infinite activation is not zero.  Zeros by address, because the loop
-// can take no more: a test or masks around the products cost up to 16 %, a last iteration of its own up to 11 %.
-static __device__ const uint4_t kZeroChunk = {0, 0, 0, 0};
+// Position of the 16-byte chunk c of row r of a slab (256 bytes a row): c ^ slab_swizzle(r).  LDS serves a 16-byte read by
+// lanes 0 .. 3, 12 .. 15, 20 .. 27 and by 4 .. 11, 16 .. 19, 28 .. 31 together (and the same from 32 on), and an operand's
+// lanes 0 .. 15 / 16 .. 31 take chunks 4 apart of rows 0 .. 15: rows 0 .. 3 and 12 .. 15 must not differ in the bit that
+// tells those chunks apart from what rows 4 .. 11 hold.  With r itself every read met another one in its banks.
+__device__ __forceinline__ int slab_swizzle(int r) { return (r & 3) | ((r & 8) >> 1) | ((r & 8) ^ ((r & 4) << 1)); }
+
+// Byte offsets inside the activations and inside 16 columns of weights fit 31 bits below this K; from here on, and where
+// the scales reach further, one arrangement with 64-bit addresses serves (WIDE).
+constexpr int64_t kSkinnyMaxK = 1 << 23;
+constexpr uint32_t kOutside = 0x80000000u;  // bytes that a descriptor spans; an offset from here on brings zeros
+static __device__ const uint4_t kZeroChunk = {0, 0, 0, 0};  // ... as this does for loads without a descriptor
+__device__ __forceinline__ void direct_load16(const char* base, wq_lptr_t dst, uint32_t off, int step_off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(base, (int)kOutside), dst, 16, off, step_off, 0, 0);
+}
+__device__ __forceinline__ void direct_load4(const char* base, wq_lptr_t dst, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(base, (int)kOutside), dst, 4, off, 0, 0, 0);
+}
 
 template <typename Policy, int TH, int NW, int WAVES, bool SB = false>
 struct SkinnyCfg {
@@ -135,6 +154,7 @@ struct SkinnyCfg {
   static constexpr int kLoadsPerStep = kXLoads + Policy::kPieces + (kStepScale ? 1 : 0);
   static constexpr int kMaxAhead = 63 / kLoadsPerStep;   // vmcnt holds 6 bits
   static constexpr int kRedBytes = WAVES * TM * 4 * 64 * 4;
+  static constexpr bool kOddStart = OddStart<Policy>::value;
 };
 
 // s_waitcnt vmcnt(groups * L) for a wavefront-uniform run-time `groups` (<= 8)
@@ -153,7 +173,7 @@ __device__ __forceinline__ void wait_newer_groups(int groups) {
   }
 }
 
-template <typename Policy, typename Epilogue, int TH, int NW, int WAVES, bool SB, bool EVEN>
+template <typename Policy, typename Epilogue, int TH, int NW, int WAVES, bool SB, bool EVEN, bool WIDE>
 __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
     typename Policy::Args pargs, const half_t* __restrict__ X, half_t* __restrict__ Y, Epilogue epi,
     int M, int N, int K, int stages) {
@@ -170,24 +190,43 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
   const int nsteps = (total_steps + KW - 1) / KW;       // per wavefront (the last may be partly empty)
   const int ahead = stages - 1;
 
-  // ---- per-lane sources ----
-  // slab load i of this wavefront: rows 4*li .. 4*li+3 of the slab, li = nw*kXLoads + i;
-  // LDS position p of a row holds the 16-byte chunk p ^ (row & 15) (bank-conflict-free reads)
-  // kAhead: the arrangements where the choice of source below cost up to 4 % (AutoGPTQ, N = 4096, K = 11008, M = 48:
-  // 25.5 -> 26.6 us) request the operands of the next MFMAs before the last ones are multiplied and count addresses from the
-  // chunk of step 0, and are as fast as they were or faster (22.6 us); with eight wavefronts side by side that loses 5 %
-  constexpr bool kAhead = !EVEN && TH >= 4 && NW < 8;
-  const char* x_row[Cfg::kXLoads];
-  int x_chunk[Cfg::kXLoads];
+  // ---- per-lane sources: buffer descriptors at the activations and at the wavefront's first column, byte offsets ----
+  // slab load i of this wavefront: rows 4*li .. 4*li+3 of the slab, li = nw*kXLoads + i
+  // Buffer loads, because behind a global_load_lds the compiler waits for all LDS reads wherever it waits for one, and
+  // since they take 32-bit offsets and bring zeros past K by themselves.  With the operands of the next MFMAs requested
+  // before the last ones are multiplied (kAhead) and the slab's order above, at 8 shapes x M = 3 .. 64, 4 formats: 6 % faster
+  // on average (q4f16_1, N = 12288, K = 4096, M = 19: 17.5 -> 13.9 us; int8, N = 5120, K = 13824, M = 48: 50.4 -> 39.0).
+  // Slower is only int8 with 17 .. 32 rows and two wavefronts side by side, for a reason not known: from 26 rows on 27.0 ->
+  // 32.4 us (N = 5120, K = 13824).  It keeps the loads it had: as fast as before up to 28 rows, up to 7 % slower at 29 .. 32.
+  constexpr bool kBuffer = !WIDE && !(P == 2 && TH == 4 && NW == 2);
+  constexpr bool kAhead = kBuffer && TH >= 4;
+  using Off = std::conditional_t<kBuffer, uint32_t, int64_t>;
+  Off x_off[Cfg::kXLoads];
+  int x_k[Cfg::kXLoads];  // first k of the chunk in step 0
 #pragma unroll
   for (int i = 0; i < Cfg::kXLoads; ++i) {
     const int li = nw * Cfg::kXLoads + i;
     const int row = 4 * li + (lane >> 4);
-    x_chunk[i] = (lane & 15) ^ (row & 15);
-    x_row[i] = reinterpret_cast<const char*>(X + (int64_t)min(row, M - 1) * K + (kAhead ? 8 * x_chunk[i] : 0));
+    x_k[i] = 8 * ((lane & 15) ^ slab_swizzle(row & 15));
+    x_off[i] = (Off)min(row, M - 1) * (Off)(2 * (int64_t)K) + 2 * x_k[i];
   }
-  typename Policy::Lane pl;
+  typename Policy::Lane pl, pl0;
   Policy::init(pl, pargs, min(n0 + 16 * nw + lj, N - 1), K, N);  // clamped columns are never stored
+  Policy::init(pl0, pargs, min(n0 + 16 * nw, N - 1), K, N);
+  const char* const w_base = Policy::w_addr(pl0, 0, 0);
+  Off w_off[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) w_off[p] = (Off)(Policy::w_addr(pl, 32 * kq, p) - w_base);
+  const char* s_base = w_base;
+  Off s_off = 0;
+  if constexpr (Policy::kScaleDma) {
+    s_base = Policy::s_lane(pl0);
+    s_off = (Off)(Policy::s_lane(pl) - s_base);
+    if constexpr (Cfg::kOddStart) {  // a pair may begin in front of its column
+      s_base -= 4;
+      s_off += 4;
+    }
+  }
   typename Policy::Scale s_fixed = Policy::null_scale();
   if (!Policy::kScaleDma) s_fixed = Policy::const_scale(pl);
 
@@ -201,32 +240,34 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
     const int stage_off = slot * Cfg::kStageBytes;
     const int ks = it * KW + kw;
     const int k0 = 128 * ks + 32 * kq;             // this lane's 32 weights
-    const int k0c = k0 < K ? k0 : 0;               // past the end: any valid address (scale is zeroed)
+    const int k0c = EVEN || k0 < K ? k0 : 0;       // past the end: any valid address (scale is zeroed)
 #pragma unroll
     for (int i = 0; i < Cfg::kXLoads; ++i) {
-      const int kchunk = ks * 16 + x_chunk[i];     // 16-byte chunk index along the row
-      const char* src;
-      if constexpr (EVEN) {
-        // always inside the row; without the test the compiler puts the LDS reads of the loop one behind the other in
-        // some arrangements (q4f16_1, N = 22016, K = 4096, M = 64: 32.1 -> 36.6 us)
-        const int64_t off = (kchunk * 8 < K) ? (int64_t)kchunk * 16 : 0;
-        src = x_row[i] + off;
-      } else if constexpr (kAhead) {
-        src = 8 * x_chunk[i] < K - 128 * ks ? x_row[i] + (int64_t)ks * 256 : reinterpret_cast<const char*>(&kZeroChunk);
+      // past K the slab holds zeros: the weights there are exact zeros, and zero times an infinite activation is not
+      const wq_lptr_t dst = (wq_lptr_t)(lds + stage_off + kw * Cfg::kSlabBytes + (nw * Cfg::kXLoads + i) * 1024);
+      const bool in_row = EVEN || x_k[i] < K - 128 * ks;
+      if constexpr (!kBuffer) {
+        const char* const src = reinterpret_cast<const char*>(X) + x_off[i] + (int64_t)ks * 256;
+        __builtin_amdgcn_global_load_lds((wq_gptr_t)(in_row ? src : reinterpret_cast<const char*>(&kZeroChunk)), dst, 16, 0, 0);
       } else {
-        src = kchunk * 8 < K ? x_row[i] + (int64_t)kchunk * 16 : reinterpret_cast<const char*>(&kZeroChunk);
+        direct_load16(reinterpret_cast<const char*>(X), dst, in_row ? x_off[i] : kOutside, ks * 256);
       }
-      __builtin_amdgcn_global_load_lds(
-          (wq_sk_gptr_t)src,
-          (wq_sk_lptr_t)(lds + stage_off + kw * Cfg::kSlabBytes + (nw * Cfg::kXLoads + i) * 1024), 16, 0, 0);
     }
 #pragma unroll
-    for (int p = 0; p < P; ++p)
-      __builtin_amdgcn_global_load_lds((wq_sk_gptr_t)Policy::w_addr(pl, k0c, p),
-                                       (wq_sk_lptr_t)(w_area + stage_off + p * 1024), 16, 0, 0);
-    if constexpr (Cfg::kStepScale)
-      __builtin_amdgcn_global_load_lds((wq_sk_gptr_t)Policy::s_addr(pl, k0c),
-                                       (wq_sk_lptr_t)(s_area + stage_off), 4, 0, 0);
+    for (int p = 0; p < P; ++p) {
+      const wq_lptr_t dst = (wq_lptr_t)(w_area + stage_off + p * 1024);
+      if constexpr (!kBuffer)
+        __builtin_amdgcn_global_load_lds((wq_gptr_t)Policy::w_addr(pl, k0c, p), dst, 16, 0, 0);
+      else
+        direct_load16(w_base, dst, EVEN || k0 < K ? w_off[p] : kOutside, ks * Policy::kStepStride);
+    }
+    if constexpr (Cfg::kStepScale) {
+      const wq_lptr_t dst = (wq_lptr_t)(s_area + stage_off);
+      if constexpr (!kBuffer)
+        __builtin_amdgcn_global_load_lds((wq_gptr_t)Policy::s_addr(pl, k0c), dst, 4, 0, 0);
+      else
+        direct_load4(s_base, dst, s_off + Policy::s_rel(pl, k0c));
+    }
   };
 
   float4_t acc[TM];
@@ -241,7 +282,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       const int k0 = 128 * (it * KW + kw);
       const int row = lj < Cfg::kRows ? lj : lj & 7;
       mul_group_sums<Policy>(acc[0], pl, w_area + stage_off, s_area + stage_off, lj, kq, live_groups(k0, K, 4), 0, [&](int g) {
-        return *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * g + kq) ^ (row & 15)) << 4));
+        return *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * g + kq) ^ slab_swizzle(row & 15)) << 4));
       });
       return;
     }
@@ -254,17 +295,17 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
     if constexpr (Cfg::kStepScale)
       s = Policy::pick_scale(pl, *reinterpret_cast<const half2_t*>(s_area + stage_off + lane * 4), kq);
     if constexpr (SB) {
-      const int g = (k0 < K ? k0 : 0) >> 5;  // chunk g / 32, fetched by lane (j, (g / 8) % 4)
+      const int g = (EVEN || k0 < K ? k0 : 0) >> 5;  // chunk g / 32, fetched by lane (j, (g / 8) % 4)
       s = *reinterpret_cast<const half_t*>(s_block + (g >> 5) * 1024 + (((g >> 3) & 3) * 16 + lj) * 16 +
                                            (g & 7) * 2);
     }
-    if (k0 >= K) s = Policy::null_scale();  // code * 0 = exact zero for the weights past K
+    if (!EVEN && k0 >= K) s = Policy::null_scale();  // code * 0 = exact zero for the weights past K
     half8_t bop[4];
     Policy::dequant(pieces, s, bop);
     // rows past the slab (M <= 8 uses half a tile) re-read a held row: never stored
     auto a_operand = [&](int t, int i) {
       const int row = (16 * i + lj < Cfg::kRows) ? 16 * i + lj : 16 * i + (lj & 7);
-      return *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * kq + t) ^ (row & 15)) << 4));
+      return *reinterpret_cast<const half8_t*>(slab + row * 256 + (((4 * kq + t) ^ slab_swizzle(row & 15)) << 4));
     };
     if constexpr (kAhead) {
       half8_t aop[2][TM];
@@ -298,16 +339,14 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
   if constexpr (SB) {
     for (int c = kw; c * 1024 < K; c += KW) {
       const int g = 32 * c + 8 * kq;
-      __builtin_amdgcn_global_load_lds((wq_sk_gptr_t)Policy::sblock_addr(pl, g * 32 < K ? g : 0),
-                                       (wq_sk_lptr_t)(s_block + c * 1024), 16, 0, 0);
+      direct_load16(s_base, (wq_lptr_t)(s_block + c * 1024), s_off + (g * 32 < K ? g : 0) * 2, 0);
     }
   }
   for (int p = 0; p < ahead && p < nsteps; ++p) issue(p, p);
   int cslot = 0;                       // slot of the step being computed
   int islot = ahead % stages;          // slot the next issue goes to
   for (int it = 0; it < nsteps; ++it) {
-    const int newer = min(ahead - 1, nsteps - 1 - it);  // steps issued after step `it`
-    wait_newer_groups<Cfg::kLoadsPerStep>(newer);
+    wait_newer_groups<Cfg::kLoadsPerStep>(min(ahead - 1, nsteps - 1 - it));  // steps issued after step `it`
     if (NW > 1 || (SB && KW > 1 && it == 0)) __builtin_amdgcn_s_barrier();
     // the slot refilled now was computed in the previous iteration (by everyone: barrier above)
     if (it + ahead < nsteps) {
@@ -442,11 +481,11 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
 #pragma unroll
     for (int p = 0; p < P; ++p)
       __builtin_amdgcn_global_load_lds(
-          (wq_sk_gptr_t)(valid[which] ? Policy::w_addr(pl[which], k0c[s], p) : reinterpret_cast<const char*>(X)),
-          (wq_sk_lptr_t)(dst + p * 1024), 16, 0, 0);
+          (wq_gptr_t)(valid[which] ? Policy::w_addr(pl[which], k0c[s], p) : reinterpret_cast<const char*>(X)),
+          (wq_lptr_t)(dst + p * 1024), 16, 0, 0);
     __builtin_amdgcn_global_load_lds(
-        (wq_sk_gptr_t)(valid[which] ? Policy::s_pair_addr(pl[which], k0c[s]) : reinterpret_cast<const char*>(X)),
-        (wq_sk_lptr_t)(dst + P * 1024), 4, 0, 0);
+        (wq_gptr_t)(valid[which] ? Policy::s_pair_addr(pl[which], k0c[s]) : reinterpret_cast<const char*>(X)),
+        (wq_lptr_t)(dst + P * 1024), 4, 0, 0);
   };
 
   // ---- prologue: the first D steps (slot = flat step % D) ----
@@ -566,13 +605,13 @@ inline SkinnyTuning skinny_tuning() {
   return SkinnyTuning{t.skinny_nw, t.skinny_stages, t.skinny_waves};
 }
 
-template <typename Policy, typename Epilogue, int TH, int NW, int WAVES, bool SB, bool EVEN>
+template <typename Policy, typename Epilogue, int TH, int NW, int WAVES, bool SB, bool EVEN, bool WIDE = false>
 static int launch_skinny_form(const char* who, const typename Policy::Args& pargs, const uint16_t* x, uint16_t* y,
                               const Epilogue& epi, int64_t M, int64_t N, int64_t K, int want_stages,
                               hipStream_t stream) {
   // one fetch of all scales where the policy allows it and the block is small (two column
   // blocks at most: more would cost a workgroup per CU)
-  if constexpr (!SB && Policy::kCanScaleBlock && NW <= 2) {
+  if constexpr (!SB && !WIDE && Policy::kCanScaleBlock && NW <= 2) {
     if (K <= kScaleBlockMaxK && Policy::scale_block_ok(pargs, K) &&
         2 * SkinnyCfg<Policy, TH, NW, WAVES, true>::kStageBytes + NW * scale_block_stride((int)K) <=
             kSkinnyLdsBudget)
@@ -580,7 +619,7 @@ static int launch_skinny_form(const char* who, const typename Policy::Args& parg
                                                                              want_stages, stream);
   }
   using Cfg = SkinnyCfg<Policy, TH, NW, WAVES, SB>;
-  auto kern = skinny_gemm_kernel<Policy, Epilogue, TH, NW, WAVES, SB, EVEN>;
+  auto kern = skinny_gemm_kernel<Policy, Epilogue, TH, NW, WAVES, SB, EVEN, WIDE>;
   const int64_t blocks = (N + 16 * NW - 1) / (16 * NW);
   int stages = want_stages;
   if (stages > Cfg::kMaxAhead + 1) stages = Cfg::kMaxAhead + 1;
@@ -626,6 +665,8 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
   // 60 -> 48 us; with two tiles per CU, or at K = 4096, the ring kernel is the faster one)
   if (xreg_fits(M, K) && Policy::pair_aligned(pargs) && (t.waves == 2 || (t.waves == 0 && K > 4096 && N / 16 >= 4 * (int64_t)cu_count())))
     return launch_xreg_auto<Policy, Epilogue>(who, pargs, x, y, epi, M, N, K, stream);
+  if (K >= kSkinnyMaxK || Policy::s_reach(pargs, N, K) >= (int64_t)kOutside)  // (four wavefronts, two ring slots)
+    return launch_skinny_form<Policy, Epilogue, GroupSums<Policy>::value ? 1 : 8, 1, 4, false, false, true>(who, pargs, x, y, epi, M, N, K, 2, stream);
   const int64_t per_cu = (N / 16) / cu_count();
   int nw = 1;
   if (per_cu >= 2) nw = M <= 8 ? (per_cu >= 4 ? 2 : 1) : M <= 16 ? 2 : 4;

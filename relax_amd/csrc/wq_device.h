@@ -89,6 +89,17 @@ __device__ __forceinline__ half2_t q4_pair_dequant_natural(uint32_t w, int j, ha
   return (as_half2(q4_pair_bits_natural(w, j)) - off) * s2;
 }
 
+typedef const void __attribute__((address_space(1))) * wq_gptr_t;
+typedef void __attribute__((address_space(3))) * wq_lptr_t;
+// The direct loads are buffer loads and not global_load_lds: behind one of those, which may touch either memory, the
+// compiler waits for ALL outstanding LDS reads and loads wherever it waits for one.
+typedef __amdgpu_buffer_rsrc_t wq_rsrc_t;
+// Raw buffer descriptor from `base` on, which must be the same for the whole wavefront.  With `live` 0 instead of -1 nothing
+// lies inside it: a load brings zeros and touches no memory.
+__device__ __forceinline__ wq_rsrc_t wq_rsrc(const char* base, int live) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, live, 0x00027000);
+}
+
 // fp32 += a.x*b.x + a.y*b.y with exact fp16 products (v_dot2_f32_f16).
 __device__ __forceinline__ float dot2(half2_t a, half2_t b, float c) {
   return __builtin_amdgcn_fdot2(a, b, c, false);

@@ -445,3 +445,22 @@ def test_gemm_k_loop_ends_bit_exact(ops, u, oracle, cfg, K):
     finally:
         _lib.lib().wq_debug_set_gemm_config(0)
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("M,K", [(5, (1 << 23) + 32), (20, (1 << 23) - 64), (40, (1 << 23) + 64)])
+def test_small_batch_where_offsets_leave_32_bits(ops, u, M, K):
+    """K around 2^23, from where on the small-batch kernel takes 64-bit addresses.  One activation per row is not zero, so
+    the product is a weight, bit for bit."""
+    import torch
+
+    N = 34
+    g = torch.Generator(device="cuda").manual_seed(7)
+    W = torch.randint(-2**31, 2**31 - 1, (N, K // 8), dtype=torch.int32, device="cuda", generator=g)
+    S = (torch.rand((N, K // 32), device="cuda", generator=g) * 0.015 + 0.005).half()
+    x = torch.zeros((M, K), dtype=torch.float16, device="cuda")
+    ks = torch.cat([torch.tensor([0, K // 2, K - 33, K - 32, K - 1]),
+                    torch.randint(0, K, (M - 5,), generator=torch.Generator().manual_seed(8))]).cuda()
+    x[torch.arange(M, device="cuda"), ks] = 1.0
+    y = ops.q4g32_linear(W, S, x)
+    codes = (W[:, ks // 8] >> (4 * (ks % 8)).int()[None, :]) & 15
+    assert torch.equal(y, ((codes.half() - 7) * S[:, ks // 32]).t())
