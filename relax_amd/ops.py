@@ -28,7 +28,9 @@ UNARY_OPS = {"identity": 0, "relu": 1}
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle of torch.cuda.current_stream() without building the Stream object: 0.14 instead of 2.57 us, of the
+    # 9.4 us that a call took the host
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(t: torch.Tensor, dtype, name: str) -> torch.Tensor:
@@ -77,6 +79,10 @@ def q4g32_dequantize(W: torch.Tensor, S: torch.Tensor) -> torch.Tensor:
     return out
 
 
+_Q4G32_KERNELS = {"auto": "wq_q4g32_linear", "gemv": "wq_q4g32_gemv", "gemm": "wq_q4g32_gemm",
+                  "small_batch": "wq_q4g32_small_batch"}
+
+
 def q4g32_linear(W: torch.Tensor, S: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor] = None,
                  residual: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
                  kernel: str = "auto") -> torch.Tensor:
@@ -109,8 +115,7 @@ def q4g32_linear(W: torch.Tensor, S: torch.Tensor, x: torch.Tensor, bias: Option
         out = _dev(out, torch.float16, "out")
         if out.numel() != M * N:
             raise ValueError("out must have M*N elements")
-    fn = {"auto": _lib.lib().wq_q4g32_linear, "gemv": _lib.lib().wq_q4g32_gemv,
-          "gemm": _lib.lib().wq_q4g32_gemm, "small_batch": _lib.lib().wq_q4g32_small_batch}[kernel]
+    fn = getattr(_lib.lib(), _Q4G32_KERNELS[kernel])
     check(fn(_ptr(W), _ptr(S), _ptr(x), _ptr(bias), _ptr(residual), _ptr(out), M, N, K, _stream()),
           f"wq_q4g32_{kernel}")
     return out

@@ -464,3 +464,27 @@ def test_small_batch_where_offsets_leave_32_bits(ops, u, M, K):
     y = ops.q4g32_linear(W, S, x)
     codes = (W[:, ks // 8] >> (4 * (ks % 8)).int()[None, :]) & 15
     assert torch.equal(y, ((codes.half() - 7) * S[:, ks // 32]).t())
+
+
+def test_calls_go_to_the_current_stream(ops):
+    """The raw handle that every call passes on: default stream, side streams, one thread beside another, a capture."""
+    import threading
+
+    import torch
+
+    def same():
+        assert ops._stream() == torch.cuda.current_stream().cuda_stream
+        return ops._stream()
+
+    default, side = same(), torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert same() == side.cuda_stream != default
+        seen = []
+        t = threading.Thread(target=lambda: seen.append(same()))
+        t.start()
+        t.join()
+        assert seen == [default]
+    assert same() == default
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        torch.zeros(1, device="cuda")
+        assert same() != default
