@@ -141,7 +141,7 @@ __device__ __forceinline__ void direct_load4(const char* base, wq_lptr_t dst, ui
 template <typename Policy, int TH, int NW, int WAVES, bool SB = false>
 struct SkinnyCfg {
   static constexpr int KW = WAVES / NW;
-  static_assert(NW * KW == WAVES && (WAVES == 4 || WAVES == 8), "wavefront arrangement");
+  static_assert(NW * KW == WAVES && (WAVES == 4 || WAVES == 6 || WAVES == 8), "wavefront arrangement");
   static constexpr int kRows = 8 * TH;                   // activation rows held (M <= kRows)
   static constexpr int TM = (TH + 1) / 2;                // 16-row MFMA tiles
   static_assert((2 * TH) % NW == 0, "the slab loads divide among the wavefronts of one kw");
@@ -687,13 +687,23 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
     while (nw > 1 && cost(nw / 2) < cost(nw) - 1e-9) nw /= 2;
     if (nw == 1 && cost(2) < cost(1) - 1e-9) nw = 2;
   }
+  // 17 .. 24 rows: slabs of 24 rows and three wavefronts side by side where four or eight leave a second, partly filled
+  // round: between four and six tiles per CU in every format (M = 19, q4f16_1 / int8: N = 18432, K = 4096 28.8 -> 20.0 /
+  // 32.3 -> 20.4 us, N = 24576, K = 6144 36.7 -> 30.8 / 40.1 -> 35.1; N = 16384 and N = 24640 lose 10 .. 30 %), and between
+  // two and three, where it makes one whole round, for int8 (N = 12288, K = 4096 16.5 -> 14.2, N = 10240, K = 8192 25.5 ->
+  // 22.9; N = 8192 loses 16 %; int4 is as fast either way and up to N = 9216 slower).
+  if (M > 16 && M <= 24) {
+    const int64_t tiles = (N + 15) / 16, cus = cu_count();
+    if ((tiles > 4 * cus && tiles <= 6 * cus) || (Policy::kPieces == 2 && tiles > 2 * cus && tiles <= 3 * cus)) nw = 3;
+  }
   if (t.nw) nw = t.nw;
+  if (nw == 3 && (M <= 16 || M > 24)) nw = 4;
   if (M <= 8 && nw >= 4) nw = 2;  // 8 rows are two slab loads: at most two wavefronts share them
   // three ring slots for four or more wavefronts side by side, and for two when every workgroup has a CU of
   // its own anyway (N = 8192, K = 28672, M = 16: 67 -> 46 us; with more workgroups than CUs the third slot
   // costs a resident workgroup: N = 10240, K = 8192, M = 16: 20.9 -> 27.4 us)
   const int64_t wgs = ((N + 15) / 16 + nw - 1) / nw;
-  const int stages = t.stages ? t.stages : (nw >= 4 || (nw == 2 && M > 8 && wgs <= cu_count()) ? 3 : 2);
+  const int stages = t.stages ? t.stages : (nw >= 4 || (nw >= 2 && M > 8 && wgs <= cu_count()) ? 3 : 2);
   // eight wavefronts where two ring slots of that arrangement fit LDS, else four
 #define WQ_SK_GO(TH, NW, WAVES)                                                                        \
   do {                                                                                                 \
@@ -716,6 +726,7 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
     if (nw == 2) WQ_SK_GO(2, 2, 8);
     WQ_SK_GO(2, 1, 8);
   }
+  if (nw == 3) WQ_SK_GO(3, 3, 6);
   if (M <= 32) {
     if (nw == 8) WQ_SK_GO(4, 8, 8);
     if (nw == 4) WQ_SK_GO(4, 4, 8);

@@ -144,6 +144,21 @@ def test_small_batch_work_splits(ops, u, oracle, nbit, group_size, nw, stages, w
         _lib.lib().wq_debug_set_skinny_config(0, 0, 0)
 
 
+@pytest.mark.parametrize("nbit", [8, 4])
+@pytest.mark.parametrize("group_size", [-1, 64])
+@pytest.mark.parametrize("M,N,K,nw,stages", [(17, 64, 64, 3, 2), (19, 320, 448, 3, 3), (24, 2048, 512, 3, 2), (21, 192, 2112, 3, 0),
+                                             (18, 8256, 576, 0, 0), (23, 16448, 512, 0, 0)])
+def test_slabs_of_24_rows(ops, u, oracle, nbit, group_size, M, N, K, nw, stages):
+    """17 .. 24 rows with three wavefronts side by side, forced and (the last two) by shape."""
+    from relax_amd import _lib
+
+    _lib.lib().wq_debug_set_skinny_config(nw, stages, 0)
+    try:
+        _run(ops, u, oracle, M, N, K, nbit, seed=M, group_size=group_size)
+    finally:
+        _lib.lib().wq_debug_set_skinny_config(0, 0, 0)
+
+
 @pytest.mark.parametrize("rows", [0, 1, 2])
 @pytest.mark.parametrize("nbit", [8, 4])
 @pytest.mark.parametrize("group_size", [-1, 64])

@@ -488,3 +488,21 @@ def test_calls_go_to_the_current_stream(ops):
     with torch.cuda.graph(torch.cuda.CUDAGraph()):
         torch.zeros(1, device="cuda")
         assert same() != default
+
+
+@pytest.mark.parametrize("N,K", [(16, 64), (40, 96), (300, 256), (300, 4096), (1000, 1184), (16400, 576)])
+@pytest.mark.parametrize("M,stages", [(17, 2), (19, 3), (24, 0)])
+def test_slabs_of_24_rows(ops, u, oracle, M, stages, N, K):
+    """17 .. 24 rows with three wavefronts side by side: workgroups whose last columns lie past N, K that ends inside a step,
+    K % 64 == 32, and (the last) the choice by shape."""
+    from relax_amd import _lib
+
+    x, W, S = oracle.make_q4g32_inputs(M, N, K, seed=M + N + K)
+    rng = np.random.default_rng(M)
+    res = rng.standard_normal((M, N)).astype(np.float16)
+    _lib.lib().wq_debug_set_skinny_config(0 if N > 16384 else 3, stages, 1)
+    try:
+        got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(x), residual=u.dev(res)))
+    finally:
+        _lib.lib().wq_debug_set_skinny_config(0, 0, 0)
+    u.assert_close(got, oracle.q4g32_linear(W, S, x, residual=res, nthreads=8), f"24-row slabs {M}x{N}x{K}")
