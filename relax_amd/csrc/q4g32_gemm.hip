@@ -121,6 +121,7 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
     }
   }
   if (cfg >= 11 && K % 64 == 0 && lds_ok) {
+    if (cfg == 15 || cfg == 16 || cfg > 19) return fail(WQ_EINVAL, "wq_q4g32_gemm: unknown tile configuration %d", cfg);
     if (K < 256)  // fewer steps than the weights are requested ahead
       return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
     if (cfg == 19 && K % 128 != 0) cfg = 17;
@@ -132,8 +133,7 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
       case 14: return launch_gemm_lds<P, Q4G32Epilogue, 4, 4, 2, 2, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 17: return launch_gemm_lds<P, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
       case 18: return launch_gemm_lds<P, Q4G32Epilogue, 8, 1, 1, 4, 1>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
-      case 19: return launch_gemm_lds<P, Q4G32Epilogue, 4, 1, 1, 4, 2, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
-      default: return fail(WQ_EINVAL, "wq_q4g32_gemm: unknown tile configuration %d", cfg);
+      default: return launch_gemm_lds<P, Q4G32Epilogue, 4, 1, 1, 4, 2, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
     }
   }
   if (cfg >= 11) cfg = (cfg == 17 || cfg == 19) ? 4 : (cfg == 11 || cfg == 14) ? 1 : 2;  // 12, 13, 18 -> 128 x 256  // not eligible: register-staged kernel, same tile
