@@ -794,7 +794,7 @@ def main():
         tf = tot_flops / tot_ms / 1e9
         gtraffic, gsrc = offline_traffic("gemm_lds_kernel")
         out["gemm"] = {
-            "kernel": "gemm_lds_kernel<Q4G32LdsPolicy>",
+            "kernel": "gemm_lds_kernel<Q4G32RegPolicy>",
             "value": round(tf, 1),
             "unit": "TFLOP/s",
             "shapes": gem,
