@@ -50,6 +50,12 @@ def _compile(src: str) -> str:
     return obj
 
 
+def check_asm(name: str) -> None:
+    from relax_amd import check_ring_asm
+
+    check_ring_asm.check_source(HIPCC, [*(f for f in FLAGS if f != "-fPIC"), *SOURCE_FLAGS.get(name, ())], name)
+
+
 def _deps(src: str, seen=None):
     """`src` and every file it includes with quotes, transitively."""
     seen = seen if seen is not None else set()
@@ -78,20 +84,23 @@ def build(verbose: bool = True, incremental: bool = False) -> str:
     os.makedirs(OBJDIR, exist_ok=True)
     srcs = sources()
     todo = [s for s in srcs if _stale(s)] if incremental else srcs
-    if todo:
-        with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(todo))) as ex:
-            list(ex.map(_compile, todo))
     from relax_amd import check_ring_asm
 
-    ring = [os.path.basename(s) for s in todo if os.path.basename(s) in check_ring_asm.SOURCES]
-    if ring:
-        # those kernels wait for their inline-assembly loads by hand: verify the generated code
-        try:
-            check_ring_asm.main(HIPCC, [f for f in FLAGS if f != "-fPIC"], ring)
-        except Exception:
-            for name in ring:  # an incremental build must not take the refused objects for up to date
-                os.remove(os.path.join(OBJDIR, name + ".o"))
-            raise
+    # some kernels wait by hand for loads that the compiler does not see: the code generated for them is verified
+    checked = [s for s in todo if os.path.basename(s) in check_ring_asm.SOURCES + check_ring_asm.DIRECT_LOAD_SOURCES]
+    if todo:
+        with concurrent.futures.ThreadPoolExecutor(max_workers=8) as ex:
+            compiled = [ex.submit(_compile, s) for s in todo]
+            checks = [ex.submit(check_asm, os.path.basename(s)) for s in checked]
+            for f in compiled:
+                f.result()
+            try:
+                for f in checks:
+                    f.result()
+            except Exception:
+                for s in checked:  # an incremental build must not take the refused objects for up to date
+                    os.remove(os.path.join(OBJDIR, os.path.basename(s) + ".o"))
+                raise
     for lib, want in ((LIB, False), (CALIBRATE_LIB, True)):
         objs = [os.path.join(OBJDIR, os.path.basename(s) + ".o") for s in srcs
                 if (os.path.basename(s) in CALIBRATE_SOURCES) == want]

@@ -1,6 +1,7 @@
-"""Build-time check of the generated code of ``csrc/q4g32_gemv_list.hip`` and ``csrc/q4g32_batch_list.hip``.
+"""Build-time checks of the generated code: of ``csrc/q4g32_gemv_list.hip`` and ``csrc/q4g32_batch_list.hip``, and of the
+tiled GEMMs.
 
-The compute wavefronts of those kernels load their weight stream with inline-assembly loads into a
+The compute wavefronts of the first two load their weight stream with inline-assembly loads into a
 ring of registers and wait for them by hand, so the compiler does not know that those registers are
 in flight between a load and its wait.  The source makes every read of a ring register an asm
 statement that depends on the wait; what is left to chance is register allocation (a copy or a
@@ -25,6 +26,9 @@ Kernels with such a ring must also be free of register spills (no ``scratch_*`` 
 A second check (``check_asm_results``) covers what inline assembly costs besides: the compiler does
 not keep the hardware's wait states between an inline-assembly VALU result and an MFMA or DPP
 instruction that reads it.
+
+A third one (``check_direct_loads_drained``) is for the tiled GEMMs: no result is staged in LDS before every direct load to
+it has landed.
 """
 from __future__ import annotations
 
@@ -36,6 +40,8 @@ import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ("q4g32_gemv_list.hip", "q4g32_batch_list.hip")
+# the tiled GEMMs (mfma_gemm_lds.h)
+DIRECT_LOAD_SOURCES = ("gemm_256.hip", "gptq.hip", "intb_gemm.hip", "q4g32_gemm.hip", "q4n32.hip")
 ALLOWED_READERS = ("v_and_or_b32", "v_lshrrev_b32", "v_cvt_f32_f16", "v_mov_b32_dpp")
 
 
@@ -131,22 +137,28 @@ def check_asm_results(asm_text: str) -> list[str]:
     return errors
 
 
-def check(asm_text: str) -> list[str]:
-    """Checks every kernel of the file on its own (register names mean nothing across kernels)."""
-    lines = [l.split(";")[0].strip() for l in asm_text.splitlines()]
+def _functions(asm_text: str, labels: bool = False):
+    """(name, instructions) of every function of the file, with its local labels if asked for."""
     functions, cur = [], None
-    for l in lines:
+    for raw in asm_text.splitlines():
+        l = raw.split(";")[0].strip()
         if not l:
             continue
         if l.endswith(":") and not l.startswith("."):  # a function label
             cur = []
-            functions.append(cur)
+            functions.append((l[:-1], cur))
         elif l.startswith(".Lfunc_end"):
             cur = None
-        elif cur is not None and not l.startswith(".") and not l.endswith(":"):
-            cur.append(l)
+        elif cur is not None and (l.startswith(".LBB") if l.endswith(":") else not l.startswith(".")):
+            if labels or not l.endswith(":"):
+                cur.append(l)
+    return functions
+
+
+def check(asm_text: str) -> list[str]:
+    """Checks every kernel of the file on its own (register names mean nothing across kernels)."""
     errors, with_ring = [], 0
-    for body in functions:
+    for _, body in _functions(asm_text):
         if any(_is_ring_load(l) for l in body):
             with_ring += 1
             errors += _check_function(body)
@@ -161,25 +173,101 @@ def check(asm_text: str) -> list[str]:
     return errors
 
 
-def main(hipcc="/opt/rocm/bin/hipcc", flags=(), sources=SOURCES):
-    for name in sources:
-        with tempfile.TemporaryDirectory() as td:
-            out = os.path.join(td, "k.s")
-            subprocess.check_call([hipcc, *flags, "-S", "--cuda-device-only", os.path.join(HERE, "csrc", name), "-o", out],
-                                  stderr=subprocess.DEVNULL)
-            text = open(out).read()
-            errs = check(text)
-            hazards = check_asm_results(text)
-        if errs:
-            raise RuntimeError(f"{name}: the generated code touches in-flight ring registers:\n  " + "\n  ".join(errs[:20]))
-        if hazards:
-            raise RuntimeError(f"{name}: an inline-assembly result reaches an MFMA / DPP instruction without wait states:\n  "
-                               + "\n  ".join(hazards[:20]))
-    return True
+def _blocks(body: list[str]):
+    """Basic blocks of a function's text as (instructions, indices of the blocks behind it)."""
+    blocks, labels = [[]], {}
+    for l in body:
+        if l.endswith(":"):
+            if blocks[-1]:
+                blocks.append([])
+            labels[l[:-1]] = len(blocks) - 1
+        else:
+            blocks[-1].append(l)
+            if l.startswith(("s_branch", "s_cbranch", "s_endpgm", "s_setpc")):
+                blocks.append([])
+    out = []
+    for i, b in enumerate(blocks):
+        succ = []
+        if b and b[-1].startswith(("s_branch", "s_cbranch")):
+            succ.append(labels[b[-1].split()[1]])
+        if i + 1 < len(blocks) and not (b and b[-1].startswith(("s_branch", "s_endpgm", "s_setpc"))):
+            succ.append(i + 1)
+        out.append((b, succ))
+    return out
+
+
+def _is_direct_load(l: str) -> bool:
+    """A load from memory to LDS."""
+    return l.startswith("global_load_lds_") or (l.startswith("buffer_load_") and l.endswith(" lds"))
+
+
+def check_direct_loads_drained(asm_text: str) -> list[str]:
+    """The tiled GEMMs keep direct loads (memory to LDS) in flight all through their K loop, past its end too, and then stage
+    the results in the same LDS.  Such a load is nobody's register, so the compiler puts no wait in front of a write to the
+    place it fills; and it may fill a place where another wavefront writes.  So in every ``gemm_lds_kernel``, on every
+    way from such a load to a ``ds_write``, there must be an ``s_waitcnt vmcnt(0)`` and an ``s_barrier`` behind it."""
+    CLEAN, DRAINED, PENDING = 0, 1, 2
+    errors, kernels = [], 0
+    for name, body in _functions(asm_text, labels=True):
+        if "gemm_lds_kernel" not in name or not any(_is_direct_load(l) for l in body):
+            continue
+        kernels += 1
+        blocks = _blocks(body)
+        entry = [CLEAN] * len(blocks)
+        todo, seen, bad = [0], set(), set()
+        while todo:
+            i = todo.pop()
+            seen.add(i)
+            state = entry[i]
+            for l in blocks[i][0]:
+                if _is_direct_load(l):
+                    state = PENDING
+                elif l.startswith("s_waitcnt") and "vmcnt(0)" in l and state == PENDING:
+                    state = DRAINED
+                elif l.startswith("s_barrier") and state == DRAINED:
+                    state = CLEAN
+                elif l.startswith("ds_write") and state != CLEAN:
+                    bad.add((l, state))
+            for j in blocks[i][1]:
+                if state > entry[j] or j not in seen:
+                    entry[j] = max(state, entry[j])
+                    todo.append(j)
+        for l, state in sorted(bad)[:3]:
+            errors.append(f"{name}: `{l}` with direct loads " + ("on their way" if state == PENDING else "of other wavefronts on their way"))
+    if kernels == 0:
+        return ["no direct loads found (expected global_load_lds_* or buffer_load_* ... lds in a gemm_lds_kernel)"]
+    return errors
+
+
+def _assembly(hipcc: str, flags, name: str) -> str:
+    with tempfile.TemporaryDirectory() as td:
+        out = os.path.join(td, "k.s")
+        subprocess.check_call([hipcc, *flags, "-S", "--cuda-device-only", os.path.join(HERE, "csrc", name), "-o", out],
+                              stderr=subprocess.DEVNULL)
+        with open(out) as f:
+            return f.read()
+
+
+def check_source(hipcc: str, flags, name: str) -> None:
+    """Raises if the code generated for one of SOURCES or DIRECT_LOAD_SOURCES is not as it has to be."""
+    text = _assembly(hipcc, flags, name)
+    if name in DIRECT_LOAD_SOURCES:
+        found = check_direct_loads_drained(text)
+        if found:
+            raise RuntimeError(f"{name}: LDS is written while direct loads to it may be on their way:\n  " + "\n  ".join(found[:20]))
+        return
+    errs = check(text)
+    hazards = check_asm_results(text)
+    if errs:
+        raise RuntimeError(f"{name}: the generated code touches in-flight ring registers:\n  " + "\n  ".join(errs[:20]))
+    if hazards:
+        raise RuntimeError(f"{name}: an inline-assembly result reaches an MFMA / DPP instruction without wait states:\n  "
+                           + "\n  ".join(hazards[:20]))
 
 
 if __name__ == "__main__":
     from relax_amd import build as _b  # noqa: E402
 
-    main(_b.HIPCC, [f for f in _b.FLAGS if f != "-fPIC"])
-    print("ring registers: ok")
+    for _name in SOURCES + DIRECT_LOAD_SOURCES:
+        _b.check_asm(_name)
+    print("ring registers, direct loads: ok")

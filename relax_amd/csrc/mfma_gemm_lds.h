@@ -118,7 +118,9 @@ struct Wide<P, std::void_t<decltype(P::kWide)>> : std::bool_constant<P::kWide> {
 // ... which they do below this one (256 rows of activations)
 constexpr int64_t kLdsGemmMaxK = 1 << 23;
 
-// What follows the K loop: the sums of the two sets of wavefronts (KW = 2), then the epilogue.
+// What follows the K loop: the sums of the two sets of wavefronts (KW = 2), then the epilogue.  Both stage in the ring, so
+// it has to be idle: no direct load of any wavefront on its way, loads past the last step included, and a barrier behind
+// the wait for them.  Both tile bodies end with that (check_ring_asm.py refuses a build without it).
 template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME, int KW>
 __device__ __forceinline__ void finish_tile(float16_t (&acc)[TME][TN], half_t* __restrict__ Y, const Epilogue& epilogue,
                                             int M, int N, int m0, int n0, unsigned char* lds_all, int set, int wave,
@@ -132,7 +134,7 @@ __device__ __forceinline__ void finish_tile(float16_t (&acc)[TME][TN], half_t* _
     constexpr int kSumBytes = 4 * TME * TN * 4096;
     static_assert(kSumBytes + 4 * RowwiseEpilogueCfg<TME, TN>::kBytesPerWave <= 2 * Cfg::kLdsBytes);
     float4_t* const sums = reinterpret_cast<float4_t*>(lds_all) + wave * (TME * TN * 256) + lane;
-    __syncthreads();  // both rings are idle
+    __syncthreads();
     if (set == 1) {
 #pragma unroll
       for (int i = 0; i < TME; ++i)
@@ -158,8 +160,7 @@ __device__ __forceinline__ void finish_tile(float16_t (&acc)[TME][TN], half_t* _
   }
 
   // ---- epilogue ----
-  // Row-wise through LDS (gemm_epilogue.h); the ring is idle now: every real read of it was
-  // waited for before the last barrier, and each wavefront stages in a piece of its own.
+  // Row-wise through LDS (gemm_epilogue.h); each wavefront stages in a piece of its own.
   using ECfg = RowwiseEpilogueCfg<TME, TN>;
   static_assert(4 * ECfg::kBytesPerWave <= Cfg::kLdsBytes, "epilogue staging exceeds the ring");
   store_tile_rowwise<Epilogue, TME, TN>(acc, epilogue, Y, M, N, m0 + wm * TME * 32, n0 + wn * TN * 32,
@@ -405,6 +406,10 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
     }
   }
 
+  // The loads past the last step write to the ring like all others (zeros; in the wide form the last step again), and their
+  // places overlap the pieces in which other wavefronts stage: all of them land before anyone goes on.
+  WQ_WAITCNT_VM(0);
+  __builtin_amdgcn_s_barrier();
   finish_tile<Policy, Epilogue, TM, TN, WM, WN, WPE, TME, KW>(acc, Y, epilogue, M, N, m0, n0, lds_all, set, wave, lane);
 }
 

@@ -1,4 +1,4 @@
-"""The build-time checks of the generated code of the list kernels (relax_amd/check_ring_asm.py), on small
+"""The build-time checks of the generated code (relax_amd/check_ring_asm.py), on small
 hand-written listings: what they must accept and what they must refuse."""
 from relax_amd import check_ring_asm as c
 
@@ -61,3 +61,53 @@ def test_inline_assembly_results_must_not_reach_mfma_or_dpp_at_once():
     assert _hazards(bare + "\tv_mov_b32_dpp v10, v51 row_ror:8 row_mask:0xf bank_mask:0xc\n")  # the old value of a DPP destination counts
     # loads inside inline assembly are waited for by s_waitcnt, not by wait states
     assert _hazards("\t;;#ASMSTART\n\tglobal_load_dwordx4 v[10:13], v6, s[0:1] nt\n\t;;#ASMEND\n" + mfma) == []
+
+
+GEMM = """
+_ZN2wq15gemm_lds_kernelEv:
+\tbuffer_load_dwordx4 v1, s[0:3], 0 offen lds
+.LBB0_1:
+\ts_waitcnt vmcnt(3) lgkmcnt(0)
+\ts_barrier
+\tbuffer_load_dwordx4 v1, s[0:3], s4 offen lds
+\ts_cbranch_scc1 .LBB0_1
+{tail}
+\ts_endpgm
+.Lfunc_end0:
+"""
+
+
+def test_direct_loads_have_landed_in_front_of_the_staging():
+    def errors(tail, text=GEMM):
+        return c.check_direct_loads_drained(text.format(tail=tail))
+
+    wait, barrier, write = "\ts_waitcnt vmcnt(0)\n", "\ts_barrier\n", "\tds_write_b128 v2, v[4:7]"
+    assert errors(wait + barrier + write) == []
+    assert errors("\ts_waitcnt vmcnt(0) lgkmcnt(0)\n" + barrier + write) == []
+    assert errors(write)                                        # the loop ends with loads on their way
+    assert errors(barrier + write)
+    assert errors(barrier + wait + write)                       # the barrier lies in front of the wait
+    assert "other wavefronts" in errors(wait + write)[0]        # those of the others may still be
+    assert errors("\ts_waitcnt vmcnt(1)\n" + barrier + write)
+    # one way around the wait is enough
+    assert errors("\ts_cbranch_vccz .LBB0_3\n" + wait + barrier + ".LBB0_3:\n" + write)
+    # a second tile body behind the first
+    again = "\tglobal_load_lds_dwordx4 v[2:3], off\n"
+    assert errors(wait + barrier + write + "\n" + again + write)
+    assert errors(wait + barrier + write + "\n" + again + wait + barrier + write) == []
+    # nothing to check, or other kernels only
+    assert errors(write, GEMM.replace(" lds", ""))
+    assert errors(write, GEMM.replace("gemm_lds", "other"))
+
+
+def test_the_build_checks_every_source_with_the_tiled_gemm():
+    import os
+
+    csrc = os.path.join(c.HERE, "csrc")
+    with_gemm = set()
+    for name in os.listdir(csrc):
+        if name.endswith(".hip"):
+            with open(os.path.join(csrc, name)) as f:
+                if "launch_gemm_lds<" in f.read():
+                    with_gemm.add(name)
+    assert with_gemm == set(c.DIRECT_LOAD_SOURCES)
