@@ -27,8 +27,9 @@ A second check (``check_asm_results``) covers what inline assembly costs besides
 not keep the hardware's wait states between an inline-assembly VALU result and an MFMA or DPP
 instruction that reads it.
 
-A third one (``check_direct_loads_drained``) is for the tiled GEMMs: no result is staged in LDS before every direct load to
-it has landed.
+Two are for the tiled GEMMs: no result is staged in LDS before every direct load to it has landed
+(``check_direct_loads_drained``), and the loads past the last step of K lie outside their empty descriptors however the range
+check counts a scalar offset (``check_empty_descriptors``).
 """
 from __future__ import annotations
 
@@ -239,6 +240,67 @@ def check_direct_loads_drained(asm_text: str) -> list[str]:
     return errors
 
 
+_SGPRS = re.compile(r"(?:s(\d+)|s\[(\d+):(\d+)\])$")
+_BUFFER_LOAD = re.compile(r"buffer_load_\w+ .*s\[\d+:\d+\], (\S+)(?: offen.*)?$")
+
+
+def _sgprs(operand: str) -> range:
+    m = _SGPRS.match(operand)
+    if not m:
+        return range(0)
+    return range(int(m[1]), int(m[1]) + 1) if m[1] else range(int(m[2]), int(m[3]) + 1)
+
+
+def check_empty_descriptors(asm_text: str) -> list[str]:
+    """Past the last step of K the tiled GEMMs load against a buffer descriptor of 0 bytes.  If the range check subtracts the
+    scalar offset from those 0 bytes, such a load lies outside only with a scalar offset of 0.  So in every
+    ``gemm_lds_kernel`` the scalar offset of a buffer load is 0, or a register that on every way to the load was
+    last written by a choice between an offset and 0 (or by an AND with the mask that makes the descriptor empty)."""
+    errors, loads = [], 0
+
+    def after(block, guarded, bad):
+        guarded = set(guarded)
+        for l in block:
+            m = _BUFFER_LOAD.match(l)
+            if m:
+                if m[1] != "0" and not (m[1][0] == "s" and guarded.issuperset(_sgprs(m[1]))):
+                    bad.add(l)
+                continue
+            op, _, rest = l.partition(" ")
+            operands = [o.strip() for o in rest.split(",")]
+            written = set(_sgprs(operands[0]))
+            masked = (op == "s_cselect_b32" and "0" in operands[1:]) or op == "s_and_b32"
+            copied = op == "s_mov_b32" and (operands[1] == "0" or (_sgprs(operands[1]) and guarded.issuperset(_sgprs(operands[1]))))
+            guarded = guarded | written if masked or copied else guarded - written
+        return guarded
+
+    for name, body in _functions(asm_text, labels=True):
+        if "gemm_lds_kernel" not in name or not any(_BUFFER_LOAD.match(l) for l in body):
+            continue
+        blocks = _blocks(body)
+        entry = [None] * len(blocks)
+        entry[0] = set()
+        todo = [0]
+        while todo:
+            i = todo.pop()
+            out = after(blocks[i][0], entry[i], set())
+            for j in blocks[i][1]:
+                joined = out if entry[j] is None else entry[j] & out
+                if joined != entry[j]:
+                    entry[j] = joined
+                    todo.append(j)
+        bad = set()
+        for (block, _), guarded in zip(blocks, entry):
+            if guarded is not None:
+                after(block, guarded, bad)
+        loads += sum(1 for l in body if _BUFFER_LOAD.match(l))
+        for l in sorted(bad)[:3]:
+            errors.append(f"{name}: `{l}` may have a scalar offset against an empty descriptor")
+    if loads == 0:
+        return ["no buffer loads found in a gemm_lds_kernel"]
+    return errors
+
+
 def _assembly(hipcc: str, flags, name: str) -> str:
     with tempfile.TemporaryDirectory() as td:
         out = os.path.join(td, "k.s")
@@ -255,6 +317,9 @@ def check_source(hipcc: str, flags, name: str) -> None:
         found = check_direct_loads_drained(text)
         if found:
             raise RuntimeError(f"{name}: LDS is written while direct loads to it may be on their way:\n  " + "\n  ".join(found[:20]))
+        found = check_empty_descriptors(text)
+        if found:
+            raise RuntimeError(f"{name}: a load past the last step may touch memory:\n  " + "\n  ".join(found[:20]))
         return
     errs = check(text)
     hazards = check_asm_results(text)

@@ -265,9 +265,9 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
       else __builtin_amdgcn_global_load_lds((wq_gptr_t)src, (wq_lptr_t)dst, 4, 0, 0);
     } else {
       const int live = __builtin_amdgcn_readfirstlane(ks < ksteps ? -1 : 0);
-      if (is_a) __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(a_base, live), (wq_lptr_t)dst, 16, a_off[i], k * 128, 0, 0);
-      else if (is_b) __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(b_base, live), (wq_lptr_t)dst, 16, b_off[i], k * Policy::kStepStride, 0, 0);
-      else __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(s_base, live), (wq_lptr_t)dst, 4, s_off[i], (int)Policy::s_offset(wargs, k), 0, 0);
+      if (is_a) direct_load16_if(live, a_base, (wq_lptr_t)dst, a_off[i], k * 128);
+      else if (is_b) direct_load16_if(live, b_base, (wq_lptr_t)dst, b_off[i], k * Policy::kStepStride);
+      else direct_load4_if(live, s_base, (wq_lptr_t)dst, s_off[i], (int)Policy::s_offset(wargs, k));
     }
   };
 
@@ -480,22 +480,21 @@ __device__ __forceinline__ void gemm_rb_tile(const typename Policy::Args& wargs,
   // past the last step: descriptors that hold nothing
   auto live = [&](int ks) { return __builtin_amdgcn_readfirstlane(ks < ksteps ? -1 : 0); };
   auto issue_a = [&](int ks, int slot, int i) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(a_base, live(ks)), (wq_lptr_t)(lds + slot * Cfg::kStageBytes + (wave * kA + i) * 1024), 16,
-                                             a_off[i], (ks0 + ks) * 128, 0, 0);
+    direct_load16_if(live(ks), a_base, (wq_lptr_t)(lds + slot * Cfg::kStageBytes + (wave * kA + i) * 1024), a_off[i], (ks0 + ks) * 128);
   };
   auto load_b2 = [&](int ks, int slot, int idx) {  // what two steps need, idx 0 .. kB2 - 1
     if (idx < 2 * TN) {
       const int t = idx / 2, st = idx % 2;
-      bq[slot + st][t].w = __builtin_amdgcn_raw_buffer_load_b128(wq_rsrc(b_base, live(ks + st)), b_off[t], (ks0 + ks + st) * Policy::kStepStride, 0);
+      bq[slot + st][t].w = load_b128_if(live(ks + st), b_base, b_off[t], (ks0 + ks + st) * Policy::kStepStride);
     } else if constexpr (!kFour) {
       const int t = idx - 2 * TN;
-      s_pair[slot >> 1][t] = as_half2(__builtin_amdgcn_raw_buffer_load_b32(wq_rsrc(s_base, live(ks)), s_off[t], Policy::s_step(wargs, ks0 + ks), 0));
+      s_pair[slot >> 1][t] = as_half2(load_b32_if(live(ks), s_base, s_off[t], Policy::s_step(wargs, ks0 + ks)));
     }
   };
   // four steps' scales: the 8 from 2 ks on, or the last 8 of the row, moved down when they are taken over
   auto s_start = [&](int ks) { return min(2 * (ks0 + ks), (K >> 5) - 8); };
   auto load_s = [&](int ks, int t) {
-    s_next[t] = __builtin_amdgcn_raw_buffer_load_b128(wq_rsrc(s_base, live(ks)), s_off[t], 2 * s_start(ks), 0);
+    s_next[t] = load_b128_if(live(ks), s_base, s_off[t], 2 * s_start(ks));
   };
   auto take_s = [&](int ks, int t) {
     const int d = (2 * (ks0 + ks) - s_start(ks)) >> 1;

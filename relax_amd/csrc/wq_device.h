@@ -94,10 +94,24 @@ typedef void __attribute__((address_space(3))) * wq_lptr_t;
 // The direct loads are buffer loads and not global_load_lds: behind one of those, which may touch either memory, the
 // compiler waits for ALL outstanding LDS reads and loads wherever it waits for one.
 typedef __amdgpu_buffer_rsrc_t wq_rsrc_t;
-// Raw buffer descriptor from `base` on, which must be the same for the whole wavefront.  With `live` 0 instead of -1 nothing
-// lies inside it: a load brings zeros and touches no memory.
-__device__ __forceinline__ wq_rsrc_t wq_rsrc(const char* base, int live) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, live, 0x00027000);
+// Raw buffer descriptor of `bytes` bytes from `base` on, which must be the same for the whole wavefront.
+__device__ __forceinline__ wq_rsrc_t wq_rsrc(const char* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00027000);
+}
+// Loads from base + off + step_off (of which step_off is the same for the wavefront) with `live` -1.  With `live` 0 the
+// descriptor is empty: they bring zeros and touch no memory.  That must not depend on whether the range check counts the
+// scalar offset (0 bytes less an offset would be many), so the scalar offset of such a load is 0.
+__device__ __forceinline__ void direct_load16_if(int live, const char* base, wq_lptr_t dst, uint32_t off, int step_off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(base, live), dst, 16, off, step_off & live, 0, 0);
+}
+__device__ __forceinline__ void direct_load4_if(int live, const char* base, wq_lptr_t dst, uint32_t off, int step_off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(base, live), dst, 4, off, step_off & live, 0, 0);
+}
+__device__ __forceinline__ uint4_t load_b128_if(int live, const char* base, uint32_t off, int step_off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(wq_rsrc(base, live), off, step_off & live, 0);
+}
+__device__ __forceinline__ uint32_t load_b32_if(int live, const char* base, uint32_t off, int step_off) {
+  return __builtin_amdgcn_raw_buffer_load_b32(wq_rsrc(base, live), off, step_off & live, 0);
 }
 
 // fp32 += a.x*b.x + a.y*b.y with exact fp16 products (v_dot2_f32_f16).

@@ -100,6 +100,30 @@ def test_direct_loads_have_landed_in_front_of_the_staging():
     assert errors(write, GEMM.replace("gemm_lds", "other"))
 
 
+def test_loads_past_the_end_have_no_scalar_offset():
+    def errors(body, text=GEMM):
+        return c.check_empty_descriptors(text.replace("s4 offen", "s9 offen").format(tail="").replace(".LBB0_1:\n", body + ".LBB0_1:\n"))
+
+    assert errors("\ts_cselect_b32 s9, s20, 0\n") == []
+    assert errors("\ts_cselect_b32 s9, 0, 0x80\n") == []
+    assert errors("\ts_and_b32 s9, s20, s2\n") == []
+    assert errors("\ts_cselect_b32 s8, s20, 0\n\ts_mov_b32 s9, s8\n") == []
+    assert errors("\ts_mov_b32 s9, 0\n") == []
+    assert errors("")                                                     # written nowhere
+    assert errors("\ts_lshl_b32 s9, s20, 7\n")
+    assert errors("\ts_cselect_b32 s9, s20, s21\n")
+    assert errors("\ts_mov_b32 s9, s20\n")
+    assert errors("\ts_cselect_b32 s9, s20, 0\n\ts_add_i32 s9, s9, 64\n")  # written again
+    assert errors("\ts_cselect_b32 s9, s20, 0\n\ts_mul_hi_u32 s9, s1, s2\n")
+    assert errors("\ts_cselect_b32 s9, s20, 0\n\ts_lshl_b64 s[8:9], s[20:21], 1\n")
+    # on one of two ways only
+    assert errors("\ts_cbranch_vccz .LBB0_1\n\ts_cselect_b32 s9, s20, 0\n")
+    # behind the load, so not in the second round of the loop
+    late = GEMM.replace("s4 offen", "s9 offen").replace("\ts_cbranch", "\ts_add_i32 s9, s9, 128\n\ts_cbranch")
+    assert errors("\ts_cselect_b32 s9, s20, 0\n", late)
+    assert errors("\ts_cselect_b32 s9, s20, 0\n", GEMM.replace("gemm_lds", "other"))
+
+
 def test_the_build_checks_every_source_with_the_tiled_gemm():
     import os
 
