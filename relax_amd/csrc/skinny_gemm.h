@@ -343,9 +343,17 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       direct_load16(s_base, (wq_lptr_t)(s_block + c * 1024), s_off + (g * 32 < K ? g : 0) * 2, 0);
     }
   }
-  for (int p = 0; p < ahead && p < nsteps; ++p) issue(p, p);
+  auto fill = [&](int p) { issue(p, p); };
+  if constexpr (TH <= 2) {
+    // one or two rounds; unrolled by eight, what the compiler computes in front of them delays the first load (N = K = 1024,
+    // up to 16 rows: 3.6 .. 3.9 -> 3.4 .. 3.7 us, what they took with addresses of 64 bits)
+#pragma unroll 1
+    for (int p = 0; p < ahead && p < nsteps; ++p) fill(p);
+  } else {
+    for (int p = 0; p < ahead && p < nsteps; ++p) fill(p);
+  }
   int cslot = 0;                       // slot of the step being computed
-  int islot = ahead % stages;          // slot the next issue goes to
+  int islot = ahead;                   // slot the next issue goes to
   for (int it = 0; it < nsteps; ++it) {
     wait_newer_groups<Cfg::kLoadsPerStep>(min(ahead - 1, nsteps - 1 - it));  // steps issued after step `it`
     if (NW > 1 || (SB && KW > 1 && it == 0)) __builtin_amdgcn_s_barrier();
