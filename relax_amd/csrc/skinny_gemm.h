@@ -197,9 +197,15 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
   // since they take 32-bit offsets and bring zeros past K by themselves.  With the operands of the next MFMAs requested
   // before the last ones are multiplied (kAhead) and the slab's order above, at 8 shapes x M = 3 .. 64, 4 formats: 6 % faster
   // on average (q4f16_1, N = 12288, K = 4096, M = 19: 17.5 -> 13.9 us; int8, N = 5120, K = 13824, M = 48: 50.4 -> 39.0).
-  // Slower is only int8 with 17 .. 32 rows and two wavefronts side by side, for a reason not known: from 26 rows on 27.0 ->
-  // 32.4 us (N = 5120, K = 13824).  It keeps the loads it had: as fast as before up to 28 rows, up to 7 % slower at 29 .. 32.
+  // int8 with 17 .. 32 rows and two wavefronts side by side loses by that: the faster the loads of a step follow one another
+  // the longer they take, the more so the more rows there are (the four slab loads of a wavefront bring as many lines as rows;
+  // N = 4160, K = 13824, M = 32: 27.3 us with a test for the end of the row in front of each, 29.2 without, 32.4 as buffer
+  // loads).  Without the tests the weights follow behind the products there, so that a burst is two thirds as long: 26.7 us;
+  // over N = 4160 .. 8192, K = 8704 .. 28672, M = 17 .. 32 7 % faster on average than with the tests, 5 % than in one burst.
+  // Where K does not come out even, the tests are needed anyway and the burst is the faster one up to 24 rows (N = 8192,
+  // K = 8768, M = 17: 21.0 us, with the weights behind the products 21.7).
   constexpr bool kBuffer = !WIDE && !(P == 2 && TH == 4 && NW == 2);
+  constexpr bool kLateWeights = !WIDE && !kBuffer && EVEN;
   constexpr bool kAhead = kBuffer && TH >= 4;
   using Off = std::conditional_t<kBuffer, uint32_t, int64_t>;
   Off x_off[Cfg::kXLoads];
@@ -237,15 +243,12 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
   // one load of one wavefront, lane (j, q) bringing scales 32c + 8q .. + 7 of column j
   unsigned char* const s_block = lds + stages * Cfg::kStageBytes + nw * ((((K + 1023) >> 10)) << 10);
 
-  auto issue = [&](int it, int slot) {
-    const int stage_off = slot * Cfg::kStageBytes;
+  auto issue_slab = [&](int it, int slot) {
     const int ks = it * KW + kw;
-    const int k0 = 128 * ks + 32 * kq;             // this lane's 32 weights
-    const int k0c = EVEN || k0 < K ? k0 : 0;       // past the end: any valid address (scale is zeroed)
 #pragma unroll
     for (int i = 0; i < Cfg::kXLoads; ++i) {
       // past K the slab holds zeros: the weights there are exact zeros, and zero times an infinite activation is not
-      const wq_lptr_t dst = (wq_lptr_t)(lds + stage_off + kw * Cfg::kSlabBytes + (nw * Cfg::kXLoads + i) * 1024);
+      const wq_lptr_t dst = (wq_lptr_t)(lds + slot * Cfg::kStageBytes + kw * Cfg::kSlabBytes + (nw * Cfg::kXLoads + i) * 1024);
       const bool in_row = EVEN || x_k[i] < K - 128 * ks;
       if constexpr (!kBuffer) {
         const char* const src = reinterpret_cast<const char*>(X) + x_off[i] + (int64_t)ks * 256;
@@ -254,6 +257,12 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
         direct_load16(reinterpret_cast<const char*>(X), dst, in_row ? x_off[i] : kOutside, ks * 256);
       }
     }
+  };
+  auto issue_weights = [&](int it, int slot) {
+    const int stage_off = slot * Cfg::kStageBytes;
+    const int ks = it * KW + kw;
+    const int k0 = 128 * ks + 32 * kq;             // this lane's 32 weights
+    const int k0c = EVEN || k0 < K ? k0 : 0;       // past the end: any valid address (scale is zeroed)
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const wq_lptr_t dst = (wq_lptr_t)(w_area + stage_off + p * 1024);
@@ -343,7 +352,10 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       direct_load16(s_base, (wq_lptr_t)(s_block + c * 1024), s_off + (g * 32 < K ? g : 0) * 2, 0);
     }
   }
-  auto fill = [&](int p) { issue(p, p); };
+  auto fill = [&](int p) {
+    issue_slab(p, p);
+    issue_weights(p, p);
+  };
   if constexpr (TH <= 2) {
     // one or two rounds; unrolled by eight, what the compiler computes in front of them delays the first load (N = K = 1024,
     // up to 16 rows: 3.6 .. 3.9 -> 3.4 .. 3.7 us, what they took with addresses of 64 bits)
@@ -359,10 +371,19 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
     if (NW > 1 || (SB && KW > 1 && it == 0)) __builtin_amdgcn_s_barrier();
     // the slot refilled now was computed in the previous iteration (by everyone: barrier above)
     if (it + ahead < nsteps) {
-      issue(it + ahead, islot);
-      islot = islot + 1 == stages ? 0 : islot + 1;
+      issue_slab(it + ahead, islot);
+      if constexpr (!kLateWeights) {
+        issue_weights(it + ahead, islot);
+        islot = islot + 1 == stages ? 0 : islot + 1;
+      }
     }
     compute(it, cslot);
+    if constexpr (kLateWeights) {
+      if (it + ahead < nsteps) {
+        issue_weights(it + ahead, islot);
+        islot = islot + 1 == stages ? 0 : islot + 1;
+      }
+    }
     cslot = cslot + 1 == stages ? 0 : cslot + 1;
   }
 

@@ -159,6 +159,21 @@ def test_slabs_of_24_rows(ops, u, oracle, nbit, group_size, M, N, K, nw, stages)
         _lib.lib().wq_debug_set_skinny_config(0, 0, 0)
 
 
+@pytest.mark.parametrize("stages", [2, 3, 4])
+@pytest.mark.parametrize("group_size", [-1, 64])
+@pytest.mark.parametrize("M,N,K", [(17, 64, 512), (24, 192, 1024), (25, 64, 1536), (32, 320, 4608), (32, 192, 576), (29, 64, 64)])
+def test_int8_two_column_blocks(ops, u, oracle, group_size, M, N, K, stages):
+    """int8, 17 .. 32 rows, two wavefronts side by side: the weights of a later step are requested behind the products
+    where K comes out even (K % 512 == 0: one step, as many as the ring holds, more), with the activations elsewhere."""
+    from relax_amd import _lib
+
+    _lib.lib().wq_debug_set_skinny_config(2, stages, 1)
+    try:
+        _run(ops, u, oracle, M, N, K, 8, seed=M + K, group_size=group_size)
+    finally:
+        _lib.lib().wq_debug_set_skinny_config(0, 0, 0)
+
+
 @pytest.mark.parametrize("rows", [0, 1, 2])
 @pytest.mark.parametrize("nbit", [8, 4])
 @pytest.mark.parametrize("group_size", [-1, 64])
