@@ -47,7 +47,8 @@ struct IntbSkinnyPolicy {
   static constexpr int kStepStride = 256;
   __device__ __forceinline__ static const char* s_lane(const Lane& l) { return reinterpret_cast<const char*>(l.s); }
   __device__ __forceinline__ static uint32_t s_rel(const Lane& l, int k0) { return (uint32_t)(k0 >> 6) * (uint32_t)l.N * 2; }
-  static int64_t s_reach(const Args&, int64_t N, int64_t K) { return GROUPED ? (K / 64) * N * 2 : 0; }
+  __device__ __forceinline__ static int s_step(int N) { return 4 * N; }
+  static int64_t s_reach(const Args&, int64_t N, int64_t K) { return GROUPED ? (K / 64 + 16) * N * 2 : 0; }
   static bool pair_aligned(const Args& a) { return (reinterpret_cast<uintptr_t>(a.scales) & 3u) == 0; }
   __device__ __forceinline__ static half_t pick_scale(const Lane& l, half2_t pair, int) { return l.odd ? pair.y : pair.x; }
   using Scale = half_t;

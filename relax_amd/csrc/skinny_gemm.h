@@ -63,6 +63,8 @@ namespace wq {
 //   kStepStride                bytes between a lane's pieces of consecutive steps (128 k)
 //   s_lane(lane), s_rel(lane, k0)   s_addr(lane, k0) as a pointer and a 32-bit offset from it           (kScaleDma)
 //   s_reach(args, N, K)        host: no such offset inside 16 columns goes beyond this
+//   s_step(N)                  optional: bytes between a lane's scales of consecutive steps, where they lie evenly (then
+//                              s_reach has room for 8 steps past K)
 // and, for weights that are not rounded (up to 8 rows, kPieces == 1),
 //   codes8(word)               the codes of a word of codes as halves, exact (8 consecutive k); the products of a
 //                              group of 32 k are summed alone and scaled in fp32
@@ -79,6 +81,11 @@ template <class P, class = void>
 struct OddStart : std::false_type {};
 template <class P>
 struct OddStart<P, std::void_t<decltype(P::kOddStart)>> : std::bool_constant<P::kOddStart> {};
+
+template <class P, class = void>
+struct ScaleStep : std::false_type {};
+template <class P>
+struct ScaleStep<P, std::void_t<decltype(&P::s_step)>> : std::true_type {};
 
 // bits 0 .. n - 1 of `groups` groups, of which those up to K exist
 __device__ __forceinline__ uint32_t live_groups(int k0, int K, int groups) {
@@ -135,8 +142,8 @@ static __device__ const uint4_t kZeroChunk = {0, 0, 0, 0};  // ... as this does 
 __device__ __forceinline__ void direct_load16(const char* base, wq_lptr_t dst, uint32_t off, int step_off) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(base, (int)kOutside), dst, 16, off, step_off, 0, 0);
 }
-__device__ __forceinline__ void direct_load4(const char* base, wq_lptr_t dst, uint32_t off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(base, (int)kOutside), dst, 4, off, 0, 0, 0);
+__device__ __forceinline__ void direct_load4(const char* base, wq_lptr_t dst, uint32_t off, int step_off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(wq_rsrc(base, (int)kOutside), dst, 4, off, step_off, 0, 0);
 }
 
 template <typename Policy, int TH, int NW, int WAVES, bool SB = false>
@@ -234,6 +241,14 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       s_off += 4;
     }
   }
+  // Where K does not come out even and a lane's scales lie evenly, the step goes into the scalar offset: with a test and a
+  // multiplication per lane and load in its place int8 with a scale per 64 took up to 9 % longer than with 64-bit addresses
+  // (N = 4096, K = 11008: M = 16 14.4 -> 13.7 us, M = 24 21.1 -> 19.9; N = 3072, K = 8768, M = 12 12.4 -> 11.3).  Where
+  // K comes out even it is faster or slower by as much, depending on the shape (int8 with a scale per 64, N = 4096, K = 13824,
+  // M = 24 26.9 -> 28.1 us; int4 with one, N = 8192, K = 8192, M = 24 17.3 -> 16.4).
+  constexpr bool kScaleStep = Cfg::kStepScale && kBuffer && ScaleStep<Policy>::value && !EVEN;
+  uint32_t s_first = 0;
+  if constexpr (kScaleStep) s_first = Policy::s_rel(pl, 32 * kq);
   typename Policy::Scale s_fixed = Policy::null_scale();
   if (!Policy::kScaleDma) s_fixed = Policy::const_scale(pl);
 
@@ -275,8 +290,10 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       const wq_lptr_t dst = (wq_lptr_t)(s_area + stage_off);
       if constexpr (!kBuffer)
         __builtin_amdgcn_global_load_lds((wq_gptr_t)Policy::s_addr(pl, k0c), dst, 4, 0, 0);
+      else if constexpr (kScaleStep)
+        direct_load4(s_base, dst, k0 < K ? s_off + s_first : kOutside, ks * Policy::s_step(N));
       else
-        direct_load4(s_base, dst, s_off + Policy::s_rel(pl, k0c));
+        direct_load4(s_base, dst, s_off + Policy::s_rel(pl, k0c), 0);
     }
   };
 
