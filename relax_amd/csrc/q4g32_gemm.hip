@@ -122,7 +122,11 @@ extern "C" int wq_q4g32_gemm(const uint32_t* W, const uint16_t* S, const uint16_
   }
   if (cfg >= 11 && K % 64 == 0 && lds_ok) {
     if (cfg == 15 || cfg == 16 || cfg > 19) return fail(WQ_EINVAL, "wq_q4g32_gemm: unknown tile configuration %d", cfg);
-    if (K < 256)  // fewer steps than the weights are requested ahead
+    // fewer steps than the weights are requested ahead; 256 x 256 tiles up to K = 320, where filling that pipeline, with
+    // one workgroup per CU, costs more than it brings (N = 22016: K = 256, M = 2048 51.2 -> 42.6 us, M = 8192 174.7 -> 160.0,
+    // K = 320, M = 1024 31.9 -> 29.9; 7 % on average over N = 4096 .. 28672, M = 512 .. 8192, N = 16384, K = 256,
+    // M = 4096 5 % slower; at K = 384 as many shapes lose as gain)
+    if (K < 256 || (K <= 320 && cfg == 11 && !tuning().gemm_cfg))
       return launch_gemm_lds<Q4G32LdsPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_q4g32_gemm", largs, x, y, ep, M, N, K, stream);
     if (cfg == 19 && K % 128 != 0) cfg = 17;
     using P = Q4G32RegPolicy;

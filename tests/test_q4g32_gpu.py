@@ -447,6 +447,16 @@ def test_gemm_k_loop_ends_bit_exact(ops, u, oracle, cfg, K):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("K", [192, 256, 320, 384])
+def test_short_k_and_256_row_tiles_bit_exact(ops, u, oracle, K):
+    """More than one round of 256 x 128 tiles: 128 x 128 tiles with the weights in LDS up to K = 320, 256 x 256 tiles with
+    the weights in registers above.  One activation per row is not zero, so the product is a weight."""
+    M, N = 1030, 8200
+    _, W, S = oracle.make_q4g32_inputs(1, N, K, seed=K)
+    got = u.host(ops.q4g32_linear(u.dev(W), u.dev(S), u.dev(np.eye(K, dtype=np.float16)[np.arange(M) % K])))
+    np.testing.assert_array_equal(got, oracle.q4g32_dequant(W, S).T[np.arange(M) % K])
+
+
 @pytest.mark.parametrize("M,K", [(5, (1 << 23) + 32), (20, (1 << 23) - 64), (40, (1 << 23) + 64)])
 def test_small_batch_where_offsets_leave_32_bits(ops, u, M, K):
     """K around 2^23, from where on the small-batch kernel takes 64-bit addresses.  One activation per row is not zero, so
