@@ -599,7 +599,11 @@ static int wq::gptq_linear_impl(const uint32_t* W_nk, const uint16_t* SZ, const 
   const GptqLdsPolicy::Args largs{W_nk, (const half2_t*)SZ, (int)G, spg,
                                   spg > 1 ? (uint32_t)(((1ull << 32) + spg - 1) / spg) : 0u};
   const int cfg = choose_q4_lds_cfg(M, N, cu_count());
-  if (spg % 2 == 0 && K >= 256) {
+  // weights in registers from four steps on; with 256 x 256 tiles (one workgroup per CU, so nobody works while its ring
+  // fills) from K = 640 on, below that they stay in LDS (N = 28672, M = 1024: K = 256 36.8 -> 31.3 us, K = 512 48.2 -> 43.8;
+  // N = 11008, M = 4096, K = 384 58.6 -> 55.5; N = 22016, M = 4096, K = 512 119.9 -> 123.0; K = 1024, M = 4096 190 in
+  // registers, 194 in LDS)
+  if (spg % 2 == 0 && K >= (cfg == 11 ? 640 : 256)) {
     switch (cfg) {
       case 17: return launch_gemm_lds<GptqRegPolicy, Q4G32Epilogue, 4, 1, 1, 4, 2>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);
       case 18: return launch_gemm_lds<GptqRegPolicy, Q4G32Epilogue, 8, 1, 1, 4, 1>("wq_gptq_linear", largs, x, y, ep, M, N, K, stream);

@@ -275,3 +275,14 @@ def test_gemm_returns_the_weights_bit_exact(ops, u, oracle, M, N, K, gs):
     w = ops.gptq_prepare(u.dev(qw), u.dev(qz), u.dev(s), u.dev(g_idx))
     got = u.host(ops.gptq_linear(w, u.dev(np.eye(K, dtype=np.float16))))
     np.testing.assert_array_equal(got, oracle.gptq_dequant(qw, qz, s, g_idx))
+
+
+@pytest.mark.parametrize("K,gs", [(256, 128), (512, 128), (640, 128), (768, 384)])
+def test_256_row_tiles_return_the_weights_bit_exact(ops, u, oracle, K, gs):
+    """More than one round of 256 x 128 tiles, so 256 x 256 tiles: weights in LDS below K = 640, in registers from there on.
+    One activation per row is not zero, so the product is a weight."""
+    M, N = 1030, 8200
+    _, qw, qz, s, g_idx = oracle.make_gptq_inputs(1, N, K, gs, seed=K + gs, act_order=False)
+    w = ops.gptq_prepare(u.dev(qw), u.dev(qz), u.dev(s), u.dev(g_idx))
+    got = u.host(ops.gptq_linear(w, u.dev(np.eye(K, dtype=np.float16)[np.arange(M) % K])))
+    np.testing.assert_array_equal(got, oracle.gptq_dequant(qw, qz, s, g_idx)[np.arange(M) % K])
