@@ -92,15 +92,13 @@ def build(verbose: bool = True, incremental: bool = False) -> str:
         with concurrent.futures.ThreadPoolExecutor(max_workers=8) as ex:
             compiled = [ex.submit(_compile, s) for s in todo]
             checks = [ex.submit(check_asm, os.path.basename(s)) for s in checked]
-            for f in compiled:
+            concurrent.futures.wait(compiled + checks)
+            for f, s in zip(checks, checked):  # an incremental build must not take a refused object for up to date
+                obj = os.path.join(OBJDIR, os.path.basename(s) + ".o")
+                if f.exception() is not None and os.path.exists(obj):
+                    os.remove(obj)
+            for f in compiled + checks:
                 f.result()
-            try:
-                for f in checks:
-                    f.result()
-            except Exception:
-                for s in checked:  # an incremental build must not take the refused objects for up to date
-                    os.remove(os.path.join(OBJDIR, os.path.basename(s) + ".o"))
-                raise
     for lib, want in ((LIB, False), (CALIBRATE_LIB, True)):
         objs = [os.path.join(OBJDIR, os.path.basename(s) + ".o") for s in srcs
                 if (os.path.basename(s) in CALIBRATE_SOURCES) == want]

@@ -135,3 +135,31 @@ def test_the_build_checks_every_source_with_the_tiled_gemm():
                 if "launch_gemm_lds<" in f.read():
                     with_gemm.add(name)
     assert with_gemm == set(c.DIRECT_LOAD_SOURCES)
+
+
+def test_an_incremental_build_does_not_keep_what_was_refused(tmp_path, monkeypatch):
+    """A source that does not compile must not hide that another one was refused: its object would pass for up to date."""
+    import os
+
+    import pytest
+
+    from relax_amd import build as b
+
+    refused, broken, fine = "gptq.hip", "common.cc", "q4n32.hip"
+    monkeypatch.setattr(b, "OBJDIR", str(tmp_path))
+    monkeypatch.setattr(b, "sources", lambda: [os.path.join(b.CSRC, n) for n in (refused, broken, fine)])
+
+    def compile_(src):
+        if src.endswith(broken):
+            raise RuntimeError("does not compile")
+        (tmp_path / (os.path.basename(src) + ".o")).write_text("object")
+
+    def check(name):
+        if name == refused:
+            raise RuntimeError("refused")
+
+    monkeypatch.setattr(b, "_compile", compile_)
+    monkeypatch.setattr(b, "check_asm", check)
+    with pytest.raises(RuntimeError):
+        b.build(verbose=False, incremental=True)
+    assert sorted(p.name for p in tmp_path.iterdir()) == [fine + ".o"]
