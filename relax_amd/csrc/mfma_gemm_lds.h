@@ -28,8 +28,7 @@
 //   kColBytes            packed bytes per column and K-step (32 or 64)
 //   kScaleBytes          bytes of scales per column and K-step staged in LDS (0, 4, or 8 as two planes of 4)
 //   Args, Frag, Scale    kernel arguments; a lane's packed codes of one column for one step; what
-//                        pair() needs besides the codes (the scale in both halves of a register,
-//                        plus the zero point where the format has one)
+//                        pair() needs besides the codes (the scale, with the zero point where the format has one)
 //   b_src(args, n0, q, N, K)   global address (step 0) of 16-byte chunk q of the B tile at column n0
 //   kStepStride          bytes between consecutive K-steps of a chunk
 //   s_src(args, n, K)    global address (step 0) of the 4 scale bytes of column n       (kScaleBytes > 0)
@@ -41,10 +40,10 @@
 //   const_scale(args, n) the Scale of column n                                          (kScaleBytes == 0)
 //   read(frag, bslot, n_local, lh)   LDS -> registers
 //   pair(frag, kk, j, scale)   dequantized weights (k = 8kk + 2j, 8kk + 2j + 1) of the lane's column,
-//                              = pair_finish(pair_bits(frag, kk, j), scale): the two exact fp16 integers
-//                              as a bit pattern, then (integer - offset) * scale.  The K loop runs the two
-//                              halves in different MFMA slots: a chain of four dependent VALU operations
-//                              does not fit behind one MFMA, two do.
+//                              = pair_finish(pair_bits(frag, kk, j), scale): the two exact fp16 integers as a bit
+//                              pattern, the offset of the codes subtracted where it is known beforehand, then
+//                              times the scale (after the zero point, where there is one).  The K loop runs the
+//                              two halves in different MFMA slots: the whole chain does not fit behind one MFMA.
 // and, only where the scale of a weight depends on its k inside the step (scales along N):
 //   phase_begin(scale, kk)     called once per column sub-tile in front of the phase that unpacks the weights
 //                              of MFMA kk: fetches what pair_finish_at needs for them
@@ -184,7 +183,8 @@ __device__ __forceinline__ void finish_tile(float16_t (&acc)[TME][TN], half_t* _
 //               weights, the first activation fragments and the first weight pairs of
 //               step ks+1, so that step ks+1 starts multiplying at once.
 // The K loop is one basic block: the loads past the last step are issued too, against a descriptor that holds nothing, so
-// that the waits are constants.  Branches around them cost more than themselves, since the compiler moves the unpacking
+// that the waits are constants (and leave the last of those loads on their way: the ring is drained behind the loop, in
+// front of finish_tile).  Branches around them cost more than themselves, since the compiler moves the unpacking
 // across the end of a block, behind the barrier.  With buffer loads, the integers of a pair finished in its first slot and
 // no wait for the scale in front of phase 3: 540 -> 308 instructions per step, N = 22016, K = 4096, M = 8192 1292 -> 1207 us,
 // int4 N = 28672, K = 8192, M = 500 232 -> 219 us, N = 11008, K = 4096, M = 200 36.4 -> 35.4 us.
@@ -424,11 +424,11 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
 //
 // Order of the loads (all of a wavefront's loads retire in order, and the wait for the activations counts them): step ks
 // requests the activations of step ks + 3 in phase 0, the scales of the next four steps in phase 1 where ks % 4 == 0, and in
-// phase 3 of odd steps the weights of steps ks + 3 and ks + 4, whose registers it has just emptied.  The prologue issues its loads in the order that the steps before the first would have had.
+// phase 3 of odd steps the weights of steps ks + 3 and ks + 4, whose registers it has just emptied.  The prologue issues
+// its loads in the order that the steps before the first would have had.
 //
 // Such a policy provides besides pair_bits / pair_finish
 //   kStepStride            bytes between the steps of a column, of which a lane takes 16
-//   b_base(args, n0, K)    where the columns from n0 on begin, b_lane(n, n0, lh, K) the lane's first piece from there
 //   kFourScales            true: a scale per 32 k, contiguous along K, taken for four steps at a time;
 //                          false: a pair of halves that serves two steps
 //   b_base(args, n0, K)    where the columns from n0 on begin, b_lane(n, n0, lh, K) the lane's first piece from there
@@ -436,7 +436,9 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
 //   s_step(args, ks)       bytes from there to the pair of step ks (not kFourScales)
 // Measured with the K loop below it, start of that change / before / now: N = 22016, K = 4096, M = 8192 1307 / 1219 / 1191 us;
 // N = 4096, K = 11008, M = 2048 194 / 187 / 178; N = 11008, K = 4096, M = 200 37.2 / 35.5 / 32.4; AutoGPTQ with a group of 128,
-// 128 x 128 tiles, 36.2 / - / 26.6 us.  fpA_intB stays with LDS: its 128-byte units are whole lines there, eight a load
+// 128 x 128 tiles, 36.2 / - / 26.6 us.  With two wavefronts above one another (WM = 2: shapes 13 and 14, which the choice by
+// size does not take on 256 CUs) both fetch the same weights, and it is the faster form all the same (256 x 128, N = 4096,
+// K = 11008, M = 1024 135 -> 120 us; 256 x 256, N = 11008, K = 4096, M = 1024 107 -> 98).  fpA_intB stays with LDS: its 128-byte units are whole lines there, eight a load
 // (int8, N = 28672, K = 8192, M = 128: 84 us, in registers 88).
 template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME, int KW = 1>
 __device__ __forceinline__ void gemm_rb_tile(const typename Policy::Args& wargs, const half_t* __restrict__ X,
@@ -722,10 +724,6 @@ struct FineTail : std::false_type {};
 template <class P>
 struct FineTail<P, std::void_t<decltype(P::kFineTail)>> : std::bool_constant<P::kFineTail> {};
 
-// Workgroup -> work item.  The first n_full workgroups compute whole tiles (as many
-// as fill complete rounds of the machine); the tiles of the last, partially filled
-// round are cut into `split` row slices of TM/split sub-tiles so that the round is
-// shorter instead of leaving most CUs idle while a few finish whole tiles.
 template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WPE, int TME, int KW>
 __device__ __forceinline__ void gemm_tile(const typename Policy::Args& wargs, const half_t* __restrict__ X,
                                           half_t* __restrict__ Y, const Epilogue& epilogue, int M, int N, int K, int m0,
@@ -736,6 +734,10 @@ __device__ __forceinline__ void gemm_tile(const typename Policy::Args& wargs, co
     gemm_lds_tile<Policy, Epilogue, TM, TN, WM, WN, WPE, TME, KW>(wargs, X, Y, epilogue, M, N, K, m0, n0, lds);
 }
 
+// Workgroup -> work item.  The first n_full workgroups compute whole tiles (as many
+// as fill complete rounds of the machine); the tiles of the last, partially filled
+// round are cut into `split` row slices of TM/split sub-tiles so that the round is
+// shorter instead of leaving most CUs idle while a few finish whole tiles.
 template <class Policy, class Epilogue, int TM, int TN, int WM, int WN, int WAVES_PER_EU, int KW>
 __global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU, WAVES_PER_EU)))
 void gemm_lds_kernel(typename Policy::Args wargs, const half_t* __restrict__ X, half_t* __restrict__ Y,

@@ -203,7 +203,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
   // Buffer loads, because behind a global_load_lds the compiler waits for all LDS reads wherever it waits for one, and
   // since they take 32-bit offsets and bring zeros past K by themselves.  With the operands of the next MFMAs requested
   // before the last ones are multiplied (kAhead) and the slab's order above, at 8 shapes x M = 3 .. 64, 4 formats: 6 % faster
-  // on average (q4f16_1, N = 12288, K = 4096, M = 19: 17.5 -> 13.9 us; int8, N = 5120, K = 13824, M = 48: 50.4 -> 39.0).
+  // on average (q4f16_1, N = 12288, K = 4096, M = 19: 17.5 -> 13.9 us; int8, N = 5120, K = 13824, M = 48: 50.4 -> 41.0).
   // int8 with 17 .. 32 rows and two wavefronts side by side loses by that: the faster the loads of a step follow one another
   // the longer they take, the more so the more rows there are (the four slab loads of a wavefront bring as many lines as rows;
   // N = 4160, K = 13824, M = 32: 27.3 us with a test for the end of the row in front of each, 29.2 without, 32.4 as buffer
@@ -737,8 +737,9 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
   // 17 .. 24 rows: slabs of 24 rows and three wavefronts side by side where four or eight leave a second, partly filled
   // round: between four and six tiles per CU in every format (M = 19, q4f16_1 / int8: N = 18432, K = 4096 28.8 -> 20.0 /
   // 32.3 -> 20.4 us, N = 24576, K = 6144 36.7 -> 30.8 / 40.1 -> 35.1; N = 16384 and N = 24640 lose 10 .. 30 %), and between
-  // two and three, where it makes one whole round, for int8 (N = 12288, K = 4096 16.5 -> 14.2, N = 10240, K = 8192 25.5 ->
-  // 22.9; N = 8192 loses 16 %; int4 is as fast either way and up to N = 9216 slower).
+  // two and three, where it makes one whole round, for int8 (against what was there before: N = 8256, the first width it
+  // takes, K = 4096 15.7 -> 13.9, K = 13824 40.9 -> 36.0; 10240, 8192 26.7 -> 23.1; 12288, 4096 17.6 -> 14.0; at every width
+  // between and K = 2048 .. 13824 7 .. 20 % faster; N = 8192 loses 16 %; int4 is as fast either way and up to N = 9216 slower).
   if (M > 16 && M <= 24) {
     const int64_t tiles = (N + 15) / 16, cus = cu_count();
     if ((tiles > 4 * cus && tiles <= 6 * cus) || (Policy::kPieces == 2 && tiles > 2 * cus && tiles <= 3 * cus)) nw = 3;
