@@ -264,7 +264,7 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
       if (is_a || is_b) __builtin_amdgcn_global_load_lds((wq_gptr_t)src, (wq_lptr_t)dst, 16, 0, 0);
       else __builtin_amdgcn_global_load_lds((wq_gptr_t)src, (wq_lptr_t)dst, 4, 0, 0);
     } else {
-      const int live = __builtin_amdgcn_readfirstlane(ks < ksteps ? -1 : 0);
+      const int live = wq_live(ks, ksteps);
       if (is_a) direct_load16_if(live, a_base, (wq_lptr_t)dst, a_off[i], k * 128);
       else if (is_b) direct_load16_if(live, b_base, (wq_lptr_t)dst, b_off[i], k * Policy::kStepStride);
       else direct_load4_if(live, s_base, (wq_lptr_t)dst, s_off[i], (int)Policy::s_offset(wargs, k));
@@ -480,7 +480,7 @@ __device__ __forceinline__ void gemm_rb_tile(const typename Policy::Args& wargs,
   uint4_t s_cur[TN], s_next[TN];    // scales of this set of four steps and of the next (kFour)
   half2_t s_pair[2][TN];            // (not kFour)
   // past the last step: descriptors that hold nothing
-  auto live = [&](int ks) { return __builtin_amdgcn_readfirstlane(ks < ksteps ? -1 : 0); };
+  auto live = [&](int ks) { return wq_live(ks, ksteps); };
   auto issue_a = [&](int ks, int slot, int i) {
     direct_load16_if(live(ks), a_base, (wq_lptr_t)(lds + slot * Cfg::kStageBytes + (wave * kA + i) * 1024), a_off[i], (ks0 + ks) * 128);
   };

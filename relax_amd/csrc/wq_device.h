@@ -98,6 +98,13 @@ typedef __amdgpu_buffer_rsrc_t wq_rsrc_t;
 __device__ __forceinline__ wq_rsrc_t wq_rsrc(const char* base, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00027000);
 }
+// -1 where a < b, else 0, of two numbers that are the same for the wavefront.  As a comparison of the compiler's it goes
+// through a vector register and back, in every step of a loop.
+__device__ __forceinline__ int wq_live(int a, int b) {
+  int live;
+  asm("s_sub_i32 %0, %1, %2\n\ts_ashr_i32 %0, %0, 31" : "=&s"(live) : "s"(a), "s"(b) : "scc");
+  return live;
+}
 // Loads from base + off + step_off (of which step_off is the same for the wavefront) with `live` -1.  With `live` 0 the
 // descriptor is empty: they bring zeros and touch no memory.  That must not depend on whether the range check counts the
 // scalar offset (0 bytes less an offset would be many), so the scalar offset of such a load is 0.
