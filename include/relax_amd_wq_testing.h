@@ -47,6 +47,9 @@ void wq_debug_set_skinny_config(int nw, int stages, int waves);
  * different linears side by side, or 0 if the linears of the (short) list share the 8 XCDs in sets sized by
  * their cost; -1 for a list of one activation row. */
 int wq_debug_gemv_list_groups(const wq_gemv_list_t* list);
+/* The shape of the kernel of a list of 2 .. 16 activation rows: 0, 1 items of 32, 16 rows x 4096 k (up to 8 activation
+ * rows), 2, 3 of 32, 16 rows x 2048 k; -1 for any other list. */
+int wq_debug_gemv_list_shape(const wq_gemv_list_t* list);
 
 /* ---- librelax_amd_wq_calibrate.so ---- */
 /* Issues `iters` x 8 independent v_mfma_f32_32x32x16_f16 per wavefront, four wavefronts

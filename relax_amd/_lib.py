@@ -94,6 +94,7 @@ TESTING_SIGNATURES = {
     "wq_debug_set_skinny_config": [_int, _int, _int],
     "wq_debug_set_intb_gemv_k_split": [_int],
     "wq_debug_gemv_list_groups": [_vp],
+    "wq_debug_gemv_list_shape": [_vp],
 }
 # ... and the calibration kernels of librelax_amd_wq_calibrate.so
 CALIBRATE_LIB_PATH = os.path.join(HERE, "librelax_amd_wq_calibrate.so")
@@ -131,7 +132,7 @@ def lib() -> ctypes.CDLL:
         for name, argtypes in TESTING_SIGNATURES.items():
             fn = getattr(l, name)
             fn.argtypes = argtypes
-            fn.restype = ctypes.c_int if name == "wq_debug_gemv_list_groups" else None
+            fn.restype = ctypes.c_int if name.startswith("wq_debug_gemv_list_") else None
         _lib = l
     return _lib
 

@@ -1,8 +1,8 @@
 """Build-time checks of the generated code: of ``csrc/q4g32_gemv_list.hip`` and ``csrc/q4g32_batch_list.hip``, and of the
 tiled GEMMs.
 
-The compute wavefronts of the first two load their weight stream with inline-assembly loads into a
-ring of registers and wait for them by hand, so the compiler does not know that those registers are
+The compute wavefronts of the one-row list and of lists of more than 16 rows load their weight stream with inline-assembly
+loads into a ring of registers and wait for them by hand, so the compiler does not know that those registers are
 in flight between a load and its wait.  The source makes every read of a ring register an asm
 statement that depends on the wait; what is left to chance is register allocation (a copy or a
 spill of a ring register inserted between load and wait would read it too early).  This script
@@ -21,7 +21,7 @@ sources therefore wait for all loads (``s_waitcnt vmcnt(0)``) where the ring's l
 Registers that the compiler also uses for short-lived temporaries while a slot is empty are
 recognised by being written by another instruction first.
 
-Kernels with such a ring must also be free of register spills (no ``scratch_*`` instruction).
+Kernels with non-temporal loads, in whatever form, must also be free of register spills (no ``scratch_*`` instruction).
 
 A second check (``check_asm_results``) covers what inline assembly costs besides: the compiler does
 not keep the hardware's wait states between an inline-assembly VALU result and an MFMA or DPP
@@ -46,8 +46,11 @@ DIRECT_LOAD_SOURCES = ("gemm_256.hip", "gptq.hip", "intb_gemm.hip", "q4g32_gemm.
 ALLOWED_READERS = ("v_and_or_b32", "v_lshrrev_b32", "v_cvt_f32_f16", "v_mov_b32_dpp")
 
 
+_COMPILERS = " (waited for by the compiler)"  # behind a non-temporal load outside of inline assembly
+
+
 def _is_ring_load(l: str) -> bool:
-    """A load of the weight stream: the only non-temporal loads of these kernels."""
+    """A load of the weight stream that is waited for by hand: a non-temporal load in inline assembly."""
     return l.startswith(("global_load_", "buffer_load_")) and l.endswith(" nt")
 
 
@@ -140,11 +143,15 @@ def check_asm_results(asm_text: str) -> list[str]:
 
 def _functions(asm_text: str, labels: bool = False):
     """(name, instructions) of every function of the file, with its local labels if asked for."""
-    functions, cur = [], None
+    functions, cur, in_asm = [], None, False
     for raw in asm_text.splitlines():
+        t = raw.strip()
+        in_asm = t.startswith(";;#ASMSTART") or (in_asm and not t.startswith(";;#ASMEND"))
         l = raw.split(";")[0].strip()
         if not l:
             continue
+        if not in_asm and l.endswith(" nt"):
+            l += _COMPILERS
         if l.endswith(":") and not l.startswith("."):  # a function label
             cur = []
             functions.append((l[:-1], cur))
@@ -160,8 +167,8 @@ def check(asm_text: str) -> list[str]:
     """Checks every kernel of the file on its own (register names mean nothing across kernels)."""
     errors, with_ring = [], 0
     for _, body in _functions(asm_text):
-        if any(_is_ring_load(l) for l in body):
-            with_ring += 1
+        if any(_is_ring_load(l) or l.endswith(_COMPILERS) for l in body):
+            with_ring += any(_is_ring_load(l) for l in body)
             errors += _check_function(body)
             # These kernels are written to fit their register budget.  A spill anywhere in them (also in a service
             # wavefront's path: one extra branch there once sent 64 load registers through scratch memory and

@@ -60,6 +60,7 @@ constexpr int kBufferFlags = 0x00020000;  // buffer resource word 3: 32-bit data
 // of the signals they wait for: one linear behind the other, K = N = 1024, 7.8 us a linear at 4, 6.6 at 64; a Llama-2-7B
 // layer 30.0 -> 25.4 us.
 constexpr int kPollSleep = 64;
+constexpr int kNonTemporal = 2;           // cache policy bit nt
 constexpr int kDeviceScope = 16;          // cache policy bit sc1: the access is coherent over the whole device
 
 // error word: 1 + the linear a consumer waited for in vain, or kBatchInternalWait + a code: a hand-over
@@ -103,7 +104,7 @@ struct wq_gemv_list {
   int gather_jobs = 0, gather_blocks = 0;
   bool zp = false;         // AutoGPTQ layers: a (scale, zero point + 1) pair per group instead of a scale per 32 columns
   int M = 1;               // activation rows of the launch; > 1: the batch kernel (q4g32_batch_list.hip) and the fields below
-  int batch_u = 0;         // chunks per tile and wavefront (4: M <= 16; 2: beyond)
+  int batch_shape = 0;     // which of the kernel's shapes (M <= 16)
   int batch_groups = 1;    // groups of workgroups that run different linears side by side (0: sets of XCDs per linear)
   int batch_nxb = 0;       // panels of activations in LDS
   int batch_ring = 0;      // items the compute wavefronts may spread over (slots of scales and of partial sums)

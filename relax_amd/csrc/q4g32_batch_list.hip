@@ -8,20 +8,31 @@
 // Two kernels: up to 16 rows of activations the one described here (q4g32_batch_list_kernel), beyond that
 // q4g32_batch_rows_kernel further down, which shares the unpack, the lane exchange and the staging of activations.
 //
-// Work.  The unit is a TILE of rows of W times a PANEL of K: 16 rows x 4096 k for M <= 8, 32 rows x 2048 k for
-// M <= 16 (an item is 32 KiB of codes: what a workgroup spends per item on hand-overs does not depend on its
-// size).  A linear is run by one GROUP of
-// workgroups (see batch_assign_groups), its tiles dealt to them round-robin, with a rotation that continues
-// from linear to linear.  Inside a workgroup the 8 compute wavefronts split a tile: 16 rows x an eighth of the
-// panel each, or, with tiles of 32 rows, wavefronts 0 .. 3 a quarter of the panel of rows 0 .. 15 each and
-// wavefronts 4 .. 7 of rows 16 .. 31.  A wavefront's share is U = 4 chunks; a chunk is
-// one 16-byte load per lane: lane (i, kq) takes scale group 4u + kq of row i, the 32 codes that the four
-// v_mfma_f32_16x16x32_f16 of the chunk consume as A operands (one dword, 8 codes, each).  (The template
-// parameter R, sets of 16 activation rows per unpacked A operand, is 1 in every instantiation.)
-// Unpacking is exact: OR the code into 0x6400 (1024 + q, or 1024 + 16 q), subtract 1031 (1136),
-// multiply by the scale, all in packed fp16: 13 VALU instructions per 8 weights and lane, whatever M.
-// The B operands (the activations of the wavefront's K slice, in the k order of the unpack, the
-// 16 q positions pre-divided by 16) live in registers for the whole panel.
+// Work.  The unit is a TILE of rows of W times a PANEL of K: RT row tiles (1 or 2, 16 rows each) x 2048 or 4096 k (SP = 1 or
+// 2).  A linear is run by one GROUP of workgroups (see batch_assign_groups), its tiles dealt to them round-robin, with a
+// rotation that continues from linear to linear.  Inside a workgroup the 8 compute wavefronts split the panel 8 ways along
+// K, each for all rows of the item.  A load is 8 rows x 128 bytes, 16 a lane; a lane's 16 bytes are the 32 codes of a scale
+// group.
+//
+// Products.  What bounds this kernel is the vector unit beside the memory: with (q - 7) * s made in packed fp16, 13
+// instructions per 8 weights and lane at 4 cycles a wavefront, it was busy for more than half of the launch.  (Measured per
+// SIMD with two or more wavefronts: and, shift, add and fma of registers or literals take 2 cycles, packed and three-operand
+// bit instructions 4, lane swaps 8.)  So a weight is not made at all.  A word's codes become fp16 numbers by masks alone (4
+// ands and a shift): the code in bits 0 .. 3 of a half is the number 2^-24 q, in bits 4 .. 7 2^-20 q, and the activations of
+// those positions are divided by 16 when they are staged.  One v_mfma_f32_16x16x32_f16 takes the 32 codes of ONE group of 16
+// rows, beginning at -7 times the group's sum of activations (another such product, with -7 in the codes' place), and 4
+// fmas add the scale times that to the sums in fp32.  For one product to hold one group, the words of a group lie in
+// the four lane quarters: two lane swaps for two words.  Nothing is rounded before the sums: against 64 bits the error
+// is that of the fp16 output alone (2.08e-4; with rounded weights 2.74e-4).
+//   Up to 8 activation rows the 16 rows of the operand hold each of them twice, at the groups of the two halves of a
+// 128-byte piece, so that lanes (rows, half) of a load are columns of one product as they come: half of the results, row
+// half against other column half, are sums of nothing and are dropped.  With 9 .. 16 rows (WIDE) two loads exchange halves
+// first (2 DPP moves a word more).
+//   7 times an infinite sum is not what the products would give without it, so activations that are infinite or not a number
+// take weights as the format defines them; so do linears of fewer rows than a row tile, whose few outputs may all be
+// small, which is where the two roundings show.
+// 32 layers of Llama-2-7B, M = 2 / 8 / 16: 774 / 762 / 785 -> 654 / 690 / 790 us (unpack as above; WIDE gains where lists are
+// short: one layer, M = 16, 78 -> 52 us, hidden 8192, ffn 28672, 3 layers 582 -> 411).
 //
 // The other four wavefronts keep everything irregular away from that loop, through LDS:
 //   * 2 x wavefronts wait for a producer linear (bounded spin), load a panel of activations,
@@ -32,13 +43,14 @@
 //     (sharing every panel between them instead was slower at every M).
 //   * the scale wavefront streams the tile's scales (per row up to 256 contiguous bytes: fetched per
 //     lane they cost more than the codes) into a ring of LDS slots, a few tiles ahead.
-//   * the y wavefront adds the 8 partial sums of a tile (4 per 16 rows of a 32-row tile) in a fixed order, keeps the
+//   * the y wavefront adds the 8 partial sums of a tile in a fixed order, keeps the
 //     sum in LDS while further panels of the same rows follow, and at the last panel applies bias / cast / residual,
 //     stores y with device-scope stores and signals the linear's completion counter.
 // A linear of several panels whose kept sums would not fit the LDS is walked in CHUNKS of its tiles (all
 // panels of a chunk, then the next chunk; template parameter CH): the activations are then loaded once
 // per chunk, which the host weighs against fewer, larger groups when it plans the list.
-// Codes in flight per CU: 8 wavefronts x (NT - 1) tiles x U KiB.
+// Codes in flight: an item per wavefront, each load of which is replaced by the next item's as soon as its registers have
+// been read (8 wavefronts x 8 KiB; 16 KiB per CU in flight reach the rate of the memory, 32 all of it).
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -51,7 +63,6 @@ namespace wq {
 constexpr int kBW = 8;     // compute wavefronts: K slices of a panel
 constexpr int kBXW = 2;    // wavefronts that stage activations
 constexpr int kBRing = 4;  // LDS slots of scales and of partial sums: how far the compute wavefronts may spread
-constexpr int kBNT = 3;    // tile buffers per compute wavefront (NT - 1 tiles of loads in flight)
 constexpr int kBThreads = 64 * (kBW + kBXW + 2);
 
 // LDS words that hand the buffers over inside a workgroup (items = (linear, panel, tile) in the
@@ -94,16 +105,14 @@ struct BatchWait {
   }
 };
 
-// TW = 1: a tile is 16 rows of W and the 8 compute wavefronts split the panel 8 ways along K.  TW = 2: a tile is
-// 32 rows, wavefronts 0 .. 3 split the panel 4 ways for its rows 0 .. 15, wavefronts 4 .. 7 for rows 16 .. 31 (half
-// as many hand-overs per byte of weights, twice the activations in a wavefront's registers).
-// R: sets of 16 activation rows every wavefront holds.
-__host__ __device__ constexpr int batch_k_ways(int TW) { return kBW / TW; }
-__host__ __device__ constexpr int batch_panel_groups(int U, int TW) { return batch_k_ways(TW) * 4 * U; }
-__host__ __device__ constexpr int batch_scale_row_bytes(int U, int TW) { return batch_panel_groups(U, TW) * 2 + 16; }  // + 16: rows on different banks
-__host__ __device__ constexpr int batch_scale_slot_bytes(int U, int TW) { return 16 * TW * batch_scale_row_bytes(U, TW); }
-__host__ __device__ constexpr int batch_partial_slot_bytes(int R) { return kBW * R * 1024; }  // per wavefront R sets of 16 activation rows
-__host__ __device__ constexpr int batch_kept_bytes(int R, int TW) { return TW * R * 1024; }   // sums of a tile kept between panels
+// WIDE: 9 .. 16 activation rows (else up to 8); RT: row tiles (16 rows of W) per item; SP: the 8 compute wavefronts split a
+// panel 8 ways along K, SP 128-byte pieces of every row of the item each.
+__host__ __device__ constexpr int batch_panel_groups(int SP) { return kBW * 8 * SP; }
+__host__ __device__ constexpr int batch_scale_row_bytes(int SP) { return batch_panel_groups(SP) * 2 + 16; }  // + 16: rows on different banks
+__host__ __device__ constexpr int batch_scale_slot_bytes(int SP, int RT) { return 16 * RT * batch_scale_row_bytes(SP); }
+__host__ __device__ constexpr int batch_partial_bytes(bool wide) { return wide ? 1024 : 512; }  // of a wavefront and row tile: 8 or 16 activation rows
+__host__ __device__ constexpr int batch_partial_slot_bytes(bool wide, int RT) { return kBW * RT * batch_partial_bytes(wide); }
+__host__ __device__ constexpr int batch_kept_bytes(int RT) { return RT * 1024; }  // sums of a tile kept between panels
 
 // ---- the walk of a workgroup over its items.  All fields are wavefront-uniform.
 struct ItemCursor {
@@ -231,14 +240,14 @@ __device__ __forceinline__ void item_next(ItemCursor& c, gemv_desc_ptr descs, in
   if (++c.lt == (CH ? c.ltend : c.T)) item_next_panel<PG, CH>(c, descs, nlin, b, nwg, chunk);
 }
 
-template <int U, int R, int TW, bool CH>
+template <bool WIDE, int SP, int RT, bool CH>
 __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvListDesc* __restrict__ descs_, int nlin,
                                                                      int* __restrict__ sync, long long spin_limit,
                                                                      int M, int nxb, int ring, int chunk, int use_sync) {
-  constexpr int PG = batch_panel_groups(U, TW);  // scale groups per panel
-  constexpr int KW = batch_k_ways(TW);          // wavefronts that share a panel along K
-  constexpr int NT = kBNT;
-  constexpr int SROW = batch_scale_row_bytes(U, TW), SSLOT = batch_scale_slot_bytes(U, TW);
+  constexpr int SG = 8 * SP, PG = batch_panel_groups(SP);  // scale groups per wavefront, and per panel
+  constexpr int XO = WIDE ? 2 * SP : SP;  // sets of four operands that hold a wavefront's activations
+  constexpr int NL = 2 * RT * SP;       // loads per wavefront and item, 8 rows x 128 bytes each
+  constexpr int SROW = batch_scale_row_bytes(SP), SSLOT = batch_scale_slot_bytes(SP, RT);
   extern __shared__ uint4_t smem[];
   const gemv_desc_ptr descs = (gemv_desc_ptr)descs_;
   char* lds = reinterpret_cast<char*>(smem);
@@ -249,7 +258,7 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
   const int xbuf_bytes = M * (PG * 64);
   char* const sbuf = xbuf + nxb * xbuf_bytes;
   char* const pbuf = sbuf + ring * SSLOT;
-  char* const abuf = pbuf + ring * batch_partial_slot_bytes(R);
+  char* const abuf = pbuf + ring * batch_partial_slot_bytes(WIDE, RT);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -264,170 +273,248 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
   if (wave < kBW) {
     // =========================== compute wavefront ===========================
     const int i = lane & 15, kq = lane >> 4;
-    const int ks = wave & (KW - 1), rt = wave / KW;  // K slice of the panel; which 16 rows of the tile
-    // The tile buffers are loaded in assembly and waited for by hand (loads retire in order and a
-    // compute wavefront issues no other vector memory operation).  `magic` (0x6400 in both halves,
-    // OR-ed under every code) doubles as the token that orders the reads of a buffer behind the wait
-    // for it: the wait "modifies" magic, every first read of a buffer register takes magic as an
-    // operand, and the registers appear in no other statement (checked in the generated code at
-    // build time).
-    uint4_t tb[NT][U];
-    uint32_t magic = 0x64006400u;
-    int ahead = 0;  // items issued and not yet consumed
+    const int ks = wave;  // K slice of the panel
+    // What has been requested: the item that is multiplied next, each load of which is replaced by that of the item behind it
+    // as soon as its contents have been taken.  Past the last item the loads are issued too, against a descriptor that
+    // holds nothing: without a branch around them the compiler counts how many are younger than the one it waits for.
+    uint4_t buf[NL];
     ItemCursor ic, cc;
     ic.lin = 0;
     item_seek<PG, CH>(ic, descs, nlin, b, nwg, chunk);
-    cc = ic;
     int k = 0;    // items consumed
     int pk = -1;  // panels taken
-    half8_t xb[R][U][4];
-    const int gi0 = ks * (4 * U) + kq;  // the lane's scale group within the panel, chunk 0
+    // The activations of the slice as A operands.  Up to 8 rows: lane (i, kq) holds row i mod 8 at the groups of the half
+    // i / 8 of a 128-byte piece, so that one operand serves what both halves of the lanes have loaded.
+    half8_t xb[XO][4];
+    bool special = false;
+    const int xrows16 = WIDE ? M : 2 * M;
+    const int xrow = WIDE ? min(i, M - 1) : (i >> 3) * M + min(i & 7, M - 1);
+    const half8_t seven = __builtin_bit_cast(half8_t, uint4_t{0x80078007u, 0x80708070u, 0x80078007u, 0x80708070u});
+    auto sevenfold = [&](int v, int g) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[v][g], seven, float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0); };
 
-    auto issue = [&](uint4_t (&buf)[U]) {
-      if (ic.lin >= nlin) return;
-      const int n0 = min(((ic.lt * ic.ncu + ic.rb) * TW + rt) << 4, ic.N - 1);  // (the second 16 rows of the last tile may lie past N)
-      const int rows = min(16, ic.N - n0);                // >= 1
-      const int pg = min(PG, ic.G - ic.panel * PG);       // scale groups of this panel (the last may be short)
-      const char* base = ic.W + (int64_t)n0 * ic.row_w + ic.panel * (PG * 16);
-      // rows past N repeat the last row (never stored); groups past K repeat the last group (their
-      // activations and scales are staged as zeros)
-      if constexpr (U >= 2) {
-        // Whole 128-byte lines: the two loads of a pair of chunks take 8 rows each, lane (i, kq) the 16 bytes of
-        // group 4 (i / 8) + kq of row i mod 8 (+ 8 for the second load), so a row contributes 128 contiguous
-        // bytes to an instruction instead of 64 (measured on a 1 GiB stream with the full unpack + MFMA work:
-        // 7.1 against 5.7 TB/s).  consume() puts the halves back where the MFMA wants them.
-        const uint32_t roff_lo = __umul24((uint32_t)min(i & 7, rows - 1), (uint32_t)ic.row_w);
-        const uint32_t roff_hi = __umul24((uint32_t)min(8 + (i & 7), rows - 1), (uint32_t)ic.row_w);
-        const int gpair = ks * (4 * U) + (i >> 3) * 4 + kq;
+    struct Place {
+      wq_rsrc_t base;
+      uint32_t roff[2 * RT], goff[SP];
+    };
+    auto place_of = [&](const ItemCursor& c) {
+      Place p;
+      const int n0 = (c.lt * c.ncu + c.rb) * (16 * RT);
+      const int rows = min(16 * RT, c.N - n0);           // >= 1
+      const int pg = min(PG, c.G - c.panel * PG);        // scale groups of this panel (the last may be short)
+      const uint64_t at = (uint64_t)(c.W + (int64_t)n0 * c.row_w + c.panel * (PG * 16));
+      p.base = wq_rsrc((const char*)at, wq_live(c.lin, nlin));
+      // Whole 128-byte lines: a load takes 8 rows, lane (i, kq) the 16 bytes of group 4 (i / 8) + kq of row i mod 8 (16 rows x
+      // 64 bytes an instruction stream slower: 5.7 against 7.1 TB/s on 1 GiB with unpack and MFMAs).
+      // Rows past N repeat the last row (never stored); groups past K repeat the last group (their
+      // activations and scales are staged as zeros).
 #pragma unroll
-        for (int u = 0; u < U; u += 2) {
-          const uint32_t goff = (uint32_t)min(gpair + 4 * u, pg - 1) * 16u;
-          asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=&v"(buf[u]) : "v"(roff_lo + goff), "s"(base));
-          asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=&v"(buf[u + 1]) : "v"(roff_hi + goff), "s"(base));
-        }
-      } else {
-        const uint32_t roff = __umul24((uint32_t)min(i, rows - 1), (uint32_t)ic.row_w);
+      for (int sp = 0; sp < SP; ++sp) p.goff[sp] = (uint32_t)min(ks * SG + (i >> 3) * 4 + kq + 8 * sp, pg - 1) * 16u;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const uint32_t voff = roff + (uint32_t)min(gi0 + 4 * u, pg - 1) * 16u;
-          asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=&v"(buf[u]) : "v"(voff), "s"(base));
-        }
+      for (int r = 0; r < 2 * RT; ++r) p.roff[r] = __umul24((uint32_t)min(8 * r + (i & 7), rows - 1), (uint32_t)c.row_w);
+      return p;
+    };
+    auto request = [&](const Place& p, int sp, int r) { return __builtin_amdgcn_raw_buffer_load_b128(p.base, p.roff[r] + p.goff[sp], 0, kNonTemporal); };
+
+    // 8 codes as the B operand: fp16 numbers whose bits are the codes, that is 2^-24 (q0, q4), 2^-20 (q1, q5) and so on
+    auto codes = [&](uint32_t w) {
+      const uint32_t w8 = w >> 8;
+      return __builtin_bit_cast(half8_t, uint4_t{w & 0x000F000Fu, w & 0x00F000F0u, w8 & 0x000F000Fu, w8 & 0x00F000F0u});
+    };
+    // ... and as the weights that the format defines, (q - 7) * s rounded to fp16
+    auto weights = [&](uint32_t w, half_t s) {
+      const half2_t c7 = {(half_t)-1031.0f, (half_t)-1031.0f}, c112 = {(half_t)-1136.0f, (half_t)-1136.0f}, s2 = {s, s};
+      const uint4_t c = __builtin_bit_cast(uint4_t, codes(w)) | 0x64006400u;
+      return __builtin_bit_cast(half8_t, uint4_t{as_u32((as_half2(c.x) + c7) * s2), as_u32((as_half2(c.y) + c112) * s2),
+                                                 as_u32((as_half2(c.z) + c7) * s2), as_u32((as_half2(c.w) + c112) * s2)});
+    };
+    // a[g]: word kq of group g in lane quarter kq, from word g of group kq
+    auto spread = [&](uint32_t (&a)[4]) {
+      const auto h0 = __builtin_amdgcn_permlane32_swap(a[0], a[2], false, false);
+      const auto h1 = __builtin_amdgcn_permlane32_swap(a[1], a[3], false, false);
+      const auto q0 = __builtin_amdgcn_permlane16_swap(h0[0], h1[0], false, false);
+      const auto q1 = __builtin_amdgcn_permlane16_swap(h0[1], h1[1], false, false);
+      a[0] = q0[0], a[1] = q0[1], a[2] = q1[0], a[3] = q1[1];
+    };
+
+    // WIDE: lanes 8 .. 15 of every 16 take their half of chunk 0 (4 groups) from the second load 8 lanes below, lanes 0 .. 7
+    // their half of chunk 1 from the first load 8 lanes above (row_ror:8 turns a row of 16 lanes by 8)
+    auto exchange = [&](uint32_t (&a)[4], uint32_t (&b2)[4]) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const uint32_t lo = a[d], hi = b2[d];
+        a[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)lo, (int)hi, 0x128 /* row_ror:8 */, 0xf, 0xc, false);
+        b2[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)hi, (int)lo, 0x128, 0xf, 0x3, false);
       }
-      ++ahead;
-      item_next<PG, CH>(ic, descs, nlin, b, nwg, chunk);
+    };
+    // the lane's four scales of what load r of piece sp brought (WIDE: of chunk r mod 2 of row tile r / 2)
+    auto scales = [&](int slot, int sp, int r) {
+      const int row = WIDE ? (r >> 1) * 16 + i : 8 * r + (i & 7), group = ks * SG + 8 * sp + 4 * (WIDE ? r & 1 : i >> 3);
+      return *reinterpret_cast<const half4_t*>(sbuf + slot * SSLOT + row * SROW + group * 2);
     };
 
-    const half2_t k1031 = {(half_t)-1031.0f, (half_t)-1031.0f};
-    const half2_t k1136 = {(half_t)-1136.0f, (half_t)-1136.0f};
-    auto ring_shr8 = [&](uint32_t word) {
-      uint32_t r;
-      asm("v_lshrrev_b32 %0, 8, %1 ; %2" : "=v"(r) : "v"(word), "v"(magic));
-      return r;
+    constexpr int NA = WIDE ? RT : 2 * RT;  // accumulators: row tiles, or halves of row tiles
+    constexpr int QB = RT < 2 ? RT : 2;     // row tiles at a time
+    auto multiply = [&](const Place& next, int slot, float4_t (&acc)[NA]) {
+#pragma unroll
+      for (int blk = 0; blk < SP * (RT / QB); ++blk) {
+        const int sp = blk / (RT / QB), q0 = blk % (RT / QB) * QB;
+        uint32_t w[2 * QB][4];
+        half4_t s4[2 * QB];
+        // in steps of two products, and behind them the scaling of those of the step before
+        float4_t t[2][2], c[WIDE ? 2 : 1];
+        auto scale = [&](int step) {
+          const int g = step / QB, q = step % QB;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            float4_t& a = acc[WIDE ? q0 + q : 2 * (q0 + q) + h];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = fmaf(t[step & 1][h][e], (float)s4[2 * q + h][g], a[e]);
+          }
+        };
+#pragma unroll
+        for (int step = 0; step < 4 * QB; ++step) {
+          const int g = step / QB, q = step % QB;
+          if (g == 0) {
+#pragma unroll
+            for (int r = 2 * q; r < 2 * q + 2; ++r) {
+              const int at = sp * 2 * RT + 2 * q0 + r;
+              // (copies, and not the registers of the loads: those take the next item's)
+              asm("v_mov_b32 %0, %4\n\tv_mov_b32 %1, %5\n\tv_mov_b32 %2, %6\n\tv_mov_b32 %3, %7\n\ts_nop 1"
+                  : "=&v"(w[r][0]), "=&v"(w[r][1]), "=&v"(w[r][2]), "=&v"(w[r][3])
+                  : "v"(buf[at].x), "v"(buf[at].y), "v"(buf[at].z), "v"(buf[at].w));
+              buf[at] = request(next, sp, 2 * q0 + r);
+              s4[r] = scales(slot, sp, 2 * q0 + r);
+            }
+            if constexpr (WIDE) exchange(w[2 * q], w[2 * q + 1]);
+            spread(w[2 * q]);
+            spread(w[2 * q + 1]);
+          }
+          if (q == 0) {
+#pragma unroll
+            for (int v = 0; v < (WIDE ? 2 : 1); ++v) c[v] = sevenfold(WIDE ? 2 * sp + v : sp, g);
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            t[step & 1][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[WIDE ? 2 * sp + h : sp][g], codes(w[2 * q + h][g]), c[WIDE ? h : 0], 0, 0, 0);
+          if (step > 0) scale(step - 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        scale(4 * QB - 1);
+      }
     };
-    // (t + c) * s: two roundings, as the format defines.  Plain C++ on purpose: the products are the MFMA's A operand, and
-    // the compiler only keeps the wait states between a VALU result and the MFMA that reads it for instructions
-    // it has issued itself (written as inline assembly, v_pk_mul_f16 two instructions in front of the MFMA was
-    // read before it had been written: the weights came out unscaled)
-    auto unpack = [&](uint32_t t, half2_t c, half2_t s2) { return as_u32((as_half2(t) + c) * s2); };
+    // The same with rounded weights, straight from memory: for activations that are infinite or not a number (7 times one
+    // of those is not what the sum of the products would be without it), and for fewer rows than a row tile.
+    auto multiply_rounded = [&](const Place& next, int slot, float4_t (&acc)[NA]) {
+      const Place here = place_of(cc);
+#pragma unroll
+      for (int sp = 0; sp < SP; ++sp)
+#pragma unroll
+        for (int q = 0; q < RT; ++q) {
+          uint32_t w[2][4];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const uint4_t l = request(here, sp, 2 * q + h);
+            w[h][0] = l.x, w[h][1] = l.y, w[h][2] = l.z, w[h][3] = l.w;
+          }
+          if constexpr (WIDE) exchange(w[0], w[1]);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            spread(w[h]);
+            const half4_t s4 = scales(slot, sp, 2 * q + h);
+            float4_t& a = acc[WIDE ? q : 2 * q + h];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) a = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[WIDE ? 2 * sp + h : sp][g], weights(w[h][g], s4[g]), a, 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+      for (int q = 0; q < NA; ++q) acc[q] *= 1.0f / 16777216.0f;
+#pragma unroll
+      for (int sp = 0; sp < SP; ++sp)
+#pragma unroll
+        for (int r = 0; r < 2 * RT; ++r) {
+          buf[sp * 2 * RT + r] = request(next, sp, r);
+          __builtin_amdgcn_sched_barrier(0);  // in this order everywhere: the waits count on it
+        }
+    };
 
-    auto consume = [&](uint4_t (&buf)[U]) {
+    auto consume = [&](const Place& next) {
       if (cc.lt == (CH ? cc.lt0 : 0)) {
         // a new panel: its activations are staged (or will be); this wavefront's K slice goes to registers
         ++pk;
         const int xslot = pk % nxb;
         wait.until(&flags->x_ready[xslot], pk + 1, 1);
+        const char* xs = xbuf + xslot * xbuf_bytes + ((ks * (XO * 16) + kq) * xrows16 + xrow) * 16;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const char* xs = xbuf + xslot * xbuf_bytes + (ks * U * 16 * M + kq * M + min(i + 16 * r, M - 1)) * 16;
+        for (int v = 0; v < XO; ++v)
 #pragma unroll
-          for (int u = 0; u < U; ++u)
+          for (int g = 0; g < 4; ++g) xb[v][g] = *reinterpret_cast<const half8_t*>(xs + ((v * 4 + g) * 4 * xrows16) * 16);
+        float zero = 0.0f;  // NaN where an activation is infinite or not a number
 #pragma unroll
-            for (int d = 0; d < 4; ++d) xb[r][u][d] = *reinterpret_cast<const half8_t*>(xs + ((u * 4 + d) * 4 * M) * 16);
-        }
+        for (int v = 0; v < XO; ++v)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const float4_t c = sevenfold(v, g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) zero = fmaf(c[e], 0.0f, zero);
+          }
+        special = __builtin_amdgcn_ballot_w64(zero != 0.0f) != 0;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (lane == 0) __hip_atomic_fetch_add(&flags->x_taken[xslot], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
       wait.until(&flags->s_ready, k + 1, 2);
       const int slot = k & (ring - 1);
-      const char* sb = sbuf + slot * SSLOT + (rt * 16 + i) * SROW + gi0 * 2;
-      float4_t acc0[R], acc1[R];
+      float4_t acc[NA];
 #pragma unroll
-      for (int r = 0; r < R; ++r) acc0[r] = acc1[r] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      uint32_t cw[2][4];  // the chunks of a pair after the exchange
+      for (int q = 0; q < NA; ++q) acc[q] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      if (special || cc.N < 16) multiply_rounded(next, slot, acc);
+      else multiply(next, slot, acc);
+      if (k >= ring) wait.until(&flags->y_done, k - ring + 1, 3);
+      // sums as [row tile][activation row][row of W]
+      float* const part = reinterpret_cast<float*>(pbuf + (slot * kBW + wave) * (RT * batch_partial_bytes(WIDE)));
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const half_t sh = *reinterpret_cast<const half_t*>(sb + u * 8);
-        const half2_t s16 = {sh, sh};
-        if constexpr (U >= 2) {
-          if ((u & 1) == 0) {
-            // both loads of the pair have landed; lanes 8 .. 15 of every 16 take their half of chunk u from the second
-            // load 8 lanes below, lanes 0 .. 7 their half of chunk u + 1 from the first load 8 lanes above (row_ror:8
-            // turns a row of 16 lanes by 8).
-            if (ahead == NT) asm volatile("s_waitcnt vmcnt(%1)" : "+v"(magic) : "n"((NT - 1) * U + (U - 2 - u)));
-            else asm volatile("s_waitcnt vmcnt(0)" : "+v"(magic));
-            // every ring register is first copied by a statement that depends on the wait (a cross-lane move with the
-            // identity pattern: not an instruction the compiler would put there by itself), the exchange is the compiler's
+      for (int q = 0; q < RT; ++q) {
+        if constexpr (!WIDE) {
+          // Lane (i, kq) has activation rows 4 (kq mod 2) .. + 3 at the groups of half kq / 2, times rows i mod 8 (+ 8) of W at
+          // those of half i / 8: sums where the halves agree.  They come together in the lanes with i < 8, lane quarters 0 and
+          // 1 for rows 0 .. 7, 2 and 3 for rows 8 .. 15.
+          float sum[4];
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-              const uint32_t lo_in = d == 0 ? buf[u].x : d == 1 ? buf[u].y : d == 2 ? buf[u].z : buf[u].w;
-              const uint32_t hi_in = d == 0 ? buf[u | 1].x : d == 1 ? buf[u | 1].y : d == 2 ? buf[u | 1].z : buf[u | 1].w;
-              uint32_t lo, hi;
-              // (the s_nop: a DPP instruction must not read a register a VALU instruction wrote in the two cycles before it,
-              // and the compiler does not count inline assembly as one)
-              asm("v_mov_b32_dpp %0, %2 quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0xf\n\t"
-                  "v_mov_b32_dpp %1, %3 quad_perm:[0,1,2,3] row_mask:0xf bank_mask:0xf\n\t"
-                  "s_nop 1 ; %4"
-                  : "=&v"(lo), "=&v"(hi)
-                  : "v"(lo_in), "v"(hi_in), "v"(magic));
-              cw[0][d] = (uint32_t)__builtin_amdgcn_update_dpp((int)lo, (int)hi, 0x128 /* row_ror:8 */, 0xf, 0xc, false);
-              cw[1][d] = (uint32_t)__builtin_amdgcn_update_dpp((int)hi, (int)lo, 0x128, 0xf, 0x3, false);
-            }
+          for (int e = 0; e < 4; ++e) {
+            const float lo = acc[2 * q][e], hi = acc[2 * q + 1][e];
+            const auto p = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi), false, false);
+            const uint32_t mine = p[0], other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p[1], 0x128 /* row_ror:8 */, 0xf, 0xf, false);
+            sum[e] = __builtin_bit_cast(float, mine) + __builtin_bit_cast(float, other);
+          }
+          if (i < 8) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[q * 128 + (4 * (kq & 1) + e) * 16 + 8 * (kq >> 1) + i] = sum[e];
           }
         } else {
-          if (ahead == NT) asm volatile("s_waitcnt vmcnt(%1)" : "+v"(magic) : "n"((NT - 1) * U + (U - 1 - u)));
-          else asm volatile("s_waitcnt vmcnt(0)" : "+v"(magic));
-        }
 #pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          uint32_t word, w8;
-          if constexpr (U >= 2) {
-            word = cw[u & 1][d];
-            w8 = word >> 8;
-          } else {
-            word = d == 0 ? buf[u].x : d == 1 ? buf[u].y : d == 2 ? buf[u].z : buf[u].w;
-            w8 = ring_shr8(word);
-          }
-          const uint32_t a0 = unpack(and_or(word, 0x000F000Fu, magic), k1031, s16);  // (q0, q4)
-          const uint32_t a1 = unpack(and_or(word, 0x00F000F0u, magic), k1136, s16);  // 16 (q1, q5)
-          const uint32_t a2 = unpack(and_or(w8, 0x000F000Fu, magic), k1031, s16);    // (q2, q6)
-          const uint32_t a3 = unpack(and_or(w8, 0x00F000F0u, magic), k1136, s16);    // 16 (q3, q7)
-          const half8_t aop = __builtin_bit_cast(half8_t, uint4_t{a0, a1, a2, a3});
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            if (d & 1) acc1[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, xb[r][u][d], acc1[r], 0, 0, 0);
-            else acc0[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, xb[r][u][d], acc0[r], 0, 0, 0);
-          }
+          for (int e = 0; e < 4; ++e) part[q * 256 + (4 * kq + e) * 16 + i] = acc[q][e];
         }
       }
-      --ahead;
-      if (k >= ring) wait.until(&flags->y_done, k - ring + 1, 3);
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        *reinterpret_cast<float4_t*>(pbuf + ((slot * kBW + wave) * R + r) * 1024 + lane * 16) = acc0[r] + acc1[r];
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (lane == 0) __hip_atomic_fetch_add(&flags->done[slot], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       ++k;
-      item_next<PG, CH>(cc, descs, nlin, b, nwg, chunk);
     };
 
+    if (ic.lin >= nlin) return;
+    {
+      const Place p = place_of(ic);
 #pragma unroll
-    for (int t = 0; t < NT - 1; ++t) issue(tb[t]);
-    while (cc.lin < nlin) {
+      for (int sp = 0; sp < SP; ++sp)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        issue(tb[(t + NT - 1) % NT]);
-        if (cc.lin < nlin) consume(tb[t]);
-      }
+        for (int r = 0; r < 2 * RT; ++r) {
+          buf[sp * 2 * RT + r] = request(p, sp, r);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    while (ic.lin < nlin) {
+      cc = ic;
+      item_next<PG, CH>(ic, descs, nlin, b, nwg, chunk);
+      consume(place_of(ic));
     }
     return;
   }
@@ -466,6 +553,10 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
     const half2_t sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
     constexpr int PPR = PG * 4;  // 16-byte pieces (8 activations) per row and panel; a power of two
     constexpr int UX = 32;       // loads in flight per lane: one round trip for a panel of 8 rows x 2048 k
+    const int xrows16 = WIDE ? M : 2 * M;
+    // 64 pieces are 16 groups of a row, four dwords each: one slice, or two (WIDE).  The order is that of the operands.
+    const int c = lane >> 2, d = lane & 3;
+    const int place0 = WIDE ? c : (c >> 3) * 4 + (c & 3), half = WIDE ? 0 : (c >> 2) & 1;
     ItemCursor xc;
     xc.lin = 0;
     item_seek<PG, CH>(xc, descs, nlin, b, nwg, chunk);
@@ -496,30 +587,26 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
           uint4_t v[UX];
 #pragma unroll
           for (int t = 0; t < UX; ++t) {
-            const int idx = base + t * 64 + lane;
-            const int row = idx / PPR, o = idx & (PPR - 1);
-            const int go = xc.panel * PPR + o;  // the piece's place in the row
-            v[t] = uint4_t{0, 0, 0, 0};
-            const int src = min(row, xrows - 1);  // rows past the entry's repeat its last row (never stored)
-            if (idx < total && go < K8)
-              v[t] = dep >= 0 ? __builtin_amdgcn_raw_buffer_load_b128(xr, (src * K8 + go) * 16, 0, kDeviceScope)
-                              : __builtin_amdgcn_raw_buffer_load_b128(xr, (src * K8 + go) * 16, 0, 0);
+            const int at = base + t * 64;  // (a row of a panel is whole wavefronts of pieces)
+            const int go = xc.panel * PPR + (at & (PPR - 1));  // the place in the row of lane 0's piece
+            const int src = min(at / PPR, xrows - 1);  // rows past the entry's repeat its last row (never stored)
+            // (past the row, or the panel: an offset that the descriptor does not reach, which brings zeros)
+            const uint32_t off = at < total && go + lane < K8 ? (uint32_t)lane * 16u : 0x80000000u;
+            v[t] = dep >= 0 ? __builtin_amdgcn_raw_buffer_load_b128(xr, off, (src * K8 + go) * 16, kDeviceScope)
+                            : __builtin_amdgcn_raw_buffer_load_b128(xr, off, (src * K8 + go) * 16, 0);
           }
 #pragma unroll
           for (int t = 0; t < UX; ++t) {
-            const int idx = base + t * 64 + lane;
-            if (idx < total) {
-              const int row = idx / PPR, o = idx & (PPR - 1);
+            const int at = base + t * 64;
+            if (at < total) {
               const uint32_t in[4] = {v[t].x, v[t].y, v[t].z, v[t].w};
               uint32_t p[4];
               pair_i_i4(in, p);  // p[e] = (x_e, x_{e+4})
-              // piece o: scale group g = o / 4, dword d = o % 4 of it; the group belongs to wavefront
-              // g / 4U, chunk (g / 4) % U, lane quarter g % 4
-              const int g = o >> 2, d = o & 3;
-              const int cw = g / (4 * U), cu = (g >> 2) & (U - 1), ckq = g & 3;
-              char* dst = xdst + ((((cw * U + cu) * 4 + d) * 4 + ckq) * M + row) * 16;
-              *reinterpret_cast<uint4_t*>(dst) =
-                  uint4_t{p[0], as_u32(as_half2(p[1]) * sixteenth), p[2], as_u32(as_half2(p[3]) * sixteenth)};
+              p[1] = as_u32(as_half2(p[1]) * sixteenth);
+              p[3] = as_u32(as_half2(p[3]) * sixteenth);
+              const int row = at / PPR, first = ((at & (PPR - 1)) >> 6) * (WIDE ? 16 : 8);
+              *reinterpret_cast<uint4_t*>(xdst + (((first + place0) * 4 + d) * xrows16 + half * M + row) * 16) =
+                  uint4_t{p[0], p[1], p[2], p[3]};
             }
           }
         }
@@ -534,9 +621,9 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
 
   if (wave == kBW + kBXW) {
     // ====================== scale wavefront: the scales of a tile -> LDS ======================
-    constexpr int PD = 6;            // items in flight in registers (a round trip under load is several items long)
+    constexpr int PD = NL <= 4 ? 6 : 3;  // items in flight in registers (a round trip under load is several items long)
     constexpr int PPR = PG / 8;      // 16-byte pieces (8 scales) per row and panel
-    constexpr int LP = 16 * TW * PPR / 64;  // pieces per lane and item
+    constexpr int LP = 16 * RT * PPR / 64;  // pieces per lane and item
     uint4_t sv[PD][LP];
     ItemCursor ic, cc;
     ic.lin = 0;
@@ -545,7 +632,7 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
     int k = 0;
     auto issue = [&](uint4_t (&buf)[LP]) {
       if (ic.lin >= nlin) return;
-      const int n0 = (ic.lt * ic.ncu + ic.rb) * (16 * TW);
+      const int n0 = (ic.lt * ic.ncu + ic.rb) * (16 * RT);
       const int pg = min(PG, ic.G - ic.panel * PG);
       const char* base = ic.S + ic.panel * (PG * 2);
 #pragma unroll
@@ -619,66 +706,57 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
           for (int lt = lt0; lt < ltend; ++lt, ++k) {
             const int slot = k & (ring - 1);
             wait.until(&flags->done[slot], kBW * (k / ring + 1), 6);
-            // sum[t][r]: rows 16 t .. of the tile, activation rows 16 r ..; the K slices in a fixed order
-            const char* pb = pbuf + slot * batch_partial_slot_bytes(R) + lane * 16;
-            float4_t sum[TW][R];
+            // sum[t]: rows 16 t + 4 rq .. + 3 of the tile, activation row j16; the K slices in a fixed order
+            const char* pb = pbuf + slot * batch_partial_slot_bytes(WIDE, RT) + (WIDE ? j16 : j16 & 7) * 64 + rq * 16;
+            float4_t sum[RT];
 #pragma unroll
-            for (int t = 0; t < TW; ++t)
+            for (int t = 0; t < RT; ++t) {
+              sum[t] = *reinterpret_cast<const float4_t*>(pb + t * batch_partial_bytes(WIDE));
 #pragma unroll
-              for (int r = 0; r < R; ++r) {
-                sum[t][r] = *reinterpret_cast<const float4_t*>(pb + ((t * KW) * R + r) * 1024);
-#pragma unroll
-                for (int w = 1; w < KW; ++w) sum[t][r] += *reinterpret_cast<const float4_t*>(pb + ((t * KW + w) * R + r) * 1024);
-              }
+              for (int w = 1; w < kBW; ++w) sum[t] += *reinterpret_cast<const float4_t*>(pb + (w * RT + t) * batch_partial_bytes(WIDE));
+            }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (lane == 0) __hip_atomic_store(&flags->y_done, k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             if (P > 1) {
-              float4_t* keep = reinterpret_cast<float4_t*>(abuf + (lt - lt0) * batch_kept_bytes(R, TW) + lane * 16);
+              float4_t* keep = reinterpret_cast<float4_t*>(abuf + (lt - lt0) * batch_kept_bytes(RT) + lane * 16);
               if (panel > 0) {
 #pragma unroll
-                for (int t = 0; t < TW; ++t)
-#pragma unroll
-                  for (int r = 0; r < R; ++r) sum[t][r] += keep[(t * R + r) * 64];
+                for (int t = 0; t < RT; ++t) sum[t] += keep[t * 64];
               }
               if (panel < P - 1) {
 #pragma unroll
-                for (int t = 0; t < TW; ++t)
-#pragma unroll
-                  for (int r = 0; r < R; ++r) keep[(t * R + r) * 64] = sum[t][r];
+                for (int t = 0; t < RT; ++t) keep[t * 64] = sum[t];
                 continue;
               }
             }
 #pragma unroll
-            for (int t = 0; t < TW; ++t) {
-              // lane (j, rq) holds rows n0 + 4 rq .. + 3 of activation rows j, j + 16
-              const int n0 = (((lt * ncu + rb) * TW + t) << 4) + 4 * rq;
+            for (int t = 0; t < RT; ++t) {
+              // lane (j, rq) holds rows n0 + 4 rq .. + 3 of activation row j
+              const int n0 = (((lt * ncu + rb) * RT + t) << 4) + 4 * rq;
+              const float4_t v4 = sum[t] * 16777216.0f;  // (the codes were 2^-24 of themselves)
+              if (j16 < yrows && wide) {
+                if (n0 < N) {
+                  float4_t v = v4;
+                  if (bias) {
+                    const half4_t bv = *reinterpret_cast<const half4_t*>(bias + n0);
 #pragma unroll
-              for (int r = 0; r < R; ++r) {
-                const int j = j16 + 16 * r;
-                if (j < yrows && wide) {
-                  if (n0 < N) {
-                    float4_t v = sum[t][r];
-                    if (bias) {
-                      const half4_t bv = *reinterpret_cast<const half4_t*>(bias + n0);
-#pragma unroll
-                      for (int e = 0; e < 4; ++e) v[e] += (float)bv[e];
-                    }
-                    half4_t h = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
-                    if (residual) h = h + *reinterpret_cast<const half4_t*>(residual + (int64_t)j * N + n0);
-                    // device-scope store: written through, so that a counter update after it publishes it
-                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2_t, h), yr, (j * N + n0) * 2, 0, kDeviceScope);
+                    for (int e = 0; e < 4; ++e) v[e] += (float)bv[e];
                   }
-                } else if (j < yrows) {
+                  half4_t h = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+                  if (residual) h = h + *reinterpret_cast<const half4_t*>(residual + (int64_t)j16 * N + n0);
+                  // device-scope store: written through, so that a counter update after it publishes it
+                  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2_t, h), yr, (j16 * N + n0) * 2, 0, kDeviceScope);
+                }
+              } else if (j16 < yrows) {
 #pragma unroll
-                  for (int e = 0; e < 4; ++e) {
-                    const int n = n0 + e;
-                    if (n < N) {
-                      float v = sum[t][r][e];
-                      if (bias) v += (float)bias[n];
-                      half_t h = (half_t)v;
-                      if (residual) h = h + residual[(int64_t)j * N + n];
-                      __builtin_amdgcn_raw_buffer_store_b16(as_u16(h), yr, (j * N + n) * 2, 0, kDeviceScope);
-                    }
+                for (int e = 0; e < 4; ++e) {
+                  const int n = n0 + e;
+                  if (n < N) {
+                    float v = v4[e];
+                    if (bias) v += (float)bias[n];
+                    half_t h = (half_t)v;
+                    if (residual) h = h + residual[(int64_t)j16 * N + n];
+                    __builtin_amdgcn_raw_buffer_store_b16(as_u16(h), yr, (j16 * N + n) * 2, 0, kDeviceScope);
                   }
                 }
               }
@@ -1250,29 +1328,30 @@ __global__ __launch_bounds__(kRThreads) void q4g32_batch_rows_kernel(const GemvL
 }
 
 // ------------------------------------------------------------------ host side
-// the kernel a list of M activation rows runs: chunks per wavefront and tile, sets of 16 activation rows, tile rows / 16
+// the kernel a list of M activation rows runs: chunks per wavefront and tile, tile rows / 16
 struct BatchShape {
-  int U, R, TW;
+  bool wide;
+  int SP, RT;
 };
-static BatchShape batch_shape(int M) {
-  if (M <= 8) return {4, 1, 1};   // tiles of 16 rows, panels of 4096 k (tiles of 32 rows x 2048 k: the same time at M = 8, slower at M = 4)
-  return {4, 1, 2};               // 32 rows, 2048 k (16 rows x 2048 k, chunks of 2: 0.90 instead of 0.81 ms for the Llama-2-7B stack)
-}                                 // (more than 16 rows: q4g32_batch_rows_kernel)
+// The shapes there are.  An item of a panel of 2048 k suits K up to there, since a panel is walked whole, and that of 4096 k
+// spends least on hand-overs; two row tiles per item halve the hand-overs where there are enough rows.  (Panels of 2048 k
+// with the operands of up to 8 rows: within 2 % of those of up to 16 at M = 2 and 8, so they are not there.)
+static const BatchShape kBatchShapes[] = {{false, 2, 2}, {false, 2, 1}, {true, 1, 2}, {true, 1, 1}};
+constexpr int kBatchShapeCount = sizeof(kBatchShapes) / sizeof(kBatchShapes[0]);
 
+constexpr size_t kBatchLds = 160 * 1024;
 static size_t batch_lds_bytes(BatchShape s, int M, int nxb, int ring, int acc_tiles) {
-  return sizeof(BatchFlags) + (size_t)nxb * M * batch_panel_groups(s.U, s.TW) * 64 + (size_t)ring * batch_scale_slot_bytes(s.U, s.TW) +
-         (size_t)ring * batch_partial_slot_bytes(s.R) + (size_t)acc_tiles * batch_kept_bytes(s.R, s.TW);
+  return sizeof(BatchFlags) + (size_t)nxb * M * batch_panel_groups(s.SP) * 64 + (size_t)ring * batch_scale_slot_bytes(s.SP, s.RT) +
+         (size_t)ring * batch_partial_slot_bytes(s.wide, s.RT) + (size_t)acc_tiles * batch_kept_bytes(s.RT);
 }
 
 // Which group of workgroups runs which linear.  Every workgroup needs all M x K activations of a linear
-// it takes part in, and those bytes cost what weight bytes cost (they pass the same memory pipeline of the
-// CU): with 256 workgroups on a 4096-row linear that is twice the weights at M = 8.  So a list is run by 2^g
+// it takes part in: with 256 workgroups on a 4096-row linear that is twice the weights at M = 8.  So a list is run by 2^g
 // groups side by side, each linear by one group (group = workgroup index mod 2^g, which is one XCD for
 // g = 3: the activations then stay in that XCD's L2): a workgroup sees 1 / 2^g of the linears and 2^g times
 // as many rows of each.  Linears go, in list order, to the group that can start them first (a consumer
-// not before its producer has ended), with the duration of a linear estimated from the bytes a workgroup
-// moves for it; g is the best of 0 .. 4 by that estimate (32-layer Llama-2-7B stack, M = 8: 1.25 ms with one
-// group, 0.89 ms with 8, 0.85 ms with 16).
+// not before its producer has ended), with the duration of a linear estimated (batch_linear_cost); g is the best of
+// 0 .. 4 by that estimate, and so is the shape.
 struct BatchGroupPlan {
   std::vector<int> group;
   double makespan = 0.0;
@@ -1281,29 +1360,37 @@ struct BatchGroupPlan {
 // chunks a workgroup with `tiles` tiles of a linear walks them in (each chunk loads every panel of activations again)
 static int batch_chunks(int tiles, int panels, int chunk) { return panels > 1 && tiles > chunk ? (tiles + chunk - 1) / chunk : 1; }
 
-// bytes through one workgroup of a group of `ncu` for linear i: its tiles' codes and scales, and all activations
-// once per chunk
-static double batch_linear_cost(const wq_gemv_list* l, int i, int ncu, BatchShape s, int chunk) {
+// How long a workgroup of a group of `ncu` takes for linear i, in units near a microsecond: an item, a panel of activations
+// (beside which the items run, but little of it is hidden where LDS holds one panel only), a linear, and the wait for a
+// producer.  Fitted to the launches of 40 lists (M = 2 .. 16, hidden 1024 .. 8192, 1 .. 32 layers) under every shape and
+// number of groups, 912 in all: the plan that the estimate picks is 1.0 % slower than the fastest one on average, 9 % at
+// most (M = 8, hidden 8192, ffn 28672, three layers).  Against bytes alone, by which a list was planned before: hidden 2048, ffn
+// 5632, 32 layers, M = 8 381 -> 218 us, one layer 34.4 -> 20.6; over 45 lists, M = 2 .. 16, 21 % with the products above.
+// (64 KiB items of a linear of several panels take longer: all workgroups read the same half of its rows' bytes.)
+constexpr double kBatchAfterProducer = 22.0;
+static double batch_linear_cost(const wq_gemv_list* l, int i, int ncu, BatchShape s, int fit) {
   const GemvListDesc& g = l->descs[i];
   const int G = (int)(g.g_dep & 0xffffu);
-  const double K = (double)G * 32.0;
-  const int trows = 16 * s.TW;
-  const double tiles = (double)((((int64_t)g.N + trows - 1) / trows + ncu - 1) / ncu);  // of one workgroup
-  const int panels = (G + batch_panel_groups(s.U, s.TW) - 1) / batch_panel_groups(s.U, s.TW);
-  return tiles * trows * K * (0.5 + 1.0 / 16.0) + batch_chunks((int)tiles, panels, chunk) * l->M * K * 2.0 + 4096.0;
+  const int trows = 16 * s.RT;
+  const int tiles = (int)((((int64_t)g.N + trows - 1) / trows + ncu - 1) / ncu);  // of one workgroup
+  const int panels = (G + batch_panel_groups(s.SP) - 1) / batch_panel_groups(s.SP);
+  const int chunks = batch_chunks(tiles, panels, fit), kept = panels > 1 ? std::min(tiles, fit) : 0;
+  const double item = (0.41 + 0.44 * s.RT * s.SP) * (s.RT * s.SP == 4 && panels > 1 ? 1.2 : 1.0), x = 1.15 + 0.34 * l->M * s.SP;
+  const double seen = batch_lds_bytes(s, l->M, 2, 2, kept) <= kBatchLds ? 0.1 : 0.45;
+  return 4.1 + chunks * panels * std::max(x, (double)tiles / chunks * item + seen * x);
 }
 
 // A SHORT list has too few linears for equal groups to be both many (so that few workgroups load a linear's
 // activations) and busy.  Its linears share the 8 XCDs instead, level by level: the linears of a dependency
 // level (level = 1 + the level of the producer) run side by side, each on a set of XCDs in proportion to what
-// it costs, every set at least one XCD; levels follow each other.  cost(i, workgroups of the group) as above.
+// it costs, every set at least one XCD.  cost(i, workgroups of the group) as above.
 struct MaskPlan {
   bool ok = false;
   std::vector<uint8_t> mask;  // XCDs of linear i
   double makespan = 0.0;
 };
 template <class Cost>
-static MaskPlan plan_xcd_masks(const wq_gemv_list* l, Cost cost) {
+static MaskPlan plan_xcd_masks(const wq_gemv_list* l, Cost cost, double after_producer = 0.0) {
   MaskPlan plan;
   if (l->blocks % 8 != 0 || l->n > 64) return plan;
   const int per_xcd = l->blocks / 8;
@@ -1327,29 +1414,40 @@ static MaskPlan plan_xcd_masks(const wq_gemv_list* l, Cost cost) {
         if (cost(who[a], per_xcd * k[a]) > cost(who[worst], per_xcd * k[worst])) worst = a;
       ++k[worst];
     }
-    double t = 0.0;
     int next = 0;
     for (size_t a = 0; a < who.size(); ++a) {
       plan.mask[who[a]] = (uint8_t)(((1u << k[a]) - 1u) << next);
       next += k[a];
-      t = std::max(t, cost(who[a], per_xcd * k[a]));
     }
-    plan.makespan += t;
+  }
+  // How long that takes: an XCD walks its linears in list order, whatever their level, so one that waits for a producer holds
+  // up what follows it (as levels one behind the other the estimate chose sets that took up to 1.4 times as long as groups).
+  double free_at[8] = {};
+  std::vector<double> end(l->n, 0.0);
+  for (int i = 0; i < l->n; ++i) {
+    const int dep = (int)((l->descs[i].g_dep >> 16) & 0x7fffu) - 1;
+    const double ready = dep >= 0 ? end[dep] + after_producer : 0.0, dur = cost(i, per_xcd * __builtin_popcount(plan.mask[i]));
+    for (int x = 0; x < 8; ++x) {
+      if (!((plan.mask[i] >> x) & 1)) continue;
+      free_at[x] = std::max(free_at[x], ready) + dur;
+      end[i] = std::max(end[i], free_at[x]);
+    }
+    plan.makespan = std::max(plan.makespan, end[i]);
   }
   plan.ok = true;
   return plan;
 }
 
-static BatchGroupPlan batch_assign_groups(const wq_gemv_list* l, int gl, BatchShape s, int chunk) {
+static BatchGroupPlan batch_assign_groups(const wq_gemv_list* l, int gl, BatchShape s, int fit) {
   const int groups = 1 << gl, ncu = l->blocks >> gl;
   BatchGroupPlan plan;
   plan.group.resize(l->n);
   std::vector<double> free_at(groups, 0.0), end(l->n, 0.0);
   for (int i = 0; i < l->n; ++i) {
     const GemvListDesc& g = l->descs[i];
-    const double dur = batch_linear_cost(l, i, ncu, s, chunk);
+    const double dur = batch_linear_cost(l, i, ncu, s, fit);
     const int dep = (int)((g.g_dep >> 16) & 0x7fffu) - 1;
-    const double ready = dep >= 0 ? end[dep] : 0.0;
+    const double ready = dep >= 0 ? end[dep] + kBatchAfterProducer : 0.0;
     int best = 0;
     for (int c = 1; c < groups; ++c) {
       const double sb = std::max(free_at[best], ready), sc = std::max(free_at[c], ready);
@@ -1365,11 +1463,12 @@ static BatchGroupPlan batch_assign_groups(const wq_gemv_list* l, int gl, BatchSh
 
 // the kernel that walks the tiles of a linear in chunks carries more loop state: only where a list needs it
 typedef void (*batch_kernel_t)(const GemvListDesc*, int, int*, long long, int, int, int, int, int);
-static int batch_kernel_index(BatchShape s) { return s.TW == 2 ? 1 : 0; }
-static batch_kernel_t batch_kernel(BatchShape s, bool chunked) {
-  switch (batch_kernel_index(s)) {
-    case 1: return chunked ? q4g32_batch_list_kernel<4, 1, 2, true> : q4g32_batch_list_kernel<4, 1, 2, false>;
-    default: return chunked ? q4g32_batch_list_kernel<4, 1, 1, true> : q4g32_batch_list_kernel<4, 1, 1, false>;
+static batch_kernel_t batch_kernel(int shape, bool chunked) {
+  switch (shape) {
+    case 0: return chunked ? q4g32_batch_list_kernel<false, 2, 2, true> : q4g32_batch_list_kernel<false, 2, 2, false>;
+    case 1: return chunked ? q4g32_batch_list_kernel<false, 2, 1, true> : q4g32_batch_list_kernel<false, 2, 1, false>;
+    case 2: return chunked ? q4g32_batch_list_kernel<true, 1, 2, true> : q4g32_batch_list_kernel<true, 1, 2, false>;
+    default: return chunked ? q4g32_batch_list_kernel<true, 1, 1, true> : q4g32_batch_list_kernel<true, 1, 1, false>;
   }
 }
 
@@ -1421,7 +1520,6 @@ static int rows_list_plan(wq_gemv_list* l) {
     if ((int64_t)l->descs[i].N * (l->descs[i].g_dep & 0xffffu) * 2 >= (1ll << 31))
       return fail(WQ_EUNSUPPORTED, "wq_q4g32_gemv_list_create: linear %d: with more than 16 rows of activations the scales must stay below 2 GiB", i);
   l->batch_rows = true;
-  l->batch_u = 2;
   l->threads = kRThreads;
   l->blocks = std::min(cu_count(), 32768);
   const size_t budget = 160 * 1024;
@@ -1484,95 +1582,102 @@ static int rows_list_plan(wq_gemv_list* l) {
   return WQ_OK;
 }
 
-int batch_list_plan(wq_gemv_list* l) {
-  if (l->M > 16) return rows_list_plan(l);
-  const BatchShape s = batch_shape(l->M);
-  const int U = s.U;
-  const int trows = 16 * s.TW;
-  l->batch_u = U;
-  l->threads = kBThreads;
-  l->blocks = std::min(cu_count(), 32768);
-  const size_t budget = 160 * 1024;
-  int best_gl = -1;
-  BatchGroupPlan best;
-  int best_acc = 0;
-  bool best_chunked = false;
+// a list as one of the shapes would run it
+struct BatchPlan {
+  double makespan = -1.0;  // < 0: not possible
+  int gl = 0;              // 2^gl groups, or (masks) sets of XCDs
+  bool masks = false, chunked = false;
+  int acc_tiles = 0;
+  std::vector<int> group;
+  std::vector<uint8_t> mask;
+};
+static BatchPlan batch_plan(const wq_gemv_list* l, BatchShape s) {
+  const int trows = 16 * s.RT;
+  BatchPlan best;
+  // the sums kept between panels must fit beside one panel of activations and a ring of 2: else the tiles of
+  // a linear are walked in chunks of what fits, at the price of loading the activations once per chunk
+  const size_t base = batch_lds_bytes(s, l->M, 1, 2, 0);
+  if (base + 4 * batch_kept_bytes(s.RT) > kBatchLds) return best;
+  const int fit = (int)((kBatchLds - base) / (size_t)batch_kept_bytes(s.RT));
+  auto kept = [&](int i, int ncu) {  // tiles whose sums a workgroup keeps for linear i
+    const int64_t tiles = ((int64_t)l->descs[i].N + trows - 1) / trows;
+    return (int)(l->descs[i].g_dep & 0xffffu) > batch_panel_groups(s.SP) ? (int)((tiles + ncu - 1) / ncu) : 0;
+  };
   for (int gl = 0; gl <= 4; ++gl) {
     if (l->blocks % (1 << gl) != 0 || (l->blocks >> gl) < 1) break;
-    const int ncu = l->blocks >> gl;
-    int acc_tiles = 0;  // most tiles a workgroup holds of a linear that spans several panels
-    for (int i = 0; i < l->n; ++i) {
-      const GemvListDesc& g = l->descs[i];
-      const int64_t tiles = ((int64_t)g.N + trows - 1) / trows;
-      if ((int)(g.g_dep & 0xffffu) > batch_panel_groups(s.U, s.TW)) acc_tiles = std::max<int>(acc_tiles, (int)((tiles + ncu - 1) / ncu));
-    }
-    // the sums kept between panels must fit beside one panel of activations and a ring of 2: else the tiles of
-    // a linear are walked in chunks of what fits, at the price of loading the activations once per chunk
-    const size_t base = batch_lds_bytes(s, l->M, 1, 2, 0);
-    if (base + 4 * batch_kept_bytes(s.R, s.TW) > budget) continue;
-    const int fit = (int)((budget - base) / (size_t)batch_kept_bytes(s.R, s.TW));
-    const int chunk = std::min(acc_tiles, fit);
-    BatchGroupPlan p = batch_assign_groups(l, gl, s, std::max(chunk, 1));
-    if (best_gl < 0 || p.makespan < best.makespan * 0.98) {
-      best_gl = gl;
-      best = std::move(p);
-      best_acc = chunk;
-      best_chunked = chunk < acc_tiles;
-    }
-  }
-  if (best_gl < 0)
-    return fail(WQ_EUNSUPPORTED, "wq_q4g32_gemv_list_create: %d rows of activations do not fit the LDS", l->M);
-  int groups = 1 << best_gl;
-  // a short list: sets of XCDs in proportion to the linears' cost (plan_xcd_masks), if the estimate says so
-  const size_t mbase = batch_lds_bytes(s, l->M, 1, 2, 0);
-  const int mfit = (int)((budget - mbase) / (size_t)batch_kept_bytes(s.R, s.TW));
-  const MaskPlan mp = plan_xcd_masks(l, [&](int i, int ncu) { return batch_linear_cost(l, i, ncu, s, std::max(mfit, 1)); });
-  if (mp.ok && mp.makespan < best.makespan * 0.98) {
     int acc_tiles = 0;
-    for (int i = 0; i < l->n; ++i) {
-      GemvListDesc& g = l->descs[i];
-      const int ncu = (l->blocks / 8) * __builtin_popcount(mp.mask[i]);
-      const int64_t tiles = ((int64_t)g.N + trows - 1) / trows;
-      if ((int)(g.g_dep & 0xffffu) > batch_panel_groups(s.U, s.TW)) acc_tiles = std::max<int>(acc_tiles, (int)((tiles + ncu - 1) / ncu));
-      g.q = (int32_t)(tiles / ncu);
-      g.rem = (uint16_t)(tiles % ncu);
-      g.off = 0;
-      g.gmod_log2 = 0x80;
-      g.gidx = mp.mask[i];
-    }
-    best_acc = std::min(acc_tiles, mfit);
-    best_chunked = best_acc < acc_tiles;
-    groups = 0;  // (sets of XCDs)
-  } else {
-    const int ncu = l->blocks >> best_gl;
-    std::vector<int64_t> off(groups, 0);
-    for (int i = 0; i < l->n; ++i) {
-      GemvListDesc& g = l->descs[i];
-      const int c = best.group[i];
-      const int64_t tiles = ((int64_t)g.N + trows - 1) / trows;
-      g.q = (int32_t)(tiles / ncu);
-      g.rem = (uint16_t)(tiles % ncu);
-      g.off = (uint16_t)off[c];
-      off[c] = (off[c] + tiles) % ncu;
-      g.gmod_log2 = (uint8_t)best_gl;
-      g.gidx = (uint8_t)c;
+    for (int i = 0; i < l->n; ++i) acc_tiles = std::max(acc_tiles, kept(i, l->blocks >> gl));
+    const int chunk = std::min(acc_tiles, fit);
+    BatchGroupPlan p = batch_assign_groups(l, gl, s, fit);
+    if (best.makespan < 0 || p.makespan < best.makespan * 0.98) {
+      best.makespan = p.makespan;
+      best.gl = gl;
+      best.group = std::move(p.group);
+      best.acc_tiles = chunk;
+      best.chunked = chunk < acc_tiles;
     }
   }
-  l->batch_groups = groups;
-  l->batch_acc_tiles = best_acc;
-  l->batch_chunked = best_chunked;
-  // a ring of 4 items and up to 2 panels of activations in LDS if they fit, else a ring of 2
-  l->batch_ring = 4;
-  l->batch_nxb = batch_lds_bytes(s, l->M, 2, 4, best_acc) <= budget ? 2 : batch_lds_bytes(s, l->M, 1, 4, best_acc) <= budget ? 1 : 0;
-  if (!l->batch_nxb) {
-    l->batch_ring = 2;
-    l->batch_nxb = batch_lds_bytes(s, l->M, 2, 2, best_acc) <= budget ? 2 : 1;
+  // a short list: sets of XCDs in proportion to the linears' cost (plan_xcd_masks), if the estimate says so
+  MaskPlan mp = plan_xcd_masks(l, [&](int i, int ncu) { return batch_linear_cost(l, i, ncu, s, fit); }, kBatchAfterProducer);
+  if (mp.ok && (best.makespan < 0 || mp.makespan <= best.makespan * 1.0005)) {  // (at a tie the sets)
+    int acc_tiles = 0;
+    for (int i = 0; i < l->n; ++i) acc_tiles = std::max(acc_tiles, kept(i, (l->blocks / 8) * __builtin_popcount(mp.mask[i])));
+    best.makespan = mp.makespan;
+    best.masks = true;
+    best.mask = std::move(mp.mask);
+    best.acc_tiles = std::min(acc_tiles, fit);
+    best.chunked = best.acc_tiles < acc_tiles;
   }
-  l->lds = batch_lds_bytes(s, l->M, l->batch_nxb, l->batch_ring, best_acc);
-  const void* kern = reinterpret_cast<const void*>(batch_kernel(s, best_chunked));
+  return best;
+}
+
+int batch_list_plan(wq_gemv_list* l) {
+  if (l->M > 16) return rows_list_plan(l);
+  l->threads = kBThreads;
+  l->blocks = std::min(cu_count(), 32768);
+  BatchPlan best;
+  for (int i = 0; i < kBatchShapeCount; ++i) {
+    if (!kBatchShapes[i].wide && l->M > 8) continue;
+    BatchPlan p = batch_plan(l, kBatchShapes[i]);
+    if (p.makespan >= 0 && (best.makespan < 0 || p.makespan < best.makespan)) {
+      best = std::move(p);
+      l->batch_shape = i;
+    }
+  }
+  if (best.makespan < 0)
+    return fail(WQ_EUNSUPPORTED, "wq_q4g32_gemv_list_create: %d rows of activations do not fit the LDS", l->M);
+  const BatchShape s = kBatchShapes[l->batch_shape];
+  const int groups = 1 << best.gl;
+  std::vector<int64_t> off(groups, 0);
+  for (int i = 0; i < l->n; ++i) {
+    GemvListDesc& g = l->descs[i];
+    const int ncu = best.masks ? (l->blocks / 8) * __builtin_popcount(best.mask[i]) : l->blocks >> best.gl;
+    const int64_t tiles = ((int64_t)g.N + 16 * s.RT - 1) / (16 * s.RT);
+    g.q = (int32_t)(tiles / ncu);
+    g.rem = (uint16_t)(tiles % ncu);
+    g.off = 0;
+    g.gmod_log2 = best.masks ? 0x80 : (uint8_t)best.gl;
+    g.gidx = best.masks ? best.mask[i] : (uint8_t)best.group[i];
+    if (!best.masks) {
+      int64_t& o = off[best.group[i]];
+      g.off = (uint16_t)o;
+      o = (o + tiles) % ncu;
+    }
+  }
+  l->batch_groups = best.masks ? 0 : groups;
+  l->batch_acc_tiles = best.acc_tiles;
+  l->batch_chunked = best.chunked;
+  // two panels of activations in LDS if they fit, then a ring of 4 items
+  for (int c : {0, 1, 2, 3}) {
+    l->batch_nxb = c < 2 ? 2 : 1;
+    l->batch_ring = c % 2 ? 2 : 4;
+    l->lds = batch_lds_bytes(s, l->M, l->batch_nxb, l->batch_ring, best.acc_tiles);
+    if (l->lds <= kBatchLds) break;
+  }
+  const void* kern = reinterpret_cast<const void*>(batch_kernel(l->batch_shape, best.chunked));
   // several lists share a kernel: the limit only ever grows
-  static DynamicLdsLimit limits[2][2];
-  if (limits[batch_kernel_index(s)][best_chunked ? 1 : 0].ensure(kern, (int)l->lds) != hipSuccess)
+  static DynamicLdsLimit limits[kBatchShapeCount][2];
+  if (limits[l->batch_shape][best.chunked ? 1 : 0].ensure(kern, (int)l->lds) != hipSuccess)
     return fail(WQ_EDEVICE, "wq_q4g32_gemv_list_create: hipFuncSetAttribute failed");
   int resident = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, l->threads, l->lds) != hipSuccess || resident < 1)
@@ -1589,7 +1694,7 @@ int batch_list_launch(wq_gemv_list* l, hipStream_t stream) {
     return WQ_OK;
   }
   // chunk: at least 1 (a list without a linear of several panels keeps no sums)
-  WQ_LAUNCH("wq_q4g32_gemv_list_run", batch_kernel(batch_shape(l->M), l->batch_chunked), dim3((unsigned)l->blocks), dim3((unsigned)l->threads), l->lds,
+  WQ_LAUNCH("wq_q4g32_gemv_list_run", batch_kernel(l->batch_shape, l->batch_chunked), dim3((unsigned)l->blocks), dim3((unsigned)l->threads), l->lds,
             stream, table, l->n, l->sync, l->spin_limit, l->M, l->batch_nxb, l->batch_ring, std::max(l->batch_acc_tiles, 1),
             use_sync);
   return WQ_OK;

@@ -1032,6 +1032,7 @@ extern "C" int wq_q4g32_gemv_list_info(const wq_gemv_list_t* l, int* dependencie
 }
 
 extern "C" int wq_debug_gemv_list_groups(const wq_gemv_list_t* l) { return l && l->M > 1 ? l->batch_groups : -1; }
+extern "C" int wq_debug_gemv_list_shape(const wq_gemv_list_t* l) { return l && l->M > 1 && !l->batch_rows ? l->batch_shape : -1; }
 
 extern "C" int wq_q4g32_gemv_list_set_spin_limit(wq_gemv_list_t* l, long long ticks) {
   using namespace wq;

@@ -311,3 +311,51 @@ def test_a_wait_that_runs_out_is_reported_and_every_wavefront_exits(env, oracle)
     u.assert_close(u.host(t0), oracle.q4g32_linear(a["W"], a["S"], a["x"], nthreads=8), "bystander after a reported time-out")
     u.assert_close(u.host(mid), r_mid, "producer after a reported time-out")
     u.assert_close(u.host(t1), oracle.q4g32_linear(b["W"], b["S"], r_mid, nthreads=8), "consumer after a reported time-out")
+
+
+# every shape of the kernel up to 16 rows (0, 1: items of 32 / 16 rows x 4096 k; 2, 3: x 2048 k): rows that end inside a row tile
+# and inside the second one, K that ends inside a panel and inside a wavefront's slice of it, several panels
+WIDE4 = [(12288, 4096), (22016, 4096), (130, 3840), (33, 4096), (17, 4352)]
+SHAPED = [(2, WIDE4, 0), (8, WIDE4, 1), (7, [(6144, 2048), (130, 1792), (33, 1024), (16, 256)], 2),
+          (16, [(6144, 2048), (2048, 2048), (11264, 2048), (2048, 5632)], 3), (9, [(17, 512), (49, 4352)], 2)]
+
+
+@pytest.mark.parametrize("M,shapes,shape", SHAPED, ids=[f"{c[2]}-M{c[0]}" for c in SHAPED])
+def test_every_shape_of_the_kernel(env, oracle, M, shapes, shape):
+    """Against the oracle, with infinite and not-a-number activations in the last linear but one: those rows have the
+    infinities and NaN of the product with the format's weights (7 times an infinity is taken from no sum), and the
+    others are as they would be without them."""
+    ops, u, torch = env
+    from relax_amd import _lib
+
+    lins = [_linear(oracle, u, N, K, M, seed=500 + i) for i, (N, K) in enumerate(shapes)]
+    odd = len(lins) - 2
+    x = lins[odd]["x"]
+    x[0, 37] = np.inf
+    x[1, 5], x[1, x.shape[1] - 1] = -np.inf, np.nan
+    ys = [torch.full((M, N), 3.0, dtype=torch.float16, device="cuda") for N, _ in shapes]
+    entries = [(l["dW"], l["dS"], u.dev(l["x"]), y) for l, y in zip(lins, ys)]
+    if len(lins) == 4 and shape == 3:  # a decoder layer: the third reads what the second wrote
+        entries[2] = (lins[2]["dW"], lins[2]["dS"], ys[1], ys[2])
+        odd = 0
+        lins[2]["x"] = None
+        entries[0] = (lins[0]["dW"], lins[0]["dS"], u.dev(x[:, :2048]), ys[0])
+        lins[0]["x"] = x[:, :2048]
+    gl = ops.Q4G32GemvList(entries, M=M)
+    assert _lib.lib().wq_debug_gemv_list_shape(gl._h) == shape
+    print(f"batch list: shape {shape}, M = {M}", flush=True)
+    for _ in range(2):
+        gl.run()
+        gl.status()
+        for i, l in enumerate(lins):
+            xi = u.host(ys[1]) if l["x"] is None else l["x"]
+            if i == odd:
+                with np.errstate(invalid="ignore"):
+                    want = xi[:2].astype(np.float32) @ oracle.q4g32_dequant(l["W"], l["S"]).astype(np.float32).T
+                got = u.host(ys[i])[:2]
+                assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got > 0, want > 0), (i, M)
+                assert np.all(np.isinf(got[0]) | np.isnan(got[0]))
+            rows = slice(2, M) if i == odd else slice(0, M)
+            if rows.start < M:
+                u.assert_close(u.host(ys[i])[rows], oracle.q4g32_linear(l["W"], l["S"], np.ascontiguousarray(xi[rows]), nthreads=8),
+                               f"shape {shape}, linear {i}")
