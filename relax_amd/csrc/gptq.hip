@@ -19,6 +19,7 @@
 #include <mutex>
 #include <vector>
 
+#include "held_gemm.h"
 #include "mfma_gemm.h"
 #include "mfma_gemm_lds.h"
 #include "q4_gemv.h"
@@ -581,6 +582,9 @@ static int wq::gptq_linear_impl(const uint32_t* W_nk, const uint16_t* SZ, const 
   if (M <= 2 && !(M == 2 && K > 8192 && K % 64 == 0))
     return gemv_dispatch<true>("wq_gptq_linear", W_nk, SZ, GemvZp{ratio, (int)G}, x, bias, residual, y, M, N, K, stream);
   if (M <= WQ_SMALL_BATCH_MAX_M && K % 64 == 0) {
+    if (gs % 128 == 0 && held_takes(kHeldGptq, M, N, K))
+      return launch_held<kHeldGptq, Q4G32Epilogue>("wq_gptq_linear", HeldArgs{(const char*)W_nk, (const char*)SZ, (int)G, (int)(gs / 128)},
+                                                   x, y, ep, M, N, K, stream);
     const GptqSkinnyPolicy::Args pargs{W_nk, (const half2_t*)SZ, (int)G, ratio, inv32};
     return launch_skinny_auto<GptqSkinnyPolicy, Q4G32Epilogue>("wq_gptq_linear", pargs, x, y, ep, M, N, K, stream);
   }

@@ -1,5 +1,6 @@
 // Format A (q4f16_1) small-batch entry: the shared small-batch kernel with the
 // group-32 int4 weight policy.
+#include "held_gemm.h"
 #include "q4g32_common.h"
 #include "q4g32_dispatch.h"
 #include "skinny_gemm.h"
@@ -12,6 +13,7 @@ struct Q4G32SkinnyPolicy {
   static constexpr int kPieces = 1;
   static constexpr bool kScaleDma = true;
   static constexpr bool kCanScaleBlock = true;
+  static constexpr bool kXreg = false;  // (K % 64 == 0: held_gemm.h)
   struct Args {
     const uint32_t* W;
     const half_t* S;
@@ -58,6 +60,7 @@ struct Q4G32SkinnyPolicy {
 struct Q4G32OddGroupsSkinnyPolicy : Q4G32SkinnyPolicy {
   static constexpr bool kCanScaleBlock = false;
   static constexpr bool kOddStart = true;
+  static constexpr bool kXreg = true;
   struct Lane : Q4G32SkinnyPolicy::Lane {
     int odd;  // parity of the row
   };
@@ -124,8 +127,11 @@ extern "C" int wq_q4g32_small_batch(const uint32_t* W, const uint16_t* S, const 
   WQ_REQUIRE(aligned16(W) && aligned16(x) && (reinterpret_cast<uintptr_t>(S) & 3u) == 0,
              "wq_q4g32_small_batch: W and x must be 16-byte aligned, S 4-byte aligned");
   WQ_REQUIRE(N < (1ll << 30) && K < (1ll << 30), "wq_q4g32_small_batch: too large");
-  const Q4G32SkinnyPolicy::Args pargs{W, (const half_t*)S};
   const Q4G32Epilogue epi{(const half_t*)bias, (const half_t*)residual, (int)N};
+  if (held_takes(kHeldQ4, M, N, K))
+    return launch_held<kHeldQ4, Q4G32Epilogue>("wq_q4g32_small_batch", HeldArgs{(const char*)W, (const char*)S, 0, 1}, x, y,
+                                               epi, M, N, K, stream);
+  const Q4G32SkinnyPolicy::Args pargs{W, (const half_t*)S};
   return launch_skinny_auto<Q4G32SkinnyPolicy, Q4G32Epilogue>("wq_q4g32_small_batch", pargs, x, y, epi,
                                                              M, N, K, stream);
 }

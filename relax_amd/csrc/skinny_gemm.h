@@ -76,6 +76,12 @@ struct GroupSums : std::false_type {};
 template <class P>
 struct GroupSums<P, std::void_t<decltype(&P::codes8)>> : std::true_type {};
 
+// Policy::kXreg = false: no form with the activations in registers here
+template <class P, class = void>
+struct UsesXreg : std::true_type {};
+template <class P>
+struct UsesXreg<P, std::void_t<decltype(P::kXreg)>> : std::bool_constant<P::kXreg> {};
+
 // Policy::kOddStart = true: s_rel may be -2 (the pair begins in front of the column)
 template <class P, class = void>
 struct OddStart : std::false_type {};
@@ -708,10 +714,12 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
                               hipStream_t stream) {
   const SkinnyTuning t = skinny_tuning();
   // activations in registers where that kernel is the faster one: 4096 < K <= 8192 and at least
-  // four column tiles per CU (N = 28672, K = 8192: q4f16_1 at M = 16 58 -> 47 us, int8 at M = 4
-  // 60 -> 48 us; with two tiles per CU, or at K = 4096, the ring kernel is the faster one)
-  if (xreg_fits(M, K) && Policy::pair_aligned(pargs) && (t.waves == 2 || (t.waves == 0 && K > 4096 && N / 16 >= 4 * (int64_t)cu_count())))
-    return launch_xreg_auto<Policy, Epilogue>(who, pargs, x, y, epi, M, N, K, stream);
+  // four column tiles per CU (N = 28672, K = 8192, int8, M = 4: 60 -> 48 us; with two tiles per CU, or at
+  // K = 4096, the ring kernel is the faster one)
+  if constexpr (UsesXreg<Policy>::value) {
+    if (xreg_fits(M, K) && Policy::pair_aligned(pargs) && (t.waves == 2 || (t.waves == 0 && K > 4096 && N / 16 >= 4 * (int64_t)cu_count())))
+      return launch_xreg_auto<Policy, Epilogue>(who, pargs, x, y, epi, M, N, K, stream);
+  }
   if (K >= kSkinnyMaxK || Policy::s_reach(pargs, N, K) >= (int64_t)kOutside)  // (four wavefronts, two ring slots)
     return launch_skinny_form<Policy, Epilogue, GroupSums<Policy>::value ? 1 : 8, 1, 4, false, false, true>(who, pargs, x, y, epi, M, N, K, 2, stream);
   const int64_t per_cu = (N / 16) / cu_count();

@@ -1,0 +1,96 @@
+"""The small-batch kernel that keeps the activations in registers (up to 16 rows of q4f16_1 and AutoGPTQ), against float64."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+# one wavefront's run of 1 .. 5 pieces of 256 k; K that ends inside a piece, inside a run and before the last run; N of part
+# of a tile, and of more rounds over the CUs than tiles in flight, odd and even
+SHAPES = [(16, 64), (33, 576), (12300, 320), (8200, 2112), (130, 4096), (47, 4352), (259, 6208), (100, 8192)]
+CASES = [(M, N, K) for M in (3, 8, 9, 16) for N, K in SHAPES] + [(2, 70, 8256), (8, 260, 10240)]
+
+
+def _codes(words):  # [N, K/8] -> [N, K]
+    return ((words[:, :, None] >> torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)) & 15).flatten(1).double()
+
+
+@pytest.mark.parametrize("fmt", ["q4f16_1", "gptq"])
+@pytest.mark.parametrize("M,N,K", CASES)
+def test_against_float64(fmt, M, N, K):
+    from relax_amd import _lib, ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    half = lambda *s, lo=0.0, hi=1.0: (torch.rand(s, device="cuda", generator=g) * (hi - lo) + lo).half()
+    words = lambda *s: torch.randint(-(2**31), 2**31 - 1, s, device="cuda", dtype=torch.int32, generator=g)
+    if fmt == "gptq":
+        N, K = N // 8 * 8, (K + 127) // 128 * 128
+        gs = 256 if K % 512 == 0 else 128
+        qw, qz, s, g_idx = words(K // 8, N), words(K // gs, N // 8), half(K // gs, N, lo=0.005, hi=0.02), torch.arange(K, dtype=torch.int32) // gs
+        prep = ops.gptq_prepare(qw, qz, s, g_idx.cuda())
+        zero = _codes(qz) + 1
+        q = _codes(qw.t().contiguous())
+        w = (q - zero.repeat_interleave(gs, 0).t()) * s.double().repeat_interleave(gs, 0).t()
+        run = lambda x, r: ops.gptq_linear(prep, x, residual=r)
+    else:
+        W, S = words(N, K // 8), half(N, K // 32, lo=0.005, hi=0.02)
+        w = (_codes(W) - 7) * S.double().repeat_interleave(32, 1)
+        run = lambda x, r: ops.q4g32_linear(W, S, x, residual=r, kernel="small_batch")
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    x[0] *= 2.0**-13  # a row of small numbers loses nothing
+    res = torch.randn(M, N, device="cuda", generator=g).half()
+    tall = x.clone()
+    tall[M - 1, K // 2] = 5000.0
+    odd = x.clone()
+    odd[0, K - 1], odd[M - 1, 3] = float("inf"), float("nan")
+    _lib.lib().wq_debug_set_skinny_config(0, 0, 2)
+    try:
+        plain, with_res, y_tall, y_odd = run(x, None), run(x, res), run(tall, None), run(odd, None)
+        torch.cuda.synchronize()
+    finally:
+        _lib.lib().wq_debug_set_skinny_config(0, 0, 0)
+
+    def close(y, a, r, unit):
+        # rounding of y (2^-11 of it, 2^-25 where it is no normal number), and per product `unit`: the sums' 24 bits and the
+        # alignment of the products in the matrix core, 2^-17, or a weight rounded to fp16, 2^-11
+        exact, mass = a.double() @ w.t(), a.double().abs() @ w.abs().t()
+        room = exact.abs() * 2.0**-11 + 2.0**-25 + mass * unit
+        if r is not None:  # the product is rounded, then the sum
+            exact = exact + r.double()
+            room = room + exact.abs() * 2.0**-11 + room * 2.0**-11
+        bad = (y.double() - exact).abs() - room
+        assert bad.max().item() <= 0, f"{bad.max().item():.3e}"
+
+    close(plain, x, None, 2.0**-17)
+    close(with_res, x, res, 2.0**-17)
+    close(y_tall, tall, None, 2.0**-11)
+    assert torch.isnan(y_odd[M - 1]).all()
+    if M > 2:
+        close(y_odd[1 : M - 1], odd[1 : M - 1], None, 2.0**-11)
+    want = w[:, K - 1].sign() * float("inf")  # the sign of the weight, no number where it is zero
+    np.testing.assert_array_equal(y_odd[0].float().cpu().numpy(), want.float().cpu().numpy())
+
+
+@pytest.mark.parametrize("fmt", ["q4f16_1", "gptq"])
+def test_the_choice_by_shape_at_its_edges(fmt):
+    """More than 8 rows, four tiles per CU and one fewer column tile: both kernels are right."""
+    from relax_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for N in (64 * cus, 64 * cus - 16):
+        K = 4224
+        x = torch.randn(16, K, device="cuda", generator=g).half()
+        W = torch.randint(-(2**31), 2**31 - 1, (K // 8, N), device="cuda", dtype=torch.int32, generator=g)
+        if fmt == "gptq":
+            s = (torch.rand(K // 128, N, device="cuda", generator=g) * 0.015 + 0.005).half()
+            z = torch.randint(-(2**31), 2**31 - 1, (K // 128, N // 8), device="cuda", dtype=torch.int32, generator=g)
+            w = (_codes(W.t().contiguous()) - (_codes(z) + 1).repeat_interleave(128, 0).t()) * s.double().repeat_interleave(128, 0).t()
+            y = ops.gptq_linear(ops.gptq_prepare(W, z, s, torch.arange(K, dtype=torch.int32, device="cuda") // 128), x)
+        else:
+            Wt, s = W.t().contiguous(), (torch.rand(N, K // 32, device="cuda", generator=g) * 0.015 + 0.005).half()
+            w = (_codes(Wt) - 7) * s.double().repeat_interleave(32, 1)
+            y = ops.q4g32_linear(Wt, s, x)
+        torch.cuda.synchronize()
+        exact, mass = x.double() @ w.t(), x.double().abs() @ w.abs().t()
+        assert ((y.double() - exact).abs() <= exact.abs() * 2.0**-11 + mass * 2.0**-11).all()
