@@ -40,8 +40,8 @@ void wq_debug_set_gemv_config(int rows, int gpl);
 void wq_debug_set_intb_gemv_k_split(int ways);
 /* Decode GEMV: persistent workgroups per CU; 0 = from the shape. */
 void wq_debug_set_gemv_blocks_per_cu(int n);
-/* Small-batch kernel: wavefronts side by side (1, 2, 4, 8), ring slots, and which kernel
- * (waves 1: ring, 2: activations in registers); 0 = from the shape. */
+/* Small-batch kernel: wavefronts side by side (1, 2, 3, 4, 8), ring slots, and which kernel
+ * (waves 1: ring, 12: ring with 12 wavefronts for nw = 3, 2: activations in registers); 0 = from the shape. */
 void wq_debug_set_skinny_config(int nw, int stages, int waves);
 /* How a list of 2 .. 32 activation rows was planned: the number of equal groups of workgroups that run
  * different linears side by side, or 0 if the linears of the (short) list share the 8 XCDs in sets sized by

@@ -155,7 +155,7 @@ __device__ __forceinline__ void direct_load4(const char* base, wq_lptr_t dst, ui
 template <typename Policy, int TH, int NW, int WAVES, bool SB = false>
 struct SkinnyCfg {
   static constexpr int KW = WAVES / NW;
-  static_assert(NW * KW == WAVES && (WAVES == 4 || WAVES == 6 || WAVES == 8), "wavefront arrangement");
+  static_assert(NW * KW == WAVES && (WAVES == 4 || WAVES == 6 || WAVES == 8 || WAVES == 12), "wavefront arrangement");
   static constexpr int kRows = 8 * TH;                   // activation rows held (M <= kRows)
   static constexpr int TM = (TH + 1) / 2;                // 16-row MFMA tiles
   static_assert((2 * TH) % NW == 0, "the slab loads divide among the wavefronts of one kw");
@@ -649,7 +649,7 @@ static int launch_xreg_auto(const char* who, const typename Policy::Args& pargs,
 }
 
 // overrides for tests and measurement (tuning.h; 0 = automatic)
-// waves: 1 = the ring kernel, 2 = the kernel that holds the activations in registers (where it fits)
+// waves: 1 = the ring kernel (12: with twelve wavefronts, nw = 3), 2 = the kernel that holds the activations in registers (where it fits)
 struct SkinnyTuning {
   int nw, stages, waves;
 };
@@ -745,14 +745,20 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
   // 17 .. 24 rows: slabs of 24 rows and three wavefronts side by side where four or eight leave a second, partly filled
   // round: between four and six tiles per CU in every format (M = 19, q4f16_1 / int8: N = 18432, K = 4096 28.8 -> 20.0 /
   // 32.3 -> 20.4 us, N = 24576, K = 6144 36.7 -> 30.8 / 40.1 -> 35.1; N = 16384 and N = 24640 lose 10 .. 30 %), and between
-  // two and three, where it makes one whole round, for int8 (against what was there before: N = 8256, the first width it
-  // takes, K = 4096 15.7 -> 13.9, K = 13824 40.9 -> 36.0; 10240, 8192 26.7 -> 23.1; 12288, 4096 17.6 -> 14.0; at every width
-  // between and K = 2048 .. 13824 7 .. 20 % faster; N = 8192 loses 16 %; int4 is as fast either way and up to N = 9216 slower).
+  // two and three, where it makes one whole round.  There the one workgroup that a CU has takes twelve wavefronts, four
+  // along K: with six the matrix cores wait for the unpacking.  M = 19, weights from memory, q4f16_1 with four side by
+  // side / int8 with three and six / int4 with four -> twelve: N = 12288, K = 4096 13.9 / 14.5 / 13.6 -> 12.4 / 14.2 / 11.7 us,
+  // K = 13824 39.0 / 37.2 / 36.3 -> 32.2 / 35.7 / 27.7; N = 8256 (the first width), K = 8192 24.0 / 22.9 / 23.0 -> 19.8 / 20.0 / 17.7.
+  // Below K = 2048 a step or two per wavefront is too little (K = 1056 6.5 -> 6.7; int8, K = 1024 6.7 -> 7.1).  Between four
+  // and six tiles per CU it loses (N = 22016, K = 4096 20.5 -> 21.2).
+  bool twelve = false;
   if (M > 16 && M <= 24) {
     const int64_t tiles = (N + 15) / 16, cus = cu_count();
-    if ((tiles > 4 * cus && tiles <= 6 * cus) || (Policy::kPieces == 2 && tiles > 2 * cus && tiles <= 3 * cus)) nw = 3;
+    const bool one_round = tiles > 2 * cus && tiles <= 3 * cus;
+    twelve = one_round && K >= 2048;
+    if ((tiles > 4 * cus && tiles <= 6 * cus) || twelve || (one_round && Policy::kPieces == 2)) nw = 3;
   }
-  if (t.nw) nw = t.nw;
+  if (t.nw) nw = t.nw, twelve = t.waves == 12;
   if (nw == 3 && (M <= 16 || M > 24)) nw = 4;
   if (M <= 8 && nw >= 4) nw = 2;  // 8 rows are two slab loads: at most two wavefronts share them
   // three ring slots for four or more wavefronts side by side, and for two when every workgroup has a CU of
@@ -782,7 +788,10 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
     if (nw == 2) WQ_SK_GO(2, 2, 8);
     WQ_SK_GO(2, 1, 8);
   }
-  if (nw == 3) WQ_SK_GO(3, 3, 6);
+  if (nw == 3) {
+    if (twelve) WQ_SK_GO(3, 3, 12);
+    WQ_SK_GO(3, 3, 6);
+  }
   if (M <= 32) {
     if (nw == 8) WQ_SK_GO(4, 8, 8);
     if (nw == 4) WQ_SK_GO(4, 4, 8);
