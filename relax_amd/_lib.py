@@ -104,6 +104,7 @@ CALIBRATE_SIGNATURES = {
 }
 
 _lib = None
+_calls = None
 _calibrate_lib = None
 
 
@@ -135,6 +136,23 @@ def lib() -> ctypes.CDLL:
             fn.restype = ctypes.c_int if name.startswith("wq_debug_gemv_list_") else None
         _lib = l
     return _lib
+
+
+def calls():
+    """The extension that takes the common form of a linear of ops.py from its tensors to the launch (csrc/python/calls.cc)."""
+    global _calls
+    if _calls is None:
+        import torch
+
+        l = lib()
+        try:
+            from relax_amd import _calls as m
+        except ImportError as e:
+            raise ImportError(f"relax_amd/_calls.so cannot be loaded ({e}): build it with `python -m relax_amd.build`") from e
+        fns = (l.wq_q4g32_linear, l.wq_fpA_intB_gemm, l.wq_fpA_intB_gemm_residual, l.wq_gptq_linear, l.wq_gptq_workspace_bytes)
+        m.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in fns), torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+        _calls = m
+    return _calls
 
 
 def calibrate_lib() -> ctypes.CDLL:

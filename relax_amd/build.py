@@ -10,6 +10,7 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 if os.path.dirname(HERE) not in sys.path:
@@ -18,6 +19,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "librelax_amd_wq.so")
 CALIBRATE_LIB = os.path.join(HERE, "librelax_amd_wq_calibrate.so")
 CALIBRATE_SOURCES = ("calibrate.hip",)  # not linked into the product library
+CALLS_SOURCE = os.path.join(CSRC, "python", "calls.cc")  # the linears of ops.py as a Python extension
+CALLS_LIB = os.path.join(HERE, "_calls.so")
 OBJDIR = os.path.join(HERE, "build")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -48,6 +51,18 @@ def _compile(src: str) -> str:
     if err.strip():
         sys.stderr.write(err + "\n")
     return obj
+
+
+def _compile_calls() -> str:
+    from torch.utils import cpp_extension
+
+    dirs = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", *(f"-I{d}" for d in dirs), CALLS_SOURCE,
+           "-o", CALLS_LIB, *(f"-L{d}" for d in cpp_extension.library_paths()), "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    p = subprocess.run(cmd, capture_output=True, text=True)
+    if p.returncode != 0:
+        raise RuntimeError(f"g++ failed on {CALLS_SOURCE}:\n{p.stderr}")
+    return CALLS_LIB
 
 
 def check_asm(name: str) -> None:
@@ -99,6 +114,8 @@ def build(verbose: bool = True, incremental: bool = False) -> str:
                     os.remove(obj)
             for f in compiled + checks:
                 f.result()
+    if not incremental or not os.path.exists(CALLS_LIB) or any(os.path.getmtime(d) > os.path.getmtime(CALLS_LIB) for d in _deps(CALLS_SOURCE)):
+        _compile_calls()
     for lib, want in ((LIB, False), (CALIBRATE_LIB, True)):
         objs = [os.path.join(OBJDIR, os.path.basename(s) + ".o") for s in srcs
                 if (os.path.basename(s) in CALIBRATE_SOURCES) == want]
