@@ -109,6 +109,8 @@ struct HalfStep : std::false_type {};
 template <class P>
 struct HalfStep<P, std::void_t<decltype(&P::half_step)>> : std::true_type {};
 
+// Policy::kColumnScale = true (kScaleBytes == 0): the sums take the column's scale, pair_finish gives the codes as they are.
+
 // Policy::kWide = true: 64-bit addresses, for a K whose byte offsets inside a tile do not fit 32 bits.
 template <class P, class = void>
 struct Wide : std::false_type {};
@@ -406,6 +408,14 @@ __device__ __forceinline__ void gemm_lds_tile(const typename Policy::Args& wargs
     }
   }
 
+  if constexpr (ColumnScale<Policy>::value) {
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int i = 0; i < TME; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][t][r] *= (float)bs[t];
+  }
   // The loads past the last step write to the ring like all others (zeros; in the wide form the last step again), and their
   // places overlap the pieces in which other wavefronts stage: all of them land before anyone goes on.
   WQ_WAITCNT_VM(0);

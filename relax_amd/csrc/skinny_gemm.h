@@ -76,6 +76,15 @@ struct GroupSums : std::false_type {};
 template <class P>
 struct GroupSums<P, std::void_t<decltype(&P::codes8)>> : std::true_type {};
 
+// Policy::kColumnScale = true: one scale per column, which the sums take and not the weights (dequant gives the codes as they are;
+// Policy::kZeroCodes is a word of codes that are zero)
+// the codes past K, whose weights have to be zero
+template <class P>
+__device__ __forceinline__ void zero_codes(uint4_t (&pieces)[P::kPieces]) {
+#pragma unroll
+  for (int p = 0; p < P::kPieces; ++p) pieces[p] = uint4_t{P::kZeroCodes, P::kZeroCodes, P::kZeroCodes, P::kZeroCodes};
+}
+
 // Policy::kXreg = false: no form with the activations in registers here
 template <class P, class = void>
 struct UsesXreg : std::true_type {};
@@ -332,7 +341,11 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
       s = *reinterpret_cast<const half_t*>(s_block + (g >> 5) * 1024 + (((g >> 3) & 3) * 16 + lj) * 16 +
                                            (g & 7) * 2);
     }
-    if (!EVEN && k0 >= K) s = Policy::null_scale();  // code * 0 = exact zero for the weights past K
+    if constexpr (ColumnScale<Policy>::value) {
+      if (!EVEN && k0 >= K) zero_codes<Policy>(pieces);
+    } else {
+      if (!EVEN && k0 >= K) s = Policy::null_scale();  // code * 0 = exact zero for the weights past K
+    }
     half8_t bop[4];
     Policy::dequant(pieces, s, bop);
     // rows past the slab (M <= 8 uses half a tile) re-read a held row: never stored
@@ -436,7 +449,9 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int m = 16 * i + 4 * kq + r;
-          if (m < M) Y[(int64_t)m * N + col] = epi(acc[i][r], m, col);
+          float v = acc[i][r];
+          if constexpr (ColumnScale<Policy>::value) v *= (float)s_fixed;
+          if (m < M) Y[(int64_t)m * N + col] = epi(v, m, col);
         }
     }
   }
@@ -565,6 +580,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
     if constexpr (GroupSums<Policy>::value) asm volatile("" : "+v"(run_groups));  // or a mask per group is kept: they spill
     const uint32_t live = __builtin_amdgcn_readfirstlane(run_groups);
     float4_t acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    float column_scale = 0.0f;
 #pragma unroll
     for (int s = 0; s < NSTEP; ++s) {
       WQ_SK_WAITCNT_VM((D - 1) * L);  // issued after this step's loads: the D - 1 steps that follow it
@@ -580,7 +596,12 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
         for (int p = 0; p < P; ++p) pieces[p] = *reinterpret_cast<const uint4_t*>(src + p * 1024 + lane * 16);
         const half2_t pair = *reinterpret_cast<const half2_t*>(src + P * 1024 + lane * 4);
         typename Policy::Scale scale = Policy::pick_scale(pl0, pair, kq);
-        if (past[s]) scale = Policy::null_scale();
+        if constexpr (ColumnScale<Policy>::value) {
+          if (past[s]) zero_codes<Policy>(pieces);
+          column_scale = (float)scale;
+        } else {
+          if (past[s]) scale = Policy::null_scale();
+        }
         half8_t bop[4];
         Policy::dequant(pieces, scale, bop);
 #pragma unroll
@@ -596,6 +617,10 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_xreg_kernel(
 
     // ---- the WAVES partial sums of the tile meet in LDS (two buffers, by turns) ----
     float4_t* const buf = red + (turn & 1) * (WAVES * 64);
+    if constexpr (ColumnScale<Policy>::value) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] *= column_scale;
+    }
     buf[wave * 64 + lane] = acc;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();

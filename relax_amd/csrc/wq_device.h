@@ -4,6 +4,7 @@
 #define RELAX_AMD_CSRC_WQ_DEVICE_H_
 
 #include <hip/hip_runtime.h>
+#include <type_traits>
 
 #include <cstdint>
 
@@ -222,6 +223,12 @@ __device__ __forceinline__ float apply_activation(float v, int act) {
     default: return v;
   }
 }
+
+// Weight policies of the matrix-core kernels: Policy::kColumnScale = true where a column has one scale, which the sums take
+template <class P, class = void>
+struct ColumnScale : std::false_type {};
+template <class P>
+struct ColumnScale<P, std::void_t<decltype(P::kColumnScale)>> : std::bool_constant<P::kColumnScale> {};
 
 }  // namespace wq
 #endif  // RELAX_AMD_CSRC_WQ_DEVICE_H_
