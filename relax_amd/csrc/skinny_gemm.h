@@ -817,11 +817,31 @@ static int launch_skinny_auto(const char* who, const typename Policy::Args& parg
     if (twelve) WQ_SK_GO(3, 3, 12);
     WQ_SK_GO(3, 3, 6);
   }
+  // slabs of 24 rows also for int8 with one column block (M = 17 / 24, before -> now, weights from memory: N = 2048, K = 4096, a scale per
+  // 64 7.6 / 8.0 -> 6.0 / 6.8 us; N = 4096, K = 11008 21.4 / 21.9 -> 16.7 / 18.5; per column, K = 13824, M = 20 22.0 -> 19.7; K = 1088
+  // 5.1 / 5.5 -> 5.0 / 5.6).  int4 and AutoGPTQ gain 2 .. 4 %, q4f16_1 between 2 and -4 %.
+  if constexpr (Policy::kPieces == 2) {
+    if (M <= 24 && nw == 1 && K >= 2048) WQ_SK_GO(3, 1, 8);
+  }
   if (M <= 32) {
     if (nw == 8) WQ_SK_GO(4, 8, 8);
     if (nw == 4) WQ_SK_GO(4, 4, 8);
     if (nw == 2) WQ_SK_GO(4, 2, 8);
     WQ_SK_GO(4, 1, 8);
+  }
+  // 33 .. 48 rows: slabs of 48, a quarter less to bring and to multiply (M = 40, before -> now, weights from memory: N = K = 4096
+  // q4f16_1 9.7 -> 9.1 us, int8 12.1 -> 11.5, int4 10.0 -> 9.3; N = K = 8192 q4f16_1 28.8 -> 23.8; N = 12288, K = 4096 18.2 -> 16.9,
+  // 18.3 -> 17.3, 16.8 -> 14.6; N = 16384, K = 13824 55.6 -> 51.3, 57.5 -> 54.4, 48.4 -> 42.1).  Not with eight column blocks (the
+  // twelve loads of a slab do not divide among them), and for int8 not with two (N = 8192, K = 4096, M = 40 14.4 -> 16.7) and
+  // with four up to 40 rows (a scale per 64, N = 11008, K = 11008, M = 33 42.9 -> 40.1, M = 48 45.4 -> 47.0);
+  // with two otherwise up to 40 rows, or above K = 4096 (int4 with a scale per 64, N = 6144, M = 36 / 48: K = 4096 13.3 / 13.3 -> 12.5 / 13.9,
+  // K = 5120 17.5 / 18.6 -> 16.6 / 17.8).
+  if (M <= 48 && nw <= 4) {
+    if constexpr (Policy::kPieces == 1) {
+      if (nw == 2 && (M <= 40 || K > 4096)) WQ_SK_GO(6, 2, 8);
+    }
+    if (nw == 4 && (Policy::kPieces == 1 || M <= 40)) WQ_SK_GO(6, 4, 8);
+    if (nw == 1) WQ_SK_GO(6, 1, 8);
   }
   if (nw == 8) WQ_SK_GO(8, 8, 8);
   if (nw == 4) WQ_SK_GO(8, 4, 8);

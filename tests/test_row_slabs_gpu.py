@@ -1,21 +1,24 @@
-"""17 .. 24 rows with twelve wavefronts per workgroup (three side by side, four along K) in every format of the small-batch kernel:
-workgroups whose last columns lie past N, fewer steps of K than wavefronts along it, K that ends inside a step, and (the last)
-the choice by shape."""
+"""Slabs of 24 and 48 rows in every format of the small-batch kernel, with one, two and four column blocks and eight wavefronts, and
+with three and twelve: workgroups whose last columns lie past N, fewer steps of K than wavefronts along it, K that ends
+inside a step, and (the last) the choice by shape."""
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("fmt", ["q4f16_1", "gptq64", "int8", "int4", "int4x64"])
-@pytest.mark.parametrize("M,N,K,stages", [(17, 64, 64, 2), (19, 128, 576, 3), (24, 320, 4160, 0), (21, 8256, 2112, 0)])
-def test_against_the_oracle(fmt, M, N, K, stages):
+@pytest.mark.parametrize("M,N,K,nw,stages,waves", [
+    (17, 64, 64, 3, 2, 12), (19, 128, 576, 3, 3, 12), (24, 320, 4160, 3, 0, 12),
+    (17, 64, 2048, 1, 2, 1), (24, 320, 2112, 1, 3, 1),
+    (33, 64, 64, 1, 2, 1), (40, 320, 1088, 2, 3, 1), (48, 128, 4224, 2, 0, 1), (39, 192, 4160, 4, 2, 1), (47, 128, 192, 1, 3, 1),
+    (21, 8256, 2112, 0, 0, 0), (40, 4160, 1088, 0, 0, 0)])
+def test_against_the_oracle(fmt, M, N, K, nw, stages, waves):
     from oracle import wq_oracle as oracle
     from relax_amd import _lib, ops
     from tests import gpu_util as u
     from tests import test_gptq_gpu, test_intb_gpu
 
-    forced = N < 8192
-    _lib.lib().wq_debug_set_skinny_config(3 if forced else 0, stages, 12 if forced else 0)
+    _lib.lib().wq_debug_set_skinny_config(nw, stages, waves)
     try:
         if fmt.startswith("int"):
             test_intb_gpu._run(ops, u, oracle, M, N, K, int(fmt[3]), seed=M + N, group_size=64 if fmt.endswith("x64") else -1)
