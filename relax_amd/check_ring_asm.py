@@ -27,9 +27,10 @@ A second check (``check_asm_results``) covers what inline assembly costs besides
 not keep the hardware's wait states between an inline-assembly VALU result and an MFMA or DPP
 instruction that reads it.
 
-Two are for the tiled GEMMs: no result is staged in LDS before every direct load to it has landed
-(``check_direct_loads_drained``), and the loads past the last step of K lie outside their empty descriptors however the range
-check counts a scalar offset (``check_empty_descriptors``).
+``check_direct_loads_drained``, of the tiled GEMMs: no result is staged in LDS before every direct load to it has landed.
+
+``check_empty_descriptors``, of the tiled GEMMs and of lists of several rows: the loads past the end lie outside their
+descriptors however the range check counts a scalar offset.
 """
 from __future__ import annotations
 
@@ -43,6 +44,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ("q4g32_gemv_list.hip", "q4g32_batch_list.hip")
 # the tiled GEMMs (mfma_gemm_lds.h)
 DIRECT_LOAD_SOURCES = ("gemm_256.hip", "gptq.hip", "intb_gemm.hip", "q4g32_gemm.hip", "q4n32.hip")
+# kernels of SOURCES whose loads past the end have a scalar offset
+GUARDED_KERNELS = {"q4g32_batch_list.hip": ("q4g32_batch_list_kernel",)}
 ALLOWED_READERS = ("v_and_or_b32", "v_lshrrev_b32", "v_cvt_f32_f16", "v_mov_b32_dpp")
 
 
@@ -258,11 +261,12 @@ def _sgprs(operand: str) -> range:
     return range(int(m[1]), int(m[1]) + 1) if m[1] else range(int(m[2]), int(m[3]) + 1)
 
 
-def check_empty_descriptors(asm_text: str) -> list[str]:
-    """Past the last step of K the tiled GEMMs load against a buffer descriptor of 0 bytes.  If the range check subtracts the
-    scalar offset from those 0 bytes, such a load lies outside only with a scalar offset of 0.  So in every
-    ``gemm_lds_kernel`` the scalar offset of a buffer load is 0, or a register that on every way to the load was
-    last written by a choice between an offset and 0 (or by an AND with the mask that makes the descriptor empty)."""
+def check_empty_descriptors(asm_text: str, kernel: str = "gemm_lds_kernel") -> list[str]:
+    """Past the last step of K the tiled GEMMs load against a buffer descriptor of 0 bytes, and the lists of several rows
+    past the last piece of a row.  If the range check subtracts the scalar offset from the bytes of the descriptor, such a load
+    lies outside only with a scalar offset that the descriptor holds.  So in every function of that name the scalar
+    offset of a buffer load is 0, or a register that on every way to the load was last written by a choice between an
+    offset and 0 (or by an AND with the mask of what there is)."""
     errors, loads = [], 0
 
     def after(block, guarded, bad):
@@ -282,7 +286,7 @@ def check_empty_descriptors(asm_text: str) -> list[str]:
         return guarded
 
     for name, body in _functions(asm_text, labels=True):
-        if "gemm_lds_kernel" not in name or not any(_BUFFER_LOAD.match(l) for l in body):
+        if kernel not in name or not any(_BUFFER_LOAD.match(l) for l in body):
             continue
         blocks = _blocks(body)
         entry = [None] * len(blocks)
@@ -304,7 +308,7 @@ def check_empty_descriptors(asm_text: str) -> list[str]:
         for l in sorted(bad)[:3]:
             errors.append(f"{name}: `{l}` may have a scalar offset against an empty descriptor")
     if loads == 0:
-        return ["no buffer loads found in a gemm_lds_kernel"]
+        return [f"no buffer loads found in a {kernel}"]
     return errors
 
 
@@ -330,6 +334,9 @@ def check_source(hipcc: str, flags, name: str) -> None:
         return
     errs = check(text)
     hazards = check_asm_results(text)
+    past = [e for k in GUARDED_KERNELS.get(name, ()) for e in check_empty_descriptors(text, k)]
+    if past:
+        raise RuntimeError(f"{name}: a load past the end may touch memory:\n  " + "\n  ".join(past[:20]))
     if errs:
         raise RuntimeError(f"{name}: the generated code touches in-flight ring registers:\n  " + "\n  ".join(errs[:20]))
     if hazards:

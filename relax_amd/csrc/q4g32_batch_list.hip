@@ -590,10 +590,13 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
             const int at = base + t * 64;  // (a row of a panel is whole wavefronts of pieces)
             const int go = xc.panel * PPR + (at & (PPR - 1));  // the place in the row of lane 0's piece
             const int src = min(at / PPR, xrows - 1);  // rows past the entry's repeat its last row (never stored)
-            // (past the row, or the panel: an offset that the descriptor does not reach, which brings zeros)
+            // Past the row, or the panel: an offset that the descriptor does not reach, which brings zeros.  The scalar offset of
+            // such a load lies inside too, so that it does not matter whether the range check counts it (wq_device.h): it is 0
+            // where no lane has a piece.
             const uint32_t off = at < total && go + lane < K8 ? (uint32_t)lane * 16u : 0x80000000u;
-            v[t] = dep >= 0 ? __builtin_amdgcn_raw_buffer_load_b128(xr, off, (src * K8 + go) * 16, kDeviceScope)
-                            : __builtin_amdgcn_raw_buffer_load_b128(xr, off, (src * K8 + go) * 16, 0);
+            const int start = (src * K8 + go) * 16 & wq_live(go, K8) & wq_live(at, total);
+            v[t] = dep >= 0 ? __builtin_amdgcn_raw_buffer_load_b128(xr, off, start, kDeviceScope)
+                            : __builtin_amdgcn_raw_buffer_load_b128(xr, off, start, 0);
           }
 #pragma unroll
           for (int t = 0; t < UX; ++t) {

@@ -124,6 +124,32 @@ def test_loads_past_the_end_have_no_scalar_offset():
     assert errors("\ts_cselect_b32 s9, s20, 0\n", GEMM.replace("gemm_lds", "other"))
 
 
+LIST = """
+_ZN2wq{kernel}ILb0ELi2EEEvPKNS_12GemvListDescE:
+{body}
+\tbuffer_load_dwordx4 v[2:5], v6, s[12:15], s9 offen
+\ts_endpgm
+.Lfunc_end0:
+"""
+
+
+def test_loads_of_the_lists_of_several_rows_past_the_end_have_no_scalar_offset(monkeypatch):
+    import pytest
+
+    source = "q4g32_batch_list.hip"
+    assert c.GUARDED_KERNELS[source]
+    for kernel in c.GUARDED_KERNELS[source]:
+        bad, good = (LIST.format(kernel=kernel, body=b) for b in ("\ts_lshl_b32 s9, s20, 4", "\ts_and_b32 s9, s20, s21"))
+        assert c.check_empty_descriptors(bad, kernel) and c.check_empty_descriptors(good, kernel) == []
+        with_others = "".join(LIST.format(kernel=k, body="\ts_mov_b32 s9, 0") for k in c.GUARDED_KERNELS[source] if k != kernel)
+        monkeypatch.setattr(c, "check", lambda text: [])
+        monkeypatch.setattr(c, "_assembly", lambda *a: bad + with_others)
+        with pytest.raises(RuntimeError, match="past the end"):
+            c.check_source("hipcc", [], source)
+        monkeypatch.setattr(c, "_assembly", lambda *a: good + with_others)
+        c.check_source("hipcc", [], source)
+
+
 def test_the_build_checks_every_source_with_the_tiled_gemm():
     import os
 
