@@ -45,7 +45,7 @@ SOURCES = ("q4g32_gemv_list.hip", "q4g32_batch_list.hip")
 # the tiled GEMMs (mfma_gemm_lds.h)
 DIRECT_LOAD_SOURCES = ("gemm_256.hip", "gptq.hip", "intb_gemm.hip", "q4g32_gemm.hip", "q4n32.hip")
 # kernels of SOURCES whose loads past the end have a scalar offset
-GUARDED_KERNELS = {"q4g32_batch_list.hip": ("q4g32_batch_list_kernel",)}
+GUARDED_KERNELS = {"q4g32_batch_list.hip": ("q4g32_batch_list_kernel", "q4g32_batch_rows_kernel")}
 ALLOWED_READERS = ("v_and_or_b32", "v_lshrrev_b32", "v_cvt_f32_f16", "v_mov_b32_dpp")
 
 

@@ -812,8 +812,8 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
 //     8 rows x 128 bytes (whole lines; a lane exchange puts the halves where the MFMA wants them), 2 TR loads
 //     in all, waited for by hand.  A pair is first exchanged into registers of its own and its ring slot
 //     refilled at once, so two pairs (32 KiB per wavefront) are in flight while one is multiplied.  The loads
-//     are buffer loads on the wavefront's rows of the pass: rows past them (a short last pass, the end of W)
-//     read zeros without touching memory and are never stored; a wavefront without rows in a pass loads from
+//     are buffer loads on the wavefront's rows of the pass: past them (a short last pass, the end of W) a load brings
+//     zeros or the first rows again, which are never stored; a wavefront without rows in a pass loads from
 //     an empty buffer and only takes part in the hand-overs.
 //   * A linear's completion counter is raised by the last of the 8 compute wavefronts to have its stores
 //     written through.
@@ -990,7 +990,7 @@ __global__ __launch_bounds__(kRThreads) void q4g32_batch_rows_kernel(const GemvL
     if (wave == 0) rows_seek<TR, true>(cc, descs, nlin, b, nwg, sync, lane);
     else rows_seek<TR, false>(cc, descs, nlin, b, nwg, sync, lane);
 
-    // the buffer of this wavefront's rows in the pass the cursor is in: rows past it read zeros
+    // the buffer of this wavefront's rows in the pass the cursor is in: it ends behind them
     auto tile_rsrc = [&](const RowsCursor& c) {
       const int nt = c.tiles_of(wave, TR);
       const int row0 = c.first_of(wave) * 16;
@@ -1008,12 +1008,15 @@ __global__ __launch_bounds__(kRThreads) void q4g32_batch_rows_kernel(const GemvL
         // lane (i, kq): row i mod 8 of the half tile, scale group 4 (i / 8) + kq of the pair
         i_voff = __umul24((uint32_t)(i & 7), (uint32_t)ic.row_w) + (uint32_t)(((i >> 3) * 4 + kq) * 16);
       }
-      const uint32_t rw8 = (uint32_t)ic.row_w * 8u;
-      uint32_t soff = (uint32_t)ic.q * (kRPairGroups * 16);
+      const int rw8 = ic.row_w * 8;
+      int soff = ic.q * (kRPairGroups * 16);
 #pragma unroll
       for (int t = 0; t < TR; ++t) {
-        asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen nt" : "=&v"(buf[t][0]) : "v"(i_voff), "s"(i_rsrc), "s"(soff));
-        asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen nt" : "=&v"(buf[t][1]) : "v"(i_voff), "s"(i_rsrc), "s"(soff + rw8));
+        // (a half tile without rows: no scalar offset against a buffer that ends before it, see direct_load16_if.  Its loads read
+        // the wavefront's first rows once more, or, where it has none, zeros.)
+        const int lo = soff & wq_live(soff, (int)i_rsrc.z), hi = (soff + rw8) & wq_live(soff + rw8, (int)i_rsrc.z);
+        asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen nt" : "=&v"(buf[t][0]) : "v"(i_voff), "s"(i_rsrc), "s"(lo));
+        asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen nt" : "=&v"(buf[t][1]) : "v"(i_voff), "s"(i_rsrc), "s"(hi));
         soff += 2 * rw8;
       }
       ++ahead;
@@ -1138,7 +1141,7 @@ __global__ __launch_bounds__(kRThreads) void q4g32_batch_rows_kernel(const GemvL
               xb[r] = *reinterpret_cast<const half8_t*>(xs + ((step * 4 + d) * 4 * M) * 16 + r * xr1);
 #pragma unroll
             for (int t = 0; t < TR; ++t) {
-              const uint32_t word = cw[t][u][d];  // (row tiles past the wavefront's share of a short pass: zeros)
+              const uint32_t word = cw[t][u][d];  // (row tiles past the wavefront's share of a short pass: never stored)
               const uint32_t w8 = word >> 8;
               const uint32_t a0 = unpack(and_or(word, 0x000F000Fu, magic), k1031, s16[t]);  // (q0, q4)
               const uint32_t a1 = unpack(and_or(word, 0x00F000F0u, magic), k1136, s16[t]);  // 16 (q1, q5)
