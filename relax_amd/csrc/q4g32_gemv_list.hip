@@ -210,6 +210,7 @@ __global__ __launch_bounds__(64 * (NC + XW + 1)) void q4g32_gemv_list_kernel(con
     };
     uint4_t i_w = row_rsrc(nullptr, 0), i_s = row_rsrc(nullptr, 0);
     auto next_group = [&]() {
+      i_off = i_soff = 0;  // (where the list has run out too: no scalar offset against an empty buffer, see direct_load16_if)
       int pos;
       uint32_t lp, row;
       while (true) {
@@ -241,7 +242,6 @@ __global__ __launch_bounds__(64 * (NC + XW + 1)) void q4g32_gemv_list_kernel(con
         i_s = row_rsrc(ic.S + (woff >> 3), ic.row_s);
       }
       i_left = ic.C;
-      i_off = i_soff = 0;
       i_x = i_x0 = ic.xoff;
       i_yl = (ybuf0 + ((ic.lin & (kYSlots - 1)) * ybuf_floats + (int)lp) * 4) | (ic.lin << 18);
       i_first = kFirst;
