@@ -19,11 +19,12 @@
 // SIMD with two or more wavefronts: and, shift, add and fma of registers or literals take 2 cycles, packed and three-operand
 // bit instructions 4, lane swaps 8.)  So a weight is not made at all.  A word's codes become fp16 numbers by masks alone (4
 // ands and a shift): the code in bits 0 .. 3 of a half is the number 2^-24 q, in bits 4 .. 7 2^-20 q, and the activations of
-// those positions are divided by 16 when they are staged.  One v_mfma_f32_16x16x32_f16 takes the 32 codes of ONE group of 16
+// the former are taken 16 times when they are staged.  One v_mfma_f32_16x16x32_f16 takes the 32 codes of ONE group of 16
 // rows, beginning at -7 times the group's sum of activations (another such product, with -7 in the codes' place), and 4
 // fmas add the scale times that to the sums in fp32.  For one product to hold one group, the words of a group lie in
-// the four lane quarters: two lane swaps for two words.  Nothing is rounded before the sums: against 64 bits the error
-// is that of the fp16 output alone (2.08e-4; with rounded weights 2.74e-4).
+// the four lane quarters: two lane swaps for two words.  Nothing is rounded before the sums, in which the matrix core aligns
+// products to 2^-17 of the largest: against 64 bits the error is that of the fp16 output (2.08e-4, of which its rounding is
+// 2.07e-4; with rounded weights 2.74e-4), for activations of 1e-4 too (divided by 16 in the other positions 2.0e-3).
 //   Up to 8 activation rows the 16 rows of the operand hold each of them twice, at the groups of the two halves of a
 // 128-byte piece, so that lanes (rows, half) of a load are columns of one product as they come: half of the results, row
 // half against other column half, are sums of nothing and are dropped.  With 9 .. 16 rows (WIDE) two loads exchange halves
@@ -67,7 +68,8 @@ constexpr int kBThreads = 64 * (kBW + kBXW + 2);
 
 // LDS words that hand the buffers over inside a workgroup (items = (linear, panel, tile) in the
 // order the workgroup walks them; panels counted over all linears)
-constexpr int kBMaxXBuf = 4;  // room in the flags; the host uses 1 or 2
+constexpr int kBMaxXBuf = 2;
+constexpr int kBOddRows = 8;  // panels of which odd_rows is kept: the y wavefront is at most ring + kBMaxXBuf <= 6 behind the one staged
 struct BatchFlags {
   int x_ready[kBMaxXBuf];  // [panel mod buffers] = panel + 1 once that panel's activations are staged
   int x_taken[kBMaxXBuf];  // [panel mod buffers] += 1 by each compute wavefront that has copied the panel
@@ -77,6 +79,7 @@ struct BatchFlags {
   int abort;         // a wait of this workgroup ran into the spin limit: nobody waits any more
   int pad;
   int done[kBRing];  // += 1 by each compute wavefront per item finished, by slot (item mod ring)
+  uint16_t odd_rows[kBOddRows];  // [panel mod kBOddRows]: rows of activations staged a sixteenth as large as the others
 };
 static_assert(sizeof(BatchFlags) == 64, "flags layout");
 
@@ -428,7 +431,7 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
           __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-      for (int q = 0; q < NA; ++q) acc[q] *= 1.0f / 16777216.0f;
+      for (int q = 0; q < NA; ++q) acc[q] *= 1.0f / 16777216.0f;  // (like the products of codes, 2^-20 of the weights' of x)
 #pragma unroll
       for (int sp = 0; sp < SP; ++sp)
 #pragma unroll
@@ -550,9 +553,15 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     };
 
-    const half2_t sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
+    // A code in bits 0 .. 3 of a half counts a sixteenth of one in bits 4 .. 7: the activations of the former are staged 16
+    // times.  (Those of the latter divided by 16 lose bits below 2^-10.)  A row of the panel in which that gives an
+    // infinity, where an activation is 4096 or more, is staged once and a sixteenth, and its sums are taken 16 times: what
+    // that costs, 2^-21 of an activation, is nothing beside the large one, and no other row changes.
+    const half2_t sixteen = {(half_t)16.0f, (half_t)16.0f}, sixteenth = {(half_t)0.0625f, (half_t)0.0625f}, one = {(half_t)1.0f, (half_t)1.0f}, null2 = {(half_t)0.0f, (half_t)0.0f};
     constexpr int PPR = PG * 4;  // 16-byte pieces (8 activations) per row and panel; a power of two
     constexpr int UX = 32;       // loads in flight per lane: one round trip for a panel of 8 rows x 2048 k
+    constexpr int UR = PPR / 64; // loads of a row
+    static_assert(UX % UR == 0, "whole rows are loaded");
     const int xrows16 = WIDE ? M : 2 * M;
     // 64 pieces are 16 groups of a row, four dwords each: one slice, or two (WIDE).  The order is that of the operands.
     const int c = lane >> 2, d = lane & 3;
@@ -583,6 +592,17 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
             __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(descs[j].x), 0, xrows * K * 2, kBufferFlags);
         char* const xdst = xbuf + xslot * xbuf_bytes;
         const int total = M * PPR;
+        auto stage = [&](uint4_t v, int row, int t, half2_t low, half2_t high, float zero) {
+          const uint32_t in[4] = {v.x, v.y, v.z, v.w};
+          uint32_t p[4];
+          pair_i_i4(in, p);  // p[e] = (x_e, x_{e+4})
+          const half2_t p0 = as_half2(p[0]) * low, p2 = as_half2(p[2]) * low;
+          const int first = t * (WIDE ? 16 : 8);
+          *reinterpret_cast<uint4_t*>(xdst + (((first + place0) * 4 + d) * xrows16 + half * M + row) * 16) =
+              uint4_t{as_u32(p0), as_u32(as_half2(p[1]) * high), as_u32(p2), as_u32(as_half2(p[3]) * high)};
+          return dot2(p0, null2, dot2(p2, null2, zero));
+        };
+        uint32_t odd = 0;
         for (int base = 0; base < total; base += 64 * UX) {
           uint4_t v[UX];
 #pragma unroll
@@ -599,20 +619,27 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
                             : __builtin_amdgcn_raw_buffer_load_b128(xr, off, start, 0);
           }
 #pragma unroll
-          for (int t = 0; t < UX; ++t) {
-            const int at = base + t * 64;
-            if (at < total) {
-              const uint32_t in[4] = {v[t].x, v[t].y, v[t].z, v[t].w};
-              uint32_t p[4];
-              pair_i_i4(in, p);  // p[e] = (x_e, x_{e+4})
-              p[1] = as_u32(as_half2(p[1]) * sixteenth);
-              p[3] = as_u32(as_half2(p[3]) * sixteenth);
-              const int row = at / PPR, first = ((at & (PPR - 1)) >> 6) * (WIDE ? 16 : 8);
-              *reinterpret_cast<uint4_t*>(xdst + (((first + place0) * 4 + d) * xrows16 + half * M + row) * 16) =
-                  uint4_t{p[0], p[1], p[2], p[3]};
+          for (int r = 0; r < UX / UR; ++r) {
+            const int row = base / PPR + r;
+            if (row < M) {
+              float zero = 0.0f;  // NaN where 16 times an activation is infinite or not a number
+#pragma unroll
+              for (int t = 0; t < UR; ++t) zero = stage(v[r * UR + t], row, t, sixteen, one, zero);
+              if (__builtin_amdgcn_ballot_w64(zero != 0.0f)) odd |= 1u << row;
             }
           }
         }
+        for (uint32_t left = odd; left; left &= left - 1) {
+          const int row = __builtin_ctz(left), src = min(row, xrows - 1);
+#pragma unroll 1
+          for (int t = 0; t < UR; ++t) {
+            const int go = xc.panel * PPR + t * 64;
+            const uint32_t off = go + lane < K8 ? (uint32_t)((src * K8 + go + lane) * 16) : 0x80000000u;
+            stage(dep >= 0 ? __builtin_amdgcn_raw_buffer_load_b128(xr, off, 0, kDeviceScope) : __builtin_amdgcn_raw_buffer_load_b128(xr, off, 0, 0),
+                  row, t, one, sixteenth, 0.0f);
+          }
+        }
+        if (lane == 0) flags->odd_rows[pk % kBOddRows] = (uint16_t)odd;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (lane == 0) __hip_atomic_store(&flags->x_ready[xslot], pk + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
@@ -679,7 +706,7 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
   // ================== y wavefront: partial sums -> y, completion signals ==================
   {
     const int j16 = lane & 15, rq = lane >> 4;
-    int k = 0;
+    int k = 0, pk = -1;
     for (int lin = 0; lin < nlin; ++lin) {
       const uint32_t g_dep = descs[lin].g_dep;
       const uint32_t grp = desc_group_word(descs, lin);
@@ -706,9 +733,11 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
       for (int lt0 = 0; lt0 < T; lt0 += csize) {
         const int ltend = min(T, lt0 + csize);
         for (int panel = 0; panel < P; ++panel) {
+          ++pk;
           for (int lt = lt0; lt < ltend; ++lt, ++k) {
             const int slot = k & (ring - 1);
             wait.until(&flags->done[slot], kBW * (k / ring + 1), 6);
+            const float factor = (flags->odd_rows[pk % kBOddRows] >> j16) & 1 ? 16.0f : 1.0f;
             // sum[t]: rows 16 t + 4 rq .. + 3 of the tile, activation row j16; the K slices in a fixed order
             const char* pb = pbuf + slot * batch_partial_slot_bytes(WIDE, RT) + (WIDE ? j16 : j16 & 7) * 64 + rq * 16;
             float4_t sum[RT];
@@ -718,6 +747,8 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
 #pragma unroll
               for (int w = 1; w < kBW; ++w) sum[t] += *reinterpret_cast<const float4_t*>(pb + (w * RT + t) * batch_partial_bytes(WIDE));
             }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) sum[t] *= factor;
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (lane == 0) __hip_atomic_store(&flags->y_done, k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             if (P > 1) {
@@ -736,7 +767,7 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
             for (int t = 0; t < RT; ++t) {
               // lane (j, rq) holds rows n0 + 4 rq .. + 3 of activation row j
               const int n0 = (((lt * ncu + rb) * RT + t) << 4) + 4 * rq;
-              const float4_t v4 = sum[t] * 16777216.0f;  // (the codes were 2^-24 of themselves)
+              const float4_t v4 = sum[t] * 1048576.0f;  // (the products were 2^-20 of themselves)
               if (j16 < yrows && wide) {
                 if (n0 < N) {
                   float4_t v = v4;

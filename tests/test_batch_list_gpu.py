@@ -359,3 +359,38 @@ def test_every_shape_of_the_kernel(env, oracle, M, shapes, shape):
             if rows.start < M:
                 u.assert_close(u.host(ys[i])[rows], oracle.q4g32_linear(l["W"], l["S"], np.ascontiguousarray(xi[rows]), nthreads=8),
                                f"shape {shape}, linear {i}")
+
+
+@pytest.mark.parametrize("M", [2, 8, 9, 16])
+def test_small_and_large_activations_against_float64(env, M):
+    """Activations of 2^-13 lose nothing, and one of 5000 (whose 16-fold is no fp16 number) changes no other row and rounds no
+    weight.  Bound: the output's rounding, 2^-11 of it and 2^-25 where it is no normal number, and per product the alignment
+    in the matrix core, 2^-17, or (fewer than 16 rows of W) the rounding of the weight, 2^-11."""
+    ops, u, torch = env
+    g = torch.Generator(device="cuda").manual_seed(M)
+    lins = []
+    for N, K in ((100, 4096), (33, 2304), (7, 512), (600, 11008)):
+        W = torch.randint(-(2**31), 2**31 - 1, (N, K // 8), device="cuda", dtype=torch.int32, generator=g)
+        S = (torch.rand(N, K // 32, device="cuda", generator=g) * 0.015 + 0.005).half()
+        q = ((W[:, :, None] >> torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)) & 15).flatten(1).double()
+        x = torch.randn(M, K, device="cuda", generator=g).half()
+        x[0] *= 2.0**-13
+        lins.append((W, S, x, (q - 7) * S.double().repeat_interleave(32, 1)))
+    plain = []
+    for tall in (False, True):
+        for _, _, x, _ in lins:
+            if tall:
+                x[M - 1, x.shape[1] // 2 + 1] = 5000.0
+        ys = [torch.zeros((M, W.shape[0]), dtype=torch.float16, device="cuda") for W, _, _, _ in lins]
+        gl = ops.Q4G32GemvList([(W, S, x, y) for (W, S, x, _), y in zip(lins, ys)], M=M)
+        print(f"batch list: small activations, M = {M}, tall {tall}", flush=True)
+        gl.run()
+        gl.status()
+        for (_, _, x, w), y in zip(lins, ys):
+            exact, mass = x.double() @ w.t(), x.double().abs() @ w.abs().t()
+            over = (y.double() - exact).abs() - (exact.abs() * 2.0**-11 + 2.0**-25 + mass * (2.0**-17 if len(w) >= 16 else 2.0**-11))
+            assert over.max().item() <= 0, (tall, tuple(w.shape), over.max().item())
+        if tall:
+            for a, b in zip(plain, ys):
+                assert torch.equal(a[: M - 1], b[: M - 1])
+        plain = ys
