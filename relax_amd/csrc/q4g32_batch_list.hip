@@ -1055,8 +1055,9 @@ __global__ __launch_bounds__(kRThreads) void q4g32_batch_rows_kernel(const GemvL
     };
 
     const half2_t k1031 = {(half_t)-1031.0f, (half_t)-1031.0f};
-    const half2_t k1136 = {(half_t)-1136.0f, (half_t)-1136.0f};
-    auto unpack = [&](uint32_t t, half2_t c, half2_t s2) { return as_u32((as_half2(t) + c) * s2); };
+    const half2_t k71 = {(half_t)-71.0f, (half_t)-71.0f}, sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
+    auto unpack = [&](uint32_t t, half2_t s2) { return as_u32((as_half2(t) + k1031) * s2); };  // of codes in bits 0 .. 3
+    auto unpack4 = [&](uint32_t t, half2_t s2) { return as_u32(__builtin_elementwise_fma(as_half2(t), sixteenth, k71) * s2); };  // 4 .. 7: (1024 + 16 q) / 16 - 71
 
     float4_t acc[TR][R];
     int pk = -1, sk = -1;  // panels of activations / of scales taken (counted over the launch)
@@ -1174,10 +1175,10 @@ __global__ __launch_bounds__(kRThreads) void q4g32_batch_rows_kernel(const GemvL
             for (int t = 0; t < TR; ++t) {
               const uint32_t word = cw[t][u][d];  // (row tiles past the wavefront's share of a short pass: never stored)
               const uint32_t w8 = word >> 8;
-              const uint32_t a0 = unpack(and_or(word, 0x000F000Fu, magic), k1031, s16[t]);  // (q0, q4)
-              const uint32_t a1 = unpack(and_or(word, 0x00F000F0u, magic), k1136, s16[t]);  // 16 (q1, q5)
-              const uint32_t a2 = unpack(and_or(w8, 0x000F000Fu, magic), k1031, s16[t]);    // (q2, q6)
-              const uint32_t a3 = unpack(and_or(w8, 0x00F000F0u, magic), k1136, s16[t]);    // 16 (q3, q7)
+              const uint32_t a0 = unpack(and_or(word, 0x000F000Fu, magic), s16[t]);   // (q0, q4)
+              const uint32_t a1 = unpack4(and_or(word, 0x00F000F0u, magic), s16[t]);  // (q1, q5)
+              const uint32_t a2 = unpack(and_or(w8, 0x000F000Fu, magic), s16[t]);     // (q2, q6)
+              const uint32_t a3 = unpack4(and_or(w8, 0x00F000F0u, magic), s16[t]);    // (q3, q7)
               const half8_t aop = __builtin_bit_cast(half8_t, uint4_t{a0, a1, a2, a3});
 #pragma unroll
               for (int r = 0; r < R; ++r) acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, xb[r], acc[t][r], 0, 0, 0);
@@ -1261,7 +1262,6 @@ __global__ __launch_bounds__(kRThreads) void q4g32_batch_rows_kernel(const GemvL
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     };
-    const half2_t sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
     constexpr int PPR = kRPG * 4;  // 16-byte pieces (8 activations) per row and panel
     constexpr int UX = 32;         // loads in flight per lane: a whole panel of 32 rows
     RowsCursor xc;
@@ -1310,8 +1310,7 @@ __global__ __launch_bounds__(kRThreads) void q4g32_batch_rows_kernel(const GemvL
               // piece o: scale group g = o / 4 of the panel, dword d = o % 4 of it; step g / 4, lane quarter g % 4
               const int g = o >> 2, d = o & 3;
               char* dst = xdst + ((((g >> 2) * 4 + d) * 4 + (g & 3)) * M + row) * 16;
-              *reinterpret_cast<uint4_t*>(dst) =
-                  uint4_t{p[0], as_u32(as_half2(p[1]) * sixteenth), p[2], as_u32(as_half2(p[3]) * sixteenth)};
+              *reinterpret_cast<uint4_t*>(dst) = uint4_t{p[0], p[1], p[2], p[3]};
             }
           }
         }
