@@ -171,7 +171,7 @@ PyObject* gptq_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
       if (v[i] <= 0) return nullptr;
     }
     const int64_t N = v[0], K = v[1], M = x.t->numel() / K;
-    if (x.t->dim() < 1 || x.t->size(-1) != K || !holds(residual, M * N)) return nullptr;
+    if (x.t->dim() < 1 || x.t->size(-1) != K || (bias.t && bias.t->numel() < N) || !holds(residual, M * N)) return nullptr;
     return launched(x, N, Py_None, [&](void* y, wq_stream_t stream) {
       const size_t need = g.gptq_workspace_bytes(M, K, perm.t != nullptr);
       at::Tensor space;

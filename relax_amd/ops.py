@@ -550,6 +550,8 @@ def gptq_linear(w: GptqWeight, x: torch.Tensor, bias: Optional[torch.Tensor] = N
     M = x.numel() // w.K
     if bias is not None:
         bias = _dev(bias, torch.float16, "bias")
+        if bias.numel() < w.N:
+            raise ValueError(f"bias must hold {w.N} elements")
     if residual is not None:
         residual = _dev(residual, torch.float16, "residual")
         if residual.numel() != M * w.N:

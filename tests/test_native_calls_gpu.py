@@ -76,3 +76,20 @@ def test_taken_and_left(env, monkeypatch, form, shape):
         y = run(x)
     torch.cuda.current_stream().wait_stream(side)
     assert watch.answers[-1] is y and torch.equal(y, run(x))
+
+
+@pytest.mark.parametrize("form", ["q4", "intb", "gptq", "gptq-order"])
+@pytest.mark.parametrize("rows", [1, 70])
+def test_a_short_bias_is_refused(env, form, rows):
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    _, _, forms, half, N, K = env
+    x, bias = half(rows, K), half(N)[: N - 1]
+    with pytest.raises(ValueError):
+        forms[form](x, bias=bias)
+    with Mode(), pytest.raises(ValueError):  # the general path
+        forms[form](x, bias=bias)
