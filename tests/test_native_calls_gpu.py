@@ -93,3 +93,12 @@ def test_a_short_bias_is_refused(env, form, rows):
         forms[form](x, bias=bias)
     with Mode(), pytest.raises(ValueError):  # the general path
         forms[form](x, bias=bias)
+
+
+def test_gptq_linear_refuses_host_tensors_to_write_to(env):
+    _, ops, forms, half, N, K = env
+    for form in ("gptq", "gptq-order"):
+        x = half(3, K)
+        for kw in ({"out": half(3, N).cpu()}, {"workspace": torch.empty(1 << 16, dtype=torch.uint8)}):
+            with pytest.raises(ValueError):
+                forms[form](x, **kw)
