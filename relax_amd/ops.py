@@ -558,10 +558,10 @@ def gptq_linear(w: GptqWeight, x: torch.Tensor, bias: Optional[torch.Tensor] = N
             raise ValueError("residual must have M*N elements")
     if out is None:
         out = torch.empty((*x.shape[:-1], w.N), dtype=torch.float16, device=x.device)
-    elif not out.is_cuda or not out.is_contiguous() or out.numel() != M * w.N or out.dtype != torch.float16:
-        raise ValueError("out must be a contiguous fp16 device tensor of M*N elements")
-    if workspace is not None and not workspace.is_cuda:
-        raise ValueError("workspace must be a device tensor")
+    elif not (out.is_cuda or out.is_pinned()) or not out.is_contiguous() or out.numel() != M * w.N or out.dtype != torch.float16:
+        raise ValueError("out must be a contiguous fp16 tensor of M*N elements that the device can write")
+    if workspace is not None and not (workspace.is_cuda or workspace.is_pinned()):
+        raise ValueError("workspace must be memory that the device can write")
     KP = getattr(w, "K_padded", 0)
     if KP:
         need = _lib.lib().wq_gptq_padded_workspace_bytes(M, KP)

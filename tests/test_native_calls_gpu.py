@@ -102,3 +102,7 @@ def test_gptq_linear_refuses_host_tensors_to_write_to(env):
         for kw in ({"out": half(3, N).cpu()}, {"workspace": torch.empty(1 << 16, dtype=torch.uint8)}):
             with pytest.raises(ValueError):
                 forms[form](x, **kw)
+        out = torch.empty(3, N, dtype=torch.float16, pin_memory=True)  # which the device can write
+        assert forms[form](x, out=out) is out
+        torch.cuda.synchronize()
+        assert torch.equal(out, forms[form](x).cpu())
