@@ -1,5 +1,6 @@
 """Compiles the HIP/C++ sources under ``relax_amd/csrc`` into ``librelax_amd_wq.so`` (gfx950), and
 the calibration kernels (``calibrate.hip``: measurement only) into ``librelax_amd_wq_calibrate.so``.
+These need no torch.  Where there is one, ``csrc/python/calls.cc`` becomes ``_calls.so`` for it.
 
 hipcc cross-compiles without a GPU.  The library is built in-tree so that it
 travels with the source tree to the machine that runs it.
@@ -22,6 +23,7 @@ CALIBRATE_SOURCES = ("calibrate.hip",)  # not linked into the product library
 CALLS_SOURCE = os.path.join(CSRC, "python", "calls.cc")  # the linears of ops.py as a Python extension
 CALLS_LIB = os.path.join(HERE, "_calls.so")
 OBJDIR = os.path.join(HERE, "build")
+CALLS_STAMP = os.path.join(OBJDIR, "_calls.torch")  # the version of torch that _calls.so was compiled for
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -53,6 +55,24 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _torch_version():
+    """The version of the installed torch, or None."""
+    try:
+        import torch
+    except ImportError:
+        return None
+    return str(torch.__version__)
+
+
+def _calls_stale() -> bool:
+    if not os.path.exists(CALLS_LIB) or not os.path.exists(CALLS_STAMP):
+        return True
+    with open(CALLS_STAMP) as f:
+        if f.read() != _torch_version():
+            return True
+    return any(os.path.getmtime(d) > os.path.getmtime(CALLS_LIB) for d in _deps(CALLS_SOURCE))
+
+
 def _compile_calls() -> str:
     from torch.utils import cpp_extension
 
@@ -62,6 +82,8 @@ def _compile_calls() -> str:
     p = subprocess.run(cmd, capture_output=True, text=True)
     if p.returncode != 0:
         raise RuntimeError(f"g++ failed on {CALLS_SOURCE}:\n{p.stderr}")
+    with open(CALLS_STAMP, "w") as f:
+        f.write(_torch_version())
     return CALLS_LIB
 
 
@@ -114,12 +136,15 @@ def build(verbose: bool = True, incremental: bool = False) -> str:
                     os.remove(obj)
             for f in compiled + checks:
                 f.result()
-    if not incremental or not os.path.exists(CALLS_LIB) or any(os.path.getmtime(d) > os.path.getmtime(CALLS_LIB) for d in _deps(CALLS_SOURCE)):
-        _compile_calls()
     for lib, want in ((LIB, False), (CALIBRATE_LIB, True)):
         objs = [os.path.join(OBJDIR, os.path.basename(s) + ".o") for s in srcs
                 if (os.path.basename(s) in CALIBRATE_SOURCES) == want]
         subprocess.check_call([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib, *objs])
+    # last: the libraries above are for programs without torch too
+    if _torch_version() is None:
+        print(f"no torch: {CALLS_LIB} is not built", flush=True)
+    elif not incremental or _calls_stale():
+        _compile_calls()
     if verbose:
         print(f"built {LIB}: compiled {len(todo)} of {len(srcs)} sources", flush=True)
     return LIB
