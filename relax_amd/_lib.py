@@ -1,12 +1,13 @@
 """Loads ``librelax_amd_wq.so`` and declares the C ABI of ``include/relax_amd_wq.h`` and ``include/relax_amd_vm.h``.
 
-There is no fallback: if the library is missing or a symbol is absent the import
+There is no fallback for it: if the library is missing or a symbol is absent the import
 fails with an error that says how to build it.
 """
 from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "librelax_amd_wq.so")
@@ -138,8 +139,20 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+class _NoCalls:
+    """In the place of the extension where there is none for this torch: every call is left to the general path."""
+
+    @staticmethod
+    def _left(*args):
+        return None
+
+    q4g32_linear = fpA_intB_gemm = gptq_linear = _left
+
+
 def calls():
-    """The extension that takes the common form of a linear of ops.py from its tensors to the launch (csrc/python/calls.cc)."""
+    """The extension that takes the common form of a linear of ops.py from its tensors to the launch (csrc/python/calls.cc).
+    It is compiled for one version of torch; with another, or without it, the linears go through ctypes as all other calls do:
+    the same kernels, with 7.4 instead of 4.4 us of host time for the shortest call."""
     global _calls
     if _calls is None:
         import torch
@@ -147,8 +160,14 @@ def calls():
         l = lib()
         try:
             from relax_amd import _calls as m
+
+            made_for = getattr(m, "torch_version", "an unknown version")
+            if made_for != str(torch.__version__):
+                raise ImportError(f"compiled for torch {made_for}, this is {torch.__version__}")
         except ImportError as e:
-            raise ImportError(f"relax_amd/_calls.so cannot be loaded ({e}): build it with `python -m relax_amd.build`") from e
+            warnings.warn(f"relax_amd/_calls.so is not used ({e}), calls take longer: build it with `python -m relax_amd.build`", RuntimeWarning)
+            _calls = _NoCalls()
+            return _calls
         fns = (l.wq_q4g32_linear, l.wq_fpA_intB_gemm, l.wq_fpA_intB_gemm_residual, l.wq_gptq_linear, l.wq_gptq_workspace_bytes)
         m.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in fns), torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
         _calls = m

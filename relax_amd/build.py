@@ -77,7 +77,7 @@ def _compile_calls() -> str:
     from torch.utils import cpp_extension
 
     dirs = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", *(f"-I{d}" for d in dirs), CALLS_SOURCE,
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", f'-DRELAX_AMD_TORCH_VERSION="{_torch_version()}"', *(f"-I{d}" for d in dirs), CALLS_SOURCE,
            "-o", CALLS_LIB, *(f"-L{d}" for d in cpp_extension.library_paths()), "-lc10", "-ltorch_cpu", "-ltorch_python"]
     p = subprocess.run(cmd, capture_output=True, text=True)
     if p.returncode != 0:

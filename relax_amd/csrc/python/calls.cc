@@ -215,4 +215,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods, nul
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__calls() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__calls() {
+  PyObject* m = PyModule_Create(&module);
+  // (its layout of a tensor is that of this torch and of no other)
+  if (m && PyModule_AddStringConstant(m, "torch_version", RELAX_AMD_TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}
