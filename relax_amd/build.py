@@ -124,7 +124,7 @@ def build(verbose: bool = True, incremental: bool = False) -> str:
     from relax_amd import check_ring_asm
 
     # some kernels wait by hand for loads that the compiler does not see: the code generated for them is verified
-    checked = [s for s in todo if os.path.basename(s) in check_ring_asm.SOURCES + check_ring_asm.DIRECT_LOAD_SOURCES]
+    checked = [s for s in todo if os.path.basename(s) in check_ring_asm.SOURCES + check_ring_asm.HELD_SOURCES + check_ring_asm.DIRECT_LOAD_SOURCES]
     if todo:
         with concurrent.futures.ThreadPoolExecutor(max_workers=8) as ex:
             compiled = [ex.submit(_compile, s) for s in todo]

@@ -21,7 +21,7 @@ sources therefore wait for all loads (``s_waitcnt vmcnt(0)``) where the ring's l
 Registers that the compiler also uses for short-lived temporaries while a slot is empty are
 recognised by being written by another instruction first.
 
-Kernels with non-temporal loads, in whatever form, must also be free of register spills (no ``scratch_*`` instruction).
+Kernels of these files with non-temporal loads, in whatever form, and those of ``held_gemm.h`` must also be free of register spills (no ``scratch_*`` instruction).
 
 A second check (``check_asm_results``) covers what inline assembly costs besides: the compiler does
 not keep the hardware's wait states between an inline-assembly VALU result and an MFMA or DPP
@@ -43,6 +43,8 @@ import tempfile
 HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ("q4g32_gemv_list.hip", "q4g32_batch_list.hip")
 # the tiled GEMMs (mfma_gemm_lds.h)
+# the kernel with activations in registers (held_gemm.h)
+HELD_SOURCES = ("gptq.hip", "q4g32_skinny.hip")
 DIRECT_LOAD_SOURCES = ("gemm_256.hip", "gptq.hip", "intb_gemm.hip", "q4g32_gemm.hip", "q4n32.hip")
 # kernels of SOURCES whose loads past the end have a scalar offset
 GUARDED_KERNELS = {"q4g32_batch_list.hip": ("q4g32_batch_list_kernel", "q4g32_batch_rows_kernel")}
@@ -166,6 +168,20 @@ def _functions(asm_text: str, labels: bool = False):
     return functions
 
 
+def _spills(body: list[str]) -> list[str]:
+    """These kernels are written to fit their register budget.  A spill anywhere in them (also in a service
+    wavefront's path: one extra branch there once sent 64 load registers through scratch memory and
+    cost the 4-linear step 3 of 21 us) is a regression the tests do not show."""
+    spills = [l for l in body if l.startswith(("scratch_load", "scratch_store"))]
+    return [f"{len(spills)} scratch accesses (register spills), the first: `{spills[0]}`"] if spills else []
+
+
+def check_held(asm_text: str) -> list[str]:
+    """Every ``held_gemm_kernel`` of the file: up to 252 of 256 registers, and no spill."""
+    kernels = [body for name, body in _functions(asm_text) if "held_gemm_kernel" in name]
+    return [e for body in kernels for e in _spills(body)] if kernels else ["no held_gemm_kernel found"]
+
+
 def check(asm_text: str) -> list[str]:
     """Checks every kernel of the file on its own (register names mean nothing across kernels)."""
     errors, with_ring = [], 0
@@ -173,12 +189,7 @@ def check(asm_text: str) -> list[str]:
         if any(_is_ring_load(l) or l.endswith(_COMPILERS) for l in body):
             with_ring += any(_is_ring_load(l) for l in body)
             errors += _check_function(body)
-            # These kernels are written to fit their register budget.  A spill anywhere in them (also in a service
-            # wavefront's path: one extra branch there once sent 64 load registers through scratch memory and
-            # cost the 4-linear step 3 of 21 us) is a regression the tests do not show.
-            spills = [l for l in body if l.startswith(("scratch_load", "scratch_store"))]
-            if spills:
-                errors.append(f"{len(spills)} scratch accesses (register spills), the first: `{spills[0]}`")
+            errors += _spills(body)
     if with_ring == 0:
         return ["no ring loads found (expected global_load_* / buffer_load_* ... nt in the kernel)"]
     return errors
@@ -322,8 +333,17 @@ def _assembly(hipcc: str, flags, name: str) -> str:
 
 
 def check_source(hipcc: str, flags, name: str) -> None:
-    """Raises if the code generated for one of SOURCES or DIRECT_LOAD_SOURCES is not as it has to be."""
+    """Raises if the code generated for one of SOURCES, HELD_SOURCES or DIRECT_LOAD_SOURCES is not as it has to be."""
     text = _assembly(hipcc, flags, name)
+    if name in SOURCES + HELD_SOURCES:
+        found = check_asm_results(text)
+        if found:
+            raise RuntimeError(f"{name}: an inline-assembly result reaches an MFMA / DPP instruction without wait states:\n  "
+                               + "\n  ".join(found[:20]))
+    if name in HELD_SOURCES:
+        found = check_held(text)
+        if found:
+            raise RuntimeError(f"{name}: registers of a kernel with the activations in them are spilled:\n  " + "\n  ".join(found[:20]))
     if name in DIRECT_LOAD_SOURCES:
         found = check_direct_loads_drained(text)
         if found:
@@ -331,22 +351,19 @@ def check_source(hipcc: str, flags, name: str) -> None:
         found = check_empty_descriptors(text)
         if found:
             raise RuntimeError(f"{name}: a load past the last step may touch memory:\n  " + "\n  ".join(found[:20]))
+    if name not in SOURCES:
         return
     errs = check(text)
-    hazards = check_asm_results(text)
     past = [e for k in GUARDED_KERNELS.get(name, ()) for e in check_empty_descriptors(text, k)]
     if past:
         raise RuntimeError(f"{name}: a load past the end may touch memory:\n  " + "\n  ".join(past[:20]))
     if errs:
         raise RuntimeError(f"{name}: the generated code touches in-flight ring registers:\n  " + "\n  ".join(errs[:20]))
-    if hazards:
-        raise RuntimeError(f"{name}: an inline-assembly result reaches an MFMA / DPP instruction without wait states:\n  "
-                           + "\n  ".join(hazards[:20]))
 
 
 if __name__ == "__main__":
     from relax_amd import build as _b  # noqa: E402
 
-    for _name in SOURCES + DIRECT_LOAD_SOURCES:
+    for _name in sorted({*SOURCES, *HELD_SOURCES, *DIRECT_LOAD_SOURCES}):
         _b.check_asm(_name)
     print("ring registers, direct loads: ok")

@@ -163,6 +163,45 @@ def test_the_build_checks_every_source_with_the_tiled_gemm():
     assert with_gemm == set(c.DIRECT_LOAD_SOURCES)
 
 
+HELD = """
+_ZN2wq16held_gemm_kernelEv:
+\t;;#ASMSTART
+\tv_mov_b32 v10, v2
+{nop}\t;;#ASMEND
+\tv_mov_b32_dpp v50, v10 row_ror:8 row_mask:0xf bank_mask:0xc
+{body}
+\ts_endpgm
+.Lfunc_end0:
+"""
+
+
+def test_the_kernel_with_activations_in_registers_is_checked(monkeypatch):
+    import os
+
+    import pytest
+
+    including = set()
+    for name in os.listdir(os.path.join(c.HERE, "csrc")):
+        if name.endswith(".hip"):
+            with open(os.path.join(c.HERE, "csrc", name)) as f:
+                if '#include "held_gemm.h"' in f.read():
+                    including.add(name)
+    assert including == set(c.HELD_SOURCES)
+    monkeypatch.setattr(c, "check_direct_loads_drained", lambda text: [])
+    monkeypatch.setattr(c, "check_empty_descriptors", lambda text: [])
+    nop = "\ts_nop 1\n"
+    for name in c.HELD_SOURCES:
+        for text, refused in ((HELD.format(nop=nop, body=""), None), (HELD.format(nop="", body=""), "wait states"),
+                              (HELD.format(nop=nop, body="\tscratch_store_dword off, v9, off offset:4"), "spilled"),
+                              (HELD.format(nop=nop, body="").replace("held_gemm", "other"), "spilled")):
+            monkeypatch.setattr(c, "_assembly", lambda *a, text=text: text)
+            if refused is None:
+                c.check_source("hipcc", [], name)
+            else:
+                with pytest.raises(RuntimeError, match=refused):
+                    c.check_source("hipcc", [], name)
+
+
 def test_an_incremental_build_does_not_keep_what_was_refused(tmp_path, monkeypatch):
     """A source that does not compile must not hide that another one was refused: its object would pass for up to date."""
     import os
