@@ -29,6 +29,7 @@
 
 #include <type_traits>
 
+#include "code_products.h"
 #include "tuning.h"
 #include "wq_device.h"
 #include "wq_host.h"
@@ -102,16 +103,6 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
     return __builtin_amdgcn_raw_buffer_load_b128(from, w_off[p] + (uint32_t)(h * 8 * col_bytes), 0, 2 /* nt */);
   };
 
-  // of two loads of 8 rows or columns x 2 halves the two halves of both: lanes 8 .. 15 of every 16 take the first half from the
-  // second load 8 lanes below, lanes 0 .. 7 the second half from the first load 8 lanes above
-  auto exchange = [&](uint32_t (&a)[4], uint32_t (&b)[4]) {
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const uint32_t lo = a[d], hi = b[d];
-      a[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)lo, (int)hi, 0x128 /* row_ror:8 */, 0xf, 0xc, false);
-      b[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)hi, (int)lo, 0x128, 0xf, 0x3, false);
-    }
-  };
   // ---- everything that the first tile needs is requested at once: activations, scales of two tiles, codes ----
   half8_t xb[PW][NO];  // operand o of piece p
   uint4_t raw[PW][NO];
@@ -176,7 +167,7 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
         uint32_t in[2][4];
 #pragma unroll
         for (int h = 0; h < 2; ++h) in[h][0] = raw[p][o + h].x, in[h][1] = raw[p][o + h].y, in[h][2] = raw[p][o + h].z, in[h][3] = raw[p][o + h].w;
-        exchange(in[0], in[1]);
+        exchange_halves(in[0], in[1]);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           uint32_t q[4];
@@ -208,11 +199,7 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
     build((half_t)1.0f);
   }
 
-  // a word of codes as an operand, and as weights rounded to fp16: (code - off) * s
-  auto codes = [&](uint32_t w) {
-    const uint32_t w8 = w >> 8;
-    return __builtin_bit_cast(half8_t, uint4_t{w & 0x000F000Fu, w & 0x00F000F0u, w8 & 0x000F000Fu, w8 & 0x00F000F0u});
-  };
+  // a word of codes as weights rounded to fp16: (code - off) * s
   auto weights = [&](uint32_t w, half_t off, half_t s) {
     const half_t o = off + (half_t)1024.0f;
     const half2_t o2 = {o, o}, s2 = {s, s};
@@ -221,19 +208,11 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
     for (int d = 0; d < 4; ++d) r[d] = as_u32((as_half2(((w >> (4 * d)) & 0x000F000Fu) | 0x64006400u) - o2) * s2);
     return __builtin_bit_cast(half8_t, uint4_t{r[0], r[1], r[2], r[3]});
   };
-  // a[g]: word kq of group g in lane quarter kq, from word g of group kq
-  auto spread = [&](uint32_t (&a)[4]) {
-    const auto h0 = __builtin_amdgcn_permlane32_swap(a[0], a[2], false, false);
-    const auto h1 = __builtin_amdgcn_permlane32_swap(a[1], a[3], false, false);
-    const auto q0 = __builtin_amdgcn_permlane16_swap(h0[0], h1[0], false, false);
-    const auto q1 = __builtin_amdgcn_permlane16_swap(h0[1], h1[1], false, false);
-    a[0] = q0[0], a[1] = q0[1], a[2] = q1[0], a[3] = q1[1];
-  };
   auto arrange = [&](uint32_t (&w)[2][4]) {
-    if constexpr (!HALF) exchange(w[0], w[1]);
+    if constexpr (!HALF) exchange_halves(w[0], w[1]);
     if constexpr (FMT == kHeldQ4) {
-      spread(w[0]);
-      spread(w[1]);
+      spread_words(w[0]);
+      spread_words(w[1]);
     }
   };
   // scales of what w[h] holds after that: columns 0 .. 7, 8 .. 15 at the lane's half (HALF), or column i at half h
@@ -246,12 +225,8 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
       uint32_t w[2][4];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        uint4_t& l = word[2 * p + h];
-        // (copies, and not the registers of the loads: those take the next tile's)
-        asm("v_mov_b32 %0, %4\n\tv_mov_b32 %1, %5\n\tv_mov_b32 %2, %6\n\tv_mov_b32 %3, %7\n\ts_nop 1"
-            : "=&v"(w[h][0]), "=&v"(w[h][1]), "=&v"(w[h][2]), "=&v"(w[h][3])
-            : "v"(l.x), "v"(l.y), "v"(l.z), "v"(l.w));
-        l = request(next, p, h);
+        take_words(word[2 * p + h], w[h]);
+        word[2 * p + h] = request(next, p, h);
       }
       arrange(w);
       float4_t t[2][2];
@@ -278,7 +253,7 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
             else c[h] = sum_of(xb[p][o], kNull);
           }
 #pragma unroll
-          for (int h = 0; h < 2; ++h) t[g & 1][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[p][HALF ? g : 4 * h + g], codes(w[h][g]), c[h], 0, 0, 0);
+          for (int h = 0; h < 2; ++h) t[g & 1][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[p][HALF ? g : 4 * h + g], code_operand(w[h][g]), c[h], 0, 0, 0);
           if (g > 0) scale(g - 1);
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -292,7 +267,7 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
         for (int d = 0; d < 4; ++d)
 #pragma unroll
           for (int h = 0; h < 2; ++h)
-            t[0][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[p][HALF ? d : 4 * h + d], codes(w[h][d]), d == 0 ? kNull : t[0][h], 0, 0, 0);
+            t[0][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[p][HALF ? d : 4 * h + d], code_operand(w[h][d]), d == 0 ? kNull : t[0][h], 0, 0, 0);
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -362,16 +337,9 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
     unsigned char* const set = parts + buf * 8 * PART;
     float* const part = reinterpret_cast<float*>(set + ks * PART);
     if constexpr (HALF) {
-      // lane (i, kq): rows 4 (kq mod 2) .. + 3 at half kq / 2, times columns i mod 8 (+ 8) at half i / 8: sums where the halves
-      // agree.  They come together in the lanes with i < 8, quarters 0 and 1 for columns 0 .. 7, 2 and 3 for 8 .. 15.
       float sum[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float lo = acc[0][e], hi = acc[NA - 1][e];
-        const auto p = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi), false, false);
-        const uint32_t mine = p[0], other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p[1], 0x128 /* row_ror:8 */, 0xf, 0xf, false);
-        sum[e] = __builtin_bit_cast(float, mine) + __builtin_bit_cast(float, other);
-      }
+      for (int e = 0; e < 4; ++e) sum[e] = join_halves(acc[0][e], acc[NA - 1][e]);
       if (i < 8) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) part[(4 * (kq & 1) + e) * 16 + 8 * (kq >> 1) + i] = sum[e];

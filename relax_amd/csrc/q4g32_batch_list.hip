@@ -56,6 +56,7 @@
 #include <cmath>
 #include <vector>
 
+#include "code_products.h"
 #include "gemv_list_common.h"
 #include "tuning.h"
 
@@ -318,36 +319,12 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
     };
     auto request = [&](const Place& p, int sp, int r) { return __builtin_amdgcn_raw_buffer_load_b128(p.base, p.roff[r] + p.goff[sp], 0, kNonTemporal); };
 
-    // 8 codes as the B operand: fp16 numbers whose bits are the codes, that is 2^-24 (q0, q4), 2^-20 (q1, q5) and so on
-    auto codes = [&](uint32_t w) {
-      const uint32_t w8 = w >> 8;
-      return __builtin_bit_cast(half8_t, uint4_t{w & 0x000F000Fu, w & 0x00F000F0u, w8 & 0x000F000Fu, w8 & 0x00F000F0u});
-    };
-    // ... and as the weights that the format defines, (q - 7) * s rounded to fp16
+    // 8 codes as the weights that the format defines, (q - 7) * s rounded to fp16, times 16 in bits 4 .. 7
     auto weights = [&](uint32_t w, half_t s) {
       const half2_t c7 = {(half_t)-1031.0f, (half_t)-1031.0f}, c112 = {(half_t)-1136.0f, (half_t)-1136.0f}, s2 = {s, s};
-      const uint4_t c = __builtin_bit_cast(uint4_t, codes(w)) | 0x64006400u;
+      const uint4_t c = __builtin_bit_cast(uint4_t, code_operand(w)) | 0x64006400u;
       return __builtin_bit_cast(half8_t, uint4_t{as_u32((as_half2(c.x) + c7) * s2), as_u32((as_half2(c.y) + c112) * s2),
                                                  as_u32((as_half2(c.z) + c7) * s2), as_u32((as_half2(c.w) + c112) * s2)});
-    };
-    // a[g]: word kq of group g in lane quarter kq, from word g of group kq
-    auto spread = [&](uint32_t (&a)[4]) {
-      const auto h0 = __builtin_amdgcn_permlane32_swap(a[0], a[2], false, false);
-      const auto h1 = __builtin_amdgcn_permlane32_swap(a[1], a[3], false, false);
-      const auto q0 = __builtin_amdgcn_permlane16_swap(h0[0], h1[0], false, false);
-      const auto q1 = __builtin_amdgcn_permlane16_swap(h0[1], h1[1], false, false);
-      a[0] = q0[0], a[1] = q0[1], a[2] = q1[0], a[3] = q1[1];
-    };
-
-    // WIDE: lanes 8 .. 15 of every 16 take their half of chunk 0 (4 groups) from the second load 8 lanes below, lanes 0 .. 7
-    // their half of chunk 1 from the first load 8 lanes above (row_ror:8 turns a row of 16 lanes by 8)
-    auto exchange = [&](uint32_t (&a)[4], uint32_t (&b2)[4]) {
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const uint32_t lo = a[d], hi = b2[d];
-        a[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)lo, (int)hi, 0x128 /* row_ror:8 */, 0xf, 0xc, false);
-        b2[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)hi, (int)lo, 0x128, 0xf, 0x3, false);
-      }
     };
     // the lane's four scales of what load r of piece sp brought (WIDE: of chunk r mod 2 of row tile r / 2)
     auto scales = [&](int slot, int sp, int r) {
@@ -381,16 +358,13 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
 #pragma unroll
             for (int r = 2 * q; r < 2 * q + 2; ++r) {
               const int at = sp * 2 * RT + 2 * q0 + r;
-              // (copies, and not the registers of the loads: those take the next item's)
-              asm("v_mov_b32 %0, %4\n\tv_mov_b32 %1, %5\n\tv_mov_b32 %2, %6\n\tv_mov_b32 %3, %7\n\ts_nop 1"
-                  : "=&v"(w[r][0]), "=&v"(w[r][1]), "=&v"(w[r][2]), "=&v"(w[r][3])
-                  : "v"(buf[at].x), "v"(buf[at].y), "v"(buf[at].z), "v"(buf[at].w));
+              take_words(buf[at], w[r]);
               buf[at] = request(next, sp, 2 * q0 + r);
               s4[r] = scales(slot, sp, 2 * q0 + r);
             }
-            if constexpr (WIDE) exchange(w[2 * q], w[2 * q + 1]);
-            spread(w[2 * q]);
-            spread(w[2 * q + 1]);
+            if constexpr (WIDE) exchange_halves(w[2 * q], w[2 * q + 1]);
+            spread_words(w[2 * q]);
+            spread_words(w[2 * q + 1]);
           }
           if (q == 0) {
 #pragma unroll
@@ -398,7 +372,7 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
           }
 #pragma unroll
           for (int h = 0; h < 2; ++h)
-            t[step & 1][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[WIDE ? 2 * sp + h : sp][g], codes(w[2 * q + h][g]), c[WIDE ? h : 0], 0, 0, 0);
+            t[step & 1][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[WIDE ? 2 * sp + h : sp][g], code_operand(w[2 * q + h][g]), c[WIDE ? h : 0], 0, 0, 0);
           if (step > 0) scale(step - 1);
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -419,10 +393,10 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
             const uint4_t l = request(here, sp, 2 * q + h);
             w[h][0] = l.x, w[h][1] = l.y, w[h][2] = l.z, w[h][3] = l.w;
           }
-          if constexpr (WIDE) exchange(w[0], w[1]);
+          if constexpr (WIDE) exchange_halves(w[0], w[1]);
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            spread(w[h]);
+            spread_words(w[h]);
             const half4_t s4 = scales(slot, sp, 2 * q + h);
             float4_t& a = acc[WIDE ? q : 2 * q + h];
 #pragma unroll
@@ -478,17 +452,9 @@ __global__ __launch_bounds__(kBThreads) void q4g32_batch_list_kernel(const GemvL
 #pragma unroll
       for (int q = 0; q < RT; ++q) {
         if constexpr (!WIDE) {
-          // Lane (i, kq) has activation rows 4 (kq mod 2) .. + 3 at the groups of half kq / 2, times rows i mod 8 (+ 8) of W at
-          // those of half i / 8: sums where the halves agree.  They come together in the lanes with i < 8, lane quarters 0 and
-          // 1 for rows 0 .. 7, 2 and 3 for rows 8 .. 15.
           float sum[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float lo = acc[2 * q][e], hi = acc[2 * q + 1][e];
-            const auto p = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi), false, false);
-            const uint32_t mine = p[0], other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p[1], 0x128 /* row_ror:8 */, 0xf, 0xf, false);
-            sum[e] = __builtin_bit_cast(float, mine) + __builtin_bit_cast(float, other);
-          }
+          for (int e = 0; e < 4; ++e) sum[e] = join_halves(acc[2 * q][e], acc[2 * q + 1][e]);
           if (i < 8) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) part[q * 128 + (4 * (kq & 1) + e) * 16 + 8 * (kq >> 1) + i] = sum[e];
