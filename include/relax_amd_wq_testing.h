@@ -43,6 +43,9 @@ void wq_debug_set_gemv_blocks_per_cu(int n);
 /* Small-batch kernel: wavefronts side by side (1, 2, 3, 4, 8), ring slots, and which kernel
  * (waves 1: ring, 12: ring with 12 wavefronts for nw = 3, 2: activations in registers); 0 = from the shape. */
 void wq_debug_set_skinny_config(int nw, int stages, int waves);
+/* What the calling thread's last small-batch call launched: 1, 2: the kernels with the activations in registers (1: q4f16_1 and AutoGPTQ,
+ * products of codes); slabs of 8 TH rows, NW wavefronts side by side of WAVES: TH << 16 | NW << 8 | WAVES. */
+int wq_debug_small_batch_form(void);
 /* How a list of 2 .. 32 activation rows was planned: the number of equal groups of workgroups that run
  * different linears side by side, or 0 if the linears of the (short) list share the 8 XCDs in sets sized by
  * their cost; -1 for a list of one activation row. */

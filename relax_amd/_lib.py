@@ -94,6 +94,7 @@ TESTING_SIGNATURES = {
     "wq_debug_set_gemv_blocks_per_cu": [_int],
     "wq_debug_set_skinny_config": [_int, _int, _int],
     "wq_debug_set_intb_gemv_k_split": [_int],
+    "wq_debug_small_batch_form": [],
     "wq_debug_gemv_list_groups": [_vp],
     "wq_debug_gemv_list_shape": [_vp],
 }
@@ -134,7 +135,7 @@ def lib() -> ctypes.CDLL:
         for name, argtypes in TESTING_SIGNATURES.items():
             fn = getattr(l, name)
             fn.argtypes = argtypes
-            fn.restype = ctypes.c_int if name.startswith("wq_debug_gemv_list_") else None
+            fn.restype = None if name.startswith("wq_debug_set_") else ctypes.c_int
         _lib = l
     return _lib
 

@@ -427,6 +427,7 @@ static int launch_held_form(const char* who, const HeldArgs& args, const uint16_
   // (as few workgroups as make the same number of rounds: each of them loads all activations)
   WQ_LAUNCH(who, kern, dim3((unsigned)((tiles + rounds - 1) / rounds)), dim3(512), Cfg::kLdsBytes, stream, args, (const half_t*)x,
             (half_t*)y, epi, (int)M, (int)N, (int)K);
+  tuning().small_batch_form = kHeldForm;
   return WQ_OK;
 }
 

@@ -657,6 +657,7 @@ static int launch_xreg(const char* who, const typename Policy::Args& pargs, cons
   WQ_HIP(limit.ensure(reinterpret_cast<const void*>(kern), 160 * 1024));
   WQ_LAUNCH(who, kern, dim3((unsigned)blocks), dim3(64 * WAVES), Cfg::kLdsBytes, stream, pargs,
             (const half_t*)x, (half_t*)y, epi, (int)M, (int)N, (int)K);
+  tuning().small_batch_form = kXregForm;
   return WQ_OK;
 }
 
@@ -712,6 +713,7 @@ static int launch_skinny_form(const char* who, const typename Policy::Args& parg
   WQ_HIP(limit.ensure(reinterpret_cast<const void*>(kern), 160 * 1024));
   WQ_LAUNCH(who, kern, dim3((unsigned)blocks), dim3(64 * WAVES), lds_bytes, stream, pargs,
             (const half_t*)x, (half_t*)y, epi, (int)M, (int)N, (int)K, stages);
+  tuning().small_batch_form = small_batch_form(TH, NW, WAVES);
   return WQ_OK;
 }
 

@@ -16,9 +16,12 @@ struct Tuning {
   int gemm_tail_split = 1;   // split the tiles of the last, partial round (on by default)
   int gemv_rows = 0, gemv_gpl = 0, gemv_blocks_per_cu = 0;
   int skinny_nw = 0, skinny_stages = 0, skinny_waves = 0;
+  int small_batch_form = 0;  // not an override: what this thread's last small-batch call launched (small_batch_form(), below)
   int intb_k_split = 0;      // Format B decode GEMV: wavefronts that share a column group and split K (1, 2, 4, 8)
 };
 Tuning& tuning();
+constexpr int kHeldForm = 1, kXregForm = 2;
+constexpr int small_batch_form(int TH, int NW, int waves) { return TH << 16 | NW << 8 | waves; }
 
 // hipFuncAttributeMaxDynamicSharedMemorySize is a property of (kernel, device): it is raised when a
 // launch first needs more than has been set on that device, not on every launch.  One object per

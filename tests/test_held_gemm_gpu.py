@@ -71,26 +71,45 @@ def test_against_float64(fmt, M, N, K):
     np.testing.assert_array_equal(y_odd[0].float().cpu().numpy(), want.float().cpu().numpy())
 
 
-@pytest.mark.parametrize("fmt", ["q4f16_1", "gptq"])
-def test_the_choice_by_shape_at_its_edges(fmt):
-    """More than 8 rows, four tiles per CU and one fewer column tile: both kernels are right."""
-    from relax_amd import ops
+# (format, M, column tiles per CU, tiles beside that, K, whether the kernel takes it): each bound of the rule from both sides
+EDGES = [
+    # K above 4096 and four tiles per CU
+    ("q4f16_1", 16, 4, 0, 4160, True), ("q4f16_1", 16, 4, -1, 4160, False), ("q4f16_1", 16, 4, 0, 4096, False),
+    ("gptq", 16, 4, 0, 4224, True), ("gptq", 16, 4, -1, 4224, False),
+    # up to 8 rows: two tiles per CU, K of 4352 or (AutoGPTQ) 3072
+    ("q4f16_1", 8, 2, 1, 4352, True), ("q4f16_1", 8, 2, 0, 4352, False), ("q4f16_1", 8, 2, 1, 4288, False), ("q4f16_1", 9, 2, 1, 4352, False),
+    ("gptq", 8, 2, 1, 3072, True), ("gptq", 8, 2, 0, 3072, False), ("gptq", 8, 2, 1, 2944, False), ("gptq", 9, 2, 1, 3072, False),
+    # ... five tiles per CU, K of 3840
+    ("q4f16_1", 3, 5, 0, 3840, True), ("q4f16_1", 3, 5, -1, 3840, False), ("q4f16_1", 3, 5, 0, 3776, False),
+    # more than 8 rows: five tiles per CU, K above 3072
+    ("q4f16_1", 9, 5, 0, 3136, True), ("q4f16_1", 9, 5, -1, 3136, False), ("q4f16_1", 9, 5, 0, 3072, False),
+    ("gptq", 16, 5, 0, 3200, True), ("gptq", 16, 5, -1, 3200, False), ("gptq", 16, 5, 0, 3072, False),
+    # ... AutoGPTQ, two tiles per CU, K above 3840 that fills 15/16 of its pieces
+    ("gptq", 9, 2, 1, 3968, True), ("gptq", 9, 2, 0, 3968, False), ("gptq", 9, 2, 1, 3840, False), ("gptq", 9, 2, 1, 5760, False),
+    ("gptq", 9, 2, 1, 5888, True),
+]
+
+
+@pytest.mark.parametrize("fmt,M,per_cu,more,K,held", EDGES)
+def test_the_choice_by_shape_at_its_edges(fmt, M, per_cu, more, K, held):
+    """Which kernel ran, and that it is right: without rounded weights (2^-17 of a product, the alignment in the matrix core) where
+    this one did, and with them (2^-11) where another."""
+    from relax_amd import _lib, ops
 
     g = torch.Generator(device="cuda").manual_seed(3)
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    for N in (64 * cus, 64 * cus - 16):
-        K = 4224
-        x = torch.randn(16, K, device="cuda", generator=g).half()
-        W = torch.randint(-(2**31), 2**31 - 1, (K // 8, N), device="cuda", dtype=torch.int32, generator=g)
-        if fmt == "gptq":
-            s = (torch.rand(K // 128, N, device="cuda", generator=g) * 0.015 + 0.005).half()
-            z = torch.randint(-(2**31), 2**31 - 1, (K // 128, N // 8), device="cuda", dtype=torch.int32, generator=g)
-            w = (_codes(W.t().contiguous()) - (_codes(z) + 1).repeat_interleave(128, 0).t()) * s.double().repeat_interleave(128, 0).t()
-            y = ops.gptq_linear(ops.gptq_prepare(W, z, s, torch.arange(K, dtype=torch.int32, device="cuda") // 128), x)
-        else:
-            Wt, s = W.t().contiguous(), (torch.rand(N, K // 32, device="cuda", generator=g) * 0.015 + 0.005).half()
-            w = (_codes(Wt) - 7) * s.double().repeat_interleave(32, 1)
-            y = ops.q4g32_linear(Wt, s, x)
-        torch.cuda.synchronize()
-        exact, mass = x.double() @ w.t(), x.double().abs() @ w.abs().t()
-        assert ((y.double() - exact).abs() <= exact.abs() * 2.0**-11 + mass * 2.0**-11).all()
+    N = 16 * (per_cu * torch.cuda.get_device_properties(0).multi_processor_count + more)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    W = torch.randint(-(2**31), 2**31 - 1, (K // 8, N), device="cuda", dtype=torch.int32, generator=g)
+    if fmt == "gptq":
+        s = (torch.rand(K // 128, N, device="cuda", generator=g) * 0.015 + 0.005).half()
+        z = torch.randint(-(2**31), 2**31 - 1, (K // 128, N // 8), device="cuda", dtype=torch.int32, generator=g)
+        w = (_codes(W.t().contiguous()) - (_codes(z) + 1).repeat_interleave(128, 0).t()) * s.double().repeat_interleave(128, 0).t()
+        y = ops.gptq_linear(ops.gptq_prepare(W, z, s, torch.arange(K, dtype=torch.int32, device="cuda") // 128), x)
+    else:
+        Wt, s = W.t().contiguous(), (torch.rand(N, K // 32, device="cuda", generator=g) * 0.015 + 0.005).half()
+        w = (_codes(Wt) - 7) * s.double().repeat_interleave(32, 1)
+        y = ops.q4g32_linear(Wt, s, x)
+    torch.cuda.synchronize()
+    assert (_lib.lib().wq_debug_small_batch_form() == 1) == held
+    exact, mass = x.double() @ w.t(), x.double().abs() @ w.abs().t()
+    assert ((y.double() - exact).abs() <= exact.abs() * 2.0**-11 + mass * (2.0**-17 if held else 2.0**-11)).all()

@@ -1,6 +1,6 @@
 """Slabs of 24 and 48 rows in every format of the small-batch kernel, with one, two and four column blocks and eight wavefronts, and
 with three and twelve: workgroups whose last columns lie past N, fewer steps of K than wavefronts along it, K that ends
-inside a step, and (the last) the choice by shape."""
+inside a step; and the choice by shape."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -33,3 +33,51 @@ def test_against_the_oracle(fmt, M, N, K, nw, stages, waves):
                 u.assert_close(u.host(y), oracle.q4g32_linear(W, S, x, nthreads=8), f"{fmt} {M}x{N}x{k}")
     finally:
         _lib.lib().wq_debug_set_skinny_config(0, 0, 0)
+
+
+# (formats, M, column tiles per CU, tiles beside that (Format B: fours), K, slab rows / 8, wavefronts side by side, wavefronts or 0: either count)
+ONE, TWO = ("q4f16_1", "int4"), ("int8",)  # pieces of a weight tile
+EDGES = [
+    # 17 .. 24 rows, two to three tiles per CU: twelve wavefronts from K = 2048 on
+    (ONE + TWO, 17, 2, 4, 2048, 3, 3, 12), (ONE + TWO, 24, 3, 0, 2048, 3, 3, 12), (ONE + TWO, 24, 2, 0, 2048, 4, 2, 0), (ONE + TWO, 24, 3, 4, 2048, 4, 4, 0),
+    (ONE, 24, 3, 0, 1984, 4, 4, 0), (TWO, 24, 3, 0, 1984, 3, 3, 6), (ONE + TWO, 25, 3, 0, 2048, 4, 4, 0), (ONE + TWO, 16, 3, 0, 2048, 2, 0, 0),
+    # ... four to six
+    (ONE + TWO, 20, 4, 4, 128, 3, 3, 6), (ONE + TWO, 20, 6, 0, 128, 3, 3, 6), (ONE + TWO, 20, 4, 0, 128, 4, 4, 0),
+    # ... one column block, int8
+    (TWO, 17, 0, 64, 2048, 3, 1, 8), (TWO, 24, 0, 64, 2048, 3, 1, 8), (TWO, 25, 0, 64, 2048, 4, 1, 0), (TWO, 24, 0, 64, 1984, 4, 1, 0), (ONE, 24, 0, 64, 2048, 4, 1, 0),
+    # 33 .. 48 rows, one, two and four column blocks
+    (ONE + TWO, 32, 0, 64, 512, 4, 1, 0), (ONE + TWO, 33, 0, 64, 512, 6, 1, 0), (ONE + TWO, 48, 0, 64, 512, 6, 1, 0), (ONE + TWO, 49, 0, 64, 512, 8, 1, 0),
+    (ONE, 40, 1, 4, 4096, 6, 2, 0), (ONE, 41, 1, 4, 4096, 8, 2, 0), (ONE, 48, 1, 4, 4160, 6, 2, 0), (TWO, 33, 1, 4, 4160, 8, 2, 0),
+    (ONE, 48, 2, 4, 512, 6, 4, 0), (TWO, 40, 2, 4, 512, 6, 4, 0), (TWO, 41, 2, 4, 512, 8, 4, 0), (ONE, 49, 2, 4, 512, 8, 4, 0),
+]
+
+
+@pytest.mark.parametrize("formats,M,per_cu,more,K,TH,NW,waves", EDGES)
+def test_the_choice_by_shape_at_its_edges(formats, M, per_cu, more, K, TH, NW, waves):
+    """Which form ran (TH 0, NW 0: not looked at), and that it is right: sums against float64 with the output's and a weight's rounding."""
+    import torch
+
+    from relax_amd import _lib, ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    N = 16 * (per_cu * torch.cuda.get_device_properties(0).multi_processor_count + more)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    for fmt in formats:
+        if fmt == "q4f16_1":
+            W = torch.randint(-(2**31), 2**31 - 1, (N, K // 8), device="cuda", dtype=torch.int32, generator=g)
+            S = (torch.rand(N, K // 32, device="cuda", generator=g) * 0.015 + 0.005).half()
+            w = (((W[:, :, None] >> torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)) & 15).flatten(1).double() - 7) * S.double().repeat_interleave(32, 1)
+            y = ops.q4g32_linear(W, S, x)
+        else:
+            bits = int(fmt[3])
+            q = torch.randint(-128, 128, (K, N * bits // 8), device="cuda", dtype=torch.int8, generator=g)
+            S = (torch.rand(N, device="cuda", generator=g) * 0.015 + 0.005).half()
+            codes = q.double() if bits == 8 else torch.stack([(q << 4) >> 4, q >> 4], -1).flatten(1).double()
+            w = codes.t() * S.double()[:, None]
+            y = ops.fpA_intB_gemm(x, ops.ft_preprocess_weight(q, 80, bits == 4), S, weight_nbit=bits)
+        torch.cuda.synchronize()
+        form = _lib.lib().wq_debug_small_batch_form()
+        got = (form >> 16, form >> 8 & 255, form & 255)
+        assert got[0] == TH and NW in (0, got[1]) and waves in (0, got[2]), (fmt, got)
+        exact, mass = x.double() @ w.t(), x.double().abs() @ w.abs().t()
+        assert ((y.double() - exact).abs() <= exact.abs() * 2.0**-11 + mass * 2.0**-11).all(), fmt
