@@ -177,7 +177,7 @@ def _spills(body: list[str]) -> list[str]:
 
 
 def check_held(asm_text: str) -> list[str]:
-    """Every ``held_gemm_kernel`` of the file: up to 252 of 256 registers, and no spill."""
+    """Every ``held_gemm_kernel`` of the file: up to all 256 registers, and no spill."""
     kernels = [body for name, body in _functions(asm_text) if "held_gemm_kernel" in name]
     return [e for body in kernels for e in _spills(body)] if kernels else ["no held_gemm_kernel found"]
 

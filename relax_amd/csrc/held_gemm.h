@@ -23,7 +23,12 @@
 // a load brings (8 columns, two halves) are the columns of one product as they come; results of a row half against the
 // other column half are sums of nothing and dropped.  With more rows two loads exchange halves first.
 // Activations of 4094 and more, infinite ones and NaN (16 times them is no number, or the sum that is taken off is not what
-// the products hold) take weights as the formats define them, rounded to fp16.
+// the products hold) take weights as the formats define them, rounded to fp16: in every row, in the wavefronts whose run holds
+// one.  The codes come as ever, but the vector unit makes the weights: with such an activation in every run N = 22016, K = 4096 takes
+// 19.1 / 20.7 / 23.9 us at M = 3 / 8 / 16 in place of 13.8 / 14.6 / 17.1, N = 28672, K = 8192 37.1 / 40.2 / 46.5 in place of
+// 27.9 / 29.9 / 36.3 (25.2 / 26.9 / 30.8 and 57.5 / 60.9 / 67.3 where those wavefronts fetched a tile's codes once more and
+// waited for them).  Rounded weights of a row's own would need two sets of operands, which the registers do not hold; with
+// rows at 1/16 of their factor a weight of exactly 0 leaves 2^-17 of its two products.
 #ifndef RELAX_AMD_CSRC_HELD_GEMM_H_
 #define RELAX_AMD_CSRC_HELD_GEMM_H_
 
@@ -58,7 +63,27 @@ struct HeldCfg {
   static constexpr int kLdsBytes = 2 * kScaleBytes + 16 * kPartBytes;
   // start values of the products in registers, where there is room
   static constexpr bool kKeep = FMT == kHeldQ4 && (kHalf ? PW <= 4 : PW <= 2);
+  // AutoGPTQ: the sums of activations, the same for all 16 columns, one per lane of 16 instead of all in every lane
+  static constexpr bool kPackSums = FMT == kHeldGptq && !kHalf && PW == 4;
 };
+
+// v of lane n of every 16
+__device__ __forceinline__ float row_broadcast(float v, int n) {
+#define WQ_ROW_BROADCAST(N) \
+  case N: return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + N /* row_newbcast */, 0xf, 0xf, false))
+  switch (n) {
+    WQ_ROW_BROADCAST(0);
+    WQ_ROW_BROADCAST(1);
+    WQ_ROW_BROADCAST(2);
+    WQ_ROW_BROADCAST(3);
+    WQ_ROW_BROADCAST(4);
+    WQ_ROW_BROADCAST(5);
+    WQ_ROW_BROADCAST(6);
+    default:
+    WQ_ROW_BROADCAST(7);
+  }
+#undef WQ_ROW_BROADCAST
+}
 
 template <HeldFormat FMT, int MODE, int PW, class Epilogue>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -83,9 +108,13 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
     w_off[p] = g < groups32 ? (uint32_t)((i & 7) * col_bytes + g * 16) : kOut;
   }
   const int s_col = FMT == kHeldQ4 ? groups32 * 2 : args.groups * 4;  // bytes of a column
-  uint32_t s_off[NL], s_to[NL];
+  // (whole wavefronts per column: the second column's lie a column further)
+  constexpr int NS = Cfg::kWords % 64 == 0 ? NL / 2 : NL;
+  uint32_t s_off[NS], s_to[NS];
+  auto scale_from = [&](int t) { return s_off[t % NS] + (uint32_t)(t / NS * s_col); };  // (beyond every descriptor stays there)
+  auto scale_to = [&](int t) { return s_to[t % NS] + (uint32_t)(t / NS * COL); };
 #pragma unroll
-  for (int t = 0; t < NL; ++t) {
+  for (int t = 0; t < NS; ++t) {
     const int idx = t * 64 + lane, c = idx / Cfg::kWords, d = idx % Cfg::kWords;  // column of the wavefront's two, word
     const bool held = c < 2 && (FMT == kHeldQ4 ? 2 * d < groups32 : 128 * d < K);
     const int at = FMT == kHeldQ4 ? 4 * d : 4 * (d / args.group128);
@@ -93,14 +122,19 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
     s_to[t] = (uint32_t)(min(2 * ks + c, 15) * COL + d * 4);
   }
   auto tile_rows = [&](int tile) { return max(min(16, N - tile * 16), 0); };  // 0 past the last tile: empty descriptors
+  struct Codes {
+    wq_rsrc_t half[2];  // columns 0 .. 7 and 8 .. 15 (those that are not there bring zeros)
+  };
   auto codes_at = [&](int tile) {
-    return wq_rsrc(args.W + (int64_t)min(tile, tiles - 1) * 16 * col_bytes, __builtin_amdgcn_readfirstlane(tile_rows(tile) * col_bytes));
+    const int rows = tile_rows(tile), first = __builtin_amdgcn_readfirstlane(min(rows, 8)), second = __builtin_amdgcn_readfirstlane(rows) - first;
+    const char* const from = args.W + (int64_t)min(tile, tiles - 1) * 16 * col_bytes;
+    return Codes{{wq_rsrc(from, first * col_bytes), wq_rsrc(from + first * col_bytes, second * col_bytes)}};
   };
   auto scales_at = [&](int tile) {
     return wq_rsrc(args.S + (int64_t)min(tile, tiles - 1) * 16 * s_col, __builtin_amdgcn_readfirstlane(tile_rows(tile) * s_col));
   };
-  auto request = [&](wq_rsrc_t from, int p, int h) {
-    return __builtin_amdgcn_raw_buffer_load_b128(from, w_off[p] + (uint32_t)(h * 8 * col_bytes), 0, 2 /* nt */);
+  auto request = [&](const Codes& from, int p, int h) {
+    return __builtin_amdgcn_raw_buffer_load_b128(from.half[h], w_off[p], 0, 2 /* nt */);
   };
 
   // ---- everything that the first tile needs is requested at once: activations, scales of two tiles, codes ----
@@ -128,20 +162,20 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
   auto fetch_scales = [&](int tile, uint32_t (&to)[NL]) {
     const wq_rsrc_t from = scales_at(tile);
 #pragma unroll
-    for (int t = 0; t < NL; ++t) to[t] = __builtin_amdgcn_raw_buffer_load_b32(from, s_off[t], 0, 0);
+    for (int t = 0; t < NL; ++t) to[t] = __builtin_amdgcn_raw_buffer_load_b32(from, scale_from(t), 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto put_scales = [&](int buf, const uint32_t (&from)[NL]) {
 #pragma unroll
     for (int t = 0; t < NL; ++t)
-      if ((t + 1) * 64 <= 2 * Cfg::kWords || t * 64 + lane < 2 * Cfg::kWords) *reinterpret_cast<uint32_t*>(lds + buf * Cfg::kScaleBytes + s_to[t]) = from[t];
+      if ((t + 1) * 64 <= 2 * Cfg::kWords || t * 64 + lane < 2 * Cfg::kWords) *reinterpret_cast<uint32_t*>(lds + buf * Cfg::kScaleBytes + scale_to(t)) = from[t];
   };
   int tile = blockIdx.x;
   fetch_scales(tile, sw0);
   fetch_scales(tile + grid, sw);
 #pragma unroll
   for (int a = 0; a < D; ++a) {
-    const wq_rsrc_t from = codes_at(tile + a * grid);
+    const Codes from = codes_at(tile + a * grid);
 #pragma unroll
     for (int l = 0; l < 2 * PW; ++l) {
       word[a][l] = request(from, l >> 1, l & 1);
@@ -151,7 +185,8 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
 
   // ---- activations as operands ----
   float4_t start[Cfg::kKeep ? PW : 1][NO];      // q4f16_1: what the products begin at
-  float4_t xsum[PW][HALF ? 1 : 2];              // AutoGPTQ: sums over 128 k
+  float4_t xsum[Cfg::kPackSums ? 1 : PW][HALF || Cfg::kPackSums ? 1 : 2];  // AutoGPTQ: sums over 128 k
+  if constexpr (Cfg::kPackSums) xsum[0][0] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
   const uint4_t kSeven = {0x80078007u, 0x80708070u, 0x80078007u, 0x80708070u};
   const uint4_t kOne = {0x00010001u, 0x00100010u, 0x00010001u, 0x00100010u};
   const half8_t weigh = __builtin_bit_cast(half8_t, FMT == kHeldQ4 ? kSeven : kOne);
@@ -179,13 +214,19 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
   build((half_t)16.0f);
   float zero = 0.0f;  // NaN where 16 times an activation is infinite or not a number
 #pragma unroll
-  for (int p = 0; p < PW; ++p)
+  for (int p = 0; p < PW; ++p) {
+    float4_t c;
 #pragma unroll
     for (int o = 0; o < NO; ++o) {
-      float4_t c;
       if constexpr (FMT == kHeldQ4) {
         c = sum_of(xb[p][o], kNull);
         if constexpr (Cfg::kKeep) start[p][o] = c;
+      } else if constexpr (Cfg::kPackSums) {
+        c = sum_of(xb[p][o], (o & 3) == 0 ? kNull : c);
+        if ((o & 3) == 3) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) xsum[0][0][e] = i == 2 * p + (o >> 2) ? c[e] : xsum[0][0][e];
+        }
       } else {
         c = sum_of(xb[p][o], (o & 3) == 0 ? kNull : xsum[p][o >> 2]);
         xsum[p][o >> 2] = c;
@@ -193,7 +234,10 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
 #pragma unroll
       for (int e = 0; e < 4; ++e) zero = fmaf(c[e], 0.0f, zero);
     }
-  const bool special = __builtin_amdgcn_ballot_w64(zero != 0.0f) != 0;
+  }
+  // (a number in a scalar register: as a lane mask it makes ways through the loop on which no loads are issued, and the compiler
+  // waits for all that are on their way)
+  const int special = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_ballot_w64(zero != 0.0f) != 0 ? 1 : 0);
   if (special) {
     fetch_x();
     build((half_t)1.0f);
@@ -219,7 +263,7 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
   auto scale_row = [&](int buf, int h) { return lds + buf * Cfg::kScaleBytes + (HALF ? 8 * h + (i & 7) : i) * COL; };
 
   constexpr int NA = HALF ? 2 : 1;
-  auto multiply = [&](wq_rsrc_t next, uint4_t (&word)[2 * PW], int buf, float4_t (&acc)[NA]) {
+  auto multiply = [&](const Codes& next, uint4_t (&word)[2 * PW], int buf, float4_t (&acc)[NA]) {
 #pragma unroll
     for (int p = 0; p < PW; ++p) {
       uint32_t w[2][4];
@@ -272,22 +316,23 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
         for (int h = 0; h < 2; ++h)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float v = fmaf(xsum[p][HALF ? 0 : h][e], -(float)sz[h].y, t[0][h][e]);
+            const float x = Cfg::kPackSums ? row_broadcast(xsum[0][0][e], 2 * p + h) : xsum[Cfg::kPackSums ? 0 : p][HALF || Cfg::kPackSums ? 0 : h][e];
+            const float v = fmaf(x, -(float)sz[h].y, t[0][h][e]);
             acc[HALF ? h : 0][e] = fmaf(v, (float)sz[h].x, acc[HALF ? h : 0][e]);
           }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  // the same with rounded weights, straight from memory
-  auto multiply_rounded = [&](wq_rsrc_t here, wq_rsrc_t next, uint4_t (&word)[2 * PW], int buf, float4_t (&acc)[NA]) {
+  // the same with rounded weights
+  auto multiply_rounded = [&](const Codes& next, uint4_t (&word)[2 * PW], int buf, float4_t (&acc)[NA]) {
 #pragma unroll
     for (int p = 0; p < PW; ++p) {
       uint32_t w[2][4];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const uint4_t l = request(here, p, h);
-        w[h][0] = l.x, w[h][1] = l.y, w[h][2] = l.z, w[h][3] = l.w;
+        take_words(word[2 * p + h], w[h]);
+        word[2 * p + h] = request(next, p, h);
       }
       arrange(w);
 #pragma unroll
@@ -308,11 +353,6 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
     }
 #pragma unroll
     for (int a = 0; a < NA; ++a) acc[a] *= 1.0f / 1048576.0f;
-#pragma unroll
-    for (int l = 0; l < 2 * PW; ++l) {
-      word[l] = request(next, l >> 1, l & 1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
   };
 
   // ---- the walk ----
@@ -325,13 +365,13 @@ void held_gemm_kernel(HeldArgs args, const half_t* __restrict__ X, half_t* __res
   meet();
   auto step = [&](int j, uint4_t (&word)[2 * PW]) {
     const int buf = j & 1;
-    const wq_rsrc_t next = codes_at(tile + D * grid);
+    const Codes next = codes_at(tile + D * grid);
     put_scales(buf ^ 1, sw);
     fetch_scales(tile + 2 * grid, sw);
     float4_t acc[NA];
 #pragma unroll
     for (int a = 0; a < NA; ++a) acc[a] = kNull;
-    if (special) multiply_rounded(codes_at(tile), next, word, buf, acc);
+    if (special) multiply_rounded(next, word, buf, acc);
     else multiply(next, word, buf, acc);
     // sums as [row][column] of the tile
     unsigned char* const set = parts + buf * 8 * PART;

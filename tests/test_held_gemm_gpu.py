@@ -9,6 +9,8 @@ pytestmark = pytest.mark.gpu
 # of a tile, and of more rounds over the CUs than tiles in flight, odd and even
 SHAPES = [(16, 64), (33, 576), (12300, 320), (8200, 2112), (130, 4096), (47, 4352), (259, 6208), (100, 8192)]
 CASES = [(M, N, K) for M in (3, 8, 9, 16) for N, K in SHAPES] + [(2, 70, 8256), (8, 260, 10240)]
+# two rounds of long runs, where the next tile's codes are requested into the registers that are being read
+CASES += [(M, 16 * 256 + 40, K) for M in (3, 8, 9, 16) for K in (4352, 6208, 8192)]
 
 
 def _codes(words):  # [N, K/8] -> [N, K]
