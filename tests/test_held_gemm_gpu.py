@@ -115,3 +115,39 @@ def test_the_choice_by_shape_at_its_edges(fmt, M, per_cu, more, K, held):
     assert (_lib.lib().wq_debug_small_batch_form() == 1) == held
     exact, mass = x.double() @ w.t(), x.double().abs() @ w.abs().t()
     assert ((y.double() - exact).abs() <= exact.abs() * 2.0**-11 + mass * (2.0**-17 if held else 2.0**-11)).all()
+
+
+@pytest.mark.parametrize("path", ["q4f16_1", "gptq", "list"])
+@pytest.mark.parametrize("M", [3, 16])
+def test_weights_that_are_exact(path, M):
+    """Scales that are powers of two: a weight is an fp16 number, so nothing but the result is rounded in any way of computing
+    it.  The sums may add a fifth of that rounding (squares add: 2 %); they are a tenth or less."""
+    from relax_amd import _lib, ops
+
+    N, K = 4096, 4096
+    g = torch.Generator(device="cuda").manual_seed(M)
+    words = lambda *s: torch.randint(-(2**31), 2**31 - 1, s, device="cuda", dtype=torch.int32, generator=g)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    _lib.lib().wq_debug_set_skinny_config(0, 0, 2)
+    try:
+        if path == "gptq":
+            qw, qz = words(K // 8, N), words(K // 128, N // 8)
+            s = torch.exp2(torch.randint(-9, -5, (K // 128, N), device="cuda", generator=g).float()).half()
+            y = ops.gptq_linear(ops.gptq_prepare(qw, qz, s, torch.arange(K, device="cuda", dtype=torch.int32) // 128), x)
+            w = (_codes(qw.t().contiguous()) - (_codes(qz) + 1).repeat_interleave(128, 0).t()) * s.double().repeat_interleave(128, 0).t()
+        else:
+            W, S = words(N, K // 8), torch.exp2(torch.randint(-9, -5, (N, K // 32), device="cuda", generator=g).float()).half()
+            w = (_codes(W) - 7) * S.double().repeat_interleave(32, 1)
+            if path == "list":
+                y = torch.zeros(M, N, device="cuda", dtype=torch.float16)
+                lin = ops.Q4G32GemvList([(W, S, x, y)], M=M)
+                lin.run()
+                lin.status()
+            else:
+                y = ops.q4g32_linear(W, S, x, kernel="small_batch")
+        torch.cuda.synchronize()
+    finally:
+        _lib.lib().wq_debug_set_skinny_config(0, 0, 0)
+    exact = x.double() @ w.t()
+    miss, rounding = (y.double() - exact).norm().item(), (exact.half().double() - exact).norm().item()
+    assert miss <= 1.02 * rounding, miss / rounding
