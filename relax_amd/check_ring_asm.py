@@ -42,9 +42,9 @@ import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ("q4g32_gemv_list.hip", "q4g32_batch_list.hip")
-# the tiled GEMMs (mfma_gemm_lds.h)
 # the kernel with activations in registers (held_gemm.h)
 HELD_SOURCES = ("gptq.hip", "q4g32_skinny.hip")
+# the tiled GEMMs (mfma_gemm_lds.h)
 DIRECT_LOAD_SOURCES = ("gemm_256.hip", "gptq.hip", "intb_gemm.hip", "q4g32_gemm.hip", "q4n32.hip")
 # kernels of SOURCES whose loads past the end have a scalar offset
 GUARDED_KERNELS = {"q4g32_batch_list.hip": ("q4g32_batch_list_kernel", "q4g32_batch_rows_kernel")}
